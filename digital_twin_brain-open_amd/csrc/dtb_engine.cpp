@@ -708,6 +708,29 @@ bool Instance::configure_run(int32_t t_steps, bool use_ou, hipStream_t s)
     return changed;
 }
 
+// Slots and strides of the next record; slots = false: one slot (records in
+// caller buffers).
+void Instance::layout_record(int64_t steps, bool freq, bool stat, bool slots)
+{
+    const uint32_t np = npop(), tiles = (n_ + kBlock - 1) / kBlock;
+    rec_slots_ = 1;
+    rec_cstride_ = np;
+    rec_sstride_ = np * kStatFields;
+    if (!slots)
+        return;
+    // whole 128-byte lines per slot
+    const uint32_t cs = (np + 31u) / 32u * 32u, ss = (np * kStatFields + 15u) / 16u * 16u;
+    const uint64_t slot_bytes = (uint64_t)steps * ((freq ? cs * sizeof(uint32_t) : 0) + (stat ? ss * sizeof(long long) : 0));
+    uint32_t k = 1;
+    while (k < kRecMaxSlots && (uint64_t)k * kRecTilesPerSlot * np < tiles && 2 * k * slot_bytes <= kRecMaxBytes)
+        k *= 2;
+    if (k > 1) {
+        rec_slots_ = k;
+        rec_cstride_ = cs;
+        rec_sstride_ = ss;
+    }
+}
+
 void Instance::begin_record(int64_t steps, bool freq, bool samples, uint32_t stat_mask, hipStream_t s)
 {
     if (samples && samples_.empty())
@@ -717,14 +740,29 @@ void Instance::begin_record(int64_t steps, bool freq, bool samples, uint32_t sta
     rec_freq_ = freq;
     rec_samples_ = samples;
     rec_stat_mask_ = stat_mask;
-    if (stat_mask != 0) {
-        rec_stat_.resize((size_t)steps * npop() * kStatFields);
+    auto allocate = [&](bool slots) {
+        layout_record(steps, freq, stat_mask != 0, slots);
+        if (stat_mask != 0) {
+            rec_stat_.resize(stat_slots() + (rec_slots_ > 1 ? (size_t)steps * npop() * kStatFields : 0));
+            rec_stat_.mutable_gpu_data();
+        }
+        if (freq) {
+            rec_counts_.resize(count_slots() + (rec_slots_ > 1 ? (size_t)steps * npop() : 0));
+            rec_counts_.mutable_gpu_data();
+        }
+    };
+    try {
+        allocate(true);
+    } catch (const Error &e) {
+        // no device memory for the slots: one per row, as without them
+        if (e.code != kOutOfMemory || rec_slots_ == 1)
+            throw;
+        allocate(false);
+    }
+    if (stat_mask != 0)
         DTB_HIP(hipMemsetAsync(rec_stat_.mutable_gpu_data(), 0, rec_stat_.size(), s));
-    }
-    if (freq) {
-        rec_counts_.resize((size_t)steps * npop());
+    if (freq)
         DTB_HIP(hipMemsetAsync(rec_counts_.mutable_gpu_data(), 0, rec_counts_.size(), s));
-    }
     if (samples) {
         const size_t m = (size_t)steps * samples_.size();
         rec_spike_.resize(m);
@@ -752,6 +790,7 @@ void Instance::begin_record_at(int64_t steps, bool freq, bool samples, uint32_t 
     rec_stat_mask_ = stat_mask;
     rec_ext_ = b;
     rec_ext_on_ = true;
+    layout_record(steps, freq, stat_mask != 0, false);
     if (stat_mask != 0)
         DTB_HIP(launch_zero_words(b.stat, (size_t)steps * npop() * kStatFields * sizeof(long long), s));
     if (freq)
@@ -775,8 +814,15 @@ void Instance::fetch_record(uint32_t *freq, uint8_t *spike, float *v, float *isy
     if (means != nullptr && rec_stat_mask_ != 0) {
         // stat_result.cpp:266-391 divides by the population size minus its
         // blocked neurons: mean = (double) sum * 2^-24 / count, as float.
-        std::vector<long long> sums(rec_stat_.count());
-        rec_stat_.download(sums.data(), sums.size(), s);
+        std::vector<long long> sums((size_t)rec_len_ * npop() * kStatFields);
+        if (rec_slots_ > 1) {
+            long long *out = rec_stat_.mutable_gpu_data() + stat_slots();
+            DTB_HIP(launch_fold_slots(rec_stat_.gpu_data(), rec_slots_, rec_sstride_, npop() * kStatFields,
+                                      (uint64_t)rec_len_, out, s));
+            DTB_HIP(hipMemcpyAsync(sums.data(), out, sums.size() * sizeof(long long), hipMemcpyDeviceToHost, s));
+        } else {
+            rec_stat_.download(sums.data(), sums.size(), s);
+        }
         DTB_HIP(hipStreamSynchronize(s));
         const uint32_t np = npop();
         std::vector<double> cnt(np, 0.0);
@@ -792,8 +838,16 @@ void Instance::fetch_record(uint32_t *freq, uint8_t *spike, float *v, float *isy
                         (float)((double)sums[((size_t)r * np + q) * kStatFields + k] * 0x1p-24 / cnt[q]);
         }
     }
-    if (freq && rec_freq_)
-        rec_counts_.download(freq, rec_counts_.count(), s);
+    if (freq && rec_freq_) {
+        if (rec_slots_ > 1) {
+            uint32_t *out = rec_counts_.mutable_gpu_data() + count_slots();
+            DTB_HIP(launch_fold_slots(rec_counts_.gpu_data(), rec_slots_, rec_cstride_, npop(), (uint64_t)rec_len_,
+                                      out, s));
+            DTB_HIP(hipMemcpyAsync(freq, out, (size_t)rec_len_ * npop() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        } else {
+            rec_counts_.download(freq, rec_counts_.count(), s);
+        }
+    }
     if (rec_samples_) {
         if (spike)
             rec_spike_.download(spike, rec_spike_.count(), s);
@@ -1002,6 +1056,9 @@ InstDev Instance::dev(uint32_t tile_base, bool gather, bool pull, uint32_t defer
     d.rec_stat = (rec_stat_mask_ != 0 && rec_len_ > 0) ? (rec_ext_on_ ? rec_ext_.stat : rec_stat_.mutable_gpu_data())
                                                        : nullptr;
     d.stat_mask = rec_stat_mask_;
+    d.rec_slots = rec_slots_;
+    d.rec_cstride = rec_cstride_;
+    d.rec_sstride = rec_sstride_;
     d.wave_ctr = counters_.mutable_gpu_data();
     d.step = step_.mutable_gpu_data();
     d.seed = seed_;

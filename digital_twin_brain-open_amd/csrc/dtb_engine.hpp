@@ -412,8 +412,14 @@ private:
     DataAllocator<PopDev> pops_;
     DataAllocator<int64_t> step_;                   // [2]
     DataAllocator<unsigned long long> counters_;   // per wave: events, spikes
+    // [steps][rec_slots_][stride], with more than one slot followed by the
+    // rows of the slots' sums ([npop], [npop][kStatFields])
     DataAllocator<uint32_t> rec_counts_;
-    DataAllocator<long long> rec_stat_;            // [steps][npop][kStatFields]
+    DataAllocator<long long> rec_stat_;
+    size_t count_slots() const { return (size_t)rec_len_ * rec_slots_ * rec_cstride_; }
+    size_t stat_slots() const { return (size_t)rec_len_ * rec_slots_ * rec_sstride_; }
+    uint32_t rec_slots_ = 1, rec_cstride_ = 0, rec_sstride_ = 0;
+    void layout_record(int64_t steps, bool freq, bool stat, bool slots);
     uint32_t rec_stat_mask_ = 0;
     DataAllocator<uint8_t> rec_spike_;
     DataAllocator<float> rec_v_, rec_isyn_, rec_iou_;
@@ -587,6 +593,7 @@ private:
     int count_layout_ = kLayoutAuto;       // requested layout
     uint32_t pass_k_ = kPassKDefault;      // synapses per lane in a binning pass
     uint32_t wfmt_ = kWeightF32;           // weight format of every instance in the tables, or kWeightAny
+    bool stat_ = false;                    // some instance in the tables records population statistics
     uint32_t queue_floor_ = 4096, queue_shift_ = 3;   // queue_capacity
     bool tuning_ = false;                  // autotune running: gather buffers are kept
     bool pull_on_ = true;                  // pull propagation where in-edges fit

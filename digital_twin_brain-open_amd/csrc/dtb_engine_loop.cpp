@@ -282,6 +282,7 @@ void Engine::rebuild()
     std::vector<SampleDev> samples;
     std::vector<SampleRecDev> recs;
     tile_base_.assign(insts_.size(), 0u);
+    stat_ = false;
     uint64_t total = 0;
     double coverage = 0.0;
     uint64_t pass_want = 0;   // split binning: pass-list entries for the queue instances
@@ -292,6 +293,7 @@ void Engine::rebuild()
             continue;
         const uint32_t idx = (uint32_t)table.size();
         tile_base_[slot] = (uint32_t)tiles.size();
+        stat_ = stat_ || p->stat_mask() != 0;
         fmt = fmt == kWeightAny + 1 || fmt == p->weight_format() ? p->weight_format() : kWeightAny;
         uint64_t qtotal = 0;   // this instance's queue slots per parity
         const auto &pb = p->pop_begin();
@@ -415,7 +417,7 @@ void Engine::launch_step_k()
 {
     launch_gather_k(par_);
     DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), ntiles_, d_insts_.gpu_data(), queues(), par_,
-                               d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, stream_));
+                               d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, stat_, stream_));
     DTB_HIP(launch_bin_kernel(d_tiles_.gpu_data(), bin_grid_, d_insts_.gpu_data(), queues(), par_,
                               d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, nullptr, nullptr, stream_));
 }
@@ -563,7 +565,8 @@ void Engine::run_timed(int64_t steps, float *ms_step)
                 DTB_HIP(launch_gather_timed(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par_, wfmt_, e[2], e[3],
                                             stream_));
             DTB_HIP(launch_step_kernel_timed(d_tiles_.gpu_data(), ntiles_, d_insts_.gpu_data(), queues(), par_,
-                                             d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, e[0], e[1], stream_));
+                                             d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, stat_, e[0], e[1],
+                                             stream_));
             if (pass_cap_ > 0)
                 DTB_HIP(launch_bin_kernel(d_tiles_.gpu_data(), bin_grid_, d_insts_.gpu_data(), queues(), par_,
                                           d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, e[4], e[5], stream_));

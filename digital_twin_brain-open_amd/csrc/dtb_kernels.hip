@@ -174,12 +174,29 @@ __device__ __forceinline__ float4 fold_delta(const float4 J, const float4 dc, co
     return r;
 }
 
+// v plus the value that DPP control kCtrl brings from another lane (0 where it
+// brings none), as two 32-bit moves and one 64-bit add.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ unsigned long long dpp_add_u64(unsigned long long v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, kCtrl, kRowMask, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), kCtrl, kRowMask, 0xf, false);
+    return v + (((unsigned long long)hi << 32) | lo);
+}
+
+// Sum over the 64 lanes (all of them active): an inclusive scan with DPP, no
+// LDS round trips; lane 63 holds the total.
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_xor(v, off, kWave);
-    return v;
+    v = dpp_add_u64<0x111, 0xf>(v);   // row_shr:1
+    v = dpp_add_u64<0x112, 0xf>(v);   // row_shr:2
+    v = dpp_add_u64<0x114, 0xf>(v);   // row_shr:4
+    v = dpp_add_u64<0x118, 0xf>(v);   // row_shr:8
+    v = dpp_add_u64<0x142, 0xa>(v);   // row_bcast:15
+    v = dpp_add_u64<0x143, 0xc>(v);   // row_bcast:31
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, kWave - 1);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), kWave - 1);
+    return ((unsigned long long)hi << 32) | lo;
 }
 
 // The LDS sums are channel-major: channel c of row i at acc[c * rows + i].
@@ -317,6 +334,40 @@ __device__ __forceinline__ float4 receptor_currents(const float4 g, const float4
     r.z = g.z * (vu.z - V) * J.z;
     r.w = g.w * (vu.w - V) * J.w;
     return r;
+}
+
+// Recorded sums of step row `row` (counts and statistics): the tile's slot.
+// Atomics on one 128-byte line are served one after the other (about 8 ns
+// each: a block of two populations and 469 tiles took 97 us per step with
+// one line per step, 9 us without statistics), so a record has rec_slots
+// slots of whole lines, a tile adding into slot (tile % slots); k_fold_slots
+// adds the slots up when the record is fetched.
+__device__ __forceinline__ uint32_t *rec_count_row(const InstDev &I, int64_t row, uint32_t begin)
+{
+    const size_t slot = (begin >> kTileBits) & (I.rec_slots - 1u);
+    return I.rec_counts + ((size_t)row * I.rec_slots + slot) * I.rec_cstride;
+}
+
+__device__ __forceinline__ long long *rec_stat_row(const InstDev &I, int64_t row, uint32_t begin)
+{
+    const size_t slot = (begin >> kTileBits) & (I.rec_slots - 1u);
+    return I.rec_stat + ((size_t)row * I.rec_slots + slot) * I.rec_sstride;
+}
+
+// The statistics selected by kmask of a tile whose neurons share one
+// population: the wave's sums into the tile's LDS sums (one global atomic
+// per tile and field follows, instead of one per wave).
+__device__ __forceinline__ void wave_tile_stats(unsigned long long *s_stat, bool valid, const long long *v,
+                                                uint32_t kmask, uint32_t lane)
+{
+#pragma unroll
+    for (int k = 0; k < kStatFields; ++k) {
+        if (!(kmask & (1u << k)))
+            continue;
+        const unsigned long long s = wave_sum_u64(valid ? (unsigned long long)v[k] : 0ull);
+        if (lane == 0)
+            atomicAdd(&s_stat[k], s);
+    }
 }
 
 // Adds this wave's per-population sums of the statistics selected by kmask
@@ -624,16 +675,24 @@ __device__ __forceinline__ void bin_pass(const uint32_t *__restrict__ col_all, c
 }
 
 
+// A tile's recorded sums in LDS (tiles of one population).
+struct TileRec {
+    unsigned long long stat[kStatFields];
+    uint32_t count;   // emitted neurons that population counts include
+};
+
 // One tile's step (the body of k_step).  kUniform: every neuron of the tile
 // has parameter class d.pcls - 1, so the parameter records are read once per
 // tile through the scalar unit instead of per lane.  K: synapses per lane in
 // a binning pass (a pass is 64 K synapses).
-template <bool kUniform, uint32_t K, uint32_t kFmt>
+// kStat: some instance records population statistics (their code costs
+// registers that a launch without them does not spend).
+template <bool kUniform, uint32_t K, uint32_t kFmt, bool kStat>
 __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__restrict__ tiles,
                                           const InstDev *__restrict__ insts, const QueueSet &qs, uint32_t par,
                                           StepCtl *__restrict__ ctl, unsigned long long *acc,
                                           unsigned long long *seg_dst, uint32_t *seg_room, long long *row_rb,
-                                          uint32_t *row_len, uint32_t &nrows, uint32_t &s_fit)
+                                          uint32_t *row_len, uint32_t &nrows, uint32_t &s_fit, TileRec &rec)
 {
     const InstDev &I = insts[d.inst];
     const uint32_t tid = threadIdx.x;
@@ -687,8 +746,15 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
     const bool over = !gat && cnt_raw > d.qcap;
     const bool pull = !gat && pull_on && (over || stamp == step + 1);
     clear_row(acc, tid);
-    if (tid == 0)
+    if (tid == 0) {
         nrows = 0u;
+        rec.count = 0u;
+    }
+    if (kStat && I.rec_stat != nullptr && tid < (uint32_t)kStatFields)
+        rec.stat[tid] = 0ull;
+    // Every neuron of the tile in one population (the usual case): its
+    // recorded sums meet in LDS first.
+    const bool one_pop = d.begin + d.count <= end_a;
     if (pull) {
         __syncthreads();
         // An overflowed queue is ignored: every emitted row then comes
@@ -744,8 +810,8 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
     // complete only now: J folded, V before this step's update); the V
     // statistic (after the update, below) to this one.
     const int64_t row_v = step - I.rec_step0;
-    const bool stat_valid = I.rec_stat != nullptr && active && !gp(I.blocked)[lc];
-    if (I.rec_stat != nullptr) {
+    const bool stat_valid = kStat && I.rec_stat != nullptr && active && !gp(I.blocked)[lc];
+    if (kStat && I.rec_stat != nullptr) {
         const uint32_t cf = current_fields(I.stat_mask);
         if (cf != 0u && row_v - 1 >= 0 && row_v - 1 < (int64_t)I.rec_len) {
             long long stv[kStatFields] = {};
@@ -755,7 +821,10 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             stv[3] = stat_q(rc.y);
             stv[4] = stat_q(rc.z);
             stv[5] = stat_q(rc.w);
-            wave_pop_stats(I.rec_stat + (size_t)(row_v - 1) * I.npop * kStatFields, stat_valid, p, stv, cf, lane);
+            if (one_pop)
+                wave_tile_stats(rec.stat, stat_valid, stv, cf, lane);
+            else
+                wave_pop_stats(rec_stat_row(I, row_v - 1, d.begin), stat_valid, p, stv, cf, lane);
         }
     }
     if (active) {
@@ -811,10 +880,13 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
         gp(I.iou)[li] = iou;
         st4(I.J, li, J);
     }
-    if (I.rec_stat != nullptr && (I.stat_mask & kStatV) && row_v >= 0 && row_v < (int64_t)I.rec_len) {
+    if (kStat && I.rec_stat != nullptr && (I.stat_mask & kStatV) && row_v >= 0 && row_v < (int64_t)I.rec_len) {
         long long stv[kStatFields] = {};
         stv[0] = stat_q(V);
-        wave_pop_stats(I.rec_stat + (size_t)row_v * I.npop * kStatFields, stat_valid, p, stv, 1u, lane);
+        if (one_pop)
+            wave_tile_stats(rec.stat, stat_valid, stv, 1u, lane);
+        else
+            wave_pop_stats(rec_stat_row(I, row_v, d.begin), stat_valid, p, stv, 1u, lane);
     }
 
     // Spike propagation (presynaptic_voltage.cpp:122-225): the tile's fired
@@ -876,24 +948,44 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             }
         }
         if (I.rec_counts != nullptr) {
-            // stat_result.cpp:161-206: one atomic per population present in
-            // the wave (blocked neurons are not counted)
+            // stat_result.cpp:161-206 (blocked neurons are not counted): one
+            // atomic per tile of one population, else one per population
+            // present in the wave
             const int64_t row = step - I.rec_step0;
             if (row >= 0 && row < (int64_t)I.rec_len) {
                 const bool counted = emit && !gp(I.blocked)[li];
                 unsigned long long rest = __ballot(counted);
+                if (one_pop) {
+                    if (lane == 0 && rest != 0ull)
+                        atomicAdd(&rec.count, (uint32_t)__popcll(rest));
+                    rest = 0ull;
+                }
                 while (rest != 0ull) {
                     const int src = __ffsll((long long)rest) - 1;
                     const uint32_t ps = __shfl(p, src, kWave);
                     const unsigned long long same = __ballot(counted && p == ps);
                     if ((int)lane == src)
-                        atomicAdd(&I.rec_counts[(size_t)row * I.npop + ps], (uint32_t)__popcll(same));
+                        atomicAdd(rec_count_row(I, row, d.begin) + ps, (uint32_t)__popcll(same));
                     rest &= ~same;
                 }
             }
         }
     }
     __syncthreads();
+    if (one_pop) {
+        // rec.count is nonzero only inside the recorded rows
+        if (tid == 0 && rec.count != 0u)
+            atomicAdd(rec_count_row(I, row_v, d.begin) + d.pop0, rec.count);
+        if (kStat && I.rec_stat != nullptr && tid < (uint32_t)kStatFields) {
+            // fields of the current step (V) and of the step before (I_syn)
+            const int64_t r = tid == 0 ? row_v : row_v - 1;
+            const uint32_t on = (I.stat_mask & kStatV ? 1u : 0u) | current_fields(I.stat_mask);
+            if (((on >> tid) & 1u) && r >= 0 && r < (int64_t)I.rec_len)
+                atomicAdd(reinterpret_cast<unsigned long long *>(rec_stat_row(I, r, d.begin)) +
+                              (size_t)d.pop0 * kStatFields + tid,
+                          rec.stat[tid]);
+        }
+    }
     const uint32_t nr = nrows;
     // A tile with many emitted rows (a synchronous volley) leaves them to
     // the consumers' pull: binning them would cost one reservation per
@@ -986,7 +1078,7 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
 // K: synapses per lane in a binning pass (the schedule; every K gives the
 // same results).  Eight waves per SIMD for K = 1, 2; K = 4's larger LDS
 // segment tables allow six.
-template <uint32_t K, uint32_t kFmt>
+template <uint32_t K, uint32_t kFmt, bool kStat>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ? 6 : 8))) void k_step(const TileDesc *__restrict__ tiles,
                                                  const InstDev *__restrict__ insts,
                                                  QueueSet qs,
@@ -1000,13 +1092,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ?
     __shared__ uint32_t row_len[kBlock];                  // and length
     __shared__ uint32_t nrows;
     __shared__ uint32_t s_fit;                            // split binning: passes in the list
+    __shared__ TileRec rec;
 
     const TileDesc d = tiles[blockIdx.x];
     if (d.pcls != 0u)
-        step_tile<true, K, kFmt>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit);
+        step_tile<true, K, kFmt, kStat>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit,
+                                 rec);
     else
-        step_tile<false, K, kFmt>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows,
-                                  s_fit);
+        step_tile<false, K, kFmt, kStat>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows,
+                                  s_fit, rec);
 }
 
 // Split binning: bins the passes that the k_step launch of parity `par`
@@ -1391,6 +1485,7 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
                                                       const InstDev *__restrict__ insts,
                                                       uint32_t par)
 {
+    __shared__ unsigned long long s_stat[kStatFields];
     const TileDesc d = tiles[blockIdx.x];
     const InstDev &I = insts[d.inst];
     const uint32_t cf = current_fields(I.stat_mask);
@@ -1423,7 +1518,35 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
         stv[5] = stat_q(rc.w);
         valid = !gp(I.blocked)[li];
     }
-    wave_pop_stats(I.rec_stat + (size_t)row * I.npop * kStatFields, valid, p, stv, cf, lane);
+    if (d.begin + d.count > I.pops[d.pop0].end) {   // more than one population
+        wave_pop_stats(rec_stat_row(I, row, d.begin), valid, p, stv, cf, lane);
+        return;
+    }
+    if (tid < (uint32_t)kStatFields)
+        s_stat[tid] = 0ull;
+    __syncthreads();
+    wave_tile_stats(s_stat, valid, stv, cf, lane);
+    __syncthreads();
+    if (tid < (uint32_t)kStatFields && ((cf >> tid) & 1u))
+        atomicAdd(reinterpret_cast<unsigned long long *>(rec_stat_row(I, row, d.begin)) +
+                      (size_t)d.pop0 * kStatFields + tid,
+                  s_stat[tid]);
+}
+
+// Adds up the slots of a record: out[row][i] = sum over slots of
+// in[row][slot][i], i < width (integers, so the order does not matter).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_fold_slots(const T *__restrict__ in, uint32_t slots, uint32_t stride,
+                                                       uint32_t width, uint64_t cells, T *__restrict__ out)
+{
+    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < cells; i += (uint64_t)gridDim.x * kBlock) {
+        const uint64_t row = i / width;
+        const T *p = in + row * slots * stride + (i - row * width);
+        T s = 0;
+        for (uint32_t k = 0; k < slots; ++k)
+            s += p[(size_t)k * stride];
+        out[i] = s;
+    }
 }
 
 // stat_result.cpp:393-433 (sampled spike flag, V, I_syn, i_ou) of the step
@@ -1499,7 +1622,11 @@ hipError_t with_kernel(uint32_t pass_k, uint32_t wfmt, F f)
 
 template <uint32_t K, uint32_t F>
 struct StepSel {
-    static auto get() { return k_step<K, F>; }
+    static auto get() { return k_step<K, F, false>; }
+};
+template <uint32_t K, uint32_t F>
+struct StepStatSel {
+    static auto get() { return k_step<K, F, true>; }
 };
 template <uint32_t K, uint32_t F>
 struct BinSel {
@@ -1507,25 +1634,30 @@ struct BinSel {
 };
 
 hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipStream_t stream)
+                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+                              hipStream_t stream)
 {
     if (ntiles == 0)
         return hipSuccess;
-    const hipError_t e = with_kernel<StepSel>(pass_k, wfmt, [&](auto kern) {
+    auto launch = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, tiles, insts, qs, par, ctl);
-    });
+    };
+    const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
+                              : with_kernel<StepSel>(pass_k, wfmt, launch);
     return e != hipSuccess ? e : hipGetLastError();
 }
 
 hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
-                                    hipEvent_t stop, hipStream_t stream)
+                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+                                    hipEvent_t start, hipEvent_t stop, hipStream_t stream)
 {
     if (ntiles == 0)
         return hipSuccess;
-    const hipError_t e = with_kernel<StepSel>(pass_k, wfmt, [&](auto kern) {
+    auto launch = [&](auto kern) {
         hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, start, stop, 0, tiles, insts, qs, par, ctl);
-    });
+    };
+    const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
+                              : with_kernel<StepSel>(pass_k, wfmt, launch);
     return e != hipSuccess ? e : hipGetLastError();
 }
 
@@ -1641,6 +1773,23 @@ hipError_t launch_stat_tail(const TileDesc *tiles, uint32_t ntiles, const InstDe
     hipLaunchKernelGGL(k_stat_tail, dim3(ntiles), dim3(kBlock), 0, stream, tiles, insts, par);
     return hipGetLastError();
 }
+
+template <typename T>
+hipError_t launch_fold_slots(const T *in, uint32_t slots, uint32_t stride, uint32_t width, uint64_t rows, T *out,
+                             hipStream_t stream)
+{
+    const uint64_t cells = rows * width;
+    if (cells == 0)
+        return hipSuccess;
+    const uint64_t nb = std::min<uint64_t>((cells + kBlock - 1) / kBlock, 4096);
+    hipLaunchKernelGGL(k_fold_slots<T>, dim3((uint32_t)nb), dim3(kBlock), 0, stream, in, slots, stride, width, cells,
+                       out);
+    return hipGetLastError();
+}
+template hipError_t launch_fold_slots<uint32_t>(const uint32_t *, uint32_t, uint32_t, uint32_t, uint64_t, uint32_t *,
+                                                hipStream_t);
+template hipError_t launch_fold_slots<long long>(const long long *, uint32_t, uint32_t, uint32_t, uint64_t,
+                                                 long long *, hipStream_t);
 
 hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_t nsamples,
                          const SampleRecDev *recs, uint32_t par, hipStream_t stream)

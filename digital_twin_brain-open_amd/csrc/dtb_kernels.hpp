@@ -8,15 +8,17 @@ namespace dtb {
 // One step of every tile, launch parity `par` (queue accumulation + fold +
 // OU + LIF + binning of the fired rows into queue set par ^ 1).
 // wfmt: the weight format of every instance in the tables, or kWeightAny
-// (each launch's kernels are specialised for it).
+// (each launch's kernels are specialised for it).  stat: some instance
+// records population statistics.
 hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipStream_t stream);
+                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+                              hipStream_t stream);
 
 // launch_step_kernel with `start` / `stop` recorded at the kernel's own
 // dispatch boundaries (kernel time without launch gaps).
 hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
-                                    hipEvent_t stop, hipStream_t stream);
+                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+                                    hipEvent_t start, hipEvent_t stop, hipStream_t stream);
 
 // Split binning: bins the passes listed by the k_step launch of parity
 // `par` (grid workgroups, each wave one pass at a time); nothing when the
@@ -61,6 +63,11 @@ hipError_t launch_settle(const TileDesc *tiles, uint32_t ntiles, const InstDev *
 // launch_materialize of the pending set); `par` = parity of the next launch.
 hipError_t launch_stat_tail(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, uint32_t par,
                             hipStream_t stream);
+
+// Sums of the slots of a record: out[rows][width] from in[rows][slots][stride].
+template <typename T>
+hipError_t launch_fold_slots(const T *in, uint32_t slots, uint32_t stride, uint32_t width, uint64_t rows, T *out,
+                             hipStream_t stream);
 
 // Samples of the step run by the k_step launch of parity `par`.
 hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_t nsamples,

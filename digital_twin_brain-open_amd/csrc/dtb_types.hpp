@@ -60,6 +60,11 @@ constexpr uint32_t kStatV = 1u;          // membrane potential (vmean)
 constexpr uint32_t kStatI = 2u;          // synaptic current (imean)
 constexpr uint32_t kStatReceptor = 4u;   // per-receptor currents (receptor imeans)
 constexpr int kStatFields = 6;           // V, I_syn, AMPA, NMDA, GABA_A, GABA_B
+// Slots of a record: one for every kRecTilesPerSlot tiles of a population (a
+// line then serves about 8 x 6 atomics of 8 ns per step), at most
+// kRecMaxSlots, and fewer where the slots of a record would pass kRecMaxBytes.
+constexpr uint32_t kRecTilesPerSlot = 8, kRecMaxSlots = 64;
+constexpr uint64_t kRecMaxBytes = (uint64_t)64 << 20;
 
 // Largest number of distinct parameter records kept as classes (2-byte class
 // index per neuron); beyond it the records are stored per neuron.
@@ -128,8 +133,11 @@ struct alignas(16) InstDev {
     int64_t *dstamp;            // [2]
     const PopDev *pops;         // [npop]
     // recording (device buffers, row = step - rec_step0)
-    uint32_t *rec_counts;       // [rec_len][npop] spikes per population
-    long long *rec_stat;        // [rec_len][npop][6] sums of V, I_syn, 4 receptor currents (x 2^24)
+    // Sums spread over rec_slots slots (a power of two) per row, a tile's
+    // into slot (tile % rec_slots); with one slot the strides are npop and
+    // npop * 6.
+    uint32_t *rec_counts;       // [rec_len][rec_slots][rec_cstride] spikes per population
+    long long *rec_stat;        // [rec_len][rec_slots][rec_sstride]: [npop][6] sums of V, I_syn, 4 receptor currents (x 2^24)
     // counters
     // per wave of 64 neurons: (synaptic events delivered = sum of fired
     // out-degrees, spikes emitted); each slot is updated only by the wave
@@ -153,7 +161,7 @@ struct alignas(16) InstDev {
     uint32_t fcap;              // rows per fired list
     uint32_t defer_min;         // pull: a tile with this many emitted rows defers them (0: never)
     uint32_t wfmt;              // weight pair format of w and cw
-    uint32_t pad2[3];
+    uint32_t rec_slots, rec_cstride, rec_sstride;   // layout of rec_counts and rec_stat
 };
 
 // Weight pair formats kept on the device (include/weights.hpp:14-21 and the

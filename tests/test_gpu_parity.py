@@ -862,3 +862,36 @@ def test_run_stream_equals_run(dtb, orc, gpu):
     ref, sim = run_oracle(orc, net, steps, seed, 1.5, vtrace=True)
     assert np.array_equal(whole["spike"], ref["raster"][:, ids])
     assert np.array_equal(bits(whole["vmemb"]), bits(ref["V"][:, ids]))
+
+
+@pytest.mark.parametrize("n", [4096, 20001])
+def test_recorded_sums_spread_over_slots(dtb, orc, gpu, n):
+    """Records of a block with many tiles per population (their sums are kept
+    in 2 and 8 slots and added up when fetched; the tile at the population
+    boundary holds two populations), with blocked neurons, against the oracle
+    and against the single-slot record of dtb_run_noalloc."""
+    seed, steps = 12, 60
+    net = dtb.gen_uniform(n, 60, seed=7)
+    net.props[::9, 1] = 1.0
+    kw = dict(freqs=True, vmean=True, imean=True, receptor_imean=True, npop=2)
+    res = []
+    for noalloc in (False, True):
+        blk = dtb.Block(net, delta_t=DT, seed=seed)
+        blk.update_ou_background_stimuli(blk.subblk_id, 4.0, 3.0, 0.2)
+        blk.run(20, freqs=False)
+        if noalloc:
+            blk.engine.run(0)
+        res.append(blk.engine.run_block(blk.inst, steps, noalloc=noalloc, **kw))
+        blk.engine.close()
+    on = orc.OracleNet.from_network(net, dt=DT, seed=seed)
+    on.set_ou(on.pop_ids, 3.0, 0.2, 4.0)
+    sim = orc.Sim(on, 32)
+    sim.run(20)
+    ref = sim.run(steps, pop_counts=True, stats=True)
+    assert ref["freq"].sum() > 0
+    for got in res:
+        assert np.array_equal(got["freq"], ref["freq"])
+        assert np.array_equal(bits(got["vmean"]), bits(ref["stat_means"][:, :, 0]))
+        assert np.array_equal(bits(got["imean"]), bits(ref["stat_means"][:, :, 1]))
+        for k in range(4):
+            assert np.array_equal(bits(got["receptor_imean"][k]), bits(ref["stat_means"][:, :, 2 + k])), k
