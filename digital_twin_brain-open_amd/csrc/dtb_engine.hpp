@@ -20,6 +20,7 @@
 #include <unordered_set>
 #include <vector>
 
+#include "dtb_kernels.hpp"
 #include "dtb_types.hpp"
 
 namespace dtb {
@@ -321,8 +322,13 @@ public:
     // defer_min > 0 with the in-edges built: pull propagation (a tile with
     // at least defer_min emitted rows defers them to the pull).
     InstDev dev(uint32_t tile_base, bool gather, bool pull, uint32_t defer_min);
+    // Descriptor of tile t for the step kernels; inst: the device address of
+    // the instance's descriptor `d`, idx its index; pop0: population of the
+    // tile's first neuron; qoff, qcap: its queue.
+    TileDesc tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, uint32_t idx, uint32_t pop0, uint64_t qoff,
+                       uint32_t qcap) const;
     // Distinct parameter records (classes); n() when stored per neuron.
-    uint32_t param_classes() const { return (uint32_t)pA_.count(); }
+    uint32_t param_classes() const { return (uint32_t)prm_.count(); }
     SampleRecDev sample_rec();
     // Synapses whose target lies in tile `tile` (2^kTileBits neurons): the
     // exact queue bound of the binning.
@@ -377,6 +383,10 @@ private:
     void derive_params(hipStream_t s);
     void derive_pops(hipStream_t s);     // population table (OU factors) only
     void init_state(hipStream_t s);
+    StateView state_view();
+    // Plain device arrays for `count` neurons' state (read_state,
+    // write_state), as many neurons as device memory holds, at most `count`.
+    struct StateStage;
     void count_tile_synapses(const NetworkHost &net);
     uint32_t find_pop(uint32_t brain_id) const;
 
@@ -394,13 +404,11 @@ private:
     std::vector<float> ou_mean_, ou_sigma_, ou_tau_;
     std::vector<uint32_t> samples_;
 
-    DataAllocator<float4> pA_, pB_, gU_, vU_, dec_;    // parameter records per class
+    DataAllocator<ParamRec> prm_;                      // parameter records per class
     DataAllocator<uint16_t> cls_;                      // parameter class per neuron
     bool dense_params_ = false;                        // one class per neuron
-    DataAllocator<float4> J_;
-    DataAllocator<uint8_t> blocked_, flag_;
-    DataAllocator<float> V_, iou_;
-    DataAllocator<int32_t> tcnt_;
+    DataAllocator<uint8_t> blocked_;
+    DataAllocator<unsigned char> state_;               // [ntiles][kStateBytes]
     DataAllocator<float4> dlt_;
     DataAllocator<unsigned long long> spill_;      // [2][n][4] Q23.40
     DataAllocator<QSyn> queue_;                    // [2][qslots_] + kQueuePrefetch
@@ -410,7 +418,7 @@ private:
     DataAllocator<uint8_t> w_;                     // [nsyn] weight pairs in format wfmt_
     uint32_t wfmt_ = kWeightF32;
     DataAllocator<PopDev> pops_;
-    DataAllocator<int64_t> step_;                   // [2]
+    DataAllocator<int64_t> step_;                   // [2] step index, [2] deferral stamps
     DataAllocator<unsigned long long> counters_;   // per wave: events, spikes
     // [steps][rec_slots_][stride], with more than one slot followed by the
     // rows of the slots' sums ([npop], [npop][kStatFields])
@@ -441,8 +449,7 @@ private:
     DataAllocator<uint32_t> crec_;        // [nsyn][grec_words] in-edges: key (source row | target in tile |
                                           // channel bit), weight pair bits
     DataAllocator<int64_t> cptr_;         // [ntiles + 1] first in-edge of each target tile
-    DataAllocator<unsigned long long> ebits_, dbits_;   // [2][ceil(n / 64)] emitted / deferred rows
-    DataAllocator<int64_t> dstamp_;       // [2] consuming step of deferred rows
+    DataAllocator<unsigned long long> bits_;   // [2][ntiles][kBitWords] emitted / deferred rows
     uint32_t gamma_calls_ = 0;            // gamma draw streams used
     std::vector<uint32_t> tile_cls_;      // per tile: 1 + shared parameter class, or 0
 };
@@ -610,6 +617,8 @@ private:
     DataAllocator<SampleDev> d_samples_;
     DataAllocator<SampleRecDev> d_recs_;
     DataAllocator<TileDesc> d_tiles_;
+    DataAllocator<QueueTile> d_qtiles_;
+    DataAllocator<QueueSet> d_queues_;     // queues() of the tables, as k_step reads it
     DataAllocator<uint32_t> d_qcnt_;       // count_words(2 * ntiles)
     DataAllocator<GroupDesc> d_groups_;    // gather groups of the gather instances
     uint32_t ngroups_ = 0;

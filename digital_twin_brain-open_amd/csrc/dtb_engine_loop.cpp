@@ -20,6 +20,8 @@ Engine::Engine(int device) : device_(device)
     DTB_HIP(hipStreamCreateWithFlags(&admit_stream_, hipStreamNonBlocking));
     d_ctl_.resize(1);
     d_ctl_.mutable_gpu_data();
+    d_queues_.resize(1);
+    d_queues_.mutable_gpu_data();
 }
 
 Engine::~Engine()
@@ -260,6 +262,8 @@ void Engine::drop_graphs()
 QueueSet Engine::queues()
 {
     QueueSet q{};
+    q.tile = d_qtiles_.gpu_data();
+    q.ctl = d_ctl_.mutable_gpu_data();
     q.count = d_qcnt_.mutable_gpu_data();
     q.ntiles = ntiles_;
     q.cshift = cshift_;
@@ -278,6 +282,22 @@ void Engine::rebuild()
     staged_.clear();
     std::vector<InstDev> table;
     std::vector<TileDesc> tiles;
+    std::vector<QueueTile> qtiles;
+    size_t ninst = 0, ntile_all = 0;
+    for (auto &p : insts_)
+        if (p) {
+            ++ninst;
+            ntile_all += (p->n() + kBlock - 1) / kBlock;
+        }
+    // The tables only grow (the kernels get their lengths as arguments), so
+    // a rebuild after the largest set so far allocates nothing.
+    auto grow = [](auto &buf, size_t n) {
+        if (buf.count() < std::max<size_t>(n, 1))
+            buf.resize(std::max<size_t>(n, 1));
+    };
+    grow(d_insts_, ninst);
+    tiles.reserve(ntile_all);
+    qtiles.reserve(ntile_all);
     std::vector<GroupDesc> groups;
     std::vector<SampleDev> samples;
     std::vector<SampleRecDev> recs;
@@ -296,21 +316,10 @@ void Engine::rebuild()
         stat_ = stat_ || p->stat_mask() != 0;
         fmt = fmt == kWeightAny + 1 || fmt == p->weight_format() ? p->weight_format() : kWeightAny;
         uint64_t qtotal = 0;   // this instance's queue slots per parity
-        const auto &pb = p->pop_begin();
-        uint32_t q = 0;
         for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
-            while (pb[q + 1] <= b)
-                ++q;
-            TileDesc d{};
-            d.inst = idx;
-            d.begin = b;
-            d.count = std::min<uint32_t>(kBlock, p->n() - b);
-            d.pop0 = q;
-            d.qcap = queue_capacity(p->tile_synapses(t));
-            d.pcls = p->tile_class(t);
-            d.qoff = qtotal;
-            qtotal += d.qcap;
-            tiles.push_back(d);
+            const uint32_t cap = queue_capacity(p->tile_synapses(t));
+            qtiles.push_back(QueueTile{qtotal, cap, 0u});
+            qtotal += cap;
         }
         // Each instance owns its queues (both parities and the read-ahead
         // slack), so instances of any size come and go without one large
@@ -330,6 +339,14 @@ void Engine::rebuild()
             try_pull(*p, stream_);
         const bool pl = !gat && pull_on_ && p->pull_built();
         table.push_back(p->dev(tile_base_[slot], gat, pl, defer_min_));
+        const auto &pb = p->pop_begin();
+        uint32_t q = 0;
+        for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
+            while (pb[q + 1] <= b)
+                ++q;
+            const QueueTile &qt = qtiles[tile_base_[slot] + t];
+            tiles.push_back(p->tile_desc(t, table.back(), d_insts_.gpu_data() + idx, idx, q, qt.off, qt.cap));
+        }
         recs.push_back(p->sample_rec());
         if (recs.back().nsample > 0) {
             const auto &ids = p->samples();
@@ -351,15 +368,9 @@ void Engine::rebuild()
     ntiles_ = (uint32_t)tiles.size();
     ngroups_ = (uint32_t)groups.size();
     nsamples_ = (uint32_t)samples.size();
-    // The tables only grow (the kernels get their lengths as arguments), so
-    // a rebuild after the largest set so far allocates nothing.
-    auto grow = [](auto &buf, size_t n) {
-        if (buf.count() < std::max<size_t>(n, 1))
-            buf.resize(std::max<size_t>(n, 1));
-    };
     grow(d_groups_, groups.size());
-    grow(d_insts_, table.size());
     grow(d_tiles_, tiles.size());
+    grow(d_qtiles_, qtiles.size());
     // sized by the samples set, recorded or not: a recording run then finds
     // the table built
     size_t sample_set = 0;
@@ -401,6 +412,9 @@ void Engine::rebuild()
         DTB_HIP(hipMemsetAsync(d_pcount_.mutable_gpu_data(), 0, d_pcount_.size(), stream_));
     d_insts_.upload(table.data(), table.size(), stream_);
     d_tiles_.upload(tiles.data(), tiles.size(), stream_);
+    d_qtiles_.upload(qtiles.data(), qtiles.size(), stream_);
+    const QueueSet qset = queues();
+    d_queues_.upload(&qset, 1, stream_);
     d_groups_.upload(groups.data(), groups.size(), stream_);
     d_samples_.upload(samples.data(), samples.size(), stream_);
     d_recs_.upload(recs.data(), recs.size(), stream_);
@@ -416,10 +430,8 @@ void Engine::launch_gather_k(uint32_t par)
 void Engine::launch_step_k()
 {
     launch_gather_k(par_);
-    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), ntiles_, d_insts_.gpu_data(), queues(), par_,
-                               d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, stat_, stream_));
-    DTB_HIP(launch_bin_kernel(d_tiles_.gpu_data(), bin_grid_, d_insts_.gpu_data(), queues(), par_,
-                              d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, nullptr, nullptr, stream_));
+    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), ntiles_, d_queues_.gpu_data(), par_, pass_k_, wfmt_, stat_, stream_));
+    DTB_HIP(launch_bin_kernel(bin_grid_, d_insts_.gpu_data(), queues(), par_, pass_k_, wfmt_, nullptr, nullptr, stream_));
 }
 
 void Engine::launch_aux()
@@ -564,12 +576,10 @@ void Engine::run_timed(int64_t steps, float *ms_step)
             if (ngroups_ > 0)
                 DTB_HIP(launch_gather_timed(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par_, wfmt_, e[2], e[3],
                                             stream_));
-            DTB_HIP(launch_step_kernel_timed(d_tiles_.gpu_data(), ntiles_, d_insts_.gpu_data(), queues(), par_,
-                                             d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, stat_, e[0], e[1],
+            DTB_HIP(launch_step_kernel_timed(d_tiles_.gpu_data(), ntiles_, d_queues_.gpu_data(), par_, pass_k_, wfmt_, stat_, e[0], e[1],
                                              stream_));
             if (pass_cap_ > 0)
-                DTB_HIP(launch_bin_kernel(d_tiles_.gpu_data(), bin_grid_, d_insts_.gpu_data(), queues(), par_,
-                                          d_ctl_.mutable_gpu_data(), pass_k_, wfmt_, e[4], e[5], stream_));
+                DTB_HIP(launch_bin_kernel(bin_grid_, d_insts_.gpu_data(), queues(), par_, pass_k_, wfmt_, e[4], e[5], stream_));
             par_ ^= 1u;
             launch_aux();
         }

@@ -71,9 +71,49 @@ __device__ __forceinline__ void st4(float4 *p, size_t i, const float4 v)
     *(__attribute__((address_space(1))) gfloat4 *)(p + i) = g;
 }
 
+// Memory that no launch reading it changes (descriptors, parameters, the step
+// index of the launch's parity), read through the scalar unit where the
+// address is uniform.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T *cp(const T *p)
+{
+    return (const __attribute__((address_space(4))) T *)p;
+}
+typedef const __attribute__((address_space(4))) InstDev *InstPtr;
+typedef const __attribute__((address_space(4))) TileDesc *TilePtr;
+typedef const __attribute__((address_space(4))) QueueSet *QueuePtr;
+
+__device__ __forceinline__ float4 ld4c(const float4 *p)
+{
+    const gfloat4 v = *(const __attribute__((address_space(4))) gfloat4 *)p;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// The same address, opaque to the compiler: what is read through it is read
+// again (scalar cache hits) instead of kept in scalar registers from an
+// earlier phase of the kernel.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T *again(
+    const __attribute__((address_space(4))) T *p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// Device-scope add on global memory (no flat access).
+template <typename T>
+__device__ __forceinline__ T gadd(T *p, T v)
+{
+    return __hip_atomic_fetch_add(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// (float)((double)q * 2^-40): the two halves meet in one rounded double, as
+// the conversion of q does; the scaling is exact on either side of the float
+// rounding (|q| >= 1 keeps the result normal).
 __device__ __forceinline__ float q40_to_f32(long long q)
 {
-    return (float)((double)q * 0x1p-40);
+    const double d = fma((double)(int32_t)(q >> 32), 0x1p32, (double)(uint32_t)q);
+    return (float)d * 0x1p-40f;
 }
 
 __device__ __forceinline__ unsigned long long f32_to_q40(float w)
@@ -147,10 +187,39 @@ __device__ __forceinline__ const void *w_row(const void *w, int64_t first, uint3
     return static_cast<const char *>(w) + (size_t)first * weight_bytes(fmt);
 }
 
-// Row of the parameter records that holds neuron li's parameters.
-__device__ __forceinline__ uint32_t param_index(const InstDev &I, uint32_t li)
+// Parameter record of neuron li.
+__device__ __forceinline__ const ParamRec *param_of(const InstDev &I, uint32_t li)
 {
-    return (li & I.pmask) + (uint32_t)gp(I.cls)[li];
+    return I.prm + ((li & I.pmask) + (uint32_t)gp(I.cls)[li]);
+}
+
+// Neuron i of a state block: field at byte offset kOff, one T per neuron.
+template <uint32_t kOff, typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T *st_at(unsigned char *block, uint32_t i)
+{
+    return (__attribute__((address_space(1))) T *)(gp(block) + (size_t)(i * (uint32_t)sizeof(T)) + kOff);
+}
+
+__device__ __forceinline__ float4 ld_J(unsigned char *block, uint32_t i)
+{
+    const gfloat4 v = *st_at<kStJ, gfloat4>(block, i);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+__device__ __forceinline__ void st_J(unsigned char *block, uint32_t i, const float4 v)
+{
+    gfloat4 g;
+    g.x = v.x;
+    g.y = v.y;
+    g.z = v.z;
+    g.w = v.w;
+    *st_at<kStJ, gfloat4>(block, i) = g;
+}
+
+// State block of the tile that holds neuron li.
+__device__ __forceinline__ unsigned char *block_of(const InstDev &I, uint32_t li)
+{
+    return I.state + (size_t)(li >> kTileBits) * kStateBytes;
 }
 
 // synaptic_current.cpp:39-43 in source order, no contraction.
@@ -208,6 +277,24 @@ __device__ __forceinline__ uint32_t acc_at(uint32_t row, uint32_t chan, uint32_t
     return chan * rows + row;
 }
 
+__device__ __forceinline__ QSyn ld_entry(const QSyn *q, size_t k)
+{
+    const auto p = gp(reinterpret_cast<const uint32_t *>(q)) + k * 3u;
+    QSyn e;
+    e.key = p[0];
+    e.w0 = __uint_as_float(p[1]);
+    e.w1 = __uint_as_float(p[2]);
+    return e;
+}
+
+__device__ __forceinline__ void st_entry(QSyn *q, size_t k, uint32_t key, float w0, float w1)
+{
+    const auto p = gp(reinterpret_cast<uint32_t *>(q)) + k * 3u;
+    p[0] = key;
+    p[1] = __float_as_uint(w0);
+    p[2] = __float_as_uint(w1);
+}
+
 // Adds the queued synapses of one tile into acc[4][256] (Q23.40, LDS): every
 // thread takes every 256th entry of the tile's queue (contiguous, so the
 // reads coalesce) and adds its weight pair with 64-bit integer LDS atomics,
@@ -217,7 +304,7 @@ __device__ __forceinline__ void accumulate_tile(unsigned long long *acc, const Q
                                                 const QSyn &pre, uint32_t npre, uint32_t tid)
 {
     for (uint32_t k = tid; k < cnt; k += kBlock) {
-        const QSyn e = (k < npre) ? pre : q[k];
+        const QSyn e = (k < npre) ? pre : ld_entry(q, k);
         const uint32_t row = e.key & 0xffu, c0 = (e.key & kQSynKind) ? 2u : 0u;
         atomicAdd(&acc[acc_at(row, c0, kBlock)], f32_to_q40(e.w0));
         atomicAdd(&acc[acc_at(row, c0 + 1u, kBlock)], f32_to_q40(e.w1));
@@ -235,10 +322,10 @@ __device__ __forceinline__ void clear_row(unsigned long long *acc, uint32_t tid)
 // Adds neuron li's spill accumulator of queue set `set` into the neuron's own
 // LDS sums (row tid of acc); `consume` clears it for the set's next use.
 // Called by the neuron's thread after the queue accumulation.
-__device__ __forceinline__ void take_spill(unsigned long long *acc, const InstDev &I, uint32_t set, uint32_t li,
-                                           uint32_t tid, bool consume)
+__device__ __forceinline__ void take_spill(unsigned long long *acc, unsigned long long *spill, uint32_t n,
+                                           uint32_t set, uint32_t li, uint32_t tid, bool consume)
 {
-    const auto s = gp(I.spill) + ((size_t)set * I.n + li) * 4u;
+    const auto s = gp(spill) + ((size_t)set * n + li) * 4u;
 #pragma unroll
     for (uint32_t c = 0; c < 4; ++c) {
         acc[acc_at(tid, c, kBlock)] += s[c];
@@ -250,9 +337,9 @@ __device__ __forceinline__ void take_spill(unsigned long long *acc, const InstDe
 // Pull propagation: adds into acc (the tile's Q23.40 LDS sums) the weight
 // pairs of tile t's in-edges whose source row was emitted by the launch that
 // filled set `set`: every emitted row (`all`: the queue overflowed and is
-// ignored) or only the rows of tiles that deferred them (dbits).  An in-edge
+// ignored) or only the rows of tiles that deferred them.  An in-edge
 // is one record (key, then the weight pair's bits: kW words), read
-// coalesced; the source's bit comes from a per-wave bitmap (n / 8 bytes,
+// coalesced; the source's bit comes from the per-tile bitmaps (n / 4 bytes,
 // cache resident; read as 32-bit words), so a batch is two dependent loads
 // (records, bit words); each thread keeps kPullItems in-edges in flight.
 // Called by the whole workgroup.
@@ -264,7 +351,7 @@ __device__ __forceinline__ void pull_loop(unsigned long long *acc, const uint32_
     constexpr uint32_t U = kPullItems;
     constexpr uint32_t kW = kFmt == kWeightF32 ? 3u : 2u;   // grec_words(kFmt)
     // uniform bases and 32-bit byte offsets (a tile's in-edges span less
-    // than 4 GB; the bitmap less than 1 MB): one VGPR per address
+    // than 4 GB; the bitmaps less than 3 MB): one VGPR per address
     using gbyte = const __attribute__((address_space(1))) unsigned char;
     gbyte *rb = reinterpret_cast<gbyte *>(gp(rec));
     gbyte *bb = reinterpret_cast<gbyte *>(gp(reinterpret_cast<const uint32_t *>(bits)));
@@ -283,7 +370,7 @@ __device__ __forceinline__ void pull_loop(unsigned long long *acc, const uint32_
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u)
             bw[u] = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t *>(
-                bb + ((kv[u] & kPullRowMask) >> 5) * 4u);
+                bb + ((kv[u] & kPullRowMask) >> kTileBits) * (kBitWords * 8u) + ((kv[u] >> 3) & 0x1cu));
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
             if (k0 + u * kBlock < len && ((bw[u] >> (kv[u] & 31u)) & 1u) != 0u) {
@@ -296,17 +383,13 @@ __device__ __forceinline__ void pull_loop(unsigned long long *acc, const uint32_
     }
 }
 
-// Not inlined: the pull is the rare path (volleys, overflowing queues), and
-// as a call it keeps its registers out of the step kernel's budget.  Its
-// registers are the ones the caller must keep free across the call, so a
-// kernel specialised for one weight format calls the loop of that format
-// only (kFmt; kWeightAny: the instance's format at run time).
-template <uint32_t kFmt>
-__device__ __attribute__((noinline)) void pull_tile(unsigned long long *acc, const InstDev &I, uint32_t set,
-                                                    uint32_t t, bool all, uint32_t tid)
+// The pull of tile t; kFmt: the launch's weight format (kWeightAny: the
+// instance's, at run time).
+template <uint32_t kFmt, typename Inst>
+__device__ __forceinline__ void pull_tile(unsigned long long *acc, const Inst &I, uint32_t set, uint32_t t, bool all,
+                                          uint32_t tid)
 {
-    const size_t nw = (I.n + kWave - 1) / kWave;
-    const unsigned long long *bits = (all ? I.ebits : I.dbits) + (size_t)set * nw;
+    const unsigned long long *bits = I.bits + (size_t)set * I.ntiles * kBitWords + (all ? 0u : 4u);
     const int64_t b = gp(I.cptr)[t];
     const uint32_t len = (uint32_t)(gp(I.cptr)[t + 1] - b);   // a tile has fewer than 2^32 in-edges
     const uint32_t fmt = kFmt != kWeightAny ? kFmt : I.wfmt;
@@ -342,13 +425,15 @@ __device__ __forceinline__ float4 receptor_currents(const float4 g, const float4
 // one line per step, 9 us without statistics), so a record has rec_slots
 // slots of whole lines, a tile adding into slot (tile % slots); k_fold_slots
 // adds the slots up when the record is fetched.
-__device__ __forceinline__ uint32_t *rec_count_row(const InstDev &I, int64_t row, uint32_t begin)
+template <typename Inst>
+__device__ __forceinline__ uint32_t *rec_count_row(const Inst &I, int64_t row, uint32_t begin)
 {
     const size_t slot = (begin >> kTileBits) & (I.rec_slots - 1u);
     return I.rec_counts + ((size_t)row * I.rec_slots + slot) * I.rec_cstride;
 }
 
-__device__ __forceinline__ long long *rec_stat_row(const InstDev &I, int64_t row, uint32_t begin)
+template <typename Inst>
+__device__ __forceinline__ long long *rec_stat_row(const Inst &I, int64_t row, uint32_t begin)
 {
     const size_t slot = (begin >> kTileBits) & (I.rec_slots - 1u);
     return I.rec_stat + ((size_t)row * I.rec_slots + slot) * I.rec_sstride;
@@ -455,7 +540,7 @@ __device__ __forceinline__ void count_over(StepCtl *__restrict__ ctl, uint32_t o
 template <uint32_t K, uint32_t kFmt>
 __device__ __forceinline__ void bin_pass_serial(const uint32_t *__restrict__ col_all, const void *w_all, uint32_t wfmt,
                                         int64_t row_begin, uint32_t len, uint32_t c0, uint32_t tile_base,
-                                        const TileDesc *__restrict__ tiles, uint32_t *__restrict__ qcnt, size_t qset, uint32_t cshift,
+                                        const QueueTile *__restrict__ qtab, uint32_t *__restrict__ qcnt, size_t qset, uint32_t cshift,
                                         QSyn *__restrict__ queue, unsigned long long *__restrict__ spill,
                                         StepCtl *__restrict__ ctl, unsigned long long *seg_dst, uint32_t *seg_room,
                                         uint32_t lane)
@@ -508,11 +593,11 @@ __device__ __forceinline__ void bin_pass_serial(const uint32_t *__restrict__ col
             if (j < len && tl[k] != nx) {
                 const uint32_t tg = tile_base + tl[k];
                 const uint32_t n = j + 1u - open;
-                const uint32_t base = atomicAdd(&qcnt[count_slot(qset + tg, cshift)], n);
-                const TileDesc td = tiles[tg];
-                const uint32_t room = td.qcap > base ? min(n, td.qcap - base) : 0u;
+                const uint32_t base = gadd(&qcnt[count_slot(qset + tg, cshift)], n);
+                const QueueTile td = qtab[tg];
+                const uint32_t room = td.cap > base ? min(n, td.cap - base) : 0u;
                 over += n - room;
-                seg_dst[open - c0] = td.qoff + base;
+                seg_dst[open - c0] = td.off + base;
                 seg_room[open - c0] = room;
             }
         }
@@ -526,15 +611,12 @@ __device__ __forceinline__ void bin_pass_serial(const uint32_t *__restrict__ col
             if (j < len) {
                 const uint32_t at = j - st[k];
                 if (at < seg_room[st[k] - c0]) {
-                    QSyn e;
-                    e.key = (cv[k] & 0xffu) | ((cv[k] & kKindBit) ? kQSynKind : 0u);
-                    e.w0 = wv[k].x;
-                    e.w1 = wv[k].y;
-                    queue[seg_dst[st[k] - c0] + at] = e;
+                    st_entry(queue, seg_dst[st[k] - c0] + at,
+                             (cv[k] & 0xffu) | ((cv[k] & kKindBit) ? kQSynKind : 0u), wv[k].x, wv[k].y);
                 } else if (spill != nullptr) {
                     unsigned long long *a = spill + (size_t)(cv[k] & kColMask) * 4u + ((cv[k] & kKindBit) ? 2u : 0u);
-                    atomicAdd(a, f32_to_q40(wv[k].x));
-                    atomicAdd(a + 1, f32_to_q40(wv[k].y));
+                    gadd(a, f32_to_q40(wv[k].x));
+                    gadd(a + 1, f32_to_q40(wv[k].y));
                 }
             }
         }
@@ -564,7 +646,7 @@ __device__ __forceinline__ void bin_pass_serial(const uint32_t *__restrict__ col
 template <uint32_t K, uint32_t kFmt>
 __device__ __forceinline__ void bin_pass(const uint32_t *__restrict__ col_all, const void *w_all, uint32_t wfmt,
                                         int64_t row_begin, uint32_t len, uint32_t c0, uint32_t tile_base,
-                                        const TileDesc *__restrict__ tiles, uint32_t *__restrict__ qcnt, size_t qset, uint32_t cshift,
+                                        const QueueTile *__restrict__ qtab, uint32_t *__restrict__ qcnt, size_t qset, uint32_t cshift,
                                         QSyn *__restrict__ queue, unsigned long long *__restrict__ spill,
                                         StepCtl *__restrict__ ctl, unsigned long long *seg_dst, uint32_t *seg_room,
                                         uint32_t lane)
@@ -632,9 +714,9 @@ __device__ __forceinline__ void bin_pass(const uint32_t *__restrict__ col_all, c
         qcap[k] = 0u;
         if (end[k]) {
             const uint32_t tg = tile_base + tl[k];
-            base[k] = atomicAdd(&qcnt[count_slot(qset + tg, cshift)], j0 + k + 1u - st[k]);
-            qoff[k] = tiles[tg].qoff;
-            qcap[k] = tiles[tg].qcap;
+            base[k] = gadd(&qcnt[count_slot(qset + tg, cshift)], j0 + k + 1u - st[k]);
+            qoff[k] = qtab[tg].off;
+            qcap[k] = qtab[tg].cap;
         }
     }
     uint32_t over = 0;   // synapses of this lane's segments past their queue's capacity
@@ -657,15 +739,12 @@ __device__ __forceinline__ void bin_pass(const uint32_t *__restrict__ col_all, c
         if (ok[k]) {
             const uint32_t at = j0 + k - st[k];
             if (at < seg_room[st[k] - c0]) {
-                QSyn e;
-                e.key = (cv[k] & 0xffu) | ((cv[k] & kKindBit) ? kQSynKind : 0u);
-                e.w0 = wv[k].x;
-                e.w1 = wv[k].y;
-                queue[seg_dst[st[k] - c0] + at] = e;
+                st_entry(queue, seg_dst[st[k] - c0] + at,
+                         (cv[k] & 0xffu) | ((cv[k] & kKindBit) ? kQSynKind : 0u), wv[k].x, wv[k].y);
             } else if (spill != nullptr) {
                 unsigned long long *a = spill + (size_t)(cv[k] & kColMask) * 4u + ((cv[k] & kKindBit) ? 2u : 0u);
-                atomicAdd(a, f32_to_q40(wv[k].x));
-                atomicAdd(a + 1, f32_to_q40(wv[k].y));
+                gadd(a, f32_to_q40(wv[k].x));
+                gadd(a + 1, f32_to_q40(wv[k].y));
             }
         }
     }
@@ -681,141 +760,159 @@ struct TileRec {
     uint32_t count;   // emitted neurons that population counts include
 };
 
-// One tile's step (the body of k_step).  kUniform: every neuron of the tile
-// has parameter class d.pcls - 1, so the parameter records are read once per
-// tile through the scalar unit instead of per lane.  K: synapses per lane in
-// a binning pass (a pass is 64 K synapses).
-// kStat: some instance records population statistics (their code costs
-// registers that a launch without them does not spend).
-template <bool kUniform, uint32_t K, uint32_t kFmt, bool kStat>
-__device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__restrict__ tiles,
-                                          const InstDev *__restrict__ insts, const QueueSet &qs, uint32_t par,
-                                          StepCtl *__restrict__ ctl, unsigned long long *acc,
-                                          unsigned long long *seg_dst, uint32_t *seg_room, long long *row_rb,
-                                          uint32_t *row_len, uint32_t &nrows, uint32_t &s_fit, TileRec &rec)
+// Neuron state of one lane.
+struct Lane {
+    float4 J;
+    float V, iou;
+    int32_t t;
+    uint32_t fl;
+};
+
+__device__ __forceinline__ Lane load_lane(unsigned char *state, uint32_t i)
 {
-    const InstDev &I = insts[d.inst];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = __lane_id();
-    const uint32_t w = tid / kWave;
-    const bool gat = I.segidx != nullptr;   // gather propagation: k_gather wrote the delta into dlt
-    const QSyn *__restrict__ q_in = I.queue + (size_t)par * I.qslots;
-    const size_t cslot_in = count_slot((size_t)par * qs.ntiles + blockIdx.x, qs.cshift);
-    QSyn *__restrict__ q_out = I.queue + (size_t)(par ^ 1u) * I.qslots;
+    Lane x;
+    x.J = ld_J(state, i);
+    x.V = *st_at<kStV, float>(state, i);
+    x.t = *st_at<kStT, int32_t>(state, i);
+    x.fl = *st_at<kStFlag, uint8_t>(state, i);
+    x.iou = *st_at<kStIou, float>(state, i);
+    return x;
+}
 
-    // Loads are issued in order of their dependence chains, before anything
-    // waits on them: the queue count and step index, the parameter class,
-    // the neuron state, the parameter records (need the class), the queue
-    // head, the deferral stamp.
-    const uint32_t cnt_raw = qs.count[cslot_in];
-    const int64_t step = gp(I.step)[par];
-    const bool pull_on = I.crec != nullptr;
-    const uint32_t li = d.begin + tid;
-    const bool active = tid < d.count;
-    const uint32_t lc = active ? li : d.begin;   // in-range index for idle lanes
-    // A tile whose neurons share one parameter class (the usual case: a
-    // population spans many tiles) reads its records without the class load.
-    const uint32_t c = kUniform ? d.pcls - 1u : (lc & I.pmask) + (uint32_t)gp(I.cls)[lc];
-    float4 J = ld4(I.J, lc);
-    float V = gp(I.V)[lc];
-    int32_t t = gp(I.tcnt)[lc];
-    uint32_t fl = gp(I.flag)[lc];
-    float iou = gp(I.iou)[lc];
-    float4 pa = ld4(I.pA, c);
-    float4 pb = ld4(I.pB, c);
-    float4 g = ld4(I.gU, c);
-    float4 vu = ld4(I.vU, c);
-    float4 dc = ld4(I.dec, c);
-    // The ends of the tile's first two populations (a tile rarely spans
-    // more) arrive with the state, not after the fold.
-    const uint32_t pop_hi = min(d.pop0 + 1u, I.npop - 1u);
-    uint32_t end_a = I.pops[d.pop0].end;
-    uint32_t end_b = I.pops[pop_hi].end;
-    // The queue is complete when the launch starts; entries past the count
-    // are ignored (the queue buffer has kQueuePrefetch slots of slack at its
-    // end, so the read needs no branch).
-    QSyn head{};
-    float4 dl = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (gat)
-        dl = ld4(I.dlt, lc);
-    else
-        head = q_in[d.qoff + min(tid, kQueuePrefetch - 1u)];
-    const int64_t stamp = pull_on ? gp(I.dstamp)[par] : 0;
-    // A tile pulls (the pull propagation, never with gather) when its queue
-    // overflowed or rows were deferred into this set: rare (volleys).
-    const bool over = !gat && cnt_raw > d.qcap;
-    const bool pull = !gat && pull_on && (over || stamp == step + 1);
-    clear_row(acc, tid);
-    if (tid == 0) {
-        nrows = 0u;
-        rec.count = 0u;
-    }
-    if (kStat && I.rec_stat != nullptr && tid < (uint32_t)kStatFields)
-        rec.stat[tid] = 0ull;
-    // Every neuron of the tile in one population (the usual case): its
-    // recorded sums meet in LDS first.
-    const bool one_pop = d.begin + d.count <= end_a;
-    if (pull) {
-        __syncthreads();
-        // An overflowed queue is ignored: every emitted row then comes
-        // through the in-edges.
-        accumulate_tile(acc, q_in + d.qoff, over ? 0u : cnt_raw, QSyn{}, 0u, tid);
-        pull_tile<kFmt>(acc, I, par, d.begin >> kTileBits, over, tid);
-        if (tid == 0)
-            atomicAdd(&ctl->slot[blockIdx.x & (kCtlSlots - 1u)].pulled, 1ull);
-        // loaded again, so that nothing loaded above is live across the call
-        J = ld4(I.J, lc);
-        V = gp(I.V)[lc];
-        t = gp(I.tcnt)[lc];
-        fl = gp(I.flag)[lc];
-        iou = gp(I.iou)[lc];
-        pa = ld4(I.pA, c);
-        pb = ld4(I.pB, c);
-        g = ld4(I.gU, c);
-        vu = ld4(I.vU, c);
-        dc = ld4(I.dec, c);
-        end_a = I.pops[d.pop0].end;
-        end_b = I.pops[pop_hi].end;
-        dl = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // (no gather here)
+// The tile's parameter record: of the tile (scalar loads), or of the lane's
+// class.
+template <bool kUniform>
+__device__ __forceinline__ ParamRec load_params(TilePtr d, uint32_t i)
+{
+    ParamRec r;
+    if (kUniform) {
+        r.a = ld4c(&d->prm->a);
+        r.b = ld4c(&d->prm->b);
+        r.g = ld4c(&d->prm->g);
+        r.v = ld4c(&d->prm->v);
+        r.d = ld4c(&d->prm->d);
     } else {
-        const uint32_t cnt = gat ? 0u : min(cnt_raw, d.qcap);
-        __syncthreads();
-        accumulate_tile(acc, q_in + d.qoff, cnt, head, kQueuePrefetch, tid);
+        const float4 *p = &d->prm[gp(d->cls)[i]].a;
+        r.a = ld4(p, 0);
+        r.b = ld4(p, 1);
+        r.g = ld4(p, 2);
+        r.v = ld4(p, 3);
+        r.d = ld4(p, 4);
     }
-    __syncthreads();
-    if (!pull_on && over && active)
-        take_spill(acc, I, par, li, tid, true);   // synapses past the queue's capacity
-    if (tid == 0)
-        qs.count[cslot_in] = 0u;   // this launch consumed the queue
-    if (d.begin == 0 && tid == 0)
-        gp(I.step)[par ^ 1u] = step + 1;   // no tile of this launch reads this slot
+    return r;
+}
 
+// LIF update of one substep (membrane_voltage.cpp:114-195): a.z = dt_sub / C.
+__device__ __forceinline__ bool lif(Lane &x, uint32_t &f, const ParamRec &q, float Ieff)
+{
+    float cvi = q.b.x * (q.a.w - x.V);
+    cvi = cvi + Ieff;
+    cvi = cvi + q.b.y;
+    const float Vn = x.V + q.a.z * cvi;
+    const bool held = x.t < 0;
+    const bool spk = !held && Vn >= q.a.y;
+    const float Vh = f ? q.a.x : x.V;   // refractory: reset once after the spike
+    x.V = held ? Vh : (spk ? q.a.y : Vn);
+    x.t = held ? x.t + 1 : (spk ? 1 - __float_as_int(q.b.w) : x.t);
+    f = spk ? 1u : 0u;
+    return spk;
+}
+
+// One OU step (extern_stimuli.cpp:39-112).
+__device__ __forceinline__ float ou_step(float iou, float mu, float f1, float f2s, float xi)
+{
+    return iou + (f1 * (mu - iou) + f2s * xi);
+}
+
+// Every substep of a tile whose neurons share one population, with one
+// substep per step (the usual case: straight-line code, the OU factors in
+// scalar registers).  Returns whether the lane's neuron emitted.
+__device__ __forceinline__ bool step_lane_one(TilePtr d, Lane &x, const ParamRec &q, float isyn, uint32_t li,
+                                              int64_t step)
+{
+    uint32_t f = x.fl & kFlagSpike;
+    float Ieff = isyn;
+    if (d->flags & kTileOuOn) {
+        x.iou = ou_step(x.iou, d->mu, d->f1, d->f2s, ou_normal(d->seed, li, (uint64_t)step));
+        Ieff = isyn + x.iou;
+    }
+    bool emit = lif(x, f, q, Ieff);
+    if (!(d->flags & kTileOu))   // spike.cpp:55-62: f_rec = f | (U < noise_rate)
+        emit = f || (noise_uniform(d->seed, li, (uint64_t)step) < q.b.z);
+    x.fl = f;
+    return emit;
+}
+
+// The same for any number of substeps and populations: p is the lane's
+// population.
+__device__ __forceinline__ bool step_lane_any(TilePtr d, InstPtr I, Lane &x, const ParamRec &q, float isyn,
+                                              uint32_t li, int64_t step, uint32_t p)
+{
+    const auto pop = gp(I->pops) + p;
+    const float mu = pop->mu, f1 = pop->f1, f2s = pop->f2s;
+    const bool ou = (d->flags & kTileOu) != 0u && pop->ou_on != 0u;
+    const int32_t T = I->t_steps;
+    uint32_t f = x.fl & kFlagSpike;
     bool emit = false;
-    uint32_t p = d.pop0;
+    for (int32_t s = 0; s < T; ++s) {
+        float Ieff = isyn;
+        if (ou) {
+            x.iou = ou_step(x.iou, mu, f1, f2s, ou_normal(d->seed, li, (uint64_t)step * (uint64_t)T + (uint64_t)s));
+            Ieff = isyn + x.iou;
+        }
+        emit = lif(x, f, q, Ieff) || emit;
+        if (s < T - 1) {
+            x.J.x = x.J.x * q.d.x;
+            x.J.y = x.J.y * q.d.y;
+            x.J.z = x.J.z * q.d.z;
+            x.J.w = x.J.w * q.d.w;
+            isyn = syn_current(q.g, q.v, x.J, x.V);
+        }
+    }
+    if (!(d->flags & kTileOu))
+        emit = f || (noise_uniform(d->seed, li, (uint64_t)step) < q.b.z);
+    x.fl = f;
+    return emit;
+}
+
+// Fold of the delta, the recorded statistics, and every substep of OU + LIF
+// (or of the noise mode) of the tile's neurons; returns whether the lane's
+// neuron emitted a spike and writes the state back.
+template <bool kStat>
+__device__ __forceinline__ bool step_lane(TilePtr d, Lane &x, const ParamRec &q, const float4 dl, bool active,
+                                          uint32_t tid, uint32_t lane, int64_t step, uint32_t &p, TileRec &rec)
+{
+    const bool one_pop = (d->flags & kTileOnePop) != 0u;
+    const uint32_t li = d->begin + tid;
+    const InstPtr I = cp(d->inst);
+    p = d->pop0;
     float isyn = 0.0f;
     if (active) {
-        if (!(fl & kFlagFolded))
-            J = fold_delta(J, dc, gat ? dl : acc_to_delta(acc, tid));
-        isyn = syn_current(g, vu, J, V);
-        // the population of neuron li (populations in order of their ends)
-        if (li >= end_a && p + 1 < I.npop) {
-            p = pop_hi;
-            if (li >= end_b)
-                while (p + 1 < I.npop && li >= I.pops[p].end)
-                    ++p;
+        if (!(x.fl & kFlagFolded))
+            x.J = fold_delta(x.J, q.d, dl);
+        isyn = syn_current(q.g, q.v, x.J, x.V);
+        if (!one_pop) {
+            // the population of neuron li (populations in order of their ends)
+            const auto pops = gp(I->pops);
+            const uint32_t npop = I->npop;
+            while (p + 1 < npop && li >= pops[p].end)
+                ++p;
         }
     }
     // stat_result.cpp:266-391: population sums, blocked neurons excluded.
     // The I_syn-based statistics belong to the previous step (its J is
     // complete only now: J folded, V before this step's update); the V
     // statistic (after the update, below) to this one.
-    const int64_t row_v = step - I.rec_step0;
-    const bool stat_valid = kStat && I.rec_stat != nullptr && active && !gp(I.blocked)[lc];
-    if (kStat && I.rec_stat != nullptr) {
-        const uint32_t cf = current_fields(I.stat_mask);
-        if (cf != 0u && row_v - 1 >= 0 && row_v - 1 < (int64_t)I.rec_len) {
+    const bool stat_on = kStat && (d->flags & kTileStat) != 0u;
+    int64_t row_v = 0;
+    bool stat_valid = false;
+    if (stat_on) {
+        row_v = step - I->rec_step0;
+        stat_valid = active && !gp(I->blocked)[active ? li : d->begin];
+        const uint32_t cf = current_fields(I->stat_mask);
+        if (cf != 0u && row_v - 1 >= 0 && row_v - 1 < (int64_t)I->rec_len) {
             long long stv[kStatFields] = {};
-            const float4 rc = receptor_currents(g, vu, J, V);
+            const float4 rc = receptor_currents(q.g, q.v, x.J, x.V);
             stv[1] = stat_q(isyn);
             stv[2] = stat_q(rc.x);
             stv[3] = stat_q(rc.y);
@@ -824,89 +921,215 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             if (one_pop)
                 wave_tile_stats(rec.stat, stat_valid, stv, cf, lane);
             else
-                wave_pop_stats(rec_stat_row(I, row_v - 1, d.begin), stat_valid, p, stv, cf, lane);
+                wave_pop_stats(rec_stat_row(*I, row_v - 1, d->begin), stat_valid, p, stv, cf, lane);
         }
     }
+    bool emit = false;
     if (active) {
-        uint32_t f = fl & kFlagSpike;
-        const PopDev pop = I.pops[p];
-        const bool ou = I.use_ou && pop.ou_on;
-        const int32_t T = I.t_steps;
-        const int32_t rsteps = __float_as_int(pb.w);
-
-        for (int32_t s = 0; s < T; ++s) {
-            float Ieff = isyn;
-            if (ou) {
-                const float xi = ou_normal(I.seed, li, (uint64_t)step * (uint64_t)T + (uint64_t)s);
-                iou = iou + (pop.f1 * (pop.mu - iou) + pop.f2s * xi);
-                Ieff = isyn + iou;
-            }
-            bool spk = false;
-            if (t < 0) {
-                if (f) {
-                    V = pa.x;
-                    f = 0;
-                }
-                t = t + 1;
-            } else {
-                float cvi = pb.x * (pa.w - V);
-                cvi = cvi + Ieff;
-                cvi = cvi + pb.y;
-                V = V + I.dt_sub * pa.z * cvi;
-                spk = V >= pa.y;
-                if (spk) {
-                    V = pa.y;
-                    t = 1 - rsteps;
-                }
-                f = spk ? 1u : 0u;
-            }
-            emit = emit || spk;
-            if (s < T - 1) {
-                J.x = J.x * dc.x;
-                J.y = J.y * dc.y;
-                J.z = J.z * dc.z;
-                J.w = J.w * dc.w;
-                isyn = syn_current(g, vu, J, V);
-            }
-        }
-        if (!I.use_ou) {
-            // spike.cpp:55-62: f_rec = f | (U < noise_rate)
-            const float u = noise_uniform(I.seed, li, (uint64_t)step);
-            emit = f || (u < pb.z);
-        }
-        gp(I.V)[li] = V;
-        gp(I.tcnt)[li] = t;
-        gp(I.flag)[li] = (uint8_t)(f | (emit ? kFlagEmit : 0u));
-        gp(I.iou)[li] = iou;
-        st4(I.J, li, J);
+        if ((d->flags & (kTileOnePop | kTileOneSub)) == (kTileOnePop | kTileOneSub))
+            emit = step_lane_one(d, x, q, isyn, li, step);
+        else
+            emit = step_lane_any(d, I, x, q, isyn, li, step, p);
+        *st_at<kStV, float>(d->state, tid) = x.V;
+        *st_at<kStT, int32_t>(d->state, tid) = x.t;
+        *st_at<kStFlag, uint8_t>(d->state, tid) = (uint8_t)(x.fl | (emit ? kFlagEmit : 0u));
+        *st_at<kStIou, float>(d->state, tid) = x.iou;
+        st_J(d->state, tid, x.J);
     }
-    if (kStat && I.rec_stat != nullptr && (I.stat_mask & kStatV) && row_v >= 0 && row_v < (int64_t)I.rec_len) {
+    if (stat_on && (I->stat_mask & kStatV) && row_v >= 0 && row_v < (int64_t)I->rec_len) {
         long long stv[kStatFields] = {};
-        stv[0] = stat_q(V);
+        stv[0] = stat_q(x.V);
         if (one_pop)
             wave_tile_stats(rec.stat, stat_valid, stv, 1u, lane);
         else
-            wave_pop_stats(rec_stat_row(I, row_v, d.begin), stat_valid, p, stv, 1u, lane);
+            wave_pop_stats(rec_stat_row(*I, row_v, d->begin), stat_valid, p, stv, 1u, lane);
+    }
+    return emit;
+}
+
+// Per-population counts of a wave with emitted neurons
+// (stat_result.cpp:161-206; blocked neurons are not counted): one LDS add
+// per wave in a tile of one population, else one atomic per population
+// present in the wave.
+__device__ __forceinline__ void count_wave(TilePtr d, InstPtr I, bool emit, uint32_t tid, uint32_t lane,
+                                           int64_t step, uint32_t p, TileRec &rec)
+{
+    const int64_t row = step - I->rec_step0;
+    if (row < 0 || row >= (int64_t)I->rec_len)
+        return;
+    const bool counted = emit && !gp(I->blocked)[d->begin + tid];
+    unsigned long long rest = __ballot(counted);
+    if (d->flags & kTileOnePop) {
+        if (lane == 0 && rest != 0ull)
+            atomicAdd(&rec.count, (uint32_t)__popcll(rest));
+        return;
+    }
+    while (rest != 0ull) {
+        const int src = __ffsll((long long)rest) - 1;
+        const uint32_t ps = __shfl(p, src, kWave);
+        const unsigned long long same = __ballot(counted && p == ps);
+        if ((int)lane == src)
+            gadd(rec_count_row(*I, row, d->begin) + ps, (uint32_t)__popcll(same));
+        rest &= ~same;
+    }
+}
+
+// The recorded sums of a tile of one population, after the barrier that
+// follows the waves' LDS adds.
+template <bool kStat>
+__device__ __forceinline__ void put_tile_rec(TilePtr d, InstPtr I, uint32_t tid, int64_t step,
+                                             const TileRec &rec)
+{
+    if (!(d->flags & kTileOnePop))
+        return;
+    // rec.count is nonzero only inside the recorded rows
+    if (tid == 0 && rec.count != 0u)
+        gadd(rec_count_row(*I, step - I->rec_step0, d->begin) + d->pop0, rec.count);
+    if (kStat && (d->flags & kTileStat) && tid < (uint32_t)kStatFields) {
+        // fields of the current step (V) and of the step before (I_syn)
+        const int64_t r = step - I->rec_step0 - (tid == 0 ? 0 : 1);
+        const uint32_t on = ((I->stat_mask & kStatV) ? 1u : 0u) | current_fields(I->stat_mask);
+        if (((on >> tid) & 1u) && r >= 0 && r < (int64_t)I->rec_len)
+            gadd(reinterpret_cast<unsigned long long *>(rec_stat_row(*I, r, d->begin)) +
+                     (size_t)d->pop0 * kStatFields + tid,
+                 rec.stat[tid]);
+    }
+}
+
+// What a tile's step reads before its queue.
+template <bool kUniform>
+struct StepIn {
+    TilePtr d;
+    QueuePtr q;
+    uint32_t cnt, lc;
+    int64_t step, stamp;
+    Lane x;
+    ParamRec prm;
+    bool active;
+
+    __device__ __forceinline__ StepIn(TilePtr tp, QueuePtr qp, uint32_t par, uint32_t tid)
+    {
+        d = tp;
+        q = qp;
+        cnt = *cp(count(par));
+        step = cp(d->step)[par];
+        stamp = cp(d->step)[2u + par];
+        active = tid < d->count;
+        lc = active ? tid : 0u;   // in-range index for idle lanes
+        x = load_lane(d->state, lc);
+        if (kUniform)
+            prm = load_params<true>(d, lc);
+    }
+    __device__ __forceinline__ uint32_t *count(uint32_t par) const
+    {
+        return q->count + count_slot((size_t)par * q->ntiles + blockIdx.x, q->cshift);
+    }
+    __device__ __forceinline__ const QSyn *queue(uint32_t par) const { return d->queue + (size_t)par * d->qslots; }
+};
+
+// One tile's step (the body of k_step).  kUniform: every neuron of the tile
+// has the same parameter class, so the parameter record is read once per
+// tile through the scalar unit instead of per lane.  K: synapses per lane in
+// a binning pass (a pass is 64 K synapses).  kStat: some instance records
+// population statistics (their code costs registers that a launch without
+// them does not spend).
+template <bool kUniform, uint32_t K, uint32_t kFmt, bool kStat>
+__device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
+                                          unsigned long long *acc,
+                                          unsigned long long *seg_dst, uint32_t *seg_room, long long *row_rb,
+                                          uint32_t *row_len, uint32_t &nrows, uint32_t &s_fit,
+                                          unsigned long long *s_bits, TileRec &rec)
+{
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = __lane_id();
+    const uint32_t w = tid / kWave;
+    bool emit, pull;
+    uint32_t p;
+    int64_t step;
+    {
+        // Everything a silent step reads is addressed from the descriptor, so
+        // all of it is in flight before anything waits: the queue count, the
+        // step index and deferral stamp, the neuron state, the parameter
+        // record and the queue head (the queue is complete when the launch
+        // starts; entries past the count are ignored, and the queue buffer has
+        // kQueuePrefetch slots of slack at its end, so the read needs no
+        // branch).
+        StepIn<kUniform> e(tp, qp, par, tid);
+        // One register quad for both: the delta that k_gather wrote (gather
+        // propagation), or the queue entry.
+        float4 ahead;
+        if (e.d->flags & kTileGather) {
+            ahead = ld4(e.d->dlt, e.lc);
+        } else {
+            const QSyn h = ld_entry(e.queue(par), min(tid, kQueuePrefetch - 1u));
+            ahead = make_float4(__uint_as_float(h.key), h.w0, h.w1, 0.0f);
+        }
+        // A tile pulls (the pull propagation, never with gather) when its
+        // queue overflowed or rows were deferred into this set: rare (volleys).
+        const bool gat = (e.d->flags & kTileGather) != 0u;
+        bool over = !gat && e.cnt > e.d->qcap;
+        uint32_t cnt = gat ? 0u : min(e.cnt, e.d->qcap);
+        pull = (e.d->flags & (kTilePull | kTileGather)) == kTilePull && (over || e.stamp == e.step + 1);
+        clear_row(acc, tid);
+        if (tid == 0) {
+            nrows = 0u;
+            rec.count = 0u;
+        }
+        if (kStat && tid < (uint32_t)kStatFields)
+            rec.stat[tid] = 0ull;
+        __syncthreads();
+        if (pull) {
+            // An overflowed queue is ignored: every emitted row then comes
+            // through the in-edges.
+            accumulate_tile(acc, e.queue(par), over ? 0u : cnt, QSyn{}, 0u, tid);
+            pull_tile<kFmt>(acc, *cp(e.d->inst), par, e.d->begin >> kTileBits, over, tid);
+            if (tid == 0)
+                gadd(&again(qp)->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].pulled, 1ull);
+            // Everything again: nothing loaded above is live across the call
+            // (what is, the compiler keeps in spilled registers from the
+            // kernel's start, in every tile).
+            e = StepIn<kUniform>(again(tp), again(qp), par, tid);
+            pull = true;
+            over = false;
+            cnt = 0u;
+        }
+        accumulate_tile(acc, e.queue(par), cnt, QSyn{__float_as_uint(ahead.x), ahead.y, ahead.z}, kQueuePrefetch, tid);
+        __syncthreads();
+        if (!kUniform)   // a rare tile: its lanes' records do not wait in registers
+            e.prm = load_params<false>(e.d, e.lc);
+        step = e.step;
+        if (over && e.active) {   // (a tile that pulls took everything)
+            const InstPtr I = cp(e.d->inst);
+            take_spill(acc, I->spill, I->n, par, e.d->begin + tid, tid, true);   // synapses past the queue's capacity
+        }
+        if (tid == 0) {
+            *gp(e.count(par)) = 0u;   // this launch consumed the queue
+            if (e.d->begin == 0)
+                gp(e.d->step)[par ^ 1u] = step + 1;   // no tile of this launch reads this slot
+        }
+        const float4 dl = (e.d->flags & kTileGather) ? ahead : acc_to_delta(acc, tid);
+        emit = step_lane<kStat>(e.d, e.x, e.prm, dl, e.active, tid, lane, step, p, rec);
     }
 
+    const TilePtr d = again(tp);
+    const InstPtr I = cp(d->inst);
+    const bool gat = (d->flags & kTileGather) != 0u;
+    const bool pull_on = (d->flags & kTilePull) != 0u;
     // Spike propagation (presynaptic_voltage.cpp:122-225): the tile's fired
     // rows are listed in LDS, and their passes of 64 K synapses are dealt
     // round-robin to the four waves, so one long row does not keep a single
     // wave busy while the others idle.
     const unsigned long long m = __ballot(emit);
-    const bool wave_in = d.begin + w * kWave < I.n;   // this wave's neurons exist
-    const size_t nw = (I.n + kWave - 1) / kWave;
-    const size_t bw = (size_t)(par ^ 1u) * nw + (d.begin >> 6) + w;   // this wave's bitmap word of set par ^ 1
-    if (pull_on && lane == 0 && wave_in)
-        gp(I.ebits)[bw] = m;
+    if (lane == 0)
+        s_bits[w] = m;
     if (m != 0ull) {
         const uint32_t cnt_w = (uint32_t)__popcll(m);
         const int leader = __ffsll((long long)m) - 1;
         long long rb = 0;
         uint32_t len = 0;
         if (emit) {
-            rb = gp(I.rowptr)[li];
-            len = (uint32_t)(gp(I.rowptr)[li + 1] - rb);
+            rb = gp(d->rowptr)[tid];
+            len = (uint32_t)(gp(d->rowptr)[tid + 1] - rb);
         }
         // events = sum of the fired rows' lengths: few per wave, read lane by
         // lane through the scalar unit
@@ -917,9 +1140,9 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
         if ((int)lane == leader) {
             // the wave's own counters, added without waiting for a read
             // (a load-add-store would stall the wave before its binning)
-            unsigned long long *c = I.wave_ctr + 2u * ((d.begin >> 6) + w);
-            atomicAdd(c, ev);
-            atomicAdd(c + 1, (unsigned long long)cnt_w);
+            unsigned long long *c = I->wave_ctr + 2u * ((d->begin >> 6) + w);
+            gadd(c, ev);
+            gadd(c + 1, (unsigned long long)cnt_w);
             if (!gat)
                 base = atomicAdd(&nrows, cnt_w);
         }
@@ -930,14 +1153,15 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             const bool has = emit && len != 0u;
             const unsigned long long mg = __ballot(has);
             if (mg != 0ull) {
-                const uint32_t list = (par ^ 1u) * kFiredLists + ((d.begin >> kTileBits) & (kFiredLists - 1u));
+                const uint32_t list = (par ^ 1u) * kFiredLists + ((d->begin >> kTileBits) & (kFiredLists - 1u));
                 const int lg = __ffsll((long long)mg) - 1;
                 uint32_t gb = 0;
                 if ((int)lane == lg)
-                    gb = atomicAdd(I.fcount + (size_t)list * kFiredCountStride, (uint32_t)__popcll(mg));
+                    gb = gadd(I->fcount + (size_t)list * kFiredCountStride, (uint32_t)__popcll(mg));
                 gb = (uint32_t)__builtin_amdgcn_readlane((int)gb, lg);
                 if (has)
-                    gp(I.fired)[(size_t)list * I.fcap + gb + (uint32_t)__popcll(mg & ((1ull << lane) - 1ull))] = li;
+                    gp(I->fired)[(size_t)list * I->fcap + gb + (uint32_t)__popcll(mg & ((1ull << lane) - 1ull))] =
+                        d->begin + tid;
             }
         } else {
             base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
@@ -947,45 +1171,12 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
                 row_len[k] = len;
             }
         }
-        if (I.rec_counts != nullptr) {
-            // stat_result.cpp:161-206 (blocked neurons are not counted): one
-            // atomic per tile of one population, else one per population
-            // present in the wave
-            const int64_t row = step - I.rec_step0;
-            if (row >= 0 && row < (int64_t)I.rec_len) {
-                const bool counted = emit && !gp(I.blocked)[li];
-                unsigned long long rest = __ballot(counted);
-                if (one_pop) {
-                    if (lane == 0 && rest != 0ull)
-                        atomicAdd(&rec.count, (uint32_t)__popcll(rest));
-                    rest = 0ull;
-                }
-                while (rest != 0ull) {
-                    const int src = __ffsll((long long)rest) - 1;
-                    const uint32_t ps = __shfl(p, src, kWave);
-                    const unsigned long long same = __ballot(counted && p == ps);
-                    if ((int)lane == src)
-                        atomicAdd(rec_count_row(I, row, d.begin) + ps, (uint32_t)__popcll(same));
-                    rest &= ~same;
-                }
-            }
-        }
+        if (I->rec_counts != nullptr)
+            count_wave(d, I, emit, tid, lane, step, p, rec);
     }
     __syncthreads();
-    if (one_pop) {
-        // rec.count is nonzero only inside the recorded rows
-        if (tid == 0 && rec.count != 0u)
-            atomicAdd(rec_count_row(I, row_v, d.begin) + d.pop0, rec.count);
-        if (kStat && I.rec_stat != nullptr && tid < (uint32_t)kStatFields) {
-            // fields of the current step (V) and of the step before (I_syn)
-            const int64_t r = tid == 0 ? row_v : row_v - 1;
-            const uint32_t on = (I.stat_mask & kStatV ? 1u : 0u) | current_fields(I.stat_mask);
-            if (((on >> tid) & 1u) && r >= 0 && r < (int64_t)I.rec_len)
-                atomicAdd(reinterpret_cast<unsigned long long *>(rec_stat_row(I, r, d.begin)) +
-                              (size_t)d.pop0 * kStatFields + tid,
-                          rec.stat[tid]);
-        }
-    }
+    const QueuePtr qs = again(qp);
+    put_tile_rec<kStat>(d, I, tid, step, rec);
     const uint32_t nr = nrows;
     // A tile with many emitted rows (a synchronous volley) leaves them to
     // the consumers' pull: binning them would cost one reservation per
@@ -993,23 +1184,33 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
     // this launch (the volley is under way) defers only from four times
     // the count: the volley's tail, where a few tiles still emit that many,
     // would otherwise cost the next step a pull of every in-edge.
-    const bool defer = pull_on && I.defer_min != 0u && nr >= (pull ? 4u * I.defer_min : I.defer_min);
+    bool defer = false;
     if (pull_on) {
-        if (lane == 0 && wave_in)
-            gp(I.dbits)[bw] = defer ? m : 0ull;
+        if (nr != 0u) {
+            const uint32_t dm = I->defer_min;
+            defer = dm != 0u && nr >= (pull ? 4u * dm : dm);
+        }
+        // the tile's emitted and deferred rows, one 64-byte store
+        if (tid < kBitWords) {
+            const unsigned long long b = s_bits[tid & 3u];
+            gp(d->bits)[(size_t)(par ^ 1u) * d->ntiles * kBitWords + tid] = (tid < 4u || defer) ? b : 0ull;
+        }
         if (defer && tid == 0) {
-            gp(I.dstamp)[par ^ 1u] = step + 2;   // consumer's step + 1 (0: none)
-            atomicAdd(&ctl->slot[blockIdx.x & (kCtlSlots - 1u)].deferred, 1ull);
+            gp(d->step)[2u + (par ^ 1u)] = step + 2;   // consumer's step + 1 (0: none)
+            gadd(&qs->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].deferred, 1ull);
         }
     }
     const uint32_t nbin = defer ? 0u : nr;
-    unsigned long long *spill_out = pull_on ? nullptr : I.spill + (size_t)(par ^ 1u) * I.n * 4u;
+    if (nbin == 0u)
+        return;
+    unsigned long long *spill_out = pull_on ? nullptr : I->spill + (size_t)(par ^ 1u) * I->n * 4u;
+    QSyn *q_out = I->queue + (size_t)(par ^ 1u) * d->qslots;
     // Split binning: the tile's passes (rows in LDS order, passes in row
     // order) go to the engine's pass list for the k_bin launch that follows,
     // where every wave of the GPU takes one; the tile bins here only the
     // passes past the list's capacity.
     uint32_t first_here = 0;   // tile pass index from which this tile bins itself
-    if (qs.pass != nullptr && nbin != 0u) {
+    if (qs->pass != nullptr) {
         if (w == 0) {
             constexpr uint32_t kPass = kWave * K;
             uint32_t total = 0;
@@ -1020,9 +1221,9 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             }
             uint32_t base = 0;
             if (lane == 0)
-                base = atomicAdd(qs.pcount + (size_t)par * kPassCountStride, total);
+                base = gadd(qs->pcount + (size_t)par * kPassCountStride, total);
             base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-            const uint32_t fit = qs.pcap > base ? min(total, qs.pcap - base) : 0u;
+            const uint32_t fit = qs->pcap > base ? min(total, qs->pcap - base) : 0u;
             uint32_t off = 0;   // passes of the rows of earlier chunks
             for (uint32_t r0 = 0; r0 < nbin; r0 += kWave) {
                 const uint32_t r = r0 + lane;
@@ -1041,8 +1242,8 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
                     PassEntry e;
                     e.first = (uint64_t)(rb + (long long)j * kPass);
                     e.len = min(kPass, len - j * kPass);
-                    e.inst = d.inst;
-                    qs.pass[base + ex + j] = e;
+                    e.inst = d->inst_idx;
+                    qs->pass[base + ex + j] = e;
                 }
                 off += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
             }
@@ -1060,14 +1261,14 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
             if ((pass & 3u) == w && pass >= first_here)
             {
                 if constexpr (K == 1)
-                    bin_pass_serial<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)rb_s, len_s, c0, I.tile_base, tiles, qs.count,
-                                       (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out,
-                                       spill_out, ctl, seg_dst + w * kWave * K,
+                    bin_pass_serial<K, kFmt>(I->col, I->w, I->wfmt, (int64_t)rb_s, len_s, c0, I->tile_base, qs->tile,
+                                       qs->count, (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out,
+                                       spill_out, qs->ctl, seg_dst + w * kWave * K,
                                        seg_room + w * kWave * K, lane);
                 else
-                    bin_pass<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)rb_s, len_s, c0, I.tile_base, tiles, qs.count,
-                                (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out,
-                                spill_out, ctl, seg_dst + w * kWave * K,
+                    bin_pass<K, kFmt>(I->col, I->w, I->wfmt, (int64_t)rb_s, len_s, c0, I->tile_base, qs->tile, qs->count,
+                                (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out,
+                                spill_out, qs->ctl, seg_dst + w * kWave * K,
                                 seg_room + w * kWave * K, lane);
             }
     }
@@ -1079,28 +1280,27 @@ __device__ __forceinline__ void step_tile(const TileDesc &d, const TileDesc *__r
 // same results).  Eight waves per SIMD for K = 1, 2; K = 4's larger LDS
 // segment tables allow six.
 template <uint32_t K, uint32_t kFmt, bool kStat>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ? 6 : 8))) void k_step(const TileDesc *__restrict__ tiles,
-                                                 const InstDev *__restrict__ insts,
-                                                 QueueSet qs,
-                                                 uint32_t par,
-                                                 StepCtl *__restrict__ ctl)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ? 6 : 8))) void k_step(const TileDesc *tiles,
+                                                 const QueueSet *queues,
+                                                 uint32_t par)
 {
     __shared__ unsigned long long acc[kBlock * 4];
     __shared__ unsigned long long seg_dst[4 * kWave * K];   // per wave: one pass
     __shared__ uint32_t seg_room[4 * kWave * K];
     __shared__ long long row_rb[kBlock];                  // fired rows of the tile: first synapse
     __shared__ uint32_t row_len[kBlock];                  // and length
+    __shared__ unsigned long long s_bits[4];              // emitted rows per wave
     __shared__ uint32_t nrows;
     __shared__ uint32_t s_fit;                            // split binning: passes in the list
     __shared__ TileRec rec;
 
-    const TileDesc d = tiles[blockIdx.x];
-    if (d.pcls != 0u)
-        step_tile<true, K, kFmt, kStat>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit,
-                                 rec);
+    const TilePtr tp = cp(tiles + blockIdx.x);
+    if (tp->flags & kTileUniform)
+        step_tile<true, K, kFmt, kStat>(tp, cp(queues), par, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit, s_bits,
+                                        rec);
     else
-        step_tile<false, K, kFmt, kStat>(d, tiles, insts, qs, par, ctl, acc, seg_dst, seg_room, row_rb, row_len, nrows,
-                                  s_fit, rec);
+        step_tile<false, K, kFmt, kStat>(tp, cp(queues), par, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit,
+                                         s_bits, rec);
 }
 
 // Split binning: bins the passes that the k_step launch of parity `par`
@@ -1110,11 +1310,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ?
 // parity's list count (its last reader was the previous k_bin; the next
 // k_step appends to it).
 template <uint32_t K, uint32_t kFmt>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_bin(const TileDesc *__restrict__ tiles,
-                                                const InstDev *__restrict__ insts,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_bin(const InstDev *__restrict__ insts,
                                                 QueueSet qs,
-                                                uint32_t par,
-                                                StepCtl *__restrict__ ctl)
+                                                uint32_t par)
 {
     __shared__ unsigned long long seg_dst[4 * kWave * K];
     __shared__ uint32_t seg_room[4 * kWave * K];
@@ -1130,12 +1328,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         QSyn *q_out = I.queue + (size_t)(par ^ 1u) * I.qslots;
         unsigned long long *spill_out = I.crec != nullptr ? nullptr : I.spill + (size_t)(par ^ 1u) * I.n * 4u;
         if constexpr (K == 1)
-            bin_pass_serial<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, tiles, qs.count,
-                               (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, ctl,
+            bin_pass_serial<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, qs.tile, qs.count,
+                               (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, qs.ctl,
                                seg_dst + w * kWave * K, seg_room + w * kWave * K, lane);
         else
-            bin_pass<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, tiles, qs.count,
-                        (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, ctl,
+            bin_pass<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, qs.tile, qs.count,
+                        (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, qs.ctl,
                         seg_dst + w * kWave * K, seg_room + w * kWave * K, lane);
     }
 }
@@ -1400,8 +1598,8 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const TileDesc *__restri
                                                         uint32_t set)
 {
     __shared__ unsigned long long acc[kBlock * 4];
-    const TileDesc d = tiles[blockIdx.x];
-    const InstDev &I = insts[d.inst];
+    const TileDesc &d = tiles[blockIdx.x];
+    const InstDev &I = insts[d.inst_idx];
     if (I.segidx != nullptr)
         return;   // gather propagation: k_gather has written dlt
     const uint32_t tid = threadIdx.x;
@@ -1409,16 +1607,16 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const TileDesc *__restri
     const uint32_t cnt_raw = qs.count[count_slot((size_t)set * qs.ntiles + blockIdx.x, qs.cshift)];
     const bool over = cnt_raw > d.qcap;
     const bool pull_on = I.crec != nullptr;
-    const bool pull = pull_on && (over || gp(I.dstamp)[set] == gp(I.step)[set] + 1);
+    const bool pull = pull_on && (over || gp(I.step)[2u + set] == gp(I.step)[set] + 1);
     const uint32_t cnt = (pull_on && over) ? 0u : min(cnt_raw, d.qcap);
     __syncthreads();
-    accumulate_tile(acc, I.queue + (size_t)set * I.qslots + d.qoff, cnt, QSyn{}, 0u, tid);
+    accumulate_tile(acc, d.queue + (size_t)set * d.qslots, cnt, QSyn{}, 0u, tid);
     if (pull)
         pull_tile<kWeightAny>(acc, I, set, d.begin >> kTileBits, over, tid);
     __syncthreads();
     if (tid < d.count) {
         if (!pull_on && over)
-            take_spill(acc, I, set, d.begin + tid, tid, false);
+            take_spill(acc, I.spill, I.n, set, d.begin + tid, tid, false);
         st4(I.dlt, d.begin + tid, acc_to_delta(acc, tid));
     }
 }
@@ -1433,18 +1631,19 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
                                                    uint32_t set)
 {
     __shared__ unsigned long long acc[kBlock * 4];
-    const TileDesc d = tiles[blockIdx.x];
-    const InstDev &I = insts[d.inst];
+    const TileDesc &d = tiles[blockIdx.x];
+    const InstDev &I = insts[d.inst_idx];
     const uint32_t tid = threadIdx.x;
     if (I.segidx != nullptr) {
         // gather propagation: k_gather has written the pending delta into
         // dlt; after the fold the fired list of this set is empty
         if (tid < d.count) {
             const uint32_t li = d.begin + tid;
-            const uint32_t fl = gp(I.flag)[li];
+            const auto flag = st_at<kStFlag, uint8_t>(d.state, tid);
+            const uint32_t fl = *flag;
             if (!(fl & kFlagFolded)) {
-                st4(I.J, li, fold_delta(ld4(I.J, li), ld4(I.dec, param_index(I, li)), ld4(I.dlt, li)));
-                gp(I.flag)[li] = (uint8_t)(fl | kFlagFolded);
+                st_J(d.state, tid, fold_delta(ld_J(d.state, tid), ld4(&param_of(I, li)->d, 0), ld4(I.dlt, li)));
+                *flag = (uint8_t)(fl | kFlagFolded);
             }
         }
         if (d.begin == 0 && tid < kFiredLists)
@@ -1456,21 +1655,22 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
     const uint32_t cnt_raw = *cnt_p;
     const bool over = cnt_raw > d.qcap;
     const bool pull_on = I.crec != nullptr;
-    const bool pull = pull_on && (over || gp(I.dstamp)[set] == gp(I.step)[set] + 1);
+    const bool pull = pull_on && (over || gp(I.step)[2u + set] == gp(I.step)[set] + 1);
     const uint32_t cnt = (pull_on && over) ? 0u : min(cnt_raw, d.qcap);
     __syncthreads();
-    accumulate_tile(acc, I.queue + (size_t)set * I.qslots + d.qoff, cnt, QSyn{}, 0u, tid);
+    accumulate_tile(acc, d.queue + (size_t)set * d.qslots, cnt, QSyn{}, 0u, tid);
     if (pull)
         pull_tile<kWeightAny>(acc, I, set, d.begin >> kTileBits, over, tid);
     __syncthreads();
     if (tid < d.count) {
         const uint32_t li = d.begin + tid;
         if (!pull_on && over)
-            take_spill(acc, I, set, li, tid, true);
-        const uint32_t fl = gp(I.flag)[li];
+            take_spill(acc, I.spill, I.n, set, li, tid, true);
+        const auto flag = st_at<kStFlag, uint8_t>(d.state, tid);
+        const uint32_t fl = *flag;
         if (!(fl & kFlagFolded)) {
-            st4(I.J, li, fold_delta(ld4(I.J, li), ld4(I.dec, param_index(I, li)), acc_to_delta(acc, tid)));
-            gp(I.flag)[li] = (uint8_t)(fl | kFlagFolded);
+            st_J(d.state, tid, fold_delta(ld_J(d.state, tid), ld4(&param_of(I, li)->d, 0), acc_to_delta(acc, tid)));
+            *flag = (uint8_t)(fl | kFlagFolded);
         }
     }
     if (tid == 0)
@@ -1486,8 +1686,8 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
                                                       uint32_t par)
 {
     __shared__ unsigned long long s_stat[kStatFields];
-    const TileDesc d = tiles[blockIdx.x];
-    const InstDev &I = insts[d.inst];
+    const TileDesc &d = tiles[blockIdx.x];
+    const InstDev &I = insts[d.inst_idx];
     const uint32_t cf = current_fields(I.stat_mask);
     if (I.rec_stat == nullptr || cf == 0u)
         return;
@@ -1504,12 +1704,12 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
     if (active) {
         while (p + 1 < I.npop && li >= I.pops[p].end)
             ++p;
-        const uint32_t c = param_index(I, li);
-        const float V = gp(I.V)[li];
-        float4 J = ld4(I.J, li);
-        if (!(gp(I.flag)[li] & kFlagFolded))
-            J = fold_delta(J, ld4(I.dec, c), ld4(I.dlt, li));
-        const float4 g = ld4(I.gU, c), vu = ld4(I.vU, c);
+        const ParamRec *c = param_of(I, li);
+        const float V = *st_at<kStV, float>(d.state, tid);
+        float4 J = ld_J(d.state, tid);
+        if (!(*st_at<kStFlag, uint8_t>(d.state, tid) & kFlagFolded))
+            J = fold_delta(J, ld4(&c->d, 0), ld4(I.dlt, li));
+        const float4 g = ld4(&c->g, 0), vu = ld4(&c->v, 0);
         const float4 rc = receptor_currents(g, vu, J, V);
         stv[1] = stat_q(syn_current(g, vu, J, V));
         stv[2] = stat_q(rc.x);
@@ -1518,7 +1718,7 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
         stv[5] = stat_q(rc.w);
         valid = !gp(I.blocked)[li];
     }
-    if (d.begin + d.count > I.pops[d.pop0].end) {   // more than one population
+    if (!(d.flags & kTileOnePop)) {
         wave_pop_stats(rec_stat_row(I, row, d.begin), valid, p, stv, cf, lane);
         return;
     }
@@ -1570,18 +1770,104 @@ __global__ __launch_bounds__(kBlock) void k_sample(const InstDev *__restrict__ i
         return;
     const uint32_t li = s.neuron;
     const size_t o = (size_t)row * R.nsample + s.slot;
-    const float V = gp(I.V)[li];
+    unsigned char *block = block_of(I, li);
+    const uint32_t k = li & (kBlock - 1u);
+    const float V = *st_at<kStV, float>(block, k);
     if (R.spike)
-        R.spike[o] = (gp(I.flag)[li] & kFlagEmit) ? 1 : 0;
+        R.spike[o] = (*st_at<kStFlag, uint8_t>(block, k) & kFlagEmit) ? 1 : 0;
     if (R.v)
         R.v[o] = V;
     if (R.isyn) {
-        const uint32_t c = param_index(I, li);
-        const float4 J = fold_delta(ld4(I.J, li), ld4(I.dec, c), ld4(I.dlt, li));   // flag bit 2 is clear here
-        R.isyn[o] = syn_current(ld4(I.gU, c), ld4(I.vU, c), J, V);
+        const ParamRec *c = param_of(I, li);
+        const float4 J = fold_delta(ld_J(block, k), ld4(&c->d, 0), ld4(I.dlt, li));   // flag bit 2 is clear here
+        R.isyn[o] = syn_current(ld4(&c->g, 0), ld4(&c->v, 0), J, V);
     }
     if (R.iou)
-        R.iou[o] = gp(I.iou)[li];
+        R.iou[o] = *st_at<kStIou, float>(block, k);
+}
+
+// Fresh state (block.cpp:136-179, membrane_voltage.cpp:18): V0 = (V_th +
+// V_reset) / 2; the rest of the blocks is zeroed before.
+__global__ __launch_bounds__(kBlock) void k_init_state(StateView v)
+{
+    const uint32_t li = blockIdx.x * kBlock + threadIdx.x;
+    if (li >= v.n)
+        return;
+    const float4 a = ld4(&v.prm[(li & v.pmask) + (uint32_t)gp(v.cls)[li]].a, 0);
+    *st_at<kStV, float>(v.state + (size_t)blockIdx.x * kStateBytes, threadIdx.x) = (a.y + a.x) / 2.0f;
+}
+
+// OU current of neurons [begin, end) set to `value`.
+__global__ __launch_bounds__(kBlock) void k_fill_iou(StateView v, uint32_t begin, uint32_t end, float value)
+{
+    const uint32_t li = begin + blockIdx.x * kBlock + threadIdx.x;
+    if (li < end)
+        *st_at<kStIou, float>(v.state + (size_t)(li >> kTileBits) * kStateBytes, li & (kBlock - 1u)) = value;
+}
+
+// Reference-visible state of `count` neurons from `first` on into plain
+// arrays (any may be null): the pending delta folded exactly as the next
+// step will fold it, I_syn of the folded J.
+__global__ __launch_bounds__(kBlock) void k_read_state(StateView v, uint32_t first, uint32_t count, StateArrays out)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= count)
+        return;
+    const uint32_t li = first + i, k = li & (kBlock - 1u);
+    unsigned char *block = v.state + (size_t)(li >> kTileBits) * kStateBytes;
+    const float V = *st_at<kStV, float>(block, k);
+    const uint32_t fl = *st_at<kStFlag, uint8_t>(block, k);
+    if (out.V)
+        out.V[i] = V;
+    if (out.t)
+        out.t[i] = *st_at<kStT, int32_t>(block, k);
+    if (out.iou)
+        out.iou[i] = *st_at<kStIou, float>(block, k);
+    if (out.f)
+        out.f[i] = fl & kFlagSpike;
+    if (out.emitted)
+        out.emitted[i] = (fl & kFlagEmit) ? 1 : 0;
+    if (out.J || out.isyn) {
+        const ParamRec *c = v.prm + ((li & v.pmask) + (uint32_t)gp(v.cls)[li]);
+        float4 J = ld_J(block, k);
+        if (!(fl & kFlagFolded))
+            J = fold_delta(J, ld4(&c->d, 0), ld4(v.dlt, li));
+        if (out.J)
+            st4(out.J, i, J);
+        if (out.isyn)
+            out.isyn[i] = syn_current(ld4(&c->g, 0), ld4(&c->v, 0), J, V);
+    }
+}
+
+// Checkpoint restore of `count` neurons from `first` on (null arrays keep
+// their field).  J is the reference-visible J of the last step: the pending
+// delta is cleared and the flag byte marks J as folded, so the next step
+// uses it as is.
+__global__ __launch_bounds__(kBlock) void k_write_state(StateView v, uint32_t first, uint32_t count, StateArrays in)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= count)
+        return;
+    const uint32_t li = first + i, k = li & (kBlock - 1u);
+    unsigned char *block = v.state + (size_t)(li >> kTileBits) * kStateBytes;
+    if (in.V)
+        *st_at<kStV, float>(block, k) = in.V[i];
+    if (in.t)
+        *st_at<kStT, int32_t>(block, k) = in.t[i];
+    if (in.iou)
+        *st_at<kStIou, float>(block, k) = in.iou[i];
+    if (in.f || in.J) {
+        uint32_t fl = *st_at<kStFlag, uint8_t>(block, k);
+        if (in.f)
+            fl = (fl & ~(uint32_t)kFlagSpike) | (in.f[i] ? kFlagSpike : 0u);
+        if (in.J)
+            fl |= kFlagFolded;
+        *st_at<kStFlag, uint8_t>(block, k) = (uint8_t)fl;
+    }
+    if (in.J) {
+        st_J(block, k, ld4(in.J, i));
+        st4(v.dlt, li, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    }
 }
 
 // Verification entry: normals of the OU stream for a range of neurons at one
@@ -1633,46 +1919,45 @@ struct BinSel {
     static auto get() { return k_bin<K, F>; }
 };
 
-hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
+                              uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
                               hipStream_t stream)
 {
     if (ntiles == 0)
         return hipSuccess;
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, tiles, insts, qs, par, ctl);
+        hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, tiles, qs, par);
     };
     const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
                               : with_kernel<StepSel>(pass_k, wfmt, launch);
     return e != hipSuccess ? e : hipGetLastError();
 }
 
-hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
+                                    uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
                                     hipEvent_t start, hipEvent_t stop, hipStream_t stream)
 {
     if (ntiles == 0)
         return hipSuccess;
     auto launch = [&](auto kern) {
-        hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, start, stop, 0, tiles, insts, qs, par, ctl);
+        hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, start, stop, 0, tiles, qs, par);
     };
     const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
                               : with_kernel<StepSel>(pass_k, wfmt, launch);
     return e != hipSuccess ? e : hipGetLastError();
 }
 
-hipError_t launch_bin_kernel(const TileDesc *tiles, uint32_t grid, const InstDev *insts, const QueueSet &qs,
-                             uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
+hipError_t launch_bin_kernel(uint32_t grid, const InstDev *insts, const QueueSet &qs,
+                             uint32_t par, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
                              hipEvent_t stop, hipStream_t stream)
 {
     if (grid == 0 || qs.pass == nullptr)
         return hipSuccess;
     const hipError_t e = with_kernel<BinSel>(pass_k, wfmt, [&](auto kern) {
         if (start != nullptr)
-            hipExtLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, start, stop, 0, tiles, insts, qs, par,
-                                  ctl);
+            hipExtLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, start, stop, 0, insts, qs, par);
         else
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, tiles, insts, qs, par, ctl);
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, insts, qs, par);
     });
     return e != hipSuccess ? e : hipGetLastError();
 }
@@ -1798,6 +2083,37 @@ hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_
         return hipSuccess;
     const uint32_t nb = (nsamples + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(k_sample, dim3(nb), dim3(kBlock), 0, stream, insts, samples, nsamples, recs, par);
+    return hipGetLastError();
+}
+
+hipError_t launch_init_state(const StateView &v, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_init_state, dim3((v.n + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, v);
+    return hipGetLastError();
+}
+
+hipError_t launch_fill_iou(const StateView &v, uint32_t begin, uint32_t end, float value, hipStream_t stream)
+{
+    if (begin >= end)
+        return hipSuccess;
+    hipLaunchKernelGGL(k_fill_iou, dim3((end - begin + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, v, begin, end,
+                       value);
+    return hipGetLastError();
+}
+
+hipError_t launch_read_state(const StateView &v, uint32_t first, uint32_t count, const StateArrays &out,
+                             hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_read_state, dim3((count + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, v, first, count,
+                       out);
+    return hipGetLastError();
+}
+
+hipError_t launch_write_state(const StateView &v, uint32_t first, uint32_t count, const StateArrays &in,
+                              hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_write_state, dim3((count + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, v, first, count,
+                       in);
     return hipGetLastError();
 }
 

@@ -10,21 +10,21 @@ namespace dtb {
 // wfmt: the weight format of every instance in the tables, or kWeightAny
 // (each launch's kernels are specialised for it).  stat: some instance
 // records population statistics.
-hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                              uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
+                              uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
                               hipStream_t stream);
 
 // launch_step_kernel with `start` / `stop` recorded at the kernel's own
 // dispatch boundaries (kernel time without launch gaps).
-hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, const QueueSet &qs,
-                                    uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, bool stat,
+hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
+                                    uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
                                     hipEvent_t start, hipEvent_t stop, hipStream_t stream);
 
 // Split binning: bins the passes listed by the k_step launch of parity
 // `par` (grid workgroups, each wave one pass at a time); nothing when the
 // queue set has no pass list.  Events may be null.
-hipError_t launch_bin_kernel(const TileDesc *tiles, uint32_t grid, const InstDev *insts, const QueueSet &qs,
-                             uint32_t par, StepCtl *ctl, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
+hipError_t launch_bin_kernel(uint32_t grid, const InstDev *insts, const QueueSet &qs,
+                             uint32_t par, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
                              hipEvent_t stop, hipStream_t stream);
 
 // Gather propagation: delta of fired list `par` into InstDev::dlt for every
@@ -72,6 +72,33 @@ hipError_t launch_fold_slots(const T *in, uint32_t slots, uint32_t stride, uint3
 // Samples of the step run by the k_step launch of parity `par`.
 hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_t nsamples,
                          const SampleRecDev *recs, uint32_t par, hipStream_t stream);
+
+// State of one instance (its blocks and what reading them needs), and plain
+// arrays of it.
+struct StateView {
+    unsigned char *state;
+    const ParamRec *prm;
+    const uint16_t *cls;
+    float4 *dlt;
+    uint32_t pmask, n;
+};
+struct StateArrays {
+    float *V;
+    int32_t *t;
+    float *iou;
+    float4 *J;
+    float *isyn;
+    uint8_t *f, *emitted;
+};
+// V of a fresh state (the blocks zeroed before); OU current of a range of
+// neurons; state of neurons [first, first + count) into / from plain device
+// arrays (null: not read / kept).
+hipError_t launch_init_state(const StateView &v, hipStream_t stream);
+hipError_t launch_fill_iou(const StateView &v, uint32_t begin, uint32_t end, float value, hipStream_t stream);
+hipError_t launch_read_state(const StateView &v, uint32_t first, uint32_t count, const StateArrays &out,
+                             hipStream_t stream);
+hipError_t launch_write_state(const StateView &v, uint32_t first, uint32_t count, const StateArrays &in,
+                              hipStream_t stream);
 
 hipError_t launch_normals(uint64_t seed, uint32_t neuron0, uint64_t substep, uint32_t count, float *out,
                           hipStream_t stream);

@@ -70,28 +70,37 @@ constexpr uint64_t kRecMaxBytes = (uint64_t)64 << 20;
 // index per neuron); beyond it the records are stored per neuron.
 constexpr size_t kMaxParamClasses = 65536;
 
+// Parameter record of a class of neurons (80 bytes, so a tile of one class
+// reads its record with two scalar loads):
+//   a = (v_reset, v_th, dt_sub / C, v_leak)
+//   b = (g_leak, i_ext, noise_rate, bits(refractory substeps))
+//   g, v, d = g_u, V_u and the decay of (AMPA, NMDA, GABA_A, GABA_B)
+struct alignas(16) ParamRec {
+    float4 a, b, g, v, d;
+};
+
+// State block of a tile of 256 neurons, one after the other in memory, so a
+// workgroup reaches all of its state from one base address: V, refractory
+// counter (reference t_actives_), OU current (i_ou_background_stimuli_),
+// flags (kFlagSpike | kFlagEmit | kFlagFolded) and J_u after the previous
+// step's decay (delta pending).  The offsets fit the immediate field of a
+// global load.
+constexpr uint32_t kStV = 0, kStT = 1024, kStIou = 2048, kStFlag = 3072, kStJ = 3328;
+constexpr uint32_t kStateBytes = 3328 + 256 * 16;   // 7424: whole 128-byte lines
+
 // Everything a kernel needs about one instance.
 struct alignas(16) InstDev {
-    // Parameter records, one float4 each, indexed by parameter class:
-    //   pA = (v_reset, v_th, 1/C, v_leak)
-    //   pB = (g_leak, i_ext, noise_rate, bits(refractory substeps))
-    //   gU, vU, dec = (AMPA, NMDA, GABA_A, GABA_B)
-    // Neurons with bit-identical records share a class (in practice one per
-    // population), so the step reads 2 bytes of class per neuron instead of
-    // 80 bytes of parameters.  The record of neuron i is
-    // (i & pmask) + cls[i]: pmask = 0 with shared classes; when the records
-    // have more than 65536 values every neuron has its own (pmask = ~0xff,
-    // cls[i] = i & 0xff, record = i).
-    const float4 *pA, *pB, *gU, *vU, *dec;
+    // Parameter records by class.  Neurons with bit-identical records share a
+    // class (in practice one per population), so the step reads 2 bytes of
+    // class per neuron at most instead of 80 bytes of parameters.  The record
+    // of neuron i is (i & pmask) + cls[i]: pmask = 0 with shared classes; when
+    // the records have more than 65536 values every neuron has its own
+    // (pmask = ~0xff, cls[i] = i & 0xff, record = i).
+    const ParamRec *prm;
     const uint16_t *cls;        // [n] parameter class
     const uint8_t *blocked;     // excluded from population statistics
-    // state
-    float *V;
-    int32_t *tcnt;              // refractory counter (reference t_actives_)
-    uint8_t *flag;              // kFlagSpike | kFlagEmit | kFlagFolded
-    float *iou;                 // OU current (reference i_ou_background_stimuli_)
-    float4 *J;                  // J_u after the previous step's decay (delta below pending)
-    float4 *dlt;                // materialised pending delta (sampling / read-back only)
+    unsigned char *state;       // [ntiles][kStateBytes]
+    float4 *dlt;                // materialised pending delta (gather, sampling, read-back)
     unsigned long long *spill;  // [2][n][4] Q23.40 sums of the synapses past a queue's capacity
     QSyn *queue;                // [2][qslots] propagation queues (+ read-ahead slack)
     uint64_t qslots;            // queue slots per parity (tile t's start: TileDesc::qoff)
@@ -117,20 +126,18 @@ struct alignas(16) InstDev {
     // in-edges of target tile t are records [cptr[t], cptr[t + 1]) of crec,
     // grec_words(wfmt) words each: key = source row (bits 0..22) | target's
     // index in the tile (bits 23..30) | channel pair (bit 31), then the
-    // weight pair's raw bits, so one load brings both.  Per wave of 64
-    // neurons, ebits[s] holds the rows emitted by the launch that filled
-    // queue set s and dbits[s] those of them whose tile deferred its
-    // propagation to the pull; dstamp[s] = 1 + the step index of the launch
-    // that consumes set s when some tile deferred into it (0: none; a stale
-    // stamp never equals a later consumer's).  A consuming tile pulls
-    // when its queue overflowed (then it ignores the queue and takes every
-    // emitted row through its in-edges) or when rows were deferred (then it
-    // adds the deferred rows to its queue).
+    // weight pair's raw bits, so one load brings both.  bits: per set and
+    // tile, the 256 rows emitted by the launch that filled the set (4 words
+    // of 64), then those of them whose tile deferred its propagation to the
+    // pull (4 words).  step[2 + s] (the deferral stamp of set s) = 1 + the
+    // step index of the launch that consumes set s when some tile deferred
+    // into it (0: none; a stale stamp never equals a later consumer's).  A
+    // consuming tile pulls when its queue overflowed (then it ignores the
+    // queue and takes every emitted row through its in-edges) or when rows
+    // were deferred (then it adds the deferred rows to its queue).
     const uint32_t *crec;       // [S][grec_words(wfmt)]
     const int64_t *cptr;        // [ntiles + 1]
-    unsigned long long *ebits;  // [2][ceil(n / 64)]
-    unsigned long long *dbits;  // [2][ceil(n / 64)]
-    int64_t *dstamp;            // [2]
+    unsigned long long *bits;   // [2][ntiles][kBitWords]
     const PopDev *pops;         // [npop]
     // recording (device buffers, row = step - rec_step0)
     // Sums spread over rec_slots slots (a power of two) per row, a tile's
@@ -143,8 +150,9 @@ struct alignas(16) InstDev {
     // out-degrees, spikes emitted); each slot is updated only by the wave
     // that owns those neurons, so no atomics are needed
     unsigned long long *wave_ctr;   // [ceil(n/64)][2]
-    int64_t *step;              // [2] step index by launch parity: the launch of
-                                // parity p reads step[p] and writes step[p^1] = step[p] + 1
+    int64_t *step;              // [0..1] step index by launch parity: the launch of
+                                // parity p reads step[p] and writes step[p^1] = step[p] + 1;
+                                // [2..3] deferral stamps by queue set
     // scalars
     uint64_t seed;
     int64_t rec_step0;
@@ -153,7 +161,6 @@ struct alignas(16) InstDev {
     uint32_t rec_len;
     int32_t t_steps;
     int32_t use_ou;
-    float dt_sub;
     uint32_t tile_base;         // engine-wide index of this instance's first tile
     uint32_t stat_mask;         // kStatV | kStatI | kStatReceptor: statistics recorded in rec_stat
     uint32_t pmask;             // parameter record of neuron i: (i & pmask) + cls[i]
@@ -162,7 +169,11 @@ struct alignas(16) InstDev {
     uint32_t defer_min;         // pull: a tile with this many emitted rows defers them (0: never)
     uint32_t wfmt;              // weight pair format of w and cw
     uint32_t rec_slots, rec_cstride, rec_sstride;   // layout of rec_counts and rec_stat
+    uint32_t ntiles;
 };
+
+// Words per tile and set of InstDev::bits.
+constexpr uint32_t kBitWords = 8;
 
 // Weight pair formats kept on the device (include/weights.hpp:14-21 and the
 // decode of presynaptic_voltage.cpp:153-176): two fp32 (8 bytes), two fp16
@@ -194,15 +205,50 @@ constexpr uint32_t kPullMaxNeurons = 1u << kPullRowBits;
 constexpr uint32_t kDeferMinDefault = 16;
 
 // One tile = one workgroup of the step kernel: up to 256 consecutive neurons
-// of one instance, and the queue of the synapses delivered to them.
-struct alignas(16) TileDesc {
-    uint32_t inst;
-    uint32_t begin;     // first instance-local neuron
-    uint32_t count;     // neurons in the tile (<= 256)
-    uint32_t pop0;      // population of the first neuron
-    uint64_t qoff;      // first slot in the instance's queue of one parity
-    uint32_t qcap;      // queue capacity: synapses targeting this tile (all rows)
-    uint32_t pcls;      // 1 + the parameter class shared by every neuron of the tile, or 0
+// of one instance.  The descriptor holds all that a step without spikes
+// needs, resolved for the tile, in 128 bytes: a workgroup issues its state,
+// parameter and queue loads after one scalar round trip (the instance's
+// descriptor behind it is only read by tiles that fire, pull or record).
+// Fields are read where a phase needs them (again() in the kernel): held in
+// scalar registers from the start, they cost about 100 spilled scalars, each
+// a vector instruction to store and one to load back.
+constexpr uint32_t kTileUniform = 1u;    // one parameter class (prm is its record)
+constexpr uint32_t kTileOnePop = 2u;     // one population (mu, f1, f2s are its OU factors)
+constexpr uint32_t kTileOu = 4u;         // the instance runs with the OU background
+constexpr uint32_t kTileOuOn = 8u;       // and the tile's one population has it configured
+constexpr uint32_t kTilePull = 16u;      // pull propagation
+constexpr uint32_t kTileGather = 32u;    // gather propagation
+constexpr uint32_t kTileOneSub = 64u;    // one substep per step
+constexpr uint32_t kTileStat = 128u;     // population statistics are recorded
+struct alignas(128) TileDesc {
+    unsigned char *state;    // the tile's state block
+    const QSyn *queue;       // its queue of set 0
+    uint64_t qslots;         // entries between the sets
+    int64_t *step;           // InstDev::step
+    uint32_t begin;          // first instance-local neuron
+    uint32_t count;          // neurons in the tile (<= 256)
+    uint32_t flags;
+    uint32_t qcap;           // queue capacity: synapses of all rows targeting this tile, at most
+    const ParamRec *prm;     // its record (kTileUniform), else record of class 0 for its neurons
+    uint64_t seed;
+    float mu, f1, f2s;       // OU of its population (kTileOnePop)
+    uint32_t pop0;           // population of the first neuron
+    const uint16_t *cls;     // classes of its neurons
+    const float4 *dlt;       // gather: its neurons' delta
+    const InstDev *inst;
+    unsigned long long *bits;   // its words of set 0 (pull)
+    const int64_t *rowptr;   // rows of its neurons
+    uint32_t ntiles;         // tiles of the instance (words between the sets of bits: ntiles * kBitWords)
+    uint32_t inst_idx;       // index of inst
+};
+static_assert(sizeof(TileDesc) == 128, "two scalar loads of 64 bytes");
+
+// Queue of a target tile as the binning sees it (a set's first slot within
+// the instance's queue, capacity).
+struct alignas(16) QueueTile {
+    uint64_t off;
+    uint32_t cap;
+    uint32_t pad;
 };
 
 // Gather propagation: one workgroup of kGatherBlock threads gathers the
@@ -280,18 +326,21 @@ constexpr uint32_t kPassCountStride = 32;
 // Most workgroups of a k_bin launch (8 per CU on 256 CUs: all resident).
 constexpr uint32_t kBinGridMax = 2048;
 
-struct QueueSet {
+struct StepCtl;
+struct alignas(16) QueueSet {
+    const QueueTile *tile;   // [ntiles]
     uint32_t *count;    // [2][ntiles], tile t of set p at word count_slot(p * ntiles + t, cshift)
-    uint32_t ntiles;
-    uint32_t cshift;    // kCountShiftDense or kCountShiftSpread
     // Split binning (pass == null: off): k_step of parity p appends its
     // tiles' passes to `pass` (count at pcount[p * kPassCountStride]) and the
     // k_bin launch after it bins them; passes past pcap are binned by their
     // own tile.
     PassEntry *pass;
     uint32_t *pcount;
+    StepCtl *ctl;
+    uint32_t ntiles;
+    uint32_t cshift;    // kCountShiftDense or kCountShiftSpread
     uint32_t pcap;
-    uint32_t pad;
+    uint32_t pad[3];
 };
 
 // Sample request (reference stat_samples_kernel, stat_result.cpp:393-433).
