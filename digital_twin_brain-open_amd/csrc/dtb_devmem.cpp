@@ -147,6 +147,11 @@ NoAlloc::~NoAlloc()
     --t_no_alloc;
 }
 
+bool NoAlloc::active()
+{
+    return t_no_alloc > 0;
+}
+
 void *alloc(size_t bytes)
 {
     if (t_no_alloc > 0)

@@ -188,7 +188,7 @@ void Instance::init_common(std::vector<float> &&props, float dt, uint64_t seed, 
     col_.resize((size_t)std::max<int64_t>(nsyn_, 1));
     w_.resize((size_t)std::max<int64_t>(nsyn_, 1) * weight_bytes(wfmt_));
     pops_.resize(np);
-    step_.resize(4);
+    step_.resize(kStepPad + 2 * (size_t)((n_ + kBlock - 1) / kBlock) * kBitWords);
     counters_.resize(2 * (size_t)((n_ + kWave - 1) / kWave));
 
     derive_params(s);
@@ -226,6 +226,7 @@ Instance::Instance(const FanoutSpec &f, float dt, uint64_t seed, hipStream_t s)
     group_coverage_ = 1.0 - std::pow(1.0 - 1.0 / ngroups(), (double)f.K);
     // rows are ordered by target, K <= 8192
     gather_ok_ = (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
+    direct_ok_ = direct_fits();
 }
 
 Instance::~Instance() = default;
@@ -241,14 +242,14 @@ void Instance::count_tile_synapses(const NetworkHost &net)
     const int nt = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(hw ? hw : 4u, 16u), nsyn_ / (1 << 20)));
     std::vector<std::vector<uint32_t>> part(nt, std::vector<uint32_t>(nfine, 0u));
     std::vector<uint64_t> segs(nt, 0), gsegs(nt, 0);
-    std::vector<char> sorted(nt, 1);
+    std::vector<char> sorted(nt, 1), tile_sorted(nt, 1);
     std::vector<std::thread> th;
     for (int t = 0; t < nt; ++t) {
         th.emplace_back([&, t]() {
             const int64_t a = (int64_t)n_ * t / nt, b = (int64_t)n_ * (t + 1) / nt;
             uint32_t *c = part[t].data();
             uint64_t sg = 0, gs = 0;
-            bool ordered = true;
+            bool ordered = true, by_tile = true;
             for (int64_t r = a; r < b; ++r) {
                 uint32_t prev = 0xffffffffu, gprev = 0xffffffffu;
                 for (int64_t j = net.rowptr[r]; j < net.rowptr[r + 1]; ++j) {
@@ -258,6 +259,7 @@ void Instance::count_tile_synapses(const NetworkHost &net)
                     sg += tl != prev;
                     gs += gr != gprev;
                     ordered = ordered && (gprev == 0xffffffffu || gr >= gprev);
+                    by_tile = by_tile && (prev == 0xffffffffu || tl >= prev);
                     prev = tl;
                     gprev = gr;
                 }
@@ -266,22 +268,25 @@ void Instance::count_tile_synapses(const NetworkHost &net)
             segs[t] = sg;
             gsegs[t] = gs;
             sorted[t] = ordered ? 1 : 0;
+            tile_sorted[t] = ordered && by_tile ? 1 : 0;
         });
     }
     for (auto &x : th)
         x.join();
     uint64_t sg = 0, gs = 0;
-    bool ordered = true;
+    bool ordered = true, by_tile = true;
     for (int t = 0; t < nt; ++t) {
         sg += segs[t];
         gs += gsegs[t];
         ordered = ordered && sorted[t];
+        by_tile = by_tile && tile_sorted[t];
         for (uint32_t k = 0; k < nfine; ++k)
             tile_syn_[k] += part[t][k];
     }
     row_coverage_ = (double)sg / ((double)n_ * (double)nfine);
     group_coverage_ = (double)gs / ((double)n_ * (double)ngroups());
     gather_ok_ = ordered && nsyn_ > 0 && (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
+    direct_ok_ = by_tile && direct_fits();
 }
 
 uint32_t Instance::fired_capacity() const
@@ -302,8 +307,8 @@ void Instance::ensure_gather(hipStream_t s)
         fired_.resize(2 * (size_t)kFiredLists * fired_capacity());
         fired_.mutable_gpu_data();
         segidx_.resize((size_t)n_ * (ngroups() + 1u));
-        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ngroups(), segidx_.mutable_gpu_data(),
-                                    s));
+        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ngroups(), kGroupBits,
+                                    segidx_.mutable_gpu_data(), s));
         grec_.resize((size_t)nsyn_ * grec_words(wfmt_));
         DTB_HIP(launch_build_grec(col_.gpu_data(), w_.gpu_data(), wfmt_, (uint64_t)nsyn_, grec_.mutable_gpu_data(),
                                   s));
@@ -317,6 +322,38 @@ void Instance::ensure_gather(hipStream_t s)
         throw;
     }
     gather_built_ = true;
+}
+
+// The lookups of an emitted row (one per tile) against the queue entries it
+// would make.  Voxel networks, rows emitted per step: time of a step by
+// queues / direct: 130k neurons x 150 synapses (4 T / k = 14): 66: 7.2 / 7.2
+// us, 749: 17.4 / 11.7; 200k x 150 (21): 98: 8.2 / 8.5, 677: 14.5 / 13.6;
+// 260k x 300 (14): 78: 9.8 / 9.1, 1465: 25.5 / 23.4.  Rows that reach many
+// tiles cost the queues more: uniform 200k x 150 (coverage 0.17), 99: 10.0 /
+// 8.1, 1920: 74.5 / 26.3.
+bool Instance::direct_fits() const
+{
+    const double ntile = (double)((n_ + kBlock - 1) / kBlock);
+    return nsyn_ > 0 && nsyn_ < ((int64_t)1 << 32) && n_ <= kDirectMaxNeurons &&
+           (double)n_ * (ntile + 1.0) * 2.0 <= 12.0 * (double)nsyn_ &&
+           ((double)n_ * ntile <= 4.0 * (double)nsyn_ || row_coverage_ >= 0.125);
+}
+
+void Instance::ensure_direct(hipStream_t s)
+{
+    if (!direct_ok_)
+        throw Error(kInvalidParameter, "this network does not allow direct propagation");
+    if (direct_built())
+        return;
+    const uint32_t ntile = (n_ + kBlock - 1) / kBlock;
+    try {
+        tidx_.resize((size_t)n_ * (ntile + 1u));
+        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ntile, kTileBits, tidx_.mutable_gpu_data(),
+                                    s));
+    } catch (...) {
+        tidx_.resize(0);
+        throw;
+    }
 }
 
 void Instance::release_gather()
@@ -337,8 +374,7 @@ void Instance::clear_fired(hipStream_t s)
 uint64_t Instance::pull_bytes() const
 {
     const uint64_t ntile = (n_ + kBlock - 1) / kBlock;
-    return (uint64_t)nsyn_ * sizeof(uint32_t) * grec_words(wfmt_) + (ntile + 1) * sizeof(int64_t) +
-           2 * ntile * kBitWords * sizeof(unsigned long long);
+    return (uint64_t)nsyn_ * sizeof(uint32_t) * grec_words(wfmt_) + (ntile + 1) * sizeof(int64_t);
 }
 
 void Instance::ensure_pull(hipStream_t s)
@@ -359,8 +395,6 @@ void Instance::ensure_pull(hipStream_t s)
         cptr_.resize((size_t)ntile + 1);
         cptr_.upload(ptr.data(), ptr.size(), s);
         crec_.resize((size_t)nsyn_ * grec_words(wfmt_));
-        bits_.resize(2 * (size_t)ntile * kBitWords);
-        bits_.mutable_gpu_data();
         DataAllocator<uint32_t> cursor(ntile);
         DTB_HIP(hipMemsetAsync(cursor.mutable_gpu_data(), 0, (size_t)ntile * sizeof(uint32_t), s));
         DTB_HIP(launch_build_pull(rowptr_.gpu_data(), col_.gpu_data(), w_.gpu_data(), wfmt_, n_, cptr_.gpu_data(),
@@ -377,14 +411,12 @@ void Instance::release_pull()
 {
     crec_.resize(0);
     cptr_.resize(0);
-    bits_.resize(0);
     pull_built_ = false;
 }
 
 void Instance::clear_deferred(hipStream_t s)
 {
-    if (pull_built_)
-        DTB_HIP(hipMemsetAsync(step_.mutable_gpu_data() + 2, 0, 2 * sizeof(int64_t), s));
+    DTB_HIP(hipMemsetAsync(step_.mutable_gpu_data() + 2, 0, step_.size() - 2 * sizeof(int64_t), s));
 }
 
 uint32_t Instance::tile_synapses(uint32_t tile) const
@@ -957,15 +989,19 @@ void Instance::clear_spill(hipStream_t s)
     DTB_HIP(hipMemsetAsync(spill_.mutable_gpu_data(), 0, spill_.size(), s));
 }
 
-InstDev Instance::dev(uint32_t tile_base, bool gather, bool pull, uint32_t defer_min)
+InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min)
 {
     InstDev d{};
+    if (direct) {
+        if (!direct_built() || gather)
+            throw Error(kInternal, "direct propagation needs the tile offsets and no gather");
+        d.tidx = tidx_.gpu_data();
+    }
     if (pull) {
         if (!pull_built_ || gather)
             throw Error(kInternal, "pull propagation needs the in-edges and no gather");
         d.crec = crec_.gpu_data();
         d.cptr = cptr_.gpu_data();
-        d.bits = bits_.mutable_gpu_data();
         d.defer_min = defer_min;
     }
     if (gather) {
@@ -983,6 +1019,7 @@ InstDev Instance::dev(uint32_t tile_base, bool gather, bool pull, uint32_t defer
     d.pmask = dense_params_ ? ~(uint32_t)(kBlock - 1) : 0u;
     d.blocked = blocked_.gpu_data();
     d.state = state_.mutable_gpu_data();
+    d.bits = reinterpret_cast<unsigned long long *>(step_.mutable_gpu_data() + kStepPad);
     d.dlt = dlt_.mutable_gpu_data();
     d.spill = spill_.mutable_gpu_data();
     d.queue = queue_.mutable_gpu_data();
@@ -1025,7 +1062,7 @@ TileDesc Instance::tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, 
     r.inst = inst;
     r.inst_idx = idx;
     r.step = d.step;
-    r.bits = d.bits ? d.bits + (size_t)t * kBitWords : nullptr;
+    r.bits = d.bits + (size_t)t * kBitWords;
     r.rowptr = d.rowptr + r.begin;
     r.seed = d.seed;
     r.queue = d.queue + qoff;
@@ -1035,6 +1072,7 @@ TileDesc Instance::tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, 
     r.pop0 = pop0;
     r.ntiles = d.ntiles;
     r.flags = (d.use_ou ? kTileOu : 0u) | (d.crec ? kTilePull : 0u) | (d.segidx ? kTileGather : 0u) |
+              (d.tidx ? kTileDirect : 0u) |
               (d.t_steps == 1 ? kTileOneSub : 0u) | (d.rec_stat ? kTileStat : 0u);
     if (tile_cls_[t] != 0u) {
         r.flags |= kTileUniform;

@@ -108,6 +108,7 @@ size_t cached_bytes(int device);     // bytes held in the cache
 struct NoAlloc {
     NoAlloc();
     ~NoAlloc();
+    static bool active();   // on this thread
     NoAlloc(const NoAlloc &) = delete;
     NoAlloc &operator=(const NoAlloc &) = delete;
 };
@@ -319,9 +320,10 @@ public:
     void counters(int64_t *step, uint64_t *events, uint64_t *spikes, hipStream_t s);
 
     // Kernel descriptor; `gather`: propagate by gather (ensure_gather first);
+    // `direct`: by direct propagation (ensure_direct first);
     // defer_min > 0 with the in-edges built: pull propagation (a tile with
     // at least defer_min emitted rows defers them to the pull).
-    InstDev dev(uint32_t tile_base, bool gather, bool pull, uint32_t defer_min);
+    InstDev dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min);
     // Descriptor of tile t for the step kernels; inst: the device address of
     // the instance's descriptor `d`, idx its index; pop0: population of the
     // tile's first neuron; qoff, qcap: its queue.
@@ -374,8 +376,18 @@ public:
     void ensure_pull(hipStream_t s);
     void release_pull();
     bool pull_built() const { return pull_built_; }
-    // Forgets deferred rows (after the pending input was folded or dropped).
+    // Forgets emitted and deferred rows (after the pending input was folded
+    // or dropped).
     void clear_deferred(hipStream_t s);
+
+    // Direct propagation: possible when every row is ordered by target and at
+    // most kGatherMaxRow long, the instance has at most kDirectMaxNeurons
+    // neurons, the tile offsets ([n][ntiles + 1] x 2 bytes) are no larger
+    // than the synapse arrays and a row has enough synapses for its lookups.
+    bool direct_allowed() const { return direct_ok_; }
+    void ensure_direct(hipStream_t s);
+    void release_direct() { tidx_.resize(0); }
+    bool direct_built() const { return tidx_.count() != 0; }
 
 private:
     void init_common(const float *props, float dt, uint64_t seed, hipStream_t s);
@@ -418,7 +430,10 @@ private:
     DataAllocator<uint8_t> w_;                     // [nsyn] weight pairs in format wfmt_
     uint32_t wfmt_ = kWeightF32;
     DataAllocator<PopDev> pops_;
-    DataAllocator<int64_t> step_;                   // [2] step index, [2] deferral stamps
+    // [2] step index, [2] deferral stamps, padded to 16 words; then the
+    // emitted and deferred rows, [2][ntiles][kBitWords]
+    DataAllocator<int64_t> step_;
+    static constexpr size_t kStepPad = 16;
     DataAllocator<unsigned long long> counters_;   // per wave: events, spikes
     // [steps][rec_slots_][stride], with more than one slot followed by the
     // rows of the slots' sums ([npop], [npop][kStatFields])
@@ -441,6 +456,9 @@ private:
     double group_coverage_ = 0.0;         // mean fraction of the gather groups one row reaches
     bool gather_ok_ = false;              // gather_allowed()
     bool gather_built_ = false;           // segidx_, fired_, fcount_ built
+    bool direct_ok_ = false;              // direct_allowed()
+    bool direct_fits() const;             // its conditions on the sizes
+    DataAllocator<uint16_t> tidx_;        // [n][ntiles + 1] tile offsets (direct propagation)
     DataAllocator<uint16_t> segidx_;      // [n][ngroups + 1] group offsets (built on demand)
     DataAllocator<uint32_t> grec_;        // [nsyn][grec_words] gather records (built with segidx_)
     DataAllocator<uint32_t> fired_;       // [2][kFiredLists][fired_capacity()] fired rows
@@ -449,7 +467,6 @@ private:
     DataAllocator<uint32_t> crec_;        // [nsyn][grec_words] in-edges: key (source row | target in tile |
                                           // channel bit), weight pair bits
     DataAllocator<int64_t> cptr_;         // [ntiles + 1] first in-edge of each target tile
-    DataAllocator<unsigned long long> bits_;   // [2][ntiles][kBitWords] emitted / deferred rows
     uint32_t gamma_calls_ = 0;            // gamma draw streams used
     std::vector<uint32_t> tile_cls_;      // per tile: 1 + shared parameter class, or 0
 };
@@ -515,11 +532,9 @@ public:
     // queues still pull).  Off: queues only, past-capacity synapses through
     // the spill accumulators.  Every setting gives the same results.
     void set_pull(bool on, uint32_t defer_min);
-    // Split binning: the fired rows' binning passes run in a second launch
-    // per step (k_bin) spread over every CU, instead of in the tiles whose
-    // neurons fired.  Results never depend on it.
-    // cap: entries of the pass list (0: sized by the instances); passes past
-    // it are binned by their own tile.
+    // Split binning: the fired rows are binned by a second launch per step
+    // (k_bin) over groups of tiles, instead of by the tiles whose neurons
+    // fired.  Results never depend on it, and nothing on cap.
     void set_split(bool on, uint32_t cap)
     {
         if (on != split_ || cap != split_cap_) {
@@ -532,6 +547,7 @@ public:
     uint32_t split_cap() const { return split_cap_; }
     bool pull_on() const { return pull_on_; }
     uint32_t defer_min() const { return defer_min_; }
+    // (a direct instance pulls the steps whose emitted rows are many)
     bool uses_pull(const Instance &p) const { return pull_on_ && p.pull_built() && !use_gather(p); }
     // Queue capacity per tile: min(synapses targeting it, floor +
     // (synapses >> shift)); shift 0 keeps the exact worst case.
@@ -581,7 +597,7 @@ public:
 private:
     void rebuild();
     void launch_step();        // one step at parity par_, then par_ ^= 1
-    void launch_step_k();
+    void launch_step_k(hipEvent_t *ev = nullptr);   // ev: 8 events (start and stop of up to four kernels)
     void launch_aux();         // materialize + sample after a step, if samples are set
     void drop_graphs();
     QueueSet queues();
@@ -601,15 +617,14 @@ private:
     uint32_t pass_k_ = kPassKDefault;      // synapses per lane in a binning pass
     uint32_t wfmt_ = kWeightF32;           // weight format of every instance in the tables, or kWeightAny
     bool stat_ = false;                    // some instance in the tables records population statistics
-    uint32_t queue_floor_ = 4096, queue_shift_ = 3;   // queue_capacity
+    static constexpr uint32_t kQueueFloorDefault = 4096, kQueueShiftDefault = 3;
+    uint32_t queue_floor_ = kQueueFloorDefault, queue_shift_ = kQueueShiftDefault;   // queue_capacity
     bool tuning_ = false;                  // autotune running: gather buffers are kept
     bool pull_on_ = true;                  // pull propagation where in-edges fit
     bool split_ = false;                   // split binning (k_bin)
-    uint32_t split_cap_ = 0;               // requested pass-list entries (0: automatic)
-    DataAllocator<PassEntry> d_pass_;      // pass list of split binning
-    DataAllocator<uint32_t> d_pcount_;     // its two counts, kPassCountStride words apart
-    uint32_t pass_cap_ = 0;                // entries of d_pass_ in use (0: split binning off)
-    uint32_t bin_grid_ = 0;                // k_bin workgroups
+    uint32_t split_cap_ = 0;               // as given to set_split
+    DataAllocator<BinDesc> d_bins_;        // source groups of the queue instances
+    uint32_t nbins_ = 0, bin_tiles_ = 0;   // groups (0: tiles bin their own rows), tiles of the largest queue instance
     uint32_t defer_min_ = kDeferMinDefault;
     void try_pull(Instance &p, hipStream_t s);   // builds p's in-edges if on and they fit
     DataAllocator<InstDev> d_insts_;
@@ -623,6 +638,19 @@ private:
     DataAllocator<GroupDesc> d_groups_;    // gather groups of the gather instances
     uint32_t ngroups_ = 0;
     void launch_gather_k(uint32_t par);    // k_gather of parity par, if any instance gathers
+    // Whether instance p takes its input by direct propagation: the automatic
+    // layout (or the autotuner's pick of it) with no propagation setting of
+    // the user's own, and p allows it.  (It then needs its in-edges, which
+    // volleys are taken through: without them 200k neurons' volley from rest
+    // takes 7.0 ms, by queues and spill 2.2.)
+    bool wants_direct(const Instance &p) const
+    {
+        return (count_layout_ == kLayoutAuto || tuned_direct_) && !split_ && pull_on_ && queue_floor_ == kQueueFloorDefault &&
+               queue_shift_ == kQueueShiftDefault && defer_min_ == kDeferMinDefault && p.direct_allowed();
+    }
+    bool try_direct(Instance &p);          // builds p's tile offsets if they fit
+    uint32_t nqueue_tiles_ = 0;            // tiles of the queue and gather instances (first in the tables)
+    bool tuned_direct_ = false;            // the autotuner's (dense, default pass) candidate ran direct
     hipGraphExec_t graph_[2] = {nullptr, nullptr};   // by starting parity
     int graph_steps_[2] = {0, 0};
 };

@@ -89,9 +89,10 @@ void Engine::set_schedule(uint32_t pass_k, int layout)
         throw Error(kInvalidParameter, "pass size must be 1, 2 or 4 synapses per lane");
     if (layout != kLayoutAuto && layout != kLayoutDense && layout != kLayoutSpread && layout != kLayoutGather)
         throw Error(kInvalidParameter, "unknown propagation layout");
-    if (pass_k != pass_k_ || layout != count_layout_) {
+    if (pass_k != pass_k_ || layout != count_layout_ || tuned_direct_) {
         pass_k_ = pass_k;
         count_layout_ = layout;
+        tuned_direct_ = false;
         dirty_ = true;   // graphs hold the old kernel; counts move to the new layout
     }
 }
@@ -99,6 +100,24 @@ void Engine::set_schedule(uint32_t pass_k, int layout)
 bool Engine::use_gather(const Instance &p) const
 {
     return p.gather_allowed() && count_layout_ == kLayoutGather;
+}
+
+bool Engine::try_direct(Instance &p)
+{
+    if (p.direct_built())
+        return true;
+    if (devmem::NoAlloc::active())
+        return false;
+    try {
+        p.ensure_direct(stream_);
+        return true;
+    } catch (const Error &e) {
+        // without device memory for the offsets the instance keeps queues
+        // (same results)
+        if (e.code != kOutOfMemory)
+            throw;
+        return false;
+    }
 }
 
 bool Engine::any_gather() const
@@ -130,6 +149,12 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
     // buffers) the seventh turn runs the default schedule and is not a
     // candidate, so the number of steps does not depend on the networks.
     int nc = gather_possible() ? 7 : 6;
+    // The default pass with dense counts stands for the automatic layout:
+    // direct propagation for the instances that allow it.
+    auto set_candidate = [&](int s) {
+        set_schedule(ks[s], layouts[s]);
+        tuned_direct_ = layouts[s] == kLayoutDense && ks[s] == kPassKDefault;
+    };
     // The cost of a step follows the network's activity, which drifts and
     // bursts; so the schedules take turns in short windows (kAutotuneWindow
     // timed steps, after 2 steps that apply the schedule) over the whole
@@ -148,7 +173,7 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
     for (int64_t r = -1; r < rounds; ++r) {
         for (int s = 0; s < 7; ++s) {
             if (s < nc)
-                set_schedule(ks[s], layouts[s]);
+                set_candidate(s);
             else
                 set_schedule(kPassKDefault, kLayoutDense);
             try {
@@ -178,7 +203,7 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
             us[i] = i < nc ? (float)(t_sum[i] * 1e3 / (double)(rounds * kAutotuneWindow)) : 0.0f;
     const uint32_t bk = ks[bi];
     const int bl = layouts[bi];
-    set_schedule(bk, bl);
+    set_candidate(bi);
     dirty_ = true;   // the next table build returns gather buffers no longer used
     if (best_k)
         *best_k = bk;
@@ -246,7 +271,7 @@ uint32_t Engine::queue_capacity(uint32_t synapses) const
     // suffice; fewer keep the queues small, and the synapses past the
     // capacity take the spill path.
     const uint64_t c = (uint64_t)queue_floor_ + (synapses >> queue_shift_);
-    return (uint32_t)std::min<uint64_t>(synapses, c);
+    return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(synapses, c), 0x7fffffffull);
 }
 
 void Engine::drop_graphs()
@@ -267,11 +292,6 @@ QueueSet Engine::queues()
     q.count = d_qcnt_.mutable_gpu_data();
     q.ntiles = ntiles_;
     q.cshift = cshift_;
-    if (pass_cap_ > 0) {
-        q.pass = d_pass_.mutable_gpu_data();
-        q.pcount = d_pcount_.mutable_gpu_data();
-        q.pcap = pass_cap_;
-    }
     return q;
 }
 
@@ -305,12 +325,26 @@ void Engine::rebuild()
     stat_ = false;
     uint64_t total = 0;
     double coverage = 0.0;
-    uint64_t pass_want = 0;   // split binning: pass-list entries for the queue instances
+    std::vector<BinDesc> bins;
+    bin_tiles_ = 0;
     uint32_t fmt = kWeightAny + 1;   // the instances' common weight format (kWeightAny: mixed)
-    for (size_t slot = 0; slot < insts_.size(); ++slot) {
+    // The tiles of the queue and gather instances come first (their index is
+    // their queue count's), then those of the direct ones.
+    std::vector<size_t> order;
+    std::vector<char> direct(insts_.size(), 0);
+    for (size_t slot = 0; slot < insts_.size(); ++slot)
+        if (insts_[slot] && wants_direct(*insts_[slot])) {
+            try_pull(*insts_[slot], stream_);
+            direct[slot] = insts_[slot]->pull_built() && try_direct(*insts_[slot]);
+        }
+    for (int d = 0; d < 2; ++d)
+        for (size_t slot = 0; slot < insts_.size(); ++slot)
+            if (insts_[slot] && direct[slot] == d)
+                order.push_back(slot);
+    nqueue_tiles_ = 0;
+    for (size_t slot : order) {
         Instance *p = insts_[slot].get();
-        if (!p)
-            continue;
+        const bool dir = direct[slot] != 0;
         const uint32_t idx = (uint32_t)table.size();
         tile_base_[slot] = (uint32_t)tiles.size();
         stat_ = stat_ || p->stat_mask() != 0;
@@ -338,7 +372,9 @@ void Engine::rebuild()
         if (!gat)
             try_pull(*p, stream_);
         const bool pl = !gat && pull_on_ && p->pull_built();
-        table.push_back(p->dev(tile_base_[slot], gat, pl, defer_min_));
+        if (!dir && !wants_direct(*p) && !tuning_)
+            p->release_direct();   // (the old tables, settled above, were the last to use it)
+        table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_));
         const auto &pb = p->pop_begin();
         uint32_t q = 0;
         for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
@@ -353,16 +389,31 @@ void Engine::rebuild()
             for (uint32_t k = 0; k < ids.size(); ++k)
                 samples.push_back(SampleDev{idx, ids[k], k, 0});
         }
-        if (!gat) {
+        if (!dir)
+            nqueue_tiles_ = (uint32_t)tiles.size();
+        if (!gat && !dir) {
             total += p->n();
             coverage += p->row_coverage() * p->n();
-            // a step listing one pass per 1/64 of the neurons and per 4096
-            // synapses fits; beyond, tiles bin their own passes
-            pass_want += p->n() / 64 + (uint64_t)p->nsyn() / 4096;
+            const uint32_t nt = split_ ? (p->n() + kBlock - 1) / kBlock : 0u;
+            bin_tiles_ = std::max(bin_tiles_, nt);
+            for (uint32_t t = 0; t < nt; t += kBinTiles)
+                bins.push_back(BinDesc{d_insts_.gpu_data() + idx, t, std::min(kBinTiles, nt - t)});
         }
     }
     if (total > 0xffffffffull || tiles.size() > 0xffffffffull)
         throw Error(kInvalidParameter, "too many neurons in one engine");
+    // Workgroups are dealt to the 8 XCDs by index mod 8: each XCD gets a
+    // contiguous range of the direct tiles, so tiles that share cache lines
+    // of a row's offsets and synapses meet in one L2.
+    {
+        const size_t nd = tiles.size() - nqueue_tiles_;
+        std::vector<TileDesc> dealt(nd);
+        for (size_t k = 0; k < nd; ++k) {
+            const size_t x = k & 7u;
+            dealt[k] = tiles[nqueue_tiles_ + x * (nd >> 3) + std::min<size_t>(x, nd & 7u) + (k >> 3)];
+        }
+        std::copy(dealt.begin(), dealt.end(), tiles.begin() + nqueue_tiles_);
+    }
     ninst_ = (uint32_t)table.size();
     wfmt_ = fmt > kWeightAny ? kWeightF32 : fmt;
     ntiles_ = (uint32_t)tiles.size();
@@ -391,16 +442,9 @@ void Engine::rebuild()
     else
         cshift_ = (total > 0 && coverage / (double)total > kSpreadCoverage) ? kCountShiftSpread : kCountShiftDense;
     grow(d_qcnt_, count_words(2 * std::max<size_t>(tiles.size(), 1), cshift_));
-    if (split_ && total > 0) {
-        pass_cap_ = split_cap_ != 0 ? split_cap_
-                                    : (uint32_t)std::min<uint64_t>(pass_want + 4096, (uint64_t)4 << 20);
-        grow(d_pass_, pass_cap_);
-        grow(d_pcount_, 2 * kPassCountStride);
-        bin_grid_ = std::min<uint32_t>(kBinGridMax, std::max<uint32_t>(64, (uint32_t)(total / kBlock)));
-    } else {
-        pass_cap_ = 0;
-        bin_grid_ = 0;
-    }
+    nbins_ = (uint32_t)bins.size();
+    grow(d_bins_, bins.size());
+    d_bins_.mutable_gpu_data();
     // Allocate (zero-filled) everything the step kernels touch before any
     // capture: no allocation may happen while a graph is being recorded.
     d_qcnt_.mutable_gpu_data();
@@ -408,11 +452,10 @@ void Engine::rebuild()
     d_recs_.mutable_gpu_data();
     d_groups_.mutable_gpu_data();
     DTB_HIP(hipMemsetAsync(d_qcnt_.mutable_gpu_data(), 0, d_qcnt_.size(), stream_));
-    if (pass_cap_ > 0)
-        DTB_HIP(hipMemsetAsync(d_pcount_.mutable_gpu_data(), 0, d_pcount_.size(), stream_));
     d_insts_.upload(table.data(), table.size(), stream_);
     d_tiles_.upload(tiles.data(), tiles.size(), stream_);
     d_qtiles_.upload(qtiles.data(), qtiles.size(), stream_);
+    d_bins_.upload(bins.data(), bins.size(), stream_);
     const QueueSet qset = queues();
     d_queues_.upload(&qset, 1, stream_);
     d_groups_.upload(groups.data(), groups.size(), stream_);
@@ -424,14 +467,20 @@ void Engine::rebuild()
 
 void Engine::launch_gather_k(uint32_t par)
 {
-    DTB_HIP(launch_gather(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par, wfmt_, stream_));
+    DTB_HIP(launch_gather(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par, wfmt_, nullptr, nullptr, stream_));
 }
 
-void Engine::launch_step_k()
+void Engine::launch_step_k(hipEvent_t *ev)
 {
-    launch_gather_k(par_);
-    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), ntiles_, d_queues_.gpu_data(), par_, pass_k_, wfmt_, stat_, stream_));
-    DTB_HIP(launch_bin_kernel(bin_grid_, d_insts_.gpu_data(), queues(), par_, pass_k_, wfmt_, nullptr, nullptr, stream_));
+    // start and stop events of the i-th kernel, or none
+    auto e = [&](int i) { return ev ? ev[i] : nullptr; };
+    DTB_HIP(launch_gather(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par_, wfmt_, e(0), e(1), stream_));
+    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), nqueue_tiles_, nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin,
+                               pass_k_, d_queues_.gpu_data(), par_, wfmt_, stat_, e(2), e(3), stream_));
+    DTB_HIP(launch_bin_kernel(d_bins_.gpu_data(), nbins_, bin_tiles_, d_queues_.gpu_data(), par_, wfmt_, e(4), e(5),
+                              stream_));
+    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data() + nqueue_tiles_, ntiles_ - nqueue_tiles_, StepMode::direct, pass_k_,
+                               d_queues_.gpu_data(), par_, wfmt_, stat_, e(6), e(7), stream_));
 }
 
 void Engine::launch_aux()
@@ -559,45 +608,37 @@ void Engine::run_timed(int64_t steps, float *ms_step)
     if (ninst_ == 0 || steps <= 0)
         return;
     pending_ = true;
-    // Every step kernel records its own start and stop events (at the
-    // dispatch boundaries, on the engine stream); they are read back once
-    // per chunk so the launch pipeline is not drained every step.
-    // With gather instances the step is two kernels (k_gather, k_step),
-    // each timed.
+    // Every kernel of a step (k_gather, k_step over the queue and gather
+    // tiles, k_bin, k_step over the direct tiles: those with a grid) records
+    // its own start and stop events at the dispatch boundaries, on the engine
+    // stream; they are read back once per chunk so the launch pipeline is not
+    // drained every step.
+    const uint32_t grid[4] = {ngroups_, nqueue_tiles_, nbins_, ntiles_ - nqueue_tiles_};
+    int last = 0;
+    for (int i = 0; i < 4; ++i)
+        if (grid[i] > 0)
+            last = i;
     const int64_t chunk = 256;
-    std::vector<hipEvent_t> ev((size_t)(6 * chunk));
+    std::vector<hipEvent_t> ev((size_t)(8 * chunk));
     for (auto &e : ev)
         DTB_HIP(hipEventCreate(&e));
     double ts = 0.0;
     for (int64_t base = 0; base < steps; base += chunk) {
         const int64_t m = std::min<int64_t>(chunk, steps - base);
         for (int64_t k = 0; k < m; ++k) {
-            hipEvent_t *e = &ev[(size_t)(6 * k)];
-            if (ngroups_ > 0)
-                DTB_HIP(launch_gather_timed(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par_, wfmt_, e[2], e[3],
-                                            stream_));
-            DTB_HIP(launch_step_kernel_timed(d_tiles_.gpu_data(), ntiles_, d_queues_.gpu_data(), par_, pass_k_, wfmt_, stat_, e[0], e[1],
-                                             stream_));
-            if (pass_cap_ > 0)
-                DTB_HIP(launch_bin_kernel(bin_grid_, d_insts_.gpu_data(), queues(), par_, pass_k_, wfmt_, e[4], e[5], stream_));
+            launch_step_k(&ev[(size_t)(8 * k)]);
             par_ ^= 1u;
             launch_aux();
         }
-        DTB_HIP(hipEventSynchronize(ev[(size_t)(6 * (m - 1) + (pass_cap_ > 0 ? 5 : 1))]));
-        for (int64_t k = 0; k < m; ++k) {
-            hipEvent_t *e = &ev[(size_t)(6 * k)];
-            float a = 0.0f;
-            DTB_HIP(hipEventElapsedTime(&a, e[0], e[1]));
-            ts += a;
-            if (ngroups_ > 0) {
-                DTB_HIP(hipEventElapsedTime(&a, e[2], e[3]));
+        DTB_HIP(hipEventSynchronize(ev[(size_t)(8 * (m - 1) + 2 * last + 1)]));
+        for (int64_t k = 0; k < m; ++k)
+            for (int i = 0; i < 4; ++i) {
+                if (grid[i] == 0)
+                    continue;
+                float a = 0.0f;
+                DTB_HIP(hipEventElapsedTime(&a, ev[(size_t)(8 * k + 2 * i)], ev[(size_t)(8 * k + 2 * i + 1)]));
                 ts += a;
             }
-            if (pass_cap_ > 0) {
-                DTB_HIP(hipEventElapsedTime(&a, e[4], e[5]));
-                ts += a;
-            }
-        }
     }
     for (auto &e : ev)
         DTB_HIP(hipEventDestroy(e));

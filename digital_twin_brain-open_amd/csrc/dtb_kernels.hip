@@ -268,6 +268,21 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Inclusive sum over the 64 lanes with DPP: shifts by 1, 2, 4, 8 within each
+// row of 16 lanes (lanes shifted in from outside the row read 0), then the
+// last lane of row 0 / 2 into rows 1 / 3 and the last lane of row 1 into rows
+// 2 and 3.
+__device__ __forceinline__ uint32_t wave_add_scan(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);   // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);   // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);   // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
 // The LDS sums are channel-major: channel c of row i at acc[c * rows + i].
 // A wave's 64-bit atomics go to random rows; with the rows 8 bytes apart
 // (not 32, as row-major would put them) they spread over twice as many LDS
@@ -400,6 +415,198 @@ __device__ __forceinline__ void pull_tile(unsigned long long *acc, const Inst &I
         pull_loop<kWeightF16>(acc, rec, bits, len, tid);
     else
         pull_loop<kWeightU8>(acc, rec, bits, len, tid);
+}
+
+// LDS of a tile's direct propagation.
+struct DirectList {
+    uint32_t row[kDirectRows];      // emitted rows
+    uint32_t first[2 * kBlock];     // of two rows per thread: first synapse of the row's segment,
+    uint32_t off[2 * kBlock];       // and items before it
+    uint16_t item[kDirectItems * kBlock];   // per synapse of a window: its row's slot
+    uint32_t n;
+    uint32_t wave[kBlock / kWave];
+};
+
+// Adds the listed rows' segments for tile t into acc.  A thread looks up two
+// rows (offsets and start), the segments (mostly none to a few synapses) are
+// laid end to end, and consecutive threads take consecutive synapses,
+// kDirectItems each in flight: a tile whose rows' segments are long (its own
+// voxel's) is not left to the few threads that found them.
+template <uint32_t kFmt, typename Inst>
+__device__ __forceinline__ void direct_rows(unsigned long long *acc, const Inst &I, DirectList &ls, uint32_t n,
+                                            uint32_t t, uint32_t tid)
+{
+    const uint32_t wfmt = kFmt != kWeightAny ? kFmt : I.wfmt;
+    const uint32_t stride = I.ntiles + 1u;
+    const uint32_t lane = tid & (kWave - 1u), w = tid / kWave;
+    const auto col = gp(I.col);
+    const void *wt = I.w;
+    for (uint32_t k0 = 0; k0 < n; k0 += 2u * kBlock) {
+        uint32_t len[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+            len[i] = 0u;
+            const uint32_t k = k0 + i * kBlock + tid;
+            if (k < n) {
+                const uint32_t r = ls.row[k];
+                const auto sg = gp(I.tidx) + ((size_t)r * stride + t);
+                const uint32_t a = sg[0], e = sg[1];
+                ls.first[i * kBlock + tid] = (uint32_t)gp(I.rowptr)[r] + a;   // (fewer than 2^32 synapses)
+                len[i] = e - a;
+            }
+        }
+        const uint32_t incl = wave_add_scan(len[0] + len[1]);
+        if (lane == kWave - 1)
+            ls.wave[w] = incl;
+        __syncthreads();
+        uint32_t off = incl - len[0] - len[1], total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < (uint32_t)kBlock / kWave; ++k) {
+            const uint32_t v = ls.wave[k];
+            off += k < w ? v : 0u;
+            total += v;
+        }
+        ls.off[tid] = off;
+        ls.off[kBlock + tid] = off + len[0];
+        constexpr uint32_t kWin = kDirectItems * kBlock;
+        for (uint32_t w0 = 0; w0 < total; w0 += kWin) {
+            // the items of this thread's segments that fall into the window
+#pragma unroll
+            for (uint32_t i = 0; i < 2u; ++i) {
+                const uint32_t b = off + (i ? len[0] : 0u);
+                for (uint32_t k = max(b, w0); k < min(b + len[i], w0 + kWin); ++k)
+                    ls.item[k - w0] = (uint16_t)(i * kBlock + tid);
+            }
+            __syncthreads();
+            const uint32_t m = min(total - w0, kWin);
+            uint32_t cv[kDirectItems];
+            unsigned long long wv[kDirectItems];
+#pragma unroll
+            for (uint32_t u = 0; u < kDirectItems; ++u) {
+                const uint32_t k = u * kBlock + tid;
+                if (k < m) {
+                    const uint32_t slot = ls.item[k];
+                    const uint32_t at = ls.first[slot] + (w0 + k - ls.off[slot]);
+                    cv[u] = col[at];
+                    wv[u] = w_raw(wt, (size_t)at, wfmt);
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kDirectItems; ++u)
+                if (u * kBlock + tid < m) {
+                    const float2 wp = w_decode(wv[u], wfmt);
+                    const uint32_t row = cv[u] & 0xffu, c0 = (cv[u] & kKindBit) ? 2u : 0u;
+                    atomicAdd(&acc[acc_at(row, c0, kBlock)], f32_to_q40(wp.x));
+                    atomicAdd(&acc[acc_at(row, c0 + 1u, kBlock)], f32_to_q40(wp.y));
+                }
+            if (w0 + kWin < total)
+                __syncthreads();
+        }
+        if (k0 + 2u * kBlock < n)
+            __syncthreads();
+    }
+}
+
+// Direct propagation: adds into acc (zeroed, as ls.n is; both visible) the
+// synapses onto tile t of every row emitted into set `set`.  Each thread
+// reads the emitted rows of up to kDirectRounds source tiles (the count and
+// the first ids; their bits where there are more) and lists them in LDS.  More rows than the list holds are taken in rounds, by rank; where
+// reading the tile's in-edges is cheaper than one segment lookup per row
+// (volleys), the tile pulls.  Called by the whole workgroup; ends without a
+// barrier.  Returns whether the tile pulled.
+template <uint32_t kFmt, typename Inst>
+__device__ __forceinline__ bool direct_tile(unsigned long long *acc, DirectList &ls, const Inst &I, uint32_t set,
+                                            uint32_t t, uint32_t tid)
+{
+    const uint32_t T = I.ntiles;
+    typedef unsigned long long u64x4 __attribute__((ext_vector_type(4)));
+    // per tile: 4 words of bits, then a word of the count and the first ids
+    const auto ids = gp(I.bits + (size_t)set * T * kBitWords + 4u);
+    const auto bits = (const __attribute__((address_space(1))) u64x4 *)gp(I.bits + (size_t)set * T * kBitWords);
+    // every round's rows in flight before the first is used
+    unsigned long long b4[kDirectRounds];
+#pragma unroll
+    for (uint32_t i = 0; i < kDirectRounds; ++i)
+        if (i * kBlock < T) {
+            const uint32_t src = i * kBlock + tid;
+            b4[i] = src < T ? ids[(size_t)src * kBitWords] : 0ull;
+        }
+    // places in the list: one LDS add per wave
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kDirectRounds; ++i)
+        if (i * kBlock < T)
+            mine += (uint32_t)b4[i] & 0xffffu;
+    const uint32_t incl = wave_add_scan(mine);
+    uint32_t at = 0;
+    if ((tid & (kWave - 1u)) == kWave - 1u)
+        at = atomicAdd(&ls.n, incl);
+    at = (uint32_t)__builtin_amdgcn_readlane((int)at, kWave - 1) + incl - mine;
+#pragma unroll
+    for (uint32_t i = 0; i < kDirectRounds; ++i) {
+        if (i * kBlock >= T)
+            continue;
+        unsigned long long b = b4[i];
+        const uint32_t c = (uint32_t)b & 0xffffu, src = i * kBlock + tid, r0 = src * kBlock;
+        const uint32_t last = min(at + c, kDirectRows);   // rows past the list are taken in rounds, below
+        if (c <= kDirectIds) {
+            // the usual case: ids in bytes 2..7
+            for (uint32_t k = at; k < last; ++k) {
+                b >>= 8;
+                ls.row[k] = r0 + ((uint32_t)(b >> 8) & 0xffu);
+            }
+        } else {
+            const u64x4 e = bits[2u * src];
+            uint32_t k = at;
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q)
+                for (unsigned long long m = e[q]; m != 0ull && k < last; m &= m - 1ull, ++k)
+                    ls.row[k] = r0 + q * kWave + (uint32_t)__ffsll((long long)m) - 1u;
+        }
+        at += c;
+    }
+    __syncthreads();
+    const uint32_t n = ls.n;
+    if (n <= kDirectRows) {
+        direct_rows<kFmt>(acc, I, ls, n, t, tid);
+        return false;
+    }
+    // Bytes either way: a lookup touches a line of offsets, and a short
+    // segment a line of columns and one of weights per few synapses; the
+    // in-edges are one stream (a volley step of 200k x 150 pulls in 110-146
+    // us, with every row in rounds 7 ms).
+    if (I.crec != nullptr) {
+        const uint64_t in_edges = (uint64_t)(gp(I.cptr)[t + 1] - gp(I.cptr)[t]);
+        if ((uint64_t)n * (64u * (uint64_t)I.n + 24u * in_edges) > 12u * in_edges * (uint64_t)I.n) {
+            pull_tile<kFmt>(acc, I, set, t, true, tid);
+            return true;
+        }
+    }
+    // ranks: rows of the threads before, then a thread's own in tile order
+    const uint32_t lane = tid & (kWave - 1u), w = tid / kWave;
+    if (lane == kWave - 1)
+        ls.wave[w] = incl;
+    __syncthreads();
+    uint32_t rank0 = incl - mine;
+    for (uint32_t k = 0; k < w; ++k)
+        rank0 += ls.wave[k];
+    for (uint32_t first = 0; first < n; first += kDirectRows) {
+        if (rank0 < first + kDirectRows && rank0 + mine > first) {
+            uint32_t at = rank0;
+            for (uint32_t src = tid; src < T; src += kBlock) {
+                const u64x4 b = bits[2u * src];
+#pragma unroll
+                for (uint32_t q = 0; q < 4u; ++q)
+                    for (unsigned long long m = b[q]; m != 0ull; m &= m - 1ull, ++at)
+                        if (at >= first && at < first + kDirectRows)
+                            ls.row[at - first] = src * kBlock + q * kWave + (uint32_t)__ffsll((long long)m) - 1u;
+            }
+        }
+        __syncthreads();
+        direct_rows<kFmt>(acc, I, ls, min(n - first, kDirectRows), t, tid);
+        __syncthreads();
+    }
+    return false;
 }
 
 // A statistic's value as the exact integer rint(x * 2^24).
@@ -996,8 +1203,14 @@ __device__ __forceinline__ void put_tile_rec(TilePtr d, InstPtr I, uint32_t tid,
     }
 }
 
+// How the tiles of a k_step launch get their input and pass on their rows:
+// from queues (or gather's delta, a flag of the tile), the emitted rows binned
+// by the tile itself (kTileBin) or left to a k_bin launch (kQueues); or from
+// the emitted rows directly (kDirect).
+enum : int { kQueues = 0, kDirect = 1, kTileBin = 2 };
+
 // What a tile's step reads before its queue.
-template <bool kUniform>
+template <bool kUniform, int kMode>
 struct StepIn {
     TilePtr d;
     QueuePtr q;
@@ -1011,7 +1224,8 @@ struct StepIn {
     {
         d = tp;
         q = qp;
-        cnt = *cp(count(par));
+        if (kMode != kDirect)
+            cnt = *cp(count(par));
         step = cp(d->step)[par];
         stamp = cp(d->step)[2u + par];
         active = tid < d->count;
@@ -1027,18 +1241,74 @@ struct StepIn {
     __device__ __forceinline__ const QSyn *queue(uint32_t par) const { return d->queue + (size_t)par * d->qslots; }
 };
 
+// The wave's own counters: events (sum of the fired rows' lengths) and
+// spikes, added without waiting for a read.
+// Returns the fired lane's row.
+struct RowSpan {
+    int64_t first;
+    uint32_t len;
+};
+
+__device__ __forceinline__ RowSpan count_fired(TilePtr d, InstPtr I, bool emit, unsigned long long m, uint32_t tid,
+                                               uint32_t lane, uint32_t w)
+{
+    RowSpan r{0, 0u};
+    if (emit) {
+        r.first = gp(d->rowptr)[tid];
+        r.len = (uint32_t)(gp(d->rowptr)[tid + 1] - r.first);
+    }
+    const unsigned long long ev = wave_sum_u64((unsigned long long)r.len);
+    if (lane == 0) {
+        unsigned long long *c = I->wave_ctr + 2u * ((d->begin >> 6) + w);
+        gadd(c, ev);
+        gadd(c + 1, (unsigned long long)__popcll(m));
+    }
+    return r;
+}
+
+// Gather propagation: the wave's fired rows with synapses go to the tile's
+// fired list of set par ^ 1 for the next launch's k_gather (one atomic per
+// wave, on a count shared with 1/64 of the tiles).
+__device__ __forceinline__ void list_fired(TilePtr d, InstPtr I, bool emit, uint32_t par, uint32_t tid, uint32_t lane)
+{
+    const uint32_t len = emit ? (uint32_t)(gp(d->rowptr)[tid + 1] - gp(d->rowptr)[tid]) : 0u;
+    const bool has = emit && len != 0u;
+    const unsigned long long mg = __ballot(has);
+    if (mg != 0ull) {
+        const uint32_t list = (par ^ 1u) * kFiredLists + ((d->begin >> kTileBits) & (kFiredLists - 1u));
+        const int lg = __ffsll((long long)mg) - 1;
+        uint32_t gb = 0;
+        if ((int)lane == lg)
+            gb = gadd(I->fcount + (size_t)list * kFiredCountStride, (uint32_t)__popcll(mg));
+        gb = (uint32_t)__builtin_amdgcn_readlane((int)gb, lg);
+        if (has)
+            gp(I->fired)[(size_t)list * I->fcap + gb + (uint32_t)__popcll(mg & ((1ull << lane) - 1ull))] =
+                d->begin + tid;
+    }
+}
+
+// LDS of a tile that bins its own rows: the rows, and per wave the segments
+// of one pass.
+template <uint32_t K>
+struct TileRows {
+    unsigned long long seg_dst[4 * kWave * K];
+    uint32_t seg_room[4 * kWave * K];
+    long long rb[kBlock];    // fired rows of the tile: first synapse
+    uint32_t len[kBlock];    // and length
+    uint32_t n;
+};
+
 // One tile's step (the body of k_step).  kUniform: every neuron of the tile
 // has the same parameter class, so the parameter record is read once per
-// tile through the scalar unit instead of per lane.  K: synapses per lane in
-// a binning pass (a pass is 64 K synapses).  kStat: some instance records
-// population statistics (their code costs registers that a launch without
-// them does not spend).
-template <bool kUniform, uint32_t K, uint32_t kFmt, bool kStat>
-__device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
-                                          unsigned long long *acc,
-                                          unsigned long long *seg_dst, uint32_t *seg_room, long long *row_rb,
-                                          uint32_t *row_len, uint32_t &nrows, uint32_t &s_fit,
-                                          unsigned long long *s_bits, TileRec &rec)
+// tile through the scalar unit instead of per lane.  kStat: some instance
+// records population statistics (their code costs registers that a launch
+// without them does not spend).
+// kMode: kQueues, kDirect or kTileBin; K: with kTileBin, synapses per lane in
+// a binning pass (a pass is 64 K synapses).
+template <bool kUniform, uint32_t kFmt, bool kStat, int kMode, uint32_t K>
+__device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par, unsigned long long *acc,
+                                          unsigned long long *s_bits, TileRec &rec, DirectList *ls,
+                                          TileRows<K> *rows)
 {
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = __lane_id();
@@ -1054,11 +1324,12 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
         // starts; entries past the count are ignored, and the queue buffer has
         // kQueuePrefetch slots of slack at its end, so the read needs no
         // branch).
-        StepIn<kUniform> e(tp, qp, par, tid);
+        StepIn<kUniform, kMode> e(tp, qp, par, tid);
         // One register quad for both: the delta that k_gather wrote (gather
         // propagation), or the queue entry.
-        float4 ahead;
-        if (e.d->flags & kTileGather) {
+        float4 ahead = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (kMode == kDirect) {
+        } else if (e.d->flags & kTileGather) {
             ahead = ld4(e.d->dlt, e.lc);
         } else {
             const QSyn h = ld_entry(e.queue(par), min(tid, kQueuePrefetch - 1u));
@@ -1066,14 +1337,17 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
         }
         // A tile pulls (the pull propagation, never with gather) when its
         // queue overflowed or rows were deferred into this set: rare (volleys).
-        const bool gat = (e.d->flags & kTileGather) != 0u;
+        const bool gat = kMode == kDirect || (e.d->flags & kTileGather) != 0u;   // no queue
         bool over = !gat && e.cnt > e.d->qcap;
         uint32_t cnt = gat ? 0u : min(e.cnt, e.d->qcap);
-        pull = (e.d->flags & (kTilePull | kTileGather)) == kTilePull && (over || e.stamp == e.step + 1);
+        pull = !gat && (e.d->flags & kTilePull) && (over || e.stamp == e.step + 1);
         clear_row(acc, tid);
         if (tid == 0) {
-            nrows = 0u;
             rec.count = 0u;
+            if (kMode == kDirect)
+                ls->n = 0u;
+            if (kMode == kTileBin)
+                rows->n = 0u;
         }
         if (kStat && tid < (uint32_t)kStatFields)
             rec.stat[tid] = 0ull;
@@ -1088,12 +1362,24 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
             // Everything again: nothing loaded above is live across the call
             // (what is, the compiler keeps in spilled registers from the
             // kernel's start, in every tile).
-            e = StepIn<kUniform>(again(tp), again(qp), par, tid);
+            e = StepIn<kUniform, kMode>(again(tp), again(qp), par, tid);
             pull = true;
             over = false;
             cnt = 0u;
         }
-        accumulate_tile(acc, e.queue(par), cnt, QSyn{__float_as_uint(ahead.x), ahead.y, ahead.z}, kQueuePrefetch, tid);
+        if (kMode == kDirect) {
+            if (direct_tile<kFmt>(acc, *ls, *cp(e.d->inst), par, e.d->begin >> kTileBits, tid) && tid == 0) {
+                // the tile pulled; and its own rows, if any, went by the pull
+                CtlSlot &c = qp->ctl->slot[blockIdx.x & (kCtlSlots - 1u)];
+                gadd(&c.pulled, 1ull);
+                const auto b = gp(e.d->bits) + (size_t)par * e.d->ntiles * kBitWords;
+                if ((b[0] | b[1] | b[2] | b[3]) != 0ull)
+                    gadd(&c.deferred, 1ull);
+            }
+        } else {
+            accumulate_tile(acc, e.queue(par), cnt, QSyn{__float_as_uint(ahead.x), ahead.y, ahead.z}, kQueuePrefetch,
+                            tid);
+        }
         __syncthreads();
         if (!kUniform)   // a rare tile: its lanes' records do not wait in registers
             e.prm = load_params<false>(e.d, e.lc);
@@ -1103,238 +1389,368 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
             take_spill(acc, I->spill, I->n, par, e.d->begin + tid, tid, true);   // synapses past the queue's capacity
         }
         if (tid == 0) {
-            *gp(e.count(par)) = 0u;   // this launch consumed the queue
+            if (kMode != kDirect)
+                *gp(e.count(par)) = 0u;   // this launch consumed the queue
             if (e.d->begin == 0)
                 gp(e.d->step)[par ^ 1u] = step + 1;   // no tile of this launch reads this slot
         }
-        const float4 dl = (e.d->flags & kTileGather) ? ahead : acc_to_delta(acc, tid);
+        const float4 dl = kMode != kDirect && (e.d->flags & kTileGather) ? ahead : acc_to_delta(acc, tid);
         emit = step_lane<kStat>(e.d, e.x, e.prm, dl, e.active, tid, lane, step, p, rec);
     }
 
     const TilePtr d = again(tp);
     const InstPtr I = cp(d->inst);
     const bool gat = (d->flags & kTileGather) != 0u;
-    const bool pull_on = (d->flags & kTilePull) != 0u;
-    // Spike propagation (presynaptic_voltage.cpp:122-225): the tile's fired
-    // rows are listed in LDS, and their passes of 64 K synapses are dealt
-    // round-robin to the four waves, so one long row does not keep a single
-    // wave busy while the others idle.
+    // Spike propagation (presynaptic_voltage.cpp:122-225): with gather the
+    // fired rows go to lists for the next k_gather; else the tile's emitted
+    // rows are left as bits for the k_bin launch that follows.
     const unsigned long long m = __ballot(emit);
     if (lane == 0)
         s_bits[w] = m;
     if (m != 0ull) {
-        const uint32_t cnt_w = (uint32_t)__popcll(m);
-        const int leader = __ffsll((long long)m) - 1;
-        long long rb = 0;
-        uint32_t len = 0;
-        if (emit) {
-            rb = gp(d->rowptr)[tid];
-            len = (uint32_t)(gp(d->rowptr)[tid + 1] - rb);
-        }
-        // events = sum of the fired rows' lengths: few per wave, read lane by
-        // lane through the scalar unit
-        unsigned long long ev = 0;
-        for (unsigned long long r = m; r != 0ull; r &= r - 1ull)
-            ev += (uint32_t)__builtin_amdgcn_readlane((int)len, __ffsll((long long)r) - 1);
-        uint32_t base = 0;
-        if ((int)lane == leader) {
-            // the wave's own counters, added without waiting for a read
-            // (a load-add-store would stall the wave before its binning)
-            unsigned long long *c = I->wave_ctr + 2u * ((d->begin >> 6) + w);
-            gadd(c, ev);
-            gadd(c + 1, (unsigned long long)cnt_w);
-            if (!gat)
-                base = atomicAdd(&nrows, cnt_w);
-        }
-        if (gat) {
-            // gather propagation: the rows with synapses go to this tile's
-            // fired list of set par ^ 1 for the next launch's k_gather (one
-            // atomic per wave, on a count shared with 1/64 of the tiles)
-            const bool has = emit && len != 0u;
-            const unsigned long long mg = __ballot(has);
-            if (mg != 0ull) {
-                const uint32_t list = (par ^ 1u) * kFiredLists + ((d->begin >> kTileBits) & (kFiredLists - 1u));
-                const int lg = __ffsll((long long)mg) - 1;
-                uint32_t gb = 0;
-                if ((int)lane == lg)
-                    gb = gadd(I->fcount + (size_t)list * kFiredCountStride, (uint32_t)__popcll(mg));
-                gb = (uint32_t)__builtin_amdgcn_readlane((int)gb, lg);
-                if (has)
-                    gp(I->fired)[(size_t)list * I->fcap + gb + (uint32_t)__popcll(mg & ((1ull << lane) - 1ull))] =
-                        d->begin + tid;
-            }
-        } else {
-            base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
-            if (emit) {
-                const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                row_rb[k] = rb;
-                row_len[k] = len;
+        if (kMode != kQueues || gat) {
+            const RowSpan r = count_fired(d, I, emit, m, tid, lane, w);
+            if (kMode == kTileBin && !gat) {
+                uint32_t base = 0;
+                if (lane == 0)
+                    base = atomicAdd(&rows->n, (uint32_t)__popcll(m));
+                base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+                if (emit) {
+                    const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                    rows->rb[k] = r.first;
+                    rows->len[k] = r.len;
+                }
             }
         }
+        if (gat)
+            list_fired(d, I, emit, par, tid, lane);
         if (I->rec_counts != nullptr)
             count_wave(d, I, emit, tid, lane, step, p, rec);
     }
     __syncthreads();
-    const QueuePtr qs = again(qp);
+    if (kMode == kDirect) {
+        // the tile's rows: their bits, then the count and the first ids
+        if (w == 0) {
+            unsigned long long word = s_bits[lane & 3u];
+            uint32_t c = (uint32_t)__popcll(word);
+            unsigned long long first = 0ull;
+            c = (uint32_t)__builtin_amdgcn_readlane((int)c, 0) + (uint32_t)__builtin_amdgcn_readlane((int)c, 1) +
+                (uint32_t)__builtin_amdgcn_readlane((int)c, 2) + (uint32_t)__builtin_amdgcn_readlane((int)c, 3);
+            if (c != 0u && c <= kDirectIds) {
+                uint32_t k = 2u;
+                for (uint32_t q = 0; q < 4u; ++q)
+                    for (unsigned long long r = s_bits[q]; r != 0ull; r &= r - 1ull, ++k)
+                        first |= (unsigned long long)(q * kWave + (uint32_t)__ffsll((long long)r) - 1u) << (8u * k);
+            }
+            if (lane < 5u)
+                gp(d->bits)[(size_t)(par ^ 1u) * d->ntiles * kBitWords + lane] = lane < 4u ? word : (first | c);
+        }
+    }
     put_tile_rec<kStat>(d, I, tid, step, rec);
-    const uint32_t nr = nrows;
+    if (kMode == kDirect || gat)
+        return;
     // A tile with many emitted rows (a synchronous volley) leaves them to
-    // the consumers' pull: binning them would cost one reservation per
-    // (row, target tile) and overflow the queues.  A tile that pulls in
-    // this launch (the volley is under way) defers only from four times
-    // the count: the volley's tail, where a few tiles still emit that many,
-    // would otherwise cost the next step a pull of every in-edge.
+    // the consumers' pull: binning them would overflow the queues.  A tile
+    // that pulls in this launch (the volley is under way) defers only from
+    // four times the count: the volley's tail, where a few tiles still emit
+    // that many, would otherwise cost the next step a pull of every in-edge.
     bool defer = false;
-    if (pull_on) {
+    const unsigned long long b = s_bits[lane & 3u];
+    if (d->flags & kTilePull) {
+        const uint32_t c = (uint32_t)__popcll(b);
+        const uint32_t nr = (uint32_t)__builtin_amdgcn_readlane((int)c, 0) +
+                            (uint32_t)__builtin_amdgcn_readlane((int)c, 1) +
+                            (uint32_t)__builtin_amdgcn_readlane((int)c, 2) +
+                            (uint32_t)__builtin_amdgcn_readlane((int)c, 3);
         if (nr != 0u) {
             const uint32_t dm = I->defer_min;
             defer = dm != 0u && nr >= (pull ? 4u * dm : dm);
-        }
-        // the tile's emitted and deferred rows, one 64-byte store
-        if (tid < kBitWords) {
-            const unsigned long long b = s_bits[tid & 3u];
-            gp(d->bits)[(size_t)(par ^ 1u) * d->ntiles * kBitWords + tid] = (tid < 4u || defer) ? b : 0ull;
-        }
-        if (defer && tid == 0) {
-            gp(d->step)[2u + (par ^ 1u)] = step + 2;   // consumer's step + 1 (0: none)
-            gadd(&qs->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].deferred, 1ull);
+            if (defer && tid == 0) {
+                gp(d->step)[2u + (par ^ 1u)] = step + 2;   // consumer's step + 1 (0: none)
+                gadd(&again(qp)->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].deferred, 1ull);
+            }
         }
     }
-    const uint32_t nbin = defer ? 0u : nr;
-    if (nbin == 0u)
-        return;
-    unsigned long long *spill_out = pull_on ? nullptr : I->spill + (size_t)(par ^ 1u) * I->n * 4u;
-    QSyn *q_out = I->queue + (size_t)(par ^ 1u) * d->qslots;
-    // Split binning: the tile's passes (rows in LDS order, passes in row
-    // order) go to the engine's pass list for the k_bin launch that follows,
-    // where every wave of the GPU takes one; the tile bins here only the
-    // passes past the list's capacity.
-    uint32_t first_here = 0;   // tile pass index from which this tile bins itself
-    if (qs->pass != nullptr) {
-        if (w == 0) {
-            constexpr uint32_t kPass = kWave * K;
-            uint32_t total = 0;
-            for (uint32_t r0 = 0; r0 < nbin; r0 += kWave) {
-                const uint32_t r = r0 + lane;
-                const uint32_t np = r < nbin ? (row_len[r] + kPass - 1u) / kPass : 0u;
-                total += (uint32_t)wave_sum_u64((unsigned long long)np);
-            }
-            uint32_t base = 0;
-            if (lane == 0)
-                base = gadd(qs->pcount + (size_t)par * kPassCountStride, total);
-            base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-            const uint32_t fit = qs->pcap > base ? min(total, qs->pcap - base) : 0u;
-            uint32_t off = 0;   // passes of the rows of earlier chunks
-            for (uint32_t r0 = 0; r0 < nbin; r0 += kWave) {
-                const uint32_t r = r0 + lane;
-                const uint32_t len = r < nbin ? row_len[r] : 0u;
-                const uint32_t np = (len + kPass - 1u) / kPass;
-                uint32_t incl = np;
-#pragma unroll
-                for (uint32_t o = 1; o < (uint32_t)kWave; o <<= 1) {
-                    const uint32_t v = __shfl_up(incl, o, kWave);
-                    if (lane >= o)
-                        incl += v;
-                }
-                const uint32_t ex = off + incl - np;   // this row's first tile pass
-                const long long rb = r < nbin ? row_rb[r] : 0;
-                for (uint32_t j = 0; j < np && ex + j < fit; ++j) {
-                    PassEntry e;
-                    e.first = (uint64_t)(rb + (long long)j * kPass);
-                    e.len = min(kPass, len - j * kPass);
-                    e.inst = d->inst_idx;
-                    qs->pass[base + ex + j] = e;
-                }
-                off += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-            }
-            if (lane == 0)
-                s_fit = fit;
-        }
-        __syncthreads();
-        first_here = s_fit;
-    }
-    uint32_t pass = 0;
-    for (uint32_t r = 0; r < nbin; ++r) {
-        const long long rb_s = row_rb[r];
-        const uint32_t len_s = row_len[r];
-        for (uint32_t c0 = 0; c0 < len_s; c0 += kWave * K, ++pass)
-            if ((pass & 3u) == w && pass >= first_here)
-            {
+    // the tile's emitted and deferred rows, one 64-byte store
+    if (tid < kBitWords && (kMode == kQueues || (d->flags & kTilePull)))
+        gp(d->bits)[(size_t)(par ^ 1u) * d->ntiles * kBitWords + tid] = (tid < 4u || defer) ? b : 0ull;
+    if constexpr (kMode == kTileBin) {
+        // The passes of the tile's rows, dealt round-robin to its four waves,
+        // so one long row does not keep a single wave busy while the others
+        // idle.
+        const uint32_t nbin = defer ? 0u : rows->n;
+        if (nbin == 0u)
+            return;
+        const QueuePtr qs = again(qp);
+        unsigned long long *spill_out =
+            (d->flags & kTilePull) ? nullptr : I->spill + (size_t)(par ^ 1u) * I->n * 4u;
+        QSyn *q_out = I->queue + (size_t)(par ^ 1u) * d->qslots;
+        uint32_t pass = 0;
+        for (uint32_t r = 0; r < nbin; ++r) {
+            const long long rb_s = rows->rb[r];
+            const uint32_t len_s = rows->len[r];
+            for (uint32_t c0 = 0; c0 < len_s; c0 += kWave * K, ++pass) {
+                if ((pass & 3u) != w)
+                    continue;
                 if constexpr (K == 1)
                     bin_pass_serial<K, kFmt>(I->col, I->w, I->wfmt, (int64_t)rb_s, len_s, c0, I->tile_base, qs->tile,
-                                       qs->count, (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out,
-                                       spill_out, qs->ctl, seg_dst + w * kWave * K,
-                                       seg_room + w * kWave * K, lane);
+                                             qs->count, (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out, spill_out,
+                                             qs->ctl, rows->seg_dst + w * kWave * K, rows->seg_room + w * kWave * K,
+                                             lane);
                 else
-                    bin_pass<K, kFmt>(I->col, I->w, I->wfmt, (int64_t)rb_s, len_s, c0, I->tile_base, qs->tile, qs->count,
-                                (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out,
-                                spill_out, qs->ctl, seg_dst + w * kWave * K,
-                                seg_room + w * kWave * K, lane);
+                    bin_pass<K, kFmt>(I->col, I->w, I->wfmt, (int64_t)rb_s, len_s, c0, I->tile_base, qs->tile,
+                                      qs->count, (size_t)(par ^ 1u) * qs->ntiles, qs->cshift, q_out, spill_out, qs->ctl,
+                                      rows->seg_dst + w * kWave * K, rows->seg_room + w * kWave * K, lane);
             }
+        }
     }
 }
 
-// The step of launch parity `par`: drains queue set par, fills set par ^ 1,
-// reads the step index from step[par] and advances it into step[par ^ 1].
-// K: synapses per lane in a binning pass (the schedule; every K gives the
-// same results).  Eight waves per SIMD for K = 1, 2; K = 4's larger LDS
-// segment tables allow six.
-template <uint32_t K, uint32_t kFmt, bool kStat>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ? 6 : 8))) void k_step(const TileDesc *tiles,
-                                                 const QueueSet *queues,
-                                                 uint32_t par)
+// The step of launch parity `par`: takes the input of set par, leaves the
+// emitted rows of set par ^ 1 as bits (fired lists with gather), reads the
+// step index from step[par] and advances it into step[par ^ 1].
+// Seven waves per SIMD: at eight the compiler spills up to 14 registers, and
+// the 2M-neuron step takes 42.3 us instead of 40.5 (1200 rows per step), a
+// 10k-neuron step by direct propagation 5.7 instead of 5.3.
+template <uint32_t kFmt, bool kStat, int kMode, uint32_t K>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ? 6 : 7))) void k_step(const TileDesc *tiles,
+                                                                                         const QueueSet *queues,
+                                                                                         uint32_t par)
 {
     __shared__ unsigned long long acc[kBlock * 4];
-    __shared__ unsigned long long seg_dst[4 * kWave * K];   // per wave: one pass
-    __shared__ uint32_t seg_room[4 * kWave * K];
-    __shared__ long long row_rb[kBlock];                  // fired rows of the tile: first synapse
-    __shared__ uint32_t row_len[kBlock];                  // and length
-    __shared__ unsigned long long s_bits[4];              // emitted rows per wave
-    __shared__ uint32_t nrows;
-    __shared__ uint32_t s_fit;                            // split binning: passes in the list
+    __shared__ unsigned long long s_bits[4];   // emitted rows per wave
     __shared__ TileRec rec;
+    DirectList *ls = nullptr;
+    if constexpr (kMode == kDirect) {
+        __shared__ DirectList list;
+        ls = &list;
+    }
+
+    TileRows<K> *rows = nullptr;
+    if constexpr (kMode == kTileBin) {
+        __shared__ TileRows<K> r;
+        rows = &r;
+    }
 
     const TilePtr tp = cp(tiles + blockIdx.x);
     if (tp->flags & kTileUniform)
-        step_tile<true, K, kFmt, kStat>(tp, cp(queues), par, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit, s_bits,
-                                        rec);
+        step_tile<true, kFmt, kStat, kMode, K>(tp, cp(queues), par, acc, s_bits, rec, ls, rows);
     else
-        step_tile<false, K, kFmt, kStat>(tp, cp(queues), par, acc, seg_dst, seg_room, row_rb, row_len, nrows, s_fit,
-                                         s_bits, rec);
+        step_tile<false, kFmt, kStat, kMode, K>(tp, cp(queues), par, acc, s_bits, rec, ls, rows);
 }
 
-// Split binning: bins the passes that the k_step launch of parity `par`
-// listed (into queue set par ^ 1, as k_step would have), one pass per wave
-// at a time over the whole grid, so a step's propagation is spread over
-// every CU instead of the tiles whose neurons fired.  Also empties the other
-// parity's list count (its last reader was the previous k_bin; the next
-// k_step appends to it).
-template <uint32_t K, uint32_t kFmt>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_bin(const InstDev *__restrict__ insts,
-                                                QueueSet qs,
-                                                uint32_t par)
+// Binning of the rows emitted by the k_step launch of parity `par` into
+// queue set par ^ 1.  A workgroup takes a group of up to kBinTiles
+// consecutive source tiles: rows of neighbouring neurons reach the same
+// target tiles (a voxel's rows share theirs), so it counts its synapses per
+// target tile in LDS, reserves each tile's share with one device atomic
+// (consecutive lanes on consecutive counts, which one request serves), and
+// writes every synapse's entry to its tile's queue at reserved start + rank.
+// Without it (one reservation per row and target tile, in the tiles whose
+// neurons fired) binning is 24 of 51 us of the 2M-neuron block's step:
+// returning atomics on single counts are served at about 2.7e10 per second,
+// and a row of 500 synapses makes 160-190 of them.  A step with / without: 2M
+// neurons x 500 47.5 / 50.9 us, 900k x 300 30.2 / 28.2, 400k x 250 19.6 /
+// 15.9 (the launch, and a group's serial phases, cost what the atomics save).
+// Rows are cut into passes of kBinPass synapses, one per wave and round;
+// deferred rows are counted (events) but not binned.  The counts of a round
+// live in min(ntiles, kBinMaxTiles) LDS words; instances with more tiles are
+// binned in windows of that many target tiles.
+template <uint32_t kFmt>
+__global__ __launch_bounds__(kBinBlock) void k_bin(const BinDesc *__restrict__ groups, const QueueSet *queues,
+                                                   uint32_t par)
 {
-    __shared__ unsigned long long seg_dst[4 * kWave * K];
-    __shared__ uint32_t seg_room[4 * kWave * K];
-    const uint32_t w = threadIdx.x / kWave;
-    const uint32_t lane = __lane_id();
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        qs.pcount[(size_t)(par ^ 1u) * kPassCountStride] = 0u;
-    const uint32_t total = min(qs.pcount[(size_t)par * kPassCountStride], qs.pcap);
-    const uint32_t nwaves = gridDim.x * (kBlock / kWave);
-    for (uint32_t i = blockIdx.x * (kBlock / kWave) + w; i < total; i += nwaves) {
-        const PassEntry e = qs.pass[i];
-        const InstDev &I = insts[e.inst];
-        QSyn *q_out = I.queue + (size_t)(par ^ 1u) * I.qslots;
-        unsigned long long *spill_out = I.crec != nullptr ? nullptr : I.spill + (size_t)(par ^ 1u) * I.n * 4u;
-        if constexpr (K == 1)
-            bin_pass_serial<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, qs.tile, qs.count,
-                               (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, qs.ctl,
-                               seg_dst + w * kWave * K, seg_room + w * kWave * K, lane);
-        else
-            bin_pass<K, kFmt>(I.col, I.w, I.wfmt, (int64_t)e.first, e.len, 0u, I.tile_base, qs.tile, qs.count,
-                        (size_t)(par ^ 1u) * qs.ntiles, qs.cshift, q_out, spill_out, qs.ctl,
-                        seg_dst + w * kWave * K, seg_room + w * kWave * K, lane);
+    constexpr uint32_t kWaves = kBinBlock / kWave;
+    extern __shared__ uint32_t hist[];               // min(ntiles, kBinMaxTiles)
+    __shared__ uint16_t s_list[kBinTiles * kBlock];  // emitted rows of the group (bit 15: deferred)
+    __shared__ uint32_t s_pass[kBinBlock];           // per row of a chunk: passes before it
+    __shared__ uint32_t s_len[kBinBlock];
+    __shared__ int64_t s_rb[kBinBlock];
+    __shared__ uint32_t s_wave[kWaves];
+    __shared__ uint16_t s_touch[kWaves * kBinDeep * kBinPass];   // target tiles of a round, each once
+    __shared__ uint32_t s_rows, s_ntouch;
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / kWave;
+    const auto bd = cp(groups + blockIdx.x);
+    const InstPtr I = cp(bd->inst);
+    const uint32_t tile0 = bd->tile0, T = I->ntiles, set = par ^ 1u;
+    if (w < kBinTiles / 16u) {
+        // one word of 64 rows per lane
+        const auto b = gp(I->bits) + ((size_t)set * T + tile0) * kBitWords;
+        const uint32_t t = tid >> 2, q = tid & 3u;
+        unsigned long long e = 0ull, df = 0ull;
+        if (t < bd->ntile) {
+            e = b[t * kBitWords + q];
+            df = b[t * kBitWords + 4u + q];
+        }
+        // the list starts where the wave before left off (its words are read
+        // again: one line each)
+        uint32_t at = 0;
+        for (uint32_t v = 0; v < w; ++v) {
+            const uint32_t tt = v * 16u + (lane >> 2);
+            const unsigned long long x = tt < bd->ntile ? b[tt * kBitWords + (lane & 3u)] : 0ull;
+            at += (uint32_t)__builtin_amdgcn_readlane((int)wave_add_scan((uint32_t)__popcll(x)), kWave - 1);
+        }
+        const uint32_t c = (uint32_t)__popcll(e), incl = wave_add_scan(c);
+        at += incl - c;
+        if (w == kBinTiles / 16u - 1u && lane == kWave - 1)
+            s_rows = at + c;
+        for (; e != 0ull; e &= e - 1ull, ++at) {
+            const uint32_t k = (uint32_t)__ffsll((long long)e) - 1u;
+            s_list[at] = (uint16_t)((tid << 6) | k | (((df >> k) & 1ull) ? 0x8000u : 0u));
+        }
+    }
+    __syncthreads();
+    const uint32_t rows = s_rows;
+    if (rows == 0u)
+        return;
+    for (uint32_t t = tid; t < min(T, (uint32_t)kBinMaxTiles); t += kBinBlock)
+        hist[t] = 0u;
+    if (tid == 0)
+        s_ntouch = 0u;
+    const QueuePtr qs = cp(queues);
+    const uint32_t wfmt = kFmt != kWeightAny ? kFmt : I->wfmt;
+    const uint32_t tb = I->tile_base;
+    uint32_t *count = qs->count;
+    const size_t cset = (size_t)set * qs->ntiles + tb;
+    const uint32_t cshift = qs->cshift;
+    const QueueTile *qtab = qs->tile + tb;
+    QSyn *q_out = I->queue + (size_t)set * I->qslots;
+    const bool pull_on = I->crec != nullptr;
+    unsigned long long events = 0;
+    for (uint32_t r0 = 0; r0 < rows; r0 += kBinBlock) {
+        const uint32_t nr = min(rows - r0, (uint32_t)kBinBlock);
+        uint32_t np = 0, len = 0;
+        int64_t rb = 0;
+        if (tid < nr) {
+            const uint32_t e = s_list[r0 + tid];
+            const uint32_t r = tile0 * kBlock + (e & 0x7fffu);
+            rb = gp(I->rowptr)[r];
+            len = (uint32_t)(gp(I->rowptr)[r + 1] - rb);
+            np = (e & 0x8000u) ? 0u : (len + kBinPass - 1u) / kBinPass;
+        }
+        events += len;
+        const uint32_t incl = wave_add_scan(np);
+        if (lane == kWave - 1)
+            s_wave[w] = incl;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kWaves; ++k) {
+            const uint32_t v = s_wave[k];
+            before += k < w ? v : 0u;
+            total += v;
+        }
+        s_pass[tid] = tid < nr ? before + incl - np : 0xffffffffu;
+        s_len[tid] = len;
+        s_rb[tid] = rb;
+        for (uint32_t t0 = 0; t0 < T; t0 += kBinMaxTiles) {
+            const uint32_t tw = min(T - t0, (uint32_t)kBinMaxTiles);
+            for (uint32_t p0 = 0; p0 < total; p0 += kWaves * kBinDeep) {
+                __syncthreads();   // s_pass, s_len, s_rb are written, hist is zero
+                constexpr uint32_t N = kBinDeep * kBinItems;
+                uint32_t cv[N], rank[N];
+                unsigned long long wv[N];
+                bool ok[N];
+#pragma unroll
+                for (uint32_t q = 0; q < kBinDeep; ++q) {
+                    const uint32_t p = p0 + q * kWaves + w;
+                    uint32_t j0 = 0, n = 0;
+                    int64_t first = 0;
+                    if (p < total) {
+                        // the row of pass p: the last one with at most p passes before it
+                        uint32_t row = 0;
+#pragma unroll
+                        for (uint32_t st = kBinBlock / 2; st > 0; st >>= 1)
+                            if (s_pass[row + st] <= p)
+                                row += st;
+                        j0 = (p - s_pass[row]) * kBinPass;
+                        n = s_len[row];
+                        first = s_rb[row];
+                    }
+#pragma unroll
+                    for (uint32_t v = 0; v < kBinItems; ++v) {
+                        const uint32_t u = q * kBinItems + v;
+                        const uint32_t j = j0 + v * kWave + lane;
+                        ok[u] = j < n;
+                        if (ok[u]) {
+                            cv[u] = gp(I->col)[first + j];
+                            wv[u] = w_raw(I->w, (size_t)(first + j), wfmt);
+                        }
+                    }
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < N; ++u)
+                    if (ok[u]) {
+                        const uint32_t t = ((cv[u] & kColMask) >> kTileBits) - t0;
+                        ok[u] = t < tw;
+                        if (ok[u]) {
+                            rank[u] = atomicAdd(&hist[t], 1u);
+                            if (rank[u] == 0u)
+                                s_touch[atomicAdd(&s_ntouch, 1u)] = (uint16_t)t;
+                        }
+                    }
+                __syncthreads();
+                const uint32_t nt = s_ntouch;
+                uint32_t over = 0;   // synapses of this thread's tiles past their queue's capacity
+                for (uint32_t k = tid; k < nt; k += kBinBlock) {
+                    const uint32_t t = s_touch[k];
+                    const uint32_t c = hist[t];
+                    const uint32_t b = gadd(&count[count_slot(cset + t0 + t, cshift)], c);
+                    const uint32_t cap = gp(qtab)[t0 + t].cap;
+                    const uint64_t off = gp(qtab)[t0 + t].off;
+                    const uint32_t room = cap > b ? min(c, cap - b) : 0u;
+                    over += c - room;
+                    // the segment's first slot; bit 31: it does not fit whole
+                    // (or the slot takes more than 31 bits), then its start
+                    // within the tile's queue
+                    hist[t] = room == c && off + b + c < 0x80000000ull ? (uint32_t)(off + b)
+                                                                      : 0x80000000u | min(b, 0x7fffffffu);
+                }
+                if (over != 0u)
+                    gadd(&qs->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].spilled, (unsigned long long)over);
+                __syncthreads();
+#pragma unroll
+                for (uint32_t u = 0; u < N; ++u) {
+                    if (!ok[u])
+                        continue;
+                    const uint32_t tile = (cv[u] & kColMask) >> kTileBits;
+                    const uint32_t h = hist[tile - t0];
+                    const uint32_t key = (cv[u] & 0xffu) | ((cv[u] & kKindBit) ? kQSynKind : 0u);
+                    const float2 wp = w_decode(wv[u], wfmt);
+                    if (!(h & 0x80000000u)) {
+                        st_entry(q_out, h + rank[u], key, wp.x, wp.y);
+                    } else {
+                        const uint64_t at = (uint64_t)(h & 0x7fffffffu) + rank[u];
+                        if (at < gp(qtab)[tile].cap) {
+                            st_entry(q_out, gp(qtab)[tile].off + at, key, wp.x, wp.y);
+                        } else if (!pull_on) {
+                            // past the capacity: the target's spill accumulator
+                            // (Q23.40 integers like the LDS sums); with the pull
+                            // the tile takes every row through its in-edges
+                            unsigned long long *a = I->spill + ((size_t)set * I->n + (cv[u] & kColMask)) * 4u +
+                                                    ((cv[u] & kKindBit) ? 2u : 0u);
+                            gadd(a, f32_to_q40(wp.x));
+                            gadd(a + 1, f32_to_q40(wp.y));
+                        }
+                    }
+                }
+                __syncthreads();
+                for (uint32_t k = tid; k < nt; k += kBinBlock)
+                    hist[s_touch[k]] = 0u;
+                if (tid == 0)
+                    s_ntouch = 0u;
+            }
+        }
+        __syncthreads();
+    }
+    // events delivered and spikes, on the counters of the group's first wave
+    const unsigned long long ev = wave_sum_u64(events);
+    if (lane == 0) {
+        unsigned long long *c = I->wave_ctr + 2u * (size_t)(tile0 * (kBlock / kWave));
+        if (ev != 0ull)
+            gadd(c, ev);
+        if (w == 0)
+            gadd(c + 1, (unsigned long long)rows);
     }
 }
 
@@ -1492,13 +1908,14 @@ __global__ __launch_bounds__(kBlock) void k_build_grec(const uint32_t *__restric
     }
 }
 
-// Group offsets of the gather propagation, one wave per row: segidx[r][g] =
-// offset in row r of the first synapse whose target lies in group g or a
-// later one, segidx[r][ngroups] = row length.  Rows must be ordered by
+// Offsets per target group of 2^shift neurons (gather groups, or tiles for
+// the direct propagation), one wave per row: segidx[r][g] = offset in row r
+// of the first synapse whose target lies in group g or a later one, segidx[r][ngroups] = row length.  Rows must be ordered by
 // target group (checked on the host).
 __global__ __launch_bounds__(kBlock) void k_build_segidx(const int64_t *__restrict__ rowptr,
                                                          const uint32_t *__restrict__ col, uint32_t n,
-                                                         uint32_t ngroups, uint16_t *__restrict__ segidx)
+                                                         uint32_t ngroups, uint32_t shift,
+                                                         uint16_t *__restrict__ segidx)
 {
     const uint32_t r = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
     const uint32_t lane = __lane_id();
@@ -1508,12 +1925,12 @@ __global__ __launch_bounds__(kBlock) void k_build_segidx(const int64_t *__restri
     const uint32_t len = (uint32_t)(rowptr[r + 1] - rb);
     uint16_t *s = segidx + (size_t)r * (ngroups + 1u);
     for (uint32_t j = lane; j < len; j += kWave) {
-        const uint32_t gc = (col[rb + j] & kColMask) >> kGroupBits;
-        const uint32_t g0 = j == 0 ? 0u : ((col[rb + j - 1] & kColMask) >> kGroupBits) + 1u;
+        const uint32_t gc = (col[rb + j] & kColMask) >> shift;
+        const uint32_t g0 = j == 0 ? 0u : ((col[rb + j - 1] & kColMask) >> shift) + 1u;
         for (uint32_t g = g0; g <= gc; ++g)
             s[g] = (uint16_t)j;
     }
-    const uint32_t tail = len == 0 ? 0u : ((col[rb + len - 1] & kColMask) >> kGroupBits) + 1u;
+    const uint32_t tail = len == 0 ? 0u : ((col[rb + len - 1] & kColMask) >> shift) + 1u;
     for (uint32_t g = tail + lane; g <= ngroups; g += kWave)
         s[g] = (uint16_t)len;
 }
@@ -1598,12 +2015,23 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const TileDesc *__restri
                                                         uint32_t set)
 {
     __shared__ unsigned long long acc[kBlock * 4];
+    __shared__ DirectList ls;
     const TileDesc &d = tiles[blockIdx.x];
     const InstDev &I = insts[d.inst_idx];
     if (I.segidx != nullptr)
         return;   // gather propagation: k_gather has written dlt
     const uint32_t tid = threadIdx.x;
     clear_row(acc, tid);
+    if (I.tidx != nullptr) {
+        if (tid == 0)
+            ls.n = 0u;
+        __syncthreads();
+        direct_tile<kWeightAny>(acc, ls, I, set, d.begin >> kTileBits, tid);
+        __syncthreads();
+        if (tid < d.count)
+            st4(I.dlt, d.begin + tid, acc_to_delta(acc, tid));
+        return;
+    }
     const uint32_t cnt_raw = qs.count[count_slot((size_t)set * qs.ntiles + blockIdx.x, qs.cshift)];
     const bool over = cnt_raw > d.qcap;
     const bool pull_on = I.crec != nullptr;
@@ -1631,6 +2059,7 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
                                                    uint32_t set)
 {
     __shared__ unsigned long long acc[kBlock * 4];
+    __shared__ DirectList ls;
     const TileDesc &d = tiles[blockIdx.x];
     const InstDev &I = insts[d.inst_idx];
     const uint32_t tid = threadIdx.x;
@@ -1650,11 +2079,18 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
             gp(I.fcount)[((size_t)set * kFiredLists + tid) * kFiredCountStride] = 0u;
         return;
     }
+    const bool direct = I.tidx != nullptr;
     uint32_t *cnt_p = qs.count + count_slot((size_t)set * qs.ntiles + blockIdx.x, qs.cshift);
     clear_row(acc, tid);
-    const uint32_t cnt_raw = *cnt_p;
+    if (direct) {
+        if (tid == 0)
+            ls.n = 0u;
+        __syncthreads();
+        direct_tile<kWeightAny>(acc, ls, I, set, d.begin >> kTileBits, tid);
+    }
+    const uint32_t cnt_raw = direct ? 0u : *cnt_p;
     const bool over = cnt_raw > d.qcap;
-    const bool pull_on = I.crec != nullptr;
+    const bool pull_on = !direct && I.crec != nullptr;
     const bool pull = pull_on && (over || gp(I.step)[2u + set] == gp(I.step)[set] + 1);
     const uint32_t cnt = (pull_on && over) ? 0u : min(cnt_raw, d.qcap);
     __syncthreads();
@@ -1673,7 +2109,7 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
             *flag = (uint8_t)(fl | kFlagFolded);
         }
     }
-    if (tid == 0)
+    if (tid == 0 && !direct)
         *cnt_p = 0u;
 }
 
@@ -1882,119 +2318,83 @@ __global__ __launch_bounds__(kBlock) void k_normals(uint64_t seed, uint32_t neur
 
 // ---- launchers ----------------------------------------------------------
 
-// Calls f(kernel) with the kernel instantiated for pass size pass_k and
-// weight format wfmt (a format of every launched instance, or kWeightAny).
-template <template <uint32_t, uint32_t> class Sel, typename F>
-hipError_t with_kernel(uint32_t pass_k, uint32_t wfmt, F f)
-{
-    auto by_fmt = [&](auto kk) -> hipError_t {
-        constexpr uint32_t K = decltype(kk)::value;
-        switch (wfmt) {
-        case kWeightF32: f(Sel<K, kWeightF32>::get()); break;
-        case kWeightF16: f(Sel<K, kWeightF16>::get()); break;
-        case kWeightU8: f(Sel<K, kWeightU8>::get()); break;
-        case kWeightAny: f(Sel<K, kWeightAny>::get()); break;
-        default: return hipErrorInvalidValue;
-        }
-        return hipSuccess;
-    };
-    switch (pass_k) {
-    case 1: return by_fmt(std::integral_constant<uint32_t, 1>{});
-    case 2: return by_fmt(std::integral_constant<uint32_t, 2>{});
-    case 4: return by_fmt(std::integral_constant<uint32_t, 4>{});
-    default: return hipErrorInvalidValue;
-    }
-}
-
-template <uint32_t K, uint32_t F>
-struct StepSel {
-    static auto get() { return k_step<K, F, false>; }
-};
-template <uint32_t K, uint32_t F>
-struct StepStatSel {
-    static auto get() { return k_step<K, F, true>; }
-};
-template <uint32_t K, uint32_t F>
-struct BinSel {
-    static auto get() { return k_bin<K, F>; }
-};
-
-hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
-                              uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
-                              hipStream_t stream)
-{
-    if (ntiles == 0)
-        return hipSuccess;
-    auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, tiles, qs, par);
-    };
-    const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
-                              : with_kernel<StepSel>(pass_k, wfmt, launch);
-    return e != hipSuccess ? e : hipGetLastError();
-}
-
-hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
-                                    uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
-                                    hipEvent_t start, hipEvent_t stop, hipStream_t stream)
-{
-    if (ntiles == 0)
-        return hipSuccess;
-    auto launch = [&](auto kern) {
-        hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, start, stop, 0, tiles, qs, par);
-    };
-    const hipError_t e = stat ? with_kernel<StepStatSel>(pass_k, wfmt, launch)
-                              : with_kernel<StepSel>(pass_k, wfmt, launch);
-    return e != hipSuccess ? e : hipGetLastError();
-}
-
-hipError_t launch_bin_kernel(uint32_t grid, const InstDev *insts, const QueueSet &qs,
-                             uint32_t par, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
-                             hipEvent_t stop, hipStream_t stream)
-{
-    if (grid == 0 || qs.pass == nullptr)
-        return hipSuccess;
-    const hipError_t e = with_kernel<BinSel>(pass_k, wfmt, [&](auto kern) {
-        if (start != nullptr)
-            hipExtLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, start, stop, 0, insts, qs, par);
-        else
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, insts, qs, par);
-    });
-    return e != hipSuccess ? e : hipGetLastError();
-}
-
 namespace {
+// Calls f with the weight format as a constant (a format of every launched
+// instance, or kWeightAny).
 template <typename F>
-hipError_t with_gather(uint32_t wfmt, F f)
+hipError_t with_format(uint32_t wfmt, F f)
 {
     switch (wfmt) {
-    case kWeightF32: f(k_gather<kWeightF32>); break;
-    case kWeightF16: f(k_gather<kWeightF16>); break;
-    case kWeightU8: f(k_gather<kWeightU8>); break;
-    case kWeightAny: f(k_gather<kWeightAny>); break;
+    case kWeightF32: f(std::integral_constant<uint32_t, kWeightF32>{}); break;
+    case kWeightF16: f(std::integral_constant<uint32_t, kWeightF16>{}); break;
+    case kWeightU8: f(std::integral_constant<uint32_t, kWeightU8>{}); break;
+    case kWeightAny: f(std::integral_constant<uint32_t, kWeightAny>{}); break;
     default: return hipErrorInvalidValue;
     }
     return hipSuccess;
 }
 }  // namespace
 
-hipError_t launch_gather(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par, uint32_t wfmt,
-                         hipStream_t stream)
+namespace {
+typedef void (*StepKernel)(const TileDesc *, const QueueSet *, uint32_t);
+
+template <uint32_t kF, bool kStat>
+StepKernel step_kernel(StepMode mode, uint32_t pass_k)
 {
-    if (ngroups == 0)
+    if (mode == StepMode::direct)
+        return k_step<kF, kStat, kDirect, 1>;
+    if (mode == StepMode::bin_launch)
+        return k_step<kF, kStat, kQueues, 1>;
+    return pass_k == 1 ? k_step<kF, kStat, kTileBin, 1>
+           : pass_k == 4 ? k_step<kF, kStat, kTileBin, 4>
+                         : k_step<kF, kStat, kTileBin, 2>;
+}
+}  // namespace
+
+hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, StepMode mode, uint32_t pass_k,
+                              const QueueSet *qs, uint32_t par, uint32_t wfmt, bool stat, hipEvent_t start,
+                              hipEvent_t stop, hipStream_t stream)
+{
+    if (ntiles == 0)
         return hipSuccess;
-    const hipError_t e = with_gather(wfmt, [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(ngroups), dim3(kGatherBlock), 0, stream, groups, insts, par);
+    const hipError_t e = with_format(wfmt, [&](auto fmt) {
+        constexpr uint32_t kF = decltype(fmt)::value;
+        const StepKernel kern = stat ? step_kernel<kF, true>(mode, pass_k) : step_kernel<kF, false>(mode, pass_k);
+        if (start != nullptr)
+            hipExtLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, start, stop, 0, tiles, qs, par);
+        else
+            hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kBlock), 0, stream, tiles, qs, par);
     });
     return e != hipSuccess ? e : hipGetLastError();
 }
 
-hipError_t launch_gather_timed(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par,
-                               uint32_t wfmt, hipEvent_t start, hipEvent_t stop, hipStream_t stream)
+hipError_t launch_bin_kernel(const BinDesc *groups, uint32_t ngroups, uint32_t max_tiles, const QueueSet *qs,
+                             uint32_t par, uint32_t wfmt, hipEvent_t start, hipEvent_t stop, hipStream_t stream)
 {
     if (ngroups == 0)
         return hipSuccess;
-    const hipError_t e = with_gather(wfmt, [&](auto kern) {
-        hipExtLaunchKernelGGL(kern, dim3(ngroups), dim3(kGatherBlock), 0, stream, start, stop, 0, groups, insts, par);
+    const uint32_t lds = std::min(max_tiles, kBinMaxTiles) * (uint32_t)sizeof(uint32_t);
+    const hipError_t e = with_format(wfmt, [&](auto fmt) {
+        auto kern = k_bin<decltype(fmt)::value>;
+        if (start != nullptr)
+            hipExtLaunchKernelGGL(kern, dim3(ngroups), dim3(kBinBlock), lds, stream, start, stop, 0, groups, qs, par);
+        else
+            hipLaunchKernelGGL(kern, dim3(ngroups), dim3(kBinBlock), lds, stream, groups, qs, par);
+    });
+    return e != hipSuccess ? e : hipGetLastError();
+}
+
+hipError_t launch_gather(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par, uint32_t wfmt,
+                         hipEvent_t start, hipEvent_t stop, hipStream_t stream)
+{
+    if (ngroups == 0)
+        return hipSuccess;
+    const hipError_t e = with_format(wfmt, [&](auto fmt) {
+        auto kern = k_gather<decltype(fmt)::value>;
+        if (start != nullptr)
+            hipExtLaunchKernelGGL(kern, dim3(ngroups), dim3(kGatherBlock), 0, stream, start, stop, 0, groups, insts, par);
+        else
+            hipLaunchKernelGGL(kern, dim3(ngroups), dim3(kGatherBlock), 0, stream, groups, insts, par);
     });
     return e != hipSuccess ? e : hipGetLastError();
 }
@@ -2010,13 +2410,13 @@ hipError_t launch_build_grec(const uint32_t *col, const void *w, uint32_t wfmt, 
 }
 
 hipError_t launch_build_segidx(const int64_t *rowptr, const uint32_t *col, uint32_t n, uint32_t ngroups,
-                               uint16_t *segidx, hipStream_t stream)
+                               uint32_t shift, uint16_t *segidx, hipStream_t stream)
 {
     if (n == 0)
         return hipSuccess;
     const uint32_t rows_per_block = kBlock / kWave;
     const uint32_t nb = (n + rows_per_block - 1) / rows_per_block;
-    hipLaunchKernelGGL(k_build_segidx, dim3(nb), dim3(kBlock), 0, stream, rowptr, col, n, ngroups, segidx);
+    hipLaunchKernelGGL(k_build_segidx, dim3(nb), dim3(kBlock), 0, stream, rowptr, col, n, ngroups, shift, segidx);
     return hipGetLastError();
 }
 

@@ -5,44 +5,41 @@
 
 namespace dtb {
 
-// One step of every tile, launch parity `par` (queue accumulation + fold +
-// OU + LIF + binning of the fired rows into queue set par ^ 1).
-// wfmt: the weight format of every instance in the tables, or kWeightAny
-// (each launch's kernels are specialised for it).  stat: some instance
-// records population statistics.
-hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
-                              uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
-                              hipStream_t stream);
+// How a k_step launch's tiles take their input and pass on their rows: queues
+// (or gather), binned by the tiles themselves or by a launch_bin_kernel after
+// it; or direct propagation.
+enum class StepMode { tile_bin, bin_launch, direct };
 
-// launch_step_kernel with `start` / `stop` recorded at the kernel's own
-// dispatch boundaries (kernel time without launch gaps).
-hipError_t launch_step_kernel_timed(const TileDesc *tiles, uint32_t ntiles, const QueueSet *qs,
-                                    uint32_t par, uint32_t pass_k, uint32_t wfmt, bool stat,
-                                    hipEvent_t start, hipEvent_t stop, hipStream_t stream);
+// One step of every tile, launch parity `par` (input of set par + fold + OU +
+// LIF; the emitted rows into set par ^ 1).  pass_k: synapses per lane in a
+// binning pass (tile_bin: 1, 2 or 4).  wfmt: the weight format of every
+// instance in the tables, or kWeightAny (each launch's kernels are
+// specialised for it).  stat: some instance records population statistics.
+// start / stop (may be null): recorded at the kernel's own dispatch
+// boundaries (kernel time without launch gaps).
+hipError_t launch_step_kernel(const TileDesc *tiles, uint32_t ntiles, StepMode mode, uint32_t pass_k,
+                              const QueueSet *qs, uint32_t par, uint32_t wfmt, bool stat, hipEvent_t start,
+                              hipEvent_t stop, hipStream_t stream);
 
-// Split binning: bins the passes listed by the k_step launch of parity
-// `par` (grid workgroups, each wave one pass at a time); nothing when the
-// queue set has no pass list.  Events may be null.
-hipError_t launch_bin_kernel(uint32_t grid, const InstDev *insts, const QueueSet &qs,
-                             uint32_t par, uint32_t pass_k, uint32_t wfmt, hipEvent_t start,
-                             hipEvent_t stop, hipStream_t stream);
+// Bins the rows emitted by the k_step launch of parity `par` into queue set
+// par ^ 1 (groups of source tiles; max_tiles: tiles of the largest instance).
+hipError_t launch_bin_kernel(const BinDesc *groups, uint32_t ngroups, uint32_t max_tiles, const QueueSet *qs,
+                             uint32_t par, uint32_t wfmt, hipEvent_t start, hipEvent_t stop, hipStream_t stream);
 
 // Gather propagation: delta of fired list `par` into InstDev::dlt for every
 // group (runs before the k_step launch of parity `par`, and before
 // materialize / settle of set `par`); empties fired list par ^ 1.
 hipError_t launch_gather(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par, uint32_t wfmt,
-                         hipStream_t stream);
-hipError_t launch_gather_timed(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par,
-                               uint32_t wfmt, hipEvent_t start, hipEvent_t stop, hipStream_t stream);
+                         hipEvent_t start, hipEvent_t stop, hipStream_t stream);
 
-// Group offsets of the gather propagation ([n][ngroups + 1], rows ordered
+// Offsets per target group of 2^shift neurons ([n][ngroups + 1], rows ordered
 // by target group).
 // Gather records ([nsyn][grec_words(wfmt)]: column, weight pair bits).
 hipError_t launch_build_grec(const uint32_t *col, const void *w, uint32_t wfmt, uint64_t nsyn, uint32_t *rec,
                              hipStream_t stream);
 
 hipError_t launch_build_segidx(const int64_t *rowptr, const uint32_t *col, uint32_t n, uint32_t ngroups,
-                               uint16_t *segidx, hipStream_t stream);
+                               uint32_t shift, uint16_t *segidx, hipStream_t stream);
 
 // In-edges of the pull propagation from the presynaptic-major CSR: cptr
 // [ntiles + 1] holds each target tile's first in-edge; cursor [ntiles] is

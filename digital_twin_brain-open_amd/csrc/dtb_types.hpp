@@ -122,6 +122,12 @@ struct alignas(16) InstDev {
     const uint32_t *grec;       // [S][grec_words(wfmt)]
     uint32_t *fired;            // [2][kFiredLists][fcap]
     uint32_t *fcount;           // [2][kFiredLists][kFiredCountStride]
+    // Direct propagation (null tidx: off; never together with gather).
+    // tidx[r][t] = offset in row r of its first synapse whose target lies in
+    // tile t or later (tidx[r][ntiles] = row length).  A tile takes its input
+    // straight from the rows of the step before: it reads the emitted bits of
+    // every tile and, per emitted row, the row's segment for itself.
+    const uint16_t *tidx;       // [n][ntiles + 1]
     // Pull propagation (null crec: off; never together with gather).  The
     // in-edges of target tile t are records [cptr[t], cptr[t + 1]) of crec,
     // grec_words(wfmt) words each: key = source row (bits 0..22) | target's
@@ -172,8 +178,22 @@ struct alignas(16) InstDev {
     uint32_t ntiles;
 };
 
-// Words per tile and set of InstDev::bits.
+// Words per tile and set of InstDev::bits: 4 of emitted rows, 4 of deferred
+// rows; with direct propagation, in place of the deferred rows, one word with
+// the count of emitted rows (2 bytes) and, up to kDirectIds, the rows
+// themselves (a byte each).
 constexpr uint32_t kBitWords = 8;
+constexpr uint32_t kDirectIds = 6;
+// Direct propagation: neurons an instance may have (every tile reads the
+// emitted rows of every tile, up to kDirectRounds words per thread, all in
+// registers: built for 2^20 neurons the kernel spilled 27 of them and every
+// size was slower), the emitted rows a tile lists in LDS at a time (with 1024
+// a 200k-neuron step of 1143 rows took 25.5 us, in two rounds, with 2048 18.2;
+// with 4096 five workgroups fit a CU and eight instances in one engine took
+// 14.7 us instead of 12.7), and the synapses a thread has in flight.
+constexpr uint32_t kDirectMaxNeurons = 1u << 18;
+constexpr uint32_t kDirectRows = 2048, kDirectItems = 4;
+constexpr uint32_t kDirectRounds = (kDirectMaxNeurons / kBlock + kBlock - 1) / kBlock;   // tiles per thread
 
 // Weight pair formats kept on the device (include/weights.hpp:14-21 and the
 // decode of presynaptic_voltage.cpp:153-176): two fp32 (8 bytes), two fp16
@@ -220,6 +240,7 @@ constexpr uint32_t kTilePull = 16u;      // pull propagation
 constexpr uint32_t kTileGather = 32u;    // gather propagation
 constexpr uint32_t kTileOneSub = 64u;    // one substep per step
 constexpr uint32_t kTileStat = 128u;     // population statistics are recorded
+constexpr uint32_t kTileDirect = 256u;   // direct propagation
 struct alignas(128) TileDesc {
     unsigned char *state;    // the tile's state block
     const QSyn *queue;       // its queue of set 0
@@ -313,34 +334,28 @@ __host__ __device__ inline size_t count_words(size_t n, uint32_t shift)
     return ((n + (1u << shift) - 1u) >> shift) * kCountLineWords;
 }
 
-// One binning pass of a fired row handed from k_step to k_bin (split
-// binning): synapses [first, first + len) of instance `inst`'s CSR, len at
-// most one pass.
-struct PassEntry {
-    uint64_t first;
-    uint32_t len;
-    uint32_t inst;
+// Split binning (k_bin): a workgroup of kBinBlock threads bins the rows of up to
+// kBinTiles consecutive source tiles (64 bit words: one per lane of a wave),
+// each wave a pass of kBinPass synapses per round, kBinItems per lane.
+constexpr int kBinBlock = 1024;
+constexpr uint32_t kBinTiles = 32;
+constexpr uint32_t kBinItems = 4, kBinDeep = 4;
+constexpr uint32_t kBinPass = kWave * kBinItems;
+constexpr uint32_t kBinMaxTiles = 16384;   // LDS counts of target tiles (64 KB)
+static_assert(kBinTiles * kBlock <= 0x8000, "rows of a group fit 15 bits");
+struct alignas(16) BinDesc {
+    const InstDev *inst;
+    uint32_t tile0;    // first source tile of the instance
+    uint32_t ntile;    // tiles (<= kBinTiles)
 };
-// Words between the two pass-list counts (each on its own 128-byte line).
-constexpr uint32_t kPassCountStride = 32;
-// Most workgroups of a k_bin launch (8 per CU on 256 CUs: all resident).
-constexpr uint32_t kBinGridMax = 2048;
 
 struct StepCtl;
 struct alignas(16) QueueSet {
     const QueueTile *tile;   // [ntiles]
     uint32_t *count;    // [2][ntiles], tile t of set p at word count_slot(p * ntiles + t, cshift)
-    // Split binning (pass == null: off): k_step of parity p appends its
-    // tiles' passes to `pass` (count at pcount[p * kPassCountStride]) and the
-    // k_bin launch after it bins them; passes past pcap are binned by their
-    // own tile.
-    PassEntry *pass;
-    uint32_t *pcount;
     StepCtl *ctl;
     uint32_t ntiles;
     uint32_t cshift;    // kCountShiftDense or kCountShiftSpread
-    uint32_t pcap;
-    uint32_t pad[3];
 };
 
 // Sample request (reference stat_samples_kernel, stat_result.cpp:393-433).

@@ -374,11 +374,10 @@ class Engine:
         return bool(o.value), int(d.value)
 
     def split(self, on=None, capacity=0):
-        """Sets (when given) and returns split binning: the fired rows'
-        binning passes run in a second launch per step over the whole GPU
-        instead of in the tiles whose neurons fired (capacity: pass-list
-        entries, 0 = sized by the instances; passes past it are binned by
-        their own tile).  Same results either way."""
+        """Sets (when given) and returns split binning: the fired rows are
+        binned by a second launch per step, in groups of 32 tiles over the
+        whole GPU, instead of by the tiles whose neurons fired (capacity has
+        no effect).  Same results either way."""
         if on is not None:
             _lib.check(self._lib.dtb_engine_split(self._h, c_int32(int(bool(on))), ctypes.c_uint32(int(capacity))))
         o, c = c_int32(0), ctypes.c_uint32(0)
@@ -398,7 +397,8 @@ class Engine:
         """Sets (when given) and returns the step kernel's schedule: synapses
         per lane in a binning pass (1, 2, 4) and the propagation layout
         ("dense" or "spread" queue counts, "gather" for every instance that
-        allows it, "auto"); every schedule gives the same results.
+        allows it, "auto": the counts by row coverage, and no queues for small
+        instances with ordered rows); every schedule gives the same results.
         Returns (pass_k, requested layout, layout in use)."""
         names = {v: k for k, v in self.LAYOUTS.items()}
         k, l, u = c_int32(0), c_int32(0), c_int32(0)

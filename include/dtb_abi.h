@@ -261,11 +261,10 @@ int dtb_engine_queue_capacity(dtb_engine_t h, uint32_t floor, uint32_t shift);
  * bit-identical results. */
 int dtb_engine_pull(dtb_engine_t h, int32_t on, uint32_t defer_min);
 /* Split binning (the binning stage of src/stage/presynaptic_voltage.cpp:
- * 122-225, scheduled differently): on = the fired rows' binning passes are
- * listed by the step kernel and binned by a second launch per step over the
- * whole GPU, instead of by the tiles whose neurons fired.  capacity = entries
- * of the pass list (0: sized by the instances); passes past it are binned by
- * their own tile.  Results never depend on either. */
+ * 122-225, scheduled differently): on = the fired rows are binned by a second
+ * launch per step, in groups of 32 tiles over the whole GPU, instead of by the
+ * tiles whose neurons fired.  capacity is kept and reported, and has no effect
+ * (there is no list to bound).  Results never depend on either. */
 int dtb_engine_split(dtb_engine_t h, int32_t on, uint32_t capacity);
 int dtb_engine_get_split(dtb_engine_t h, int32_t *on, uint32_t *capacity);
 int dtb_engine_get_pull(dtb_engine_t h, int32_t *on, uint32_t *defer_min);
@@ -279,7 +278,9 @@ int dtb_instance_pull_info(dtb_engine_t h, int inst, int32_t *allowed, int32_t *
  * schedule: pass_k synapses per lane in a binning pass (1, 2 or 4: passes of
  * 64, 128 or 256 synapses dealt to a tile's waves) and the propagation
  * layout: queues whose counts are DENSE (32 per cache line) or SPREAD (one
- * per line; DTB_LAYOUT_AUTO picks by row coverage), or GATHER (every
+ * per line; DTB_LAYOUT_AUTO picks by row coverage, and small instances with
+ * ordered rows take their input straight from the rows emitted in the step
+ * before, without queues), or GATHER (every
  * instance that allows it gathers, per group of 2048 target neurons, the
  * synapses of the last step's fired rows through per-row group offsets; the
  * others use dense queues).  Every schedule gives bit-identical results.
@@ -295,7 +296,9 @@ int dtb_engine_get_schedule(dtb_engine_t h, int32_t *pass_k, int32_t *layout, in
  * allows it; otherwise its turns run the default schedule, untimed for the
  * choice.  Steps run in all: 7 (2 + r (2 + 4)), r = ceil(trial_steps / 4).
  * us_per_step[7] (optional) = mean per schedule, [dense K=1, 2, 4, spread
- * K=1, 2, 4, gather] (gather 0 when not a candidate).  The steps advance the
+ * K=1, 2, 4, gather] (gather 0 when not a candidate; dense K=2 runs, and if
+ * chosen keeps, the automatic layout's direct propagation where an instance
+ * allows it).  The steps advance the
  * simulation exactly as any other steps would; tune in the regime that will
  * be run (after the initial transient). */
 int dtb_engine_autotune(dtb_engine_t h, int64_t trial_steps, int32_t *pass_k, int32_t *layout, float *us_per_step);
