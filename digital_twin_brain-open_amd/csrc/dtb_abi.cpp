@@ -258,7 +258,7 @@ void run_recorded(dtb::Engine &e, dtb::Instance *I, int32_t iters, int32_t t_ste
         throw dtb::Error(dtb::kInvalidParameter, "i_ou samples need the OU background");
     if (want_samples && I->samples().empty())
         throw dtb::Error(dtb::kUnsetSampleFailure, "samples are not set");
-    e.settle();
+    const int64_t step0 = e.settled_step(*I);
     I->configure_run(t_steps, use_ou, e.stream());
     const bool freq = (flags & DTB_RUN_FREQ) != 0 && out && out->freq;
     const bool samples = want_samples && out &&
@@ -285,17 +285,17 @@ void run_recorded(dtb::Engine &e, dtb::Instance *I, int32_t iters, int32_t t_ste
             means[5] = out->gabab_imean;
         }
     }
-    I->begin_record(iters, freq, samples, stat_mask, e.stream());
+    I->begin_record(step0, iters, freq, samples, stat_mask, e.stream());
     e.mark_dirty();
     e.run(iters, (flags & DTB_RUN_GRAPH) ? 64 : 0);
     if (stat_mask & (dtb::kStatI | dtb::kStatReceptor))
-        e.stat_tail();
-    e.sync();
+        e.stat_tail(false);
     if (out)
-        I->fetch_record(freq ? out->freq : nullptr, (flags & DTB_RUN_SAMPLE_SPIKE) ? out->sample_spike : nullptr,
+        I->fetch_record(e.call_stage(), freq ? out->freq : nullptr, (flags & DTB_RUN_SAMPLE_SPIKE) ? out->sample_spike : nullptr,
                         (flags & DTB_RUN_SAMPLE_VMEMB) ? out->sample_vmemb : nullptr,
                         (flags & DTB_RUN_SAMPLE_ISYN) ? out->sample_isynaptic : nullptr,
                         (flags & DTB_RUN_SAMPLE_IOU) ? out->sample_iou : nullptr, means, e.stream());
+    e.sync();
     I->end_record();
     e.mark_dirty();
 }
@@ -678,7 +678,7 @@ int dtb_read_state(dtb_engine_t h, int inst, float *v, int32_t *t_ref_count, uin
         dtb::Engine &e = engine(h);
         e.get(inst);
         e.settle();   // the pending delta of the last step is folded into J
-        e.get(inst)->read_state(v, t_ref_count, f, emitted, i_ou, j, i_syn, e.stream());
+        e.get(inst)->read_state(e.call_stage(), v, t_ref_count, f, emitted, i_ou, j, i_syn, e.stream());
     });
 }
 
@@ -689,7 +689,7 @@ int dtb_write_state(dtb_engine_t h, int inst, const float *v, const int32_t *t_r
         dtb::Engine &e = engine(h);
         e.get(inst);
         e.settle();
-        e.get(inst)->write_state(v, t_ref_count, f, i_ou, j, e.stream());
+        e.get(inst)->write_state(e.call_stage(), v, t_ref_count, f, i_ou, j, e.stream());
         if (j)
             e.clear_queues(inst);   // J already includes the delta of the restored step
     });

@@ -9,6 +9,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <unordered_set>
@@ -414,9 +416,15 @@ void Instance::release_pull()
     pull_built_ = false;
 }
 
+CopyWords Instance::deferred_words()
+{
+    return CopyWords{step_.mutable_gpu_data() + 2, nullptr, (step_.size() - 2 * sizeof(int64_t)) / 4};
+}
+
 void Instance::clear_deferred(hipStream_t s)
 {
-    DTB_HIP(hipMemsetAsync(step_.mutable_gpu_data() + 2, 0, step_.size() - 2 * sizeof(int64_t), s));
+    const CopyWords w = deferred_words();
+    DTB_HIP(launch_copy_words(&w, 1, s));
 }
 
 uint32_t Instance::tile_synapses(uint32_t tile) const
@@ -449,79 +457,170 @@ struct ParamRecEq {
 
 }  // namespace
 
+namespace {
+// Threads for a pass over n neurons' property rows (88 bytes each, so one
+// thread waits for memory): 200k neurons' parameters re-derived took 1.1 ms
+// on one thread.
+uint32_t host_parts(uint32_t n)
+{
+    const uint32_t hw = std::thread::hardware_concurrency();
+    return std::max(1u, std::min({hw ? hw : 4u, 8u, n / 16384u}));
+}
+
+// f(0) .. f(parts - 1), each on a thread of its own; rethrows the first error.
+template <typename F>
+void for_parts(uint32_t parts, F &&f)
+{
+    std::vector<std::exception_ptr> err(parts);
+    std::vector<std::thread> th;
+    auto run = [&](uint32_t k) {
+        try {
+            f(k);
+        } catch (...) {
+            err[k] = std::current_exception();
+        }
+    };
+    uint32_t k = 1;
+    try {
+        for (; k < parts; ++k)
+            th.emplace_back(run, k);
+    } catch (const std::system_error &) {
+        // no more threads: this one does the rest
+    }
+    for (; k < parts; ++k)
+        run(k);
+    run(0);
+    for (auto &t : th)
+        t.join();
+    for (auto &e : err)
+        if (e)
+            std::rethrow_exception(e);
+}
+}  // namespace
+
 void Instance::derive_params(hipStream_t s)
 {
     const float dt_sub = dt_ / (float)t_steps_;
-    const float *prev = nullptr;
-    ParamRec cur{};
-    auto derive = [&](uint32_t i) -> const ParamRec & {
-        const float *p = &props_[(size_t)i * kNumCols];
-        if (prev != nullptr && std::memcmp(p, prev, sizeof(float) * kNumCols) == 0)
-            return cur;   // same property row as the neuron before
-        prev = p;
-        cur.a = make_float4(p[kColVReset], p[kColVTh], dt_sub * (1.0f / p[kColC]), p[kColVLeak]);
-        cur.b = make_float4(p[kColGLeak], p[kColIExt], p[kColNoiseRate],
-                            bits_as_float(refractory_substeps(p[kColTRef], dt_, t_steps_)));
-        cur.g = make_float4(p[kColGU + 0], p[kColGU + 1], p[kColGU + 2], p[kColGU + 3]);
-        cur.v = make_float4(p[kColVU + 0], p[kColVU + 1], p[kColVU + 2], p[kColVU + 3]);
-        // property.cpp:19-29: exp(-dt / tau)
-        cur.d = make_float4(host_expf((-dt_sub) / p[kColTauU + 0]), host_expf((-dt_sub) / p[kColTauU + 1]),
-                            host_expf((-dt_sub) / p[kColTauU + 2]), host_expf((-dt_sub) / p[kColTauU + 3]));
-        return cur;
-    };
+    // A thread's derivation, in neuron order.
+    struct Derive {
+        const float *props;
+        float dt, dt_sub;
+        int32_t t_steps;
+        const float *prev = nullptr;
+        ParamRec cur{};
 
-    // Deduplicate the records: class per neuron + one record per class.
-    std::vector<ParamRec> recs;
-    std::vector<uint16_t> cls(n_);
-    std::unordered_map<ParamRec, uint32_t, ParamRecHash, ParamRecEq> index;
-    bool dense = false;
-    for (uint32_t i = 0; i < n_ && !dense; ++i) {
-        const ParamRec &r = derive(i);
-        if (!recs.empty() && same_bits(r, recs[cls[i - 1]])) {
-            cls[i] = cls[i - 1];
-            continue;
+        const ParamRec &operator()(uint32_t i)
+        {
+            const float *p = props + (size_t)i * kNumCols;
+            if (prev != nullptr && std::memcmp(p, prev, sizeof(float) * kNumCols) == 0)
+                return cur;   // same property row as the neuron before
+            prev = p;
+            cur.a = make_float4(p[kColVReset], p[kColVTh], dt_sub * (1.0f / p[kColC]), p[kColVLeak]);
+            cur.b = make_float4(p[kColGLeak], p[kColIExt], p[kColNoiseRate],
+                                bits_as_float(refractory_substeps(p[kColTRef], dt, t_steps)));
+            cur.g = make_float4(p[kColGU + 0], p[kColGU + 1], p[kColGU + 2], p[kColGU + 3]);
+            cur.v = make_float4(p[kColVU + 0], p[kColVU + 1], p[kColVU + 2], p[kColVU + 3]);
+            // property.cpp:19-29: exp(-dt / tau)
+            cur.d = make_float4(host_expf((-dt_sub) / p[kColTauU + 0]), host_expf((-dt_sub) / p[kColTauU + 1]),
+                                host_expf((-dt_sub) / p[kColTauU + 2]), host_expf((-dt_sub) / p[kColTauU + 3]));
+            return cur;
         }
-        auto it = index.find(r);
-        if (it == index.end()) {
-            if (recs.size() == kMaxParamClasses) {
-                dense = true;
-                break;
+    };
+    const Derive fresh{props_.data(), dt_, dt_sub, t_steps_};
+
+    // Deduplicate the records: class per neuron + one record per class, by
+    // ranges of whole tiles; a range's classes, in the order in which it
+    // meets them, then join those of the ranges before it (the same numbers
+    // as in one pass).
+    const uint32_t ntile = (n_ + kBlock - 1) / kBlock;
+    const uint32_t parts = host_parts(n_);
+    struct Part {
+        std::vector<ParamRec> recs;
+        std::vector<uint32_t> cls;   // of its own classes
+        bool dense = false;
+    };
+    std::vector<Part> part(parts);
+    auto range = [&](uint32_t k) {
+        return std::pair<uint32_t, uint32_t>(
+            std::min<uint32_t>(n_, (uint32_t)((uint64_t)ntile * k / parts) * kBlock),
+            std::min<uint32_t>(n_, (uint32_t)((uint64_t)ntile * (k + 1) / parts) * kBlock));
+    };
+    cls_.resize(n_);
+    uint16_t *cls = cls_.mutable_cpu_data();
+    uint8_t *bl = blocked_.mutable_cpu_data();
+    for_parts(parts, [&](uint32_t k) {
+        Part &p = part[k];
+        Derive derive = fresh;
+        std::unordered_map<ParamRec, uint32_t, ParamRecHash, ParamRecEq> index;
+        const auto [b, e] = range(k);
+        for (uint32_t i = b; i < e; ++i) {
+            bl[i] = props_[(size_t)i * kNumCols + kColBlocked] != 0.0f;
+            if (p.dense)
+                continue;
+            const ParamRec &r = derive(i);
+            if (i > b && same_bits(r, p.recs[cls[i - 1]])) {
+                cls[i] = cls[i - 1];
+                continue;
             }
-            it = index.emplace(r, (uint32_t)recs.size()).first;
-            recs.push_back(r);
+            auto it = index.find(r);
+            if (it == index.end()) {
+                if (p.recs.size() == kMaxParamClasses) {
+                    p.dense = true;
+                    continue;
+                }
+                it = index.emplace(r, (uint32_t)p.recs.size()).first;
+                p.recs.push_back(r);
+            }
+            cls[i] = (uint16_t)it->second;
         }
-        cls[i] = (uint16_t)it->second;
+    });
+    std::vector<ParamRec> recs;
+    bool dense = false;
+    {
+        std::unordered_map<ParamRec, uint32_t, ParamRecHash, ParamRecEq> index;
+        for (Part &p : part) {
+            dense = dense || p.dense;
+            for (const ParamRec &r : p.recs) {
+                if (dense)
+                    break;
+                auto it = index.find(r);
+                if (it == index.end()) {
+                    if (recs.size() == kMaxParamClasses) {
+                        dense = true;
+                        break;
+                    }
+                    it = index.emplace(r, (uint32_t)recs.size()).first;
+                    recs.push_back(r);
+                }
+                p.cls.push_back(it->second);
+            }
+        }
     }
     dense_params_ = dense;
-    const size_t nrec = dense ? n_ : recs.size();
-    prm_.resize(nrec);
-    cls_.resize(n_);
+    prm_.resize(dense ? n_ : recs.size());
     ParamRec *rec = prm_.mutable_cpu_data();
-    if (dense) {
-        prev = nullptr;
-        uint16_t *cl = cls_.mutable_cpu_data();
-        for (uint32_t i = 0; i < n_; ++i) {
-            rec[i] = derive(i);
-            cl[i] = (uint16_t)(i & (kBlock - 1));
-        }
-    } else {
+    if (!dense)
         std::copy(recs.begin(), recs.end(), rec);
-        std::memcpy(cls_.mutable_cpu_data(), cls.data(), sizeof(uint16_t) * n_);
-    }
-    const uint32_t ntile = (n_ + kBlock - 1) / kBlock;
     tile_cls_.assign(ntile, 0u);
-    if (!dense) {
-        for (uint32_t t = 0; t < ntile; ++t) {
-            const uint32_t b = t * kBlock, e = std::min<uint32_t>(n_, b + kBlock);
+    for_parts(parts, [&](uint32_t k) {
+        Derive derive = fresh;
+        const auto [b, e] = range(k);
+        for (uint32_t t0 = b; t0 < e; t0 += kBlock) {
+            const uint32_t t1 = std::min<uint32_t>(e, t0 + kBlock);
             bool same = true;
-            for (uint32_t i = b + 1; i < e && same; ++i)
-                same = cls[i] == cls[b];
-            tile_cls_[t] = same ? (uint32_t)cls[b] + 1u : 0u;
+            for (uint32_t i = t0; i < t1; ++i) {
+                if (dense) {
+                    rec[i] = derive(i);
+                    cls[i] = (uint16_t)(i & (kBlock - 1));
+                } else {
+                    cls[i] = (uint16_t)part[k].cls[cls[i]];
+                    same = same && cls[i] == cls[t0];
+                }
+            }
+            if (!dense)
+                tile_cls_[t0 / kBlock] = same ? (uint32_t)cls[t0] + 1u : 0u;
         }
-    }
-    uint8_t *bl = blocked_.mutable_cpu_data();
-    for (uint32_t i = 0; i < n_; ++i)
-        bl[i] = props_[(size_t)i * kNumCols + kColBlocked] != 0.0f;
+    });
     prm_.to_gpu(s);
     cls_.to_gpu(s);
     blocked_.to_gpu(s);
@@ -625,16 +724,26 @@ void Instance::update_prop_cols(const uint32_t *prop_ids, const uint32_t *brain_
         if (prop_type_column((int)prop_ids[k]) < 0)
             throw Error(kInvalidParameter, "unknown property id");
     }
+    struct Set {
+        uint32_t begin, end;
+        int col;
+        float val;
+    };
+    std::vector<Set> sets;
     for (size_t k = 0; k < n; ++k) {
         const uint32_t q = find_pop(brain_ids[k]);
-        if (q == UINT32_MAX)
-            continue;
-        const int c = prop_type_column((int)prop_ids[k]);
-        for (uint32_t i = pop_begin_[q]; i < pop_begin_[q + 1]; ++i) {
-            float &x = props_[(size_t)i * kNumCols + c];
-            x = assign ? vals[k] : x * vals[k];
-        }
+        if (q != UINT32_MAX)
+            sets.push_back(Set{pop_begin_[q], pop_begin_[q + 1], prop_type_column((int)prop_ids[k]), vals[k]});
     }
+    const uint32_t parts = host_parts(n_);
+    for_parts(parts, [&](uint32_t k) {
+        const uint32_t b = (uint32_t)((uint64_t)n_ * k / parts), e = (uint32_t)((uint64_t)n_ * (k + 1) / parts);
+        for (const Set &v : sets)   // in the caller's order
+            for (uint32_t i = std::max(b, v.begin); i < std::min(e, v.end); ++i) {
+                float &x = props_[(size_t)i * kNumCols + v.col];
+                x = assign ? v.val : x * v.val;
+            }
+    });
     derive_params(s);
 }
 
@@ -707,7 +816,8 @@ void Instance::layout_record(int64_t steps, bool freq, bool stat, bool slots)
     const uint32_t cs = (np + 31u) / 32u * 32u, ss = (np * kStatFields + 15u) / 16u * 16u;
     const uint64_t slot_bytes = (uint64_t)steps * ((freq ? cs * sizeof(uint32_t) : 0) + (stat ? ss * sizeof(long long) : 0));
     uint32_t k = 1;
-    while (k < kRecMaxSlots && (uint64_t)k * kRecTilesPerSlot * np < tiles && 2 * k * slot_bytes <= kRecMaxBytes)
+    while ((uint64_t)steps * tiles >= kRecMinMeets * np && k < kRecMaxSlots &&
+           (uint64_t)k * kRecTilesPerSlot * np < tiles && 2 * k * slot_bytes <= kRecMaxBytes)
         k *= 2;
     if (k > 1) {
         rec_slots_ = k;
@@ -716,11 +826,11 @@ void Instance::layout_record(int64_t steps, bool freq, bool stat, bool slots)
     }
 }
 
-void Instance::begin_record(int64_t steps, bool freq, bool samples, uint32_t stat_mask, hipStream_t s)
+void Instance::begin_record(int64_t step0, int64_t steps, bool freq, bool samples, uint32_t stat_mask, hipStream_t s)
 {
     if (samples && samples_.empty())
         throw Error(kUnsetSampleFailure, "samples requested but not set");
-    rec_step0_ = step(s);
+    rec_step0_ = step0;
     rec_len_ = steps;
     rec_freq_ = freq;
     rec_samples_ = samples;
@@ -728,11 +838,11 @@ void Instance::begin_record(int64_t steps, bool freq, bool samples, uint32_t sta
     auto allocate = [&](bool slots) {
         layout_record(steps, freq, stat_mask != 0, slots);
         if (stat_mask != 0) {
-            rec_stat_.resize(stat_slots() + (rec_slots_ > 1 ? (size_t)steps * npop() * kStatFields : 0));
+            rec_stat_.resize(stat_slots());
             rec_stat_.mutable_gpu_data();
         }
         if (freq) {
-            rec_counts_.resize(count_slots() + (rec_slots_ > 1 ? (size_t)steps * npop() : 0));
+            rec_counts_.resize(count_slots());
             rec_counts_.mutable_gpu_data();
         }
     };
@@ -744,10 +854,9 @@ void Instance::begin_record(int64_t steps, bool freq, bool samples, uint32_t sta
             throw;
         allocate(false);
     }
-    if (stat_mask != 0)
-        DTB_HIP(hipMemsetAsync(rec_stat_.mutable_gpu_data(), 0, rec_stat_.size(), s));
-    if (freq)
-        DTB_HIP(hipMemsetAsync(rec_counts_.mutable_gpu_data(), 0, rec_counts_.size(), s));
+    const CopyWords clear[2] = {{rec_stat_.mutable_gpu_data(), nullptr, stat_mask != 0 ? rec_stat_.size() / 4 : 0},
+                                {rec_counts_.mutable_gpu_data(), nullptr, freq ? rec_counts_.size() / 4 : 0}};
+    DTB_HIP(launch_copy_words(clear, 2, s));
     if (samples) {
         const size_t m = (size_t)steps * samples_.size();
         rec_spike_.resize(m);
@@ -791,46 +900,49 @@ void Instance::end_record()
     rec_len_ = 0;
 }
 
-void Instance::fetch_record(uint32_t *freq, uint8_t *spike, float *v, float *isyn, float *iou, float *const *means,
-                            hipStream_t s)
+void Instance::fetch_record(HostStage &stage, uint32_t *freq, uint8_t *spike, float *v, float *isyn, float *iou,
+                            float *const *means, hipStream_t s)
 {
     if (rec_ext_on_)
         throw Error(kInternal, "the recording is in caller buffers");
-    if (means != nullptr && rec_stat_mask_ != 0) {
-        // stat_result.cpp:266-391 divides by the population size minus its
-        // blocked neurons: mean = (double) sum * 2^-24 / count, as float.
-        std::vector<long long> sums((size_t)rec_len_ * npop() * kStatFields);
-        if (rec_slots_ > 1) {
-            long long *out = rec_stat_.mutable_gpu_data() + stat_slots();
-            DTB_HIP(launch_fold_slots(rec_stat_.gpu_data(), rec_slots_, rec_sstride_, npop() * kStatFields,
-                                      (uint64_t)rec_len_, out, s));
-            DTB_HIP(hipMemcpyAsync(sums.data(), out, sums.size() * sizeof(long long), hipMemcpyDeviceToHost, s));
-        } else {
-            rec_stat_.download(sums.data(), sums.size(), s);
-        }
-        DTB_HIP(hipStreamSynchronize(s));
-        const uint32_t np = npop();
+    const uint32_t np = npop();
+    const bool stats = means != nullptr && rec_stat_mask_ != 0, counts = freq && rec_freq_;
+    if (stats || counts) {
+        RecordRows r{};
+        r.stat = rec_stat_.gpu_data();
+        r.counts = rec_counts_.gpu_data();
+        r.slots = rec_slots_;
+        r.sstride = rec_sstride_;
+        r.cstride = rec_cstride_;
+        r.swidth = stats ? np * kStatFields : 0u;
+        r.cwidth = counts ? np : 0u;
         std::vector<double> cnt(np, 0.0);
-        for (uint32_t q = 0; q < np; ++q)
-            for (uint32_t i = pop_begin_[q]; i < pop_begin_[q + 1]; ++i)
-                cnt[q] += props_[(size_t)i * kNumCols + kColBlocked] != 0.0f ? 0.0 : 1.0;
-        for (int k = 0; k < kStatFields; ++k) {
-            if (means[k] == nullptr)
-                continue;
-            for (int64_t r = 0; r < rec_len_; ++r)
-                for (uint32_t q = 0; q < np; ++q)
-                    means[k][(size_t)r * np + q] =
-                        (float)((double)sums[((size_t)r * np + q) * kStatFields + k] * 0x1p-24 / cnt[q]);
+        if (stats) {
+            const uint8_t *bl = blocked_.cpu_data();
+            for (uint32_t q = 0; q < np; ++q)
+                cnt[q] = (double)std::count(bl + pop_begin_[q], bl + pop_begin_[q + 1], (uint8_t)0);
         }
-    }
-    if (freq && rec_freq_) {
-        if (rec_slots_ > 1) {
-            uint32_t *out = rec_counts_.mutable_gpu_data() + count_slots();
-            DTB_HIP(launch_fold_slots(rec_counts_.gpu_data(), rec_slots_, rec_cstride_, npop(), (uint64_t)rec_len_,
-                                      out, s));
-            DTB_HIP(hipMemcpyAsync(freq, out, (size_t)rec_len_ * npop() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        } else {
-            rec_counts_.download(freq, rec_counts_.count(), s);
+        const size_t row_bytes = (size_t)r.swidth * sizeof(long long) + (size_t)r.cwidth * sizeof(uint32_t);
+        const int64_t most = (int64_t)std::max<size_t>(1, kCallStageBytes / row_bytes);
+        unsigned char *p = stage.reserve(std::max(kCallStageBytes, row_bytes));
+        for (int64_t r0 = 0; r0 < rec_len_; r0 += most) {
+            const int64_t m = std::min(most, rec_len_ - r0);
+            r.out_stat = reinterpret_cast<long long *>(p);
+            r.out_counts = reinterpret_cast<uint32_t *>(p + (size_t)m * r.swidth * sizeof(long long));
+            DTB_HIP(launch_fetch_rows(r, (uint64_t)r0, (uint64_t)m, s));
+            DTB_HIP(hipStreamSynchronize(s));
+            // stat_result.cpp:266-391 divides by the population size minus its
+            // blocked neurons: mean = (double) sum * 2^-24 / count, as float.
+            for (int k = 0; stats && k < kStatFields; ++k) {
+                if (means[k] == nullptr)
+                    continue;
+                for (int64_t t = 0; t < m; ++t)
+                    for (uint32_t q = 0; q < np; ++q)
+                        means[k][(size_t)(r0 + t) * np + q] =
+                            (float)((double)r.out_stat[((size_t)t * np + q) * kStatFields + k] * 0x1p-24 / cnt[q]);
+            }
+            if (counts)
+                std::memcpy(freq + (size_t)r0 * np, r.out_counts, (size_t)m * np * sizeof(uint32_t));
         }
     }
     if (rec_samples_) {
@@ -886,40 +998,48 @@ void Instance::counters(int64_t *step, uint64_t *events, uint64_t *spikes, hipSt
 // arrays of as many neurons as fit (usually all), and each field is one copy:
 // 2M neurons read in 6 ms, 28 ms with the fold on the host.
 struct Instance::StateStage {
-    unsigned char *base = nullptr;
+    unsigned char *base = nullptr;   // device memory, or null: the arrays are pinned host memory
     uint32_t cap = 0;
     StateArrays a{};
 
     static constexpr size_t kPerNeuron = 4 + 4 + 4 + 16 + 4 + 1 + 1;
-    explicit StateStage(uint32_t count)
+    // A small state goes through the call's pinned memory, which the kernel
+    // reads or writes itself: a copy per field of 10k neurons was 250 us.
+    StateStage(HostStage &host, uint32_t count)
     {
-        // at most 1M neurons (34 MB) at a time; fewer when memory is short
-        for (cap = std::min<uint32_t>(count, 1u << 20);; cap /= 2) {
-            try {
-                base = static_cast<unsigned char *>(devmem::alloc((size_t)cap * kPerNeuron));
-                break;
-            } catch (const Error &e) {
-                if (e.code != kOutOfMemory || cap <= 256)
-                    throw;
+        unsigned char *p = nullptr;
+        if (count * kPerNeuron <= kCallStageBytes) {
+            cap = count;
+            p = host.reserve(kCallStageBytes);
+        } else {
+            // at most 1M neurons (34 MB) at a time; fewer when memory is short
+            for (cap = std::min<uint32_t>(count, 1u << 20);; cap /= 2) {
+                try {
+                    p = base = static_cast<unsigned char *>(devmem::alloc((size_t)cap * kPerNeuron));
+                    break;
+                } catch (const Error &e) {
+                    if (e.code != kOutOfMemory || cap <= 256)
+                        throw;
+                }
             }
         }
-        a.J = reinterpret_cast<float4 *>(base);
-        a.V = reinterpret_cast<float *>(base + (size_t)cap * 16);
-        a.t = reinterpret_cast<int32_t *>(base + (size_t)cap * 20);
-        a.iou = reinterpret_cast<float *>(base + (size_t)cap * 24);
-        a.isyn = reinterpret_cast<float *>(base + (size_t)cap * 28);
-        a.f = base + (size_t)cap * 32;
-        a.emitted = base + (size_t)cap * 33;
+        a.J = reinterpret_cast<float4 *>(p);
+        a.V = reinterpret_cast<float *>(p + (size_t)cap * 16);
+        a.t = reinterpret_cast<int32_t *>(p + (size_t)cap * 20);
+        a.iou = reinterpret_cast<float *>(p + (size_t)cap * 24);
+        a.isyn = reinterpret_cast<float *>(p + (size_t)cap * 28);
+        a.f = p + (size_t)cap * 32;
+        a.emitted = p + (size_t)cap * 33;
     }
     ~StateStage() { devmem::release(base); }
     StateStage(const StateStage &) = delete;
     StateStage &operator=(const StateStage &) = delete;
 };
 
-void Instance::read_state(float *V, int32_t *t, uint8_t *f, uint8_t *emitted, float *iou, float *J, float *isyn,
+void Instance::read_state(HostStage &stage, float *V, int32_t *t, uint8_t *f, uint8_t *emitted, float *iou, float *J, float *isyn,
                           hipStream_t s)
 {
-    StateStage st(n_);
+    StateStage st(stage, n_);
     StateArrays a = st.a;
     a.V = V ? a.V : nullptr;
     a.t = t ? a.t : nullptr;
@@ -931,8 +1051,12 @@ void Instance::read_state(float *V, int32_t *t, uint8_t *f, uint8_t *emitted, fl
     for (uint32_t b = 0; b < n_; b += st.cap) {
         const size_t m = std::min(st.cap, n_ - b);
         DTB_HIP(launch_read_state(state_view(), b, (uint32_t)m, a, s));
+        if (st.base == nullptr)
+            DTB_HIP(hipStreamSynchronize(s));
         auto copy = [&](auto *dst, const auto *src, size_t per) {
-            if (dst != nullptr)
+            if (dst != nullptr && st.base == nullptr)
+                std::memcpy(dst, src, m * per * sizeof(*dst));
+            else if (dst != nullptr)
                 DTB_HIP(hipMemcpyAsync(dst + (size_t)b * per, src, m * per * sizeof(*dst), hipMemcpyDeviceToHost, s));
         };
         copy(V, a.V, 1);
@@ -946,12 +1070,12 @@ void Instance::read_state(float *V, int32_t *t, uint8_t *f, uint8_t *emitted, fl
     DTB_HIP(hipStreamSynchronize(s));
 }
 
-void Instance::write_state(const float *V, const int32_t *t, const uint8_t *f, const float *iou, const float *J,
+void Instance::write_state(HostStage &stage, const float *V, const int32_t *t, const uint8_t *f, const float *iou, const float *J,
                            hipStream_t s)
 {
     if (!V && !t && !f && !iou && !J)
         return;
-    StateStage st(n_);
+    StateStage st(stage, n_);
     StateArrays a = st.a;
     a.V = V ? a.V : nullptr;
     a.t = t ? a.t : nullptr;
@@ -961,7 +1085,9 @@ void Instance::write_state(const float *V, const int32_t *t, const uint8_t *f, c
     for (uint32_t b = 0; b < n_; b += st.cap) {
         const size_t m = std::min(st.cap, n_ - b);
         auto copy = [&](auto *dst, const auto *src, size_t per) {
-            if (src != nullptr)
+            if (src != nullptr && st.base == nullptr)
+                std::memcpy(dst, src, m * per * sizeof(*src));
+            else if (src != nullptr)
                 DTB_HIP(hipMemcpyAsync(dst, src + (size_t)b * per, m * per * sizeof(*src), hipMemcpyHostToDevice, s));
         };
         copy(a.V, V, 1);

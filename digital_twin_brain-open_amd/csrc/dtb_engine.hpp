@@ -208,6 +208,41 @@ private:
     std::vector<T> cpu_;
 };
 
+// Pinned host memory that kernels read and write in place: what a call
+// uploads (its tables) and returns (its records, a small state), without a
+// copy call each.  Grows; freed with its owner.
+class HostStage {
+public:
+    HostStage() = default;
+    ~HostStage() { release(); }
+    HostStage(const HostStage &) = delete;
+    HostStage &operator=(const HostStage &) = delete;
+    // At least `bytes`; what it held before is lost when it grows, so no
+    // kernel may be using it.
+    unsigned char *reserve(size_t bytes)
+    {
+        if (bytes > cap_) {
+            release();
+            DTB_HIP(hipHostMalloc(&p_, bytes, hipHostMallocDefault));
+            cap_ = bytes;
+        }
+        return static_cast<unsigned char *>(p_);
+    }
+
+private:
+    void release()
+    {
+        if (p_ != nullptr)
+            (void)hipHostFree(p_);
+        p_ = nullptr;
+        cap_ = 0;
+    }
+    void *p_ = nullptr;
+    size_t cap_ = 0;
+};
+// A call's results are taken through at most this much pinned memory at a time.
+constexpr size_t kCallStageBytes = (size_t)1 << 20;
+
 // Host description of a network in the reference layout: property matrix
 // [n][22] and a presynaptic-major CSR whose synapses carry a weight pair and a
 // channel bit (0: AMPA/NMDA pair, 1: GABA_A/GABA_B pair), bit-packed in
@@ -283,7 +318,8 @@ public:
     bool configure_run(int32_t t_steps, bool use_ou, hipStream_t s);
     // Recording window of `steps` rows starting at the current step;
     // stat_mask selects per-population means (kStatV | kStatI | kStatReceptor).
-    void begin_record(int64_t steps, bool freq, bool samples, uint32_t stat_mask, hipStream_t s);
+    // step0: the step index (step()).
+    void begin_record(int64_t step0, int64_t steps, bool freq, bool samples, uint32_t stat_mask, hipStream_t s);
     // The same window recorded into caller-provided device buffers (no
     // allocation): counts [steps][npop] and sums [steps][npop][kStatFields]
     // are zeroed here; the sample rows [steps][nsample] need no clearing.
@@ -303,15 +339,15 @@ public:
     uint32_t stat_mask() const { return rec_stat_mask_; }
     // means: [6] arrays [steps][npop] (vmean, imean, AMPA, NMDA, GABA_A,
     // GABA_B), any may be null.
-    void fetch_record(uint32_t *freq, uint8_t *spike, float *v, float *isyn, float *iou, float *const *means,
+    void fetch_record(HostStage &stage, uint32_t *freq, uint8_t *spike, float *v, float *isyn, float *iou, float *const *means,
                       hipStream_t s);
 
     // Reference-visible state after the last completed step: V, refractory
     // counter, spike flag, emitted flag, i_ou, J[4] (pending delta folded
     // in), I_syn (without i_ou).
-    void read_state(float *V, int32_t *t, uint8_t *f, uint8_t *emitted, float *iou, float *J, float *isyn,
+    void read_state(HostStage &stage, float *V, int32_t *t, uint8_t *f, uint8_t *emitted, float *iou, float *J, float *isyn,
                     hipStream_t s);
-    void write_state(const float *V, const int32_t *t, const uint8_t *f, const float *iou, const float *J,
+    void write_state(HostStage &stage, const float *V, const int32_t *t, const uint8_t *f, const float *iou, const float *J,
                      hipStream_t s);
     // The step index is kept in two device slots (read and written by
     // alternating launch parities); the current step is the larger one.
@@ -379,6 +415,8 @@ public:
     // Forgets emitted and deferred rows (after the pending input was folded
     // or dropped).
     void clear_deferred(hipStream_t s);
+    CopyWords deferred_words();   // the same as a launch_copy_words segment
+    const int64_t *step_words() { return step_.gpu_data(); }   // [2], the larger one is the step index
 
     // Direct propagation: possible when every row is ordered by target and at
     // most kGatherMaxRow long, the instance has at most kDirectMaxNeurons
@@ -576,11 +614,17 @@ public:
     void clear_queues(int id);
     // Records the I_syn-based statistics of the last step run (imean,
     // receptor imeans), which the next step's launch would otherwise take.
-    void stat_tail();
+    // wait: until it is done; else only enqueued on stream().
+    void stat_tail(bool wait = true);
     // Folds every pending delta into J with the current tables and
     // parameters.  Must run before parameters, samples, recording or the
     // instance set change (a table rebuild empties the queues).
-    void settle();
+    // wait: until it is done; else only enqueued on stream().
+    void settle(bool wait = true);
+    // settle(), and the step index of instance p.
+    int64_t settled_step(Instance &p);
+    // Pinned memory for one call's results.
+    HostStage &call_stage() { return call_stage_; }
 
     // Kernel-time measurement: events recorded around every step kernel
     // (total in ms over `steps` steps).
@@ -651,6 +695,14 @@ private:
     bool try_direct(Instance &p);          // builds p's tile offsets if they fit
     uint32_t nqueue_tiles_ = 0;            // tiles of the queue and gather instances (first in the tables)
     bool tuned_direct_ = false;            // the autotuner's (dense, default pass) candidate ran direct
+    HostStage tables_stage_, call_stage_;
+    // Everything a captured step's launches take from the engine: graphs stay
+    // as long as it does (what changes from run to run is in the tables).
+    struct GraphKey {
+        const void *tiles, *insts, *queues, *qtiles, *qcnt, *bins, *groups, *samples, *recs;
+        uint32_t ntiles, nqueue_tiles, nbins, bin_tiles, ngroups, nsamples, cshift, pass_k, wfmt, stat;
+    };
+    GraphKey graph_key_{};
     hipGraphExec_t graph_[2] = {nullptr, nullptr};   // by starting parity
     int graph_steps_[2] = {0, 0};
 };

@@ -2169,19 +2169,48 @@ __global__ __launch_bounds__(kBlock) void k_stat_tail(const TileDesc *__restrict
                   s_stat[tid]);
 }
 
-// Adds up the slots of a record: out[row][i] = sum over slots of
-// in[row][slot][i], i < width (integers, so the order does not matter).
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_fold_slots(const T *__restrict__ in, uint32_t slots, uint32_t stride,
-                                                       uint32_t width, uint64_t cells, T *__restrict__ out)
+// Rows [row0, row0 + rows) of a record with each row's slots added up
+// (integers, so the order does not matter), statistics first.  The outputs
+// are the call's pinned host memory, so a small record costs one launch and
+// no copy: two folds and two copies were 45 us of a 240 us call.
+__global__ __launch_bounds__(kBlock) void k_fetch_rows(RecordRows r, uint64_t row0, uint64_t rows)
 {
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < cells; i += (uint64_t)gridDim.x * kBlock) {
-        const uint64_t row = i / width;
-        const T *p = in + row * slots * stride + (i - row * width);
-        T s = 0;
-        for (uint32_t k = 0; k < slots; ++k)
-            s += p[(size_t)k * stride];
-        out[i] = s;
+    const uint64_t ns = rows * r.swidth, nc = rows * r.cwidth;
+    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < ns + nc; i += (uint64_t)gridDim.x * kBlock) {
+        if (i < ns) {
+            const uint64_t row = i / r.swidth;
+            const long long *p = r.stat + (row0 + row) * r.slots * r.sstride + (i - row * r.swidth);
+            long long s = 0;
+            for (uint32_t k = 0; k < r.slots; ++k)
+                s += p[(size_t)k * r.sstride];
+            r.out_stat[i] = s;
+        } else {
+            const uint64_t c = i - ns, row = c / r.cwidth;
+            const uint32_t *p = r.counts + (row0 + row) * r.slots * r.cstride + (c - row * r.cwidth);
+            uint32_t s = 0;
+            for (uint32_t k = 0; k < r.slots; ++k)
+                s += p[(size_t)k * r.cstride];
+            r.out_counts[c] = s;
+        }
+    }
+}
+
+// Several small copies and fills in one launch: the tables of a run (up to
+// nine) from pinned host memory, and the words a call clears.  One hipMemcpy
+// or hipMemset each cost 3-20 us of host time, most of a short call's.
+struct CopyList {
+    CopyWords seg[kCopySegs];
+    int n;
+};
+
+__global__ __launch_bounds__(kBlock) void k_copy_words(CopyList l)
+{
+    for (int k = 0; k < l.n; ++k) {
+        uint32_t *dst = static_cast<uint32_t *>(l.seg[k].dst);
+        const uint32_t *src = static_cast<const uint32_t *>(l.seg[k].src);
+        for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < l.seg[k].words;
+             i += (uint64_t)gridDim.x * kBlock)
+            dst[i] = src != nullptr ? src[i] : 0u;
     }
 }
 
@@ -2459,22 +2488,36 @@ hipError_t launch_stat_tail(const TileDesc *tiles, uint32_t ntiles, const InstDe
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_fold_slots(const T *in, uint32_t slots, uint32_t stride, uint32_t width, uint64_t rows, T *out,
-                             hipStream_t stream)
+hipError_t launch_fetch_rows(const RecordRows &r, uint64_t row0, uint64_t rows, hipStream_t stream)
 {
-    const uint64_t cells = rows * width;
+    const uint64_t cells = rows * ((uint64_t)r.swidth + r.cwidth);
     if (cells == 0)
         return hipSuccess;
     const uint64_t nb = std::min<uint64_t>((cells + kBlock - 1) / kBlock, 4096);
-    hipLaunchKernelGGL(k_fold_slots<T>, dim3((uint32_t)nb), dim3(kBlock), 0, stream, in, slots, stride, width, cells,
-                       out);
+    hipLaunchKernelGGL(k_fetch_rows, dim3((uint32_t)nb), dim3(kBlock), 0, stream, r, row0, rows);
     return hipGetLastError();
 }
-template hipError_t launch_fold_slots<uint32_t>(const uint32_t *, uint32_t, uint32_t, uint32_t, uint64_t, uint32_t *,
-                                                hipStream_t);
-template hipError_t launch_fold_slots<long long>(const long long *, uint32_t, uint32_t, uint32_t, uint64_t,
-                                                 long long *, hipStream_t);
+
+hipError_t launch_copy_words(const CopyWords *segs, int n, hipStream_t stream)
+{
+    while (n > 0) {
+        CopyList l{};
+        uint64_t most = 0;
+        for (l.n = 0; l.n < kCopySegs && n > 0; --n, ++segs)
+            if (segs->words > 0) {
+                l.seg[l.n++] = *segs;
+                most = std::max(most, segs->words);
+            }
+        if (l.n == 0)
+            continue;
+        const uint64_t nb = std::min<uint64_t>((most + kBlock - 1) / kBlock, 1024);
+        hipLaunchKernelGGL(k_copy_words, dim3((uint32_t)nb), dim3(kBlock), 0, stream, l);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
 
 hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_t nsamples,
                          const SampleRecDev *recs, uint32_t par, hipStream_t stream)

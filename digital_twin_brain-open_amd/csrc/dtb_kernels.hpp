@@ -61,10 +61,28 @@ hipError_t launch_settle(const TileDesc *tiles, uint32_t ntiles, const InstDev *
 hipError_t launch_stat_tail(const TileDesc *tiles, uint32_t ntiles, const InstDev *insts, uint32_t par,
                             hipStream_t stream);
 
-// Sums of the slots of a record: out[rows][width] from in[rows][slots][stride].
-template <typename T>
-hipError_t launch_fold_slots(const T *in, uint32_t slots, uint32_t stride, uint32_t width, uint64_t rows, T *out,
-                             hipStream_t stream);
+// Copies `words` 4-byte words of src (null: zeros) to dst; either may be
+// pinned host memory.
+struct CopyWords {
+    void *dst;
+    const void *src;
+    uint64_t words;
+};
+// All of segs[n] (kCopySegs per launch).
+constexpr int kCopySegs = 10;
+hipError_t launch_copy_words(const CopyWords *segs, int n, hipStream_t stream);
+
+// Rows [row0, row0 + rows) of a record, each row's slots added up, as plain
+// arrays: sums [rows][swidth] and counts [rows][cwidth] (width 0: none).
+// The outputs may be pinned host memory.
+struct RecordRows {
+    const long long *stat;
+    const uint32_t *counts;
+    uint32_t slots, sstride, cstride, swidth, cwidth;
+    long long *out_stat;
+    uint32_t *out_counts;
+};
+hipError_t launch_fetch_rows(const RecordRows &r, uint64_t row0, uint64_t rows, hipStream_t stream);
 
 // Samples of the step run by the k_step launch of parity `par`.
 hipError_t launch_sample(const InstDev *insts, const SampleDev *samples, uint32_t nsamples,

@@ -64,6 +64,9 @@ constexpr int kStatFields = 6;           // V, I_syn, AMPA, NMDA, GABA_A, GABA_B
 // line then serves about 8 x 6 atomics of 8 ns per step), at most
 // kRecMaxSlots, and fewer where the slots of a record would pass kRecMaxBytes.
 constexpr uint32_t kRecTilesPerSlot = 8, kRecMaxSlots = 64;
+// Atomics that must meet on one line, over the record, before it has slots
+// (8 ns each).
+constexpr uint64_t kRecMinMeets = 1024;
 constexpr uint64_t kRecMaxBytes = (uint64_t)64 << 20;
 
 // Largest number of distinct parameter records kept as classes (2-byte class
