@@ -228,6 +228,7 @@ Instance::Instance(const FanoutSpec &f, float dt, uint64_t seed, hipStream_t s)
     group_coverage_ = 1.0 - std::pow(1.0 - 1.0 / ngroups(), (double)f.K);
     // rows are ordered by target, K <= 8192
     gather_ok_ = (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
+    choose_groups(true);
     direct_ok_ = direct_fits();
 }
 
@@ -288,7 +289,16 @@ void Instance::count_tile_synapses(const NetworkHost &net)
     row_coverage_ = (double)sg / ((double)n_ * (double)nfine);
     group_coverage_ = (double)gs / ((double)n_ * (double)ngroups());
     gather_ok_ = ordered && nsyn_ > 0 && (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
+    choose_groups(by_tile);
     direct_ok_ = by_tile && direct_fits();
+}
+
+void Instance::choose_groups(bool by_tile)
+{
+    gather_bits_ = kGroupBits;
+    while (by_tile && gather_bits_ > kGroupBitsMin && ngroups(gather_bits_) < kGatherGroups &&
+           (double)n_ * (ngroups(gather_bits_ - 1u) + 1.0) * 2.0 <= 12.0 * (double)nsyn_)
+        --gather_bits_;
 }
 
 uint32_t Instance::fired_capacity() const
@@ -308,8 +318,9 @@ void Instance::ensure_gather(hipStream_t s)
         fcount_.mutable_gpu_data();
         fired_.resize(2 * (size_t)kFiredLists * fired_capacity());
         fired_.mutable_gpu_data();
-        segidx_.resize((size_t)n_ * (ngroups() + 1u));
-        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ngroups(), kGroupBits,
+        const uint32_t ng = ngroups(gather_bits_);
+        segidx_.resize((size_t)n_ * (ng + 1u));
+        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ng, gather_bits_,
                                     segidx_.mutable_gpu_data(), s));
         grec_.resize((size_t)nsyn_ * grec_words(wfmt_));
         DTB_HIP(launch_build_grec(col_.gpu_data(), w_.gpu_data(), wfmt_, (uint64_t)nsyn_, grec_.mutable_gpu_data(),
@@ -1137,7 +1148,7 @@ InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, u
         d.grec = grec_.gpu_data();
         d.fired = fired_.mutable_gpu_data();
         d.fcount = fcount_.mutable_gpu_data();
-        d.ngroups = ngroups();
+        d.ngroups = ngroups(gather_bits_);
         d.fcap = fired_capacity();
     }
     d.prm = prm_.gpu_data();

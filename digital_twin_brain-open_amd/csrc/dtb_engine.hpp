@@ -389,9 +389,14 @@ public:
     // target group, no row is longer than kGatherMaxRow and the group offsets
     // ([n][ngroups + 1] x 2 bytes) are no larger than the synapse arrays.
     bool gather_allowed() const { return gather_ok_; }
-    // Mean over rows of the fraction of the groups that the row reaches.
+    // Mean over rows of the fraction of the groups of 2^kGroupBits neurons
+    // that the row reaches.
     double group_coverage() const { return group_coverage_; }
-    uint32_t ngroups() const { return (n_ + (1u << kGroupBits) - 1) >> kGroupBits; }
+    uint32_t ngroups(uint32_t bits = kGroupBits) const { return (n_ + (1u << bits) - 1) >> bits; }
+    // Neurons per group of k_gather (log2): 2^kGroupBits, or fewer to get
+    // kGatherGroups groups, where rows are ordered by tile and the offsets of
+    // the smaller groups keep to the same limit.
+    uint32_t gather_bits() const { return gather_bits_; }
     // Rows per fired list (the tiles of one list hold at most this many).
     uint32_t fired_capacity() const;
     // Builds the group offsets and fired lists if not built yet.
@@ -493,6 +498,8 @@ private:
     double row_coverage_ = 0.0;           // mean fraction of the tiles one row reaches
     double group_coverage_ = 0.0;         // mean fraction of the gather groups one row reaches
     bool gather_ok_ = false;              // gather_allowed()
+    uint32_t gather_bits_ = kGroupBits;   // gather_bits()
+    void choose_groups(bool by_tile);     // sets gather_bits_
     bool gather_built_ = false;           // segidx_, fired_, fcount_ built
     bool direct_ok_ = false;              // direct_allowed()
     bool direct_fits() const;             // its conditions on the sizes

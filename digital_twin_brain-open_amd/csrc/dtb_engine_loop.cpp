@@ -363,8 +363,9 @@ void Engine::rebuild()
         const bool gat = use_gather(*p);
         if (gat) {
             p->ensure_gather(stream_);
-            for (uint32_t g = 0; g < p->ngroups(); ++g)
-                groups.push_back(GroupDesc{idx, g, std::min<uint32_t>(1u << kGroupBits, p->n() - (g << kGroupBits)), 0u});
+            const uint32_t gb = p->gather_bits();
+            for (uint32_t g = 0; g < p->ngroups(gb); ++g)
+                groups.push_back(GroupDesc{idx, g, std::min<uint32_t>(1u << gb, p->n() - (g << gb)), gb});
         } else if (p->gather_built() && !tuning_) {
             // the old tables (settled above) were the last to use them;
             // device memory returns to the cache

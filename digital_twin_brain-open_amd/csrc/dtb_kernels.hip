@@ -1756,17 +1756,16 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(const BinDesc *__restrict__ g
 
 // Gather propagation (instances with InstDev::segidx; their k_step reads
 // the delta from dlt): the delta of the rows fired by the last launch (the
-// fired lists of set `par`) for one group of kGroupTiles tiles, written into
-// dlt.  A wave takes
-// 64 fired rows at a time: lane l reads row l's segment bounds for the group
+// fired lists of set `par`) for one group of consecutive neurons (GroupDesc),
+// written into dlt.  A wave takes 64 fired rows at a time: lane l reads row l's segment bounds for the group
 // from the row's group offsets, a wave prefix sum lays the segments end to
 // end, and the wave then reads them with consecutive lanes on consecutive
 // synapses (a segment is contiguous in the row), adding each weight pair
 // into the group's Q23.40 LDS sums (64-bit integer atomics, so the result
 // does not depend on the order); each lane has kGatherItems synapses in
-// flight.  Groups of 2048 neurons give segments of about 20 synapses at the
-// stress shape (in-degree 5000 on 500k neurons), which is what coalesces the
-// reads; one 1024-thread workgroup per group.  Also empties the fired lists
+// flight.  Segments of about 20 synapses (in-degree 5000, 2048 neurons of
+// 500k, 1024 of 200k) coalesce the reads; one 1024-thread workgroup per group,
+// and smaller groups where those of 2048 leave CUs idle.  Also empties the fired lists
 // of set par ^ 1 (the ones the k_step launch after this one fills; their
 // last reader was the previous k_gather).  Consecutive groups go to one XCD (workgroups
 // are dealt to the 8 XCDs round-robin by index), so the segments of
@@ -1784,11 +1783,14 @@ __global__ __launch_bounds__(kGatherBlock) __attribute__((amdgpu_waves_per_eu(8)
     const uint32_t nb = gridDim.x, x = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     const GroupDesc d = groups[x * (nb >> 3) + min(x, nb & 7u) + slot];
     const InstDev &I = insts[d.inst];
+    const uint32_t nn = 1u << d.bits;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = __lane_id();
     const uint32_t wv = tid / kWave;
-    for (uint32_t i = tid; i < kNeurons * 4; i += kGatherBlock)
-        acc[i] = 0ull;
+    for (uint32_t i = tid; i < nn; i += kGatherBlock)
+#pragma unroll
+        for (uint32_t c = 0; c < 4u; ++c)
+            acc[acc_at(i, c, kNeurons)] = 0ull;
     // the fired lists of set par laid end to end: lane l holds list l's count
     const uint32_t lcnt = gp(I.fcount)[((size_t)par * kFiredLists + lane) * kFiredCountStride];
     uint32_t lincl = lcnt;
@@ -1806,7 +1808,7 @@ __global__ __launch_bounds__(kGatherBlock) __attribute__((amdgpu_waves_per_eu(8)
     const auto fired = gp(I.fired) + (size_t)par * kFiredLists * I.fcap;
     const uint32_t wfmt = kFmt != kWeightAny ? kFmt : I.wfmt;
     const uint32_t stride = I.ngroups + 1u;
-    const uint32_t first = d.g << kGroupBits;
+    const uint32_t first = d.g << d.bits;
     for (uint32_t c0 = wv * kWave; c0 < nf; c0 += kGatherBlock) {
         const uint32_t k = c0 + lane;
         const bool valid = k < nf;

@@ -173,7 +173,7 @@ struct alignas(16) InstDev {
     uint32_t tile_base;         // engine-wide index of this instance's first tile
     uint32_t stat_mask;         // kStatV | kStatI | kStatReceptor: statistics recorded in rec_stat
     uint32_t pmask;             // parameter record of neuron i: (i & pmask) + cls[i]
-    uint32_t ngroups;           // gather groups of the instance (kGroupTiles tiles each)
+    uint32_t ngroups;           // gather groups of the instance
     uint32_t fcap;              // rows per fired list
     uint32_t defer_min;         // pull: a tile with this many emitted rows defers them (0: never)
     uint32_t wfmt;              // weight pair format of w and cw
@@ -276,11 +276,17 @@ struct alignas(16) QueueTile {
 };
 
 // Gather propagation: one workgroup of kGatherBlock threads gathers the
-// synapses of every fired row that target one group of kGroupTiles
-// consecutive tiles (2^kGroupBits neurons) into LDS, then writes their delta.
-constexpr uint32_t kGroupTiles = 8;
-constexpr uint32_t kGroupBits = kTileBits + 3;
-static_assert((1u << (kGroupBits - kTileBits)) == kGroupTiles, "a group is kGroupTiles tiles");
+// synapses of every fired row that target one group of consecutive neurons
+// (at most 2^kGroupBits; Instance::gather_bits) into LDS, then writes their
+// delta.
+constexpr uint32_t kGroupBits = kTileBits + 3, kGroupBitsMin = kTileBits;
+// Groups below which an instance is cut into smaller ones: one workgroup per
+// group, 256 CUs.  Steps with groups of 2^kGroupBits neurons / by the rule:
+// 20k neurons x 2000 synapses 67 / 18 us, 60k x 3000 49 / 17, 120k x 3000
+// 39 / 22, 200k x 5000 42 / 31 (98 / 196 groups); past it halving the group
+// costs more (every group looks every row up) than it fills: 300k x 2000, 147
+// groups 30.8 us, 293 35.4.
+constexpr uint32_t kGatherGroups = 128;
 constexpr int kGatherBlock = 1024;
 // Synapses each lane of k_gather loads before it adds them (in flight together).
 constexpr uint32_t kGatherItems = 8;
@@ -294,9 +300,9 @@ static_assert(kFiredLists == 64, "k_gather reads one list count per lane");
 
 struct alignas(16) GroupDesc {
     uint32_t inst;
-    uint32_t g;         // group index within the instance (first neuron g << kGroupBits)
+    uint32_t g;         // group index within the instance (first neuron g << bits)
     uint32_t count;     // neurons in the group
-    uint32_t pad;
+    uint32_t bits;      // Instance::gather_bits()
 };
 
 // Queues of both parities: the launch of parity p drains set p and fills set

@@ -281,7 +281,7 @@ int dtb_instance_pull_info(dtb_engine_t h, int inst, int32_t *allowed, int32_t *
  * per line; DTB_LAYOUT_AUTO picks by row coverage, and small instances with
  * ordered rows take their input straight from the rows emitted in the step
  * before, without queues), or GATHER (every
- * instance that allows it gathers, per group of 2048 target neurons, the
+ * instance that allows it gathers, per group of 256 to 2048 target neurons, the
  * synapses of the last step's fired rows through per-row group offsets; the
  * others use dense queues).  Every schedule gives bit-identical results.
  * layout_in_use: GATHER when some instance gathers, else DENSE or SPREAD. */
