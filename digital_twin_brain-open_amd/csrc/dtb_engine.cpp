@@ -228,6 +228,9 @@ Instance::Instance(const FanoutSpec &f, float dt, uint64_t seed, hipStream_t s)
     group_coverage_ = 1.0 - std::pow(1.0 - 1.0 / ngroups(), (double)f.K);
     // rows are ordered by target, K <= 8192
     gather_ok_ = (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
+    src_pass_.assign(ntile, 0u);
+    for (uint32_t t = 0; t < ntile; ++t)
+        src_pass_[t] = std::min<uint32_t>(kBlock, n_ - t * kBlock) * (((uint32_t)f.K + kBinPass - 1u) / kBinPass);
     choose_groups(true);
     direct_ok_ = direct_fits();
 }
@@ -241,6 +244,9 @@ void Instance::count_tile_synapses(const NetworkHost &net)
     // these counts are its exact capacity.
     const uint32_t nfine = (n_ + (1u << kTileBits) - 1) >> kTileBits;
     tile_syn_.assign(nfine, 0u);
+    src_pass_.assign(nfine, 0u);
+    for (uint32_t r = 0; r < n_; ++r)
+        src_pass_[r >> kTileBits] += (uint32_t)((net.rowptr[r + 1] - net.rowptr[r] + kBinPass - 1) / kBinPass);
     unsigned hw = std::thread::hardware_concurrency();
     const int nt = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(hw ? hw : 4u, 16u), nsyn_ / (1 << 20)));
     std::vector<std::vector<uint32_t>> part(nt, std::vector<uint32_t>(nfine, 0u));
@@ -367,6 +373,38 @@ void Instance::ensure_direct(hipStream_t s)
         tidx_.resize(0);
         throw;
     }
+}
+
+void Instance::ensure_passes()
+{
+    if (passes_built())
+        return;
+    // list l takes the tiles t with t * kFiredLists / ntiles == l
+    const uint64_t nt = src_pass_.size();
+    std::vector<uint64_t> cap(kFiredLists, 0);
+    for (uint64_t t = 0; t < nt; ++t)
+        cap[t * kFiredLists / nt] += src_pass_[t];
+    passcap_ = std::max<uint64_t>(1, *std::max_element(cap.begin(), cap.end()));
+    try {
+        pass_count_.resize(2 * (size_t)kFiredLists * kFiredCountStride);
+        pass_count_.mutable_gpu_data();
+        passes_.resize((size_t)(kFiredLists * passcap_));
+        passes_.mutable_gpu_data();
+    } catch (...) {
+        release_passes();
+        throw;
+    }
+}
+
+void Instance::release_passes()
+{
+    passes_.resize(0);
+    pass_count_.resize(0);
+}
+
+CopyWords Instance::pass_count_words()
+{
+    return CopyWords{pass_count_.mutable_gpu_data(), nullptr, pass_count_.count()};
 }
 
 void Instance::release_gather()
@@ -1126,9 +1164,16 @@ void Instance::clear_spill(hipStream_t s)
     DTB_HIP(hipMemsetAsync(spill_.mutable_gpu_data(), 0, spill_.size(), s));
 }
 
-InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min)
+InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min, bool passes)
 {
     InstDev d{};
+    if (passes) {
+        if (!passes_built() || gather || direct)
+            throw Error(kInternal, "binning by a launch of its own needs the pass lists and queues");
+        d.passes = passes_.mutable_gpu_data();
+        d.pass_count = pass_count_.mutable_gpu_data();
+        d.passcap = passcap_;
+    }
     if (direct) {
         if (!direct_built() || gather)
             throw Error(kInternal, "direct propagation needs the tile offsets and no gather");

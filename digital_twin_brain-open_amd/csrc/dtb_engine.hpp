@@ -359,7 +359,8 @@ public:
     // `direct`: by direct propagation (ensure_direct first);
     // defer_min > 0 with the in-edges built: pull propagation (a tile with
     // at least defer_min emitted rows defers them to the pull).
-    InstDev dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min);
+    // `passes`: binning by k_bin (ensure_passes first).
+    InstDev dev(uint32_t tile_base, bool gather, bool direct, bool pull, uint32_t defer_min, bool passes);
     // Descriptor of tile t for the step kernels; inst: the device address of
     // the instance's descriptor `d`, idx its index; pop0: population of the
     // tile's first neuron; qoff, qcap: its queue.
@@ -429,6 +430,12 @@ public:
     // than the synapse arrays and a row has enough synapses for its lookups.
     bool direct_allowed() const { return direct_ok_; }
     void ensure_direct(hipStream_t s);
+    // Pass lists of k_bin (InstDev::passes), long enough for a step in which
+    // every neuron fires.
+    void ensure_passes();
+    void release_passes();
+    bool passes_built() const { return passes_.count() != 0; }
+    CopyWords pass_count_words();   // to clear the lists
     void release_direct() { tidx_.resize(0); }
     bool direct_built() const { return tidx_.count() != 0; }
 
@@ -504,6 +511,10 @@ private:
     bool direct_ok_ = false;              // direct_allowed()
     bool direct_fits() const;             // its conditions on the sizes
     DataAllocator<uint16_t> tidx_;        // [n][ntiles + 1] tile offsets (direct propagation)
+    std::vector<uint32_t> src_pass_;      // per tile: binning passes of all its rows
+    uint64_t passcap_ = 0;
+    DataAllocator<unsigned long long> passes_;   // [kFiredLists][passcap_]
+    DataAllocator<uint32_t> pass_count_;  // [2][kFiredLists][kFiredCountStride]
     DataAllocator<uint16_t> segidx_;      // [n][ngroups + 1] group offsets (built on demand)
     DataAllocator<uint32_t> grec_;        // [nsyn][grec_words] gather records (built with segidx_)
     DataAllocator<uint32_t> fired_;       // [2][kFiredLists][fired_capacity()] fired rows
@@ -578,8 +589,9 @@ public:
     // the spill accumulators.  Every setting gives the same results.
     void set_pull(bool on, uint32_t defer_min);
     // Split binning: the fired rows are binned by a second launch per step
-    // (k_bin) over groups of tiles, instead of by the tiles whose neurons
-    // fired.  Results never depend on it, and nothing on cap.
+    // (k_bin) in equal shares, instead of by the tiles whose neurons fired;
+    // off, large engines do so (kBinLaunchTiles).  Results never depend on it,
+    // and nothing on cap.
     void set_split(bool on, uint32_t cap)
     {
         if (on != split_ || cap != split_cap_) {
@@ -674,8 +686,9 @@ private:
     bool pull_on_ = true;                  // pull propagation where in-edges fit
     bool split_ = false;                   // split binning (k_bin)
     uint32_t split_cap_ = 0;               // as given to set_split
-    DataAllocator<BinDesc> d_bins_;        // source groups of the queue instances
-    uint32_t nbins_ = 0, bin_tiles_ = 0;   // groups (0: tiles bin their own rows), tiles of the largest queue instance
+    DataAllocator<BinDesc> d_bins_;        // k_bin's workgroups
+    uint32_t nbins_ = 0, bin_tiles_ = 0;   // their number (0: tiles bin their own rows), tiles of the largest queue instance
+    bool want_bin_launch(const std::vector<char> &direct);   // and builds the pass lists; false if they do not fit
     uint32_t defer_min_ = kDeferMinDefault;
     void try_pull(Instance &p, hipStream_t s);   // builds p's in-edges if on and they fit
     DataAllocator<InstDev> d_insts_;

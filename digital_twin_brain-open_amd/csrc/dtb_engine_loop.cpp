@@ -121,6 +121,36 @@ bool Engine::try_direct(Instance &p)
     }
 }
 
+bool Engine::want_bin_launch(const std::vector<char> &direct)
+{
+    uint64_t tiles = 0;
+    bool want = false;
+    auto queued = [&](size_t i) { return insts_[i] && !direct[i] && !use_gather(*insts_[i]); };
+    for (size_t i = 0; i < insts_.size(); ++i)
+        if (queued(i))
+            tiles += (insts_[i]->n() + kBlock - 1) / kBlock;
+    want = tiles > 0 && (split_ || tiles >= kBinLaunchTiles);
+    for (size_t i = 0; i < insts_.size() && want; ++i) {
+        if (!queued(i) || insts_[i]->passes_built())
+            continue;
+        if (devmem::NoAlloc::active())
+            return false;
+        try {
+            insts_[i]->ensure_passes();
+        } catch (const Error &e) {
+            // without device memory for the lists the tiles bin their own
+            // rows (same results)
+            if (e.code != kOutOfMemory)
+                throw;
+            want = false;
+        }
+    }
+    for (auto &p : insts_)
+        if (p && !want)
+            p->release_passes();
+    return want;
+}
+
 bool Engine::any_gather() const
 {
     for (auto &p : insts_)
@@ -343,6 +373,8 @@ void Engine::rebuild()
             if (insts_[slot] && direct[slot] == d)
                 order.push_back(slot);
     nqueue_tiles_ = 0;
+    const bool bin_launch = want_bin_launch(direct);
+    std::vector<CopyWords> put;   // the tables' copies, below
     for (size_t slot : order) {
         Instance *p = insts_[slot].get();
         const bool dir = direct[slot] != 0;
@@ -376,7 +408,10 @@ void Engine::rebuild()
         const bool pl = !gat && pull_on_ && p->pull_built();
         if (!dir && !wants_direct(*p) && !tuning_)
             p->release_direct();   // (the old tables, settled above, were the last to use it)
-        table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_));
+        const bool passes = bin_launch && !gat && !dir;
+        table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_, passes));
+        if (passes)
+            put.push_back(p->pass_count_words());
         const auto &pb = p->pop_begin();
         uint32_t q = 0;
         for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
@@ -396,10 +431,13 @@ void Engine::rebuild()
         if (!gat && !dir) {
             total += p->n();
             coverage += p->row_coverage() * p->n();
-            const uint32_t nt = split_ ? (p->n() + kBlock - 1) / kBlock : 0u;
-            bin_tiles_ = std::max(bin_tiles_, nt);
-            for (uint32_t t = 0; t < nt; t += kBinTiles)
-                bins.push_back(BinDesc{d_insts_.gpu_data() + idx, t, std::min(kBinTiles, nt - t)});
+            if (passes) {
+                const uint32_t nt = (p->n() + kBlock - 1) / kBlock;
+                bin_tiles_ = std::max(bin_tiles_, nt);
+                const uint32_t parts = std::min(kBinGroups, (nt + kBinTiles - 1) / kBinTiles);
+                for (uint32_t k = 0; k < parts; ++k)
+                    bins.push_back(BinDesc{d_insts_.gpu_data() + idx, k, parts});
+            }
         }
     }
     if (total > 0xffffffffull || tiles.size() > 0xffffffffull)
@@ -456,7 +494,6 @@ void Engine::rebuild()
     // All tables in one launch, from pinned memory: a copy call each and the
     // wait for the last were 60 of a short call's 240 us.
     const std::vector<QueueSet> qset(1, queues());
-    std::vector<CopyWords> put;
     size_t bytes = 0;
     auto each_table = [&](auto &&f) {
         f(d_insts_, table);

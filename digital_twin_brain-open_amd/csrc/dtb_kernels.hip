@@ -1298,6 +1298,13 @@ struct TileRows {
     uint32_t n;
 };
 
+// The pass list of tile t of nt: contiguous ranges of tiles, so a list's rows
+// share target tiles.
+__device__ __forceinline__ uint32_t pass_list(uint32_t t, uint32_t nt)
+{
+    return (uint32_t)(((uint64_t)t * kFiredLists) / nt);
+}
+
 // One tile's step (the body of k_step).  kUniform: every neuron of the tile
 // has the same parameter class, so the parameter record is read once per
 // tile through the scalar unit instead of per lane.  kStat: some instance
@@ -1407,19 +1414,18 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
     const unsigned long long m = __ballot(emit);
     if (lane == 0)
         s_bits[w] = m;
+    RowSpan span{0, 0u};
     if (m != 0ull) {
-        if (kMode != kQueues || gat) {
-            const RowSpan r = count_fired(d, I, emit, m, tid, lane, w);
-            if (kMode == kTileBin && !gat) {
-                uint32_t base = 0;
-                if (lane == 0)
-                    base = atomicAdd(&rows->n, (uint32_t)__popcll(m));
-                base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-                if (emit) {
-                    const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                    rows->rb[k] = r.first;
-                    rows->len[k] = r.len;
-                }
+        span = count_fired(d, I, emit, m, tid, lane, w);
+        if (kMode == kTileBin && !gat) {
+            uint32_t base = 0;
+            if (lane == 0)
+                base = atomicAdd(&rows->n, (uint32_t)__popcll(m));
+            base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+            if (emit) {
+                const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                rows->rb[k] = span.first;
+                rows->len[k] = span.len;
             }
         }
         if (gat)
@@ -1472,8 +1478,26 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
         }
     }
     // the tile's emitted and deferred rows, one 64-byte store
-    if (tid < kBitWords && (kMode == kQueues || (d->flags & kTilePull)))
+    if (tid < kBitWords && (d->flags & kTilePull))
         gp(d->bits)[(size_t)(par ^ 1u) * d->ntiles * kBitWords + tid] = (tid < 4u || defer) ? b : 0ull;
+    if (kMode == kQueues && m != 0ull && !defer) {
+        // The wave's passes onto its list: one atomic on a count shared with
+        // 1/64 of the tiles.
+        const uint32_t np = (span.len + kBinPass - 1u) / kBinPass;
+        const uint32_t incl = wave_add_scan(np);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        if (total != 0u) {
+            const uint32_t list = pass_list(d->begin >> kTileBits, d->ntiles);
+            uint32_t at = 0;
+            if (lane == 0)
+                at = gadd(I->pass_count + ((par * kFiredLists + list) * kFiredCountStride), total);
+            at = (uint32_t)__builtin_amdgcn_readlane((int)at, 0) + incl - np;
+            const auto out = gp(I->passes) + ((size_t)list * I->passcap + at);
+            for (uint32_t k = 0; k < np; ++k)
+                out[k] = ((unsigned long long)(span.first + (int64_t)(k * kBinPass)) << 8) |
+                         (min(span.len - k * kBinPass, kBinPass) - 1u);
+        }
+    }
     if constexpr (kMode == kTileBin) {
         // The passes of the tile's rows, dealt round-robin to its four waves,
         // so one long row does not keep a single wave busy while the others
@@ -1539,69 +1563,45 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(K == 4 ?
         step_tile<false, kFmt, kStat, kMode, K>(tp, cp(queues), par, acc, s_bits, rec, ls, rows);
 }
 
-// Binning of the rows emitted by the k_step launch of parity `par` into
-// queue set par ^ 1.  A workgroup takes a group of up to kBinTiles
-// consecutive source tiles: rows of neighbouring neurons reach the same
-// target tiles (a voxel's rows share theirs), so it counts its synapses per
-// target tile in LDS, reserves each tile's share with one device atomic
-// (consecutive lanes on consecutive counts, which one request serves), and
-// writes every synapse's entry to its tile's queue at reserved start + rank.
+// Binning of the passes listed by the k_step launch of parity `par` into
+// queue set par ^ 1.  A workgroup takes an equal share of them, consecutive
+// ones: rows of neighbouring neurons reach the same target tiles (a voxel's
+// rows share theirs), so it counts its synapses per target tile in LDS,
+// reserves each tile's share with one device atomic, and writes every
+// synapse's entry to its tile's queue at reserved start + rank.
 // Without it (one reservation per row and target tile, in the tiles whose
-// neurons fired) binning is 24 of 51 us of the 2M-neuron block's step:
+// neurons fired) binning is 22 of 50 us of the 2M-neuron block's step:
 // returning atomics on single counts are served at about 2.7e10 per second,
-// and a row of 500 synapses makes 160-190 of them.  A step with / without: 2M
-// neurons x 500 47.5 / 50.9 us, 900k x 300 30.2 / 28.2, 400k x 250 19.6 /
-// 15.9 (the launch, and a group's serial phases, cost what the atomics save).
-// Rows are cut into passes of kBinPass synapses, one per wave and round;
-// deferred rows are counted (events) but not binned.  The counts of a round
-// live in min(ntiles, kBinMaxTiles) LDS words; instances with more tiles are
-// binned in windows of that many target tiles.
+// and a row of 500 synapses makes 160-190 of them; with it 14.5 of 43.5.
+// Groups of 32 source tiles instead of equal shares of the passes took 19 us:
+// the fullest group's time.
+// The counts of a round live in min(ntiles, kBinMaxTiles) LDS words;
+// instances with more tiles are binned in windows of that many target tiles.
+// Also empties the lists of set par ^ 1 (the next k_step's; their last reader
+// was the previous k_bin).
 template <uint32_t kFmt>
 __global__ __launch_bounds__(kBinBlock) void k_bin(const BinDesc *__restrict__ groups, const QueueSet *queues,
                                                    uint32_t par)
 {
     constexpr uint32_t kWaves = kBinBlock / kWave;
     extern __shared__ uint32_t hist[];               // min(ntiles, kBinMaxTiles)
-    __shared__ uint16_t s_list[kBinTiles * kBlock];  // emitted rows of the group (bit 15: deferred)
-    __shared__ uint32_t s_pass[kBinBlock];           // per row of a chunk: passes before it
-    __shared__ uint32_t s_len[kBinBlock];
-    __shared__ int64_t s_rb[kBinBlock];
-    __shared__ uint32_t s_wave[kWaves];
+    __shared__ uint32_t s_list[kFiredLists];         // passes of the lists before
     __shared__ uint16_t s_touch[kWaves * kBinDeep * kBinPass];   // target tiles of a round, each once
-    __shared__ uint32_t s_rows, s_ntouch;
+    __shared__ uint32_t s_ntouch;
     const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / kWave;
     const auto bd = cp(groups + blockIdx.x);
     const InstPtr I = cp(bd->inst);
-    const uint32_t tile0 = bd->tile0, T = I->ntiles, set = par ^ 1u;
-    if (w < kBinTiles / 16u) {
-        // one word of 64 rows per lane
-        const auto b = gp(I->bits) + ((size_t)set * T + tile0) * kBitWords;
-        const uint32_t t = tid >> 2, q = tid & 3u;
-        unsigned long long e = 0ull, df = 0ull;
-        if (t < bd->ntile) {
-            e = b[t * kBitWords + q];
-            df = b[t * kBitWords + 4u + q];
-        }
-        // the list starts where the wave before left off (its words are read
-        // again: one line each)
-        uint32_t at = 0;
-        for (uint32_t v = 0; v < w; ++v) {
-            const uint32_t tt = v * 16u + (lane >> 2);
-            const unsigned long long x = tt < bd->ntile ? b[tt * kBitWords + (lane & 3u)] : 0ull;
-            at += (uint32_t)__builtin_amdgcn_readlane((int)wave_add_scan((uint32_t)__popcll(x)), kWave - 1);
-        }
-        const uint32_t c = (uint32_t)__popcll(e), incl = wave_add_scan(c);
-        at += incl - c;
-        if (w == kBinTiles / 16u - 1u && lane == kWave - 1)
-            s_rows = at + c;
-        for (; e != 0ull; e &= e - 1ull, ++at) {
-            const uint32_t k = (uint32_t)__ffsll((long long)e) - 1u;
-            s_list[at] = (uint16_t)((tid << 6) | k | (((df >> k) & 1ull) ? 0x8000u : 0u));
-        }
-    }
-    __syncthreads();
-    const uint32_t rows = s_rows;
-    if (rows == 0u)
+    const uint32_t T = I->ntiles, set = par ^ 1u;
+    const uint32_t cnt = gp(I->pass_count)[(par * kFiredLists + lane) * kFiredCountStride];
+    const uint32_t incl = wave_add_scan(cnt);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    if (w == 0)
+        s_list[lane] = incl - cnt;
+    if (bd->part == 0u && tid < kFiredLists)
+        gp(I->pass_count)[(set * kFiredLists + tid) * kFiredCountStride] = 0u;
+    const uint32_t lo = (uint32_t)((uint64_t)total * bd->part / bd->parts);
+    const uint32_t hi = (uint32_t)((uint64_t)total * (bd->part + 1u) / bd->parts);
+    if (lo == hi)
         return;
     for (uint32_t t = tid; t < min(T, (uint32_t)kBinMaxTiles); t += kBinBlock)
         hist[t] = 0u;
@@ -1616,141 +1616,105 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(const BinDesc *__restrict__ g
     const QueueTile *qtab = qs->tile + tb;
     QSyn *q_out = I->queue + (size_t)set * I->qslots;
     const bool pull_on = I->crec != nullptr;
-    unsigned long long events = 0;
-    for (uint32_t r0 = 0; r0 < rows; r0 += kBinBlock) {
-        const uint32_t nr = min(rows - r0, (uint32_t)kBinBlock);
-        uint32_t np = 0, len = 0;
-        int64_t rb = 0;
-        if (tid < nr) {
-            const uint32_t e = s_list[r0 + tid];
-            const uint32_t r = tile0 * kBlock + (e & 0x7fffu);
-            rb = gp(I->rowptr)[r];
-            len = (uint32_t)(gp(I->rowptr)[r + 1] - rb);
-            np = (e & 0x8000u) ? 0u : (len + kBinPass - 1u) / kBinPass;
-        }
-        events += len;
-        const uint32_t incl = wave_add_scan(np);
-        if (lane == kWave - 1)
-            s_wave[w] = incl;
-        __syncthreads();
-        uint32_t before = 0, total = 0;
+    for (uint32_t t0 = 0; t0 < T; t0 += kBinMaxTiles) {
+        const uint32_t tw = min(T - t0, (uint32_t)kBinMaxTiles);
+        for (uint32_t p0 = lo; p0 < hi; p0 += kWaves * kBinDeep) {
+            __syncthreads();   // s_list is written, hist is zero
+            constexpr uint32_t N = kBinDeep * kBinItems;
+            uint32_t cv[N], rank[N];
+            unsigned long long wv[N];
+            bool ok[N];
+            unsigned long long pe[kBinDeep];
 #pragma unroll
-        for (uint32_t k = 0; k < kWaves; ++k) {
-            const uint32_t v = s_wave[k];
-            before += k < w ? v : 0u;
-            total += v;
-        }
-        s_pass[tid] = tid < nr ? before + incl - np : 0xffffffffu;
-        s_len[tid] = len;
-        s_rb[tid] = rb;
-        for (uint32_t t0 = 0; t0 < T; t0 += kBinMaxTiles) {
-            const uint32_t tw = min(T - t0, (uint32_t)kBinMaxTiles);
-            for (uint32_t p0 = 0; p0 < total; p0 += kWaves * kBinDeep) {
-                __syncthreads();   // s_pass, s_len, s_rb are written, hist is zero
-                constexpr uint32_t N = kBinDeep * kBinItems;
-                uint32_t cv[N], rank[N];
-                unsigned long long wv[N];
-                bool ok[N];
+            for (uint32_t q = 0; q < kBinDeep; ++q) {
+                const uint32_t p = p0 + q * kWaves + w;
+                if (p < hi) {
+                    // the list holding pass p: the last one with at most p passes before it
+                    uint32_t l = 0;
 #pragma unroll
-                for (uint32_t q = 0; q < kBinDeep; ++q) {
-                    const uint32_t p = p0 + q * kWaves + w;
-                    uint32_t j0 = 0, n = 0;
-                    int64_t first = 0;
-                    if (p < total) {
-                        // the row of pass p: the last one with at most p passes before it
-                        uint32_t row = 0;
-#pragma unroll
-                        for (uint32_t st = kBinBlock / 2; st > 0; st >>= 1)
-                            if (s_pass[row + st] <= p)
-                                row += st;
-                        j0 = (p - s_pass[row]) * kBinPass;
-                        n = s_len[row];
-                        first = s_rb[row];
-                    }
-#pragma unroll
-                    for (uint32_t v = 0; v < kBinItems; ++v) {
-                        const uint32_t u = q * kBinItems + v;
-                        const uint32_t j = j0 + v * kWave + lane;
-                        ok[u] = j < n;
-                        if (ok[u]) {
-                            cv[u] = gp(I->col)[first + j];
-                            wv[u] = w_raw(I->w, (size_t)(first + j), wfmt);
-                        }
-                    }
+                    for (uint32_t st = kFiredLists / 2; st > 0; st >>= 1)
+                        if (s_list[l + st] <= p)
+                            l += st;
+                    pe[q] = gp(I->passes)[(size_t)l * I->passcap + (p - s_list[l])];
                 }
-#pragma unroll
-                for (uint32_t u = 0; u < N; ++u)
-                    if (ok[u]) {
-                        const uint32_t t = ((cv[u] & kColMask) >> kTileBits) - t0;
-                        ok[u] = t < tw;
-                        if (ok[u]) {
-                            rank[u] = atomicAdd(&hist[t], 1u);
-                            if (rank[u] == 0u)
-                                s_touch[atomicAdd(&s_ntouch, 1u)] = (uint16_t)t;
-                        }
-                    }
-                __syncthreads();
-                const uint32_t nt = s_ntouch;
-                uint32_t over = 0;   // synapses of this thread's tiles past their queue's capacity
-                for (uint32_t k = tid; k < nt; k += kBinBlock) {
-                    const uint32_t t = s_touch[k];
-                    const uint32_t c = hist[t];
-                    const uint32_t b = gadd(&count[count_slot(cset + t0 + t, cshift)], c);
-                    const uint32_t cap = gp(qtab)[t0 + t].cap;
-                    const uint64_t off = gp(qtab)[t0 + t].off;
-                    const uint32_t room = cap > b ? min(c, cap - b) : 0u;
-                    over += c - room;
-                    // the segment's first slot; bit 31: it does not fit whole
-                    // (or the slot takes more than 31 bits), then its start
-                    // within the tile's queue
-                    hist[t] = room == c && off + b + c < 0x80000000ull ? (uint32_t)(off + b)
-                                                                      : 0x80000000u | min(b, 0x7fffffffu);
-                }
-                if (over != 0u)
-                    gadd(&qs->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].spilled, (unsigned long long)over);
-                __syncthreads();
-#pragma unroll
-                for (uint32_t u = 0; u < N; ++u) {
-                    if (!ok[u])
-                        continue;
-                    const uint32_t tile = (cv[u] & kColMask) >> kTileBits;
-                    const uint32_t h = hist[tile - t0];
-                    const uint32_t key = (cv[u] & 0xffu) | ((cv[u] & kKindBit) ? kQSynKind : 0u);
-                    const float2 wp = w_decode(wv[u], wfmt);
-                    if (!(h & 0x80000000u)) {
-                        st_entry(q_out, h + rank[u], key, wp.x, wp.y);
-                    } else {
-                        const uint64_t at = (uint64_t)(h & 0x7fffffffu) + rank[u];
-                        if (at < gp(qtab)[tile].cap) {
-                            st_entry(q_out, gp(qtab)[tile].off + at, key, wp.x, wp.y);
-                        } else if (!pull_on) {
-                            // past the capacity: the target's spill accumulator
-                            // (Q23.40 integers like the LDS sums); with the pull
-                            // the tile takes every row through its in-edges
-                            unsigned long long *a = I->spill + ((size_t)set * I->n + (cv[u] & kColMask)) * 4u +
-                                                    ((cv[u] & kKindBit) ? 2u : 0u);
-                            gadd(a, f32_to_q40(wp.x));
-                            gadd(a + 1, f32_to_q40(wp.y));
-                        }
-                    }
-                }
-                __syncthreads();
-                for (uint32_t k = tid; k < nt; k += kBinBlock)
-                    hist[s_touch[k]] = 0u;
-                if (tid == 0)
-                    s_ntouch = 0u;
             }
+#pragma unroll
+            for (uint32_t q = 0; q < kBinDeep; ++q) {
+                const bool any = p0 + q * kWaves + w < hi;
+                const uint64_t first = any ? pe[q] >> 8 : 0ull;
+                const uint32_t n = any ? (uint32_t)(pe[q] & 0xffull) + 1u : 0u;
+#pragma unroll
+                for (uint32_t v = 0; v < kBinItems; ++v) {
+                    const uint32_t u = q * kBinItems + v, j = v * kWave + lane;
+                    ok[u] = j < n;
+                    if (ok[u]) {
+                        cv[u] = gp(I->col)[first + j];
+                        wv[u] = w_raw(I->w, (size_t)(first + j), wfmt);
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < N; ++u)
+                if (ok[u]) {
+                    const uint32_t t = ((cv[u] & kColMask) >> kTileBits) - t0;
+                    ok[u] = t < tw;
+                    if (ok[u]) {
+                        rank[u] = atomicAdd(&hist[t], 1u);
+                        if (rank[u] == 0u)
+                            s_touch[atomicAdd(&s_ntouch, 1u)] = (uint16_t)t;
+                    }
+                }
+            __syncthreads();
+            const uint32_t nt = s_ntouch;
+            uint32_t over = 0;   // synapses of this thread's tiles past their queue's capacity
+            for (uint32_t k = tid; k < nt; k += kBinBlock) {
+                const uint32_t t = s_touch[k];
+                const uint32_t c = hist[t];
+                const uint32_t b = gadd(&count[count_slot(cset + t0 + t, cshift)], c);
+                const uint32_t cap = gp(qtab)[t0 + t].cap;
+                const uint64_t off = gp(qtab)[t0 + t].off;
+                const uint32_t room = cap > b ? min(c, cap - b) : 0u;
+                over += c - room;
+                // the segment's first slot; bit 31: it does not fit whole
+                // (or the slot takes more than 31 bits), then its start
+                // within the tile's queue
+                hist[t] = room == c && off + b + c < 0x80000000ull ? (uint32_t)(off + b)
+                                                                  : 0x80000000u | min(b, 0x7fffffffu);
+            }
+            if (over != 0u)
+                gadd(&qs->ctl->slot[blockIdx.x & (kCtlSlots - 1u)].spilled, (unsigned long long)over);
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < N; ++u) {
+                if (!ok[u])
+                    continue;
+                const uint32_t tile = (cv[u] & kColMask) >> kTileBits;
+                const uint32_t h = hist[tile - t0];
+                const uint32_t key = (cv[u] & 0xffu) | ((cv[u] & kKindBit) ? kQSynKind : 0u);
+                const float2 wp = w_decode(wv[u], wfmt);
+                if (!(h & 0x80000000u)) {
+                    st_entry(q_out, h + rank[u], key, wp.x, wp.y);
+                } else {
+                    const uint64_t at = (uint64_t)(h & 0x7fffffffu) + rank[u];
+                    if (at < gp(qtab)[tile].cap) {
+                        st_entry(q_out, gp(qtab)[tile].off + at, key, wp.x, wp.y);
+                    } else if (!pull_on) {
+                        // past the capacity: the target's spill accumulator
+                        // (Q23.40 integers like the LDS sums); with the pull
+                        // the tile takes every row through its in-edges
+                        unsigned long long *a = I->spill + ((size_t)set * I->n + (cv[u] & kColMask)) * 4u +
+                                                ((cv[u] & kKindBit) ? 2u : 0u);
+                        gadd(a, f32_to_q40(wp.x));
+                        gadd(a + 1, f32_to_q40(wp.y));
+                    }
+                }
+            }
+            __syncthreads();
+            for (uint32_t k = tid; k < nt; k += kBinBlock)
+                hist[s_touch[k]] = 0u;
+            if (tid == 0)
+                s_ntouch = 0u;
         }
-        __syncthreads();
-    }
-    // events delivered and spikes, on the counters of the group's first wave
-    const unsigned long long ev = wave_sum_u64(events);
-    if (lane == 0) {
-        unsigned long long *c = I->wave_ctr + 2u * (size_t)(tile0 * (kBlock / kWave));
-        if (ev != 0ull)
-            gadd(c, ev);
-        if (w == 0)
-            gadd(c + 1, (unsigned long long)rows);
     }
 }
 

@@ -131,6 +131,13 @@ struct alignas(16) InstDev {
     // straight from the rows of the step before: it reads the emitted bits of
     // every tile and, per emitted row, the row's segment for itself.
     const uint16_t *tidx;       // [n][ntiles + 1]
+    // Binning by k_bin (null passes: the tiles bin their rows): the passes of
+    // a step's rows, (first synapse << 8) | (synapses - 1), in kFiredLists
+    // lists of passcap entries, tile t's on list t * kFiredLists / ntiles;
+    // their counts at pass_count[(set * kFiredLists + list) * kFiredCountStride].
+    unsigned long long *passes;
+    uint32_t *pass_count;
+    uint64_t passcap;
     // Pull propagation (null crec: off; never together with gather).  The
     // in-edges of target tile t are records [cptr[t], cptr[t + 1]) of crec,
     // grec_words(wfmt) words each: key = source row (bits 0..22) | target's
@@ -343,19 +350,28 @@ __host__ __device__ inline size_t count_words(size_t n, uint32_t shift)
     return ((n + (1u << shift) - 1u) >> shift) * kCountLineWords;
 }
 
-// Split binning (k_bin): a workgroup of kBinBlock threads bins the rows of up to
-// kBinTiles consecutive source tiles (64 bit words: one per lane of a wave),
-// each wave a pass of kBinPass synapses per round, kBinItems per lane.
+// Binning by a launch of its own (k_bin): passes of kBinPass synapses, taken
+// by workgroups of kBinBlock threads, each wave kBinDeep passes per round and
+// each lane kBinItems synapses of a pass.
 constexpr int kBinBlock = 1024;
-constexpr uint32_t kBinTiles = 32;
-constexpr uint32_t kBinItems = 4, kBinDeep = 4;
+constexpr uint32_t kBinItems = 4, kBinDeep = 1;
 constexpr uint32_t kBinPass = kWave * kBinItems;
+static_assert(kBinPass == 256, "a pass entry holds its length less one in 8 bits");
 constexpr uint32_t kBinMaxTiles = 16384;   // LDS counts of target tiles (64 KB)
-static_assert(kBinTiles * kBlock <= 0x8000, "rows of a group fit 15 bits");
+// Workgroups: one per kBinTiles source tiles, at most kBinGroups (two per CU)
+// per instance.
+constexpr uint32_t kBinTiles = 16, kBinGroups = 512;
+// Queue tiles from which an engine bins by k_bin instead of in the tiles that
+// fired: its launch and its chain of waits are 8 us of a step, its atomics a
+// third as many.  Steps in the tiles / by k_bin, voxel networks at 10, 16 and
+// 33 spikes per second: 400k neurons (1563 tiles) 13.5 / 15.3, 15.7 / 16.0 and
+// 22.9 / 20.7 us; 600k (2344) 16.3 / 18.0, 19.5 / 19.6 and 28.8 / 25.9; 900k
+// (3516) 22.9 / 23.1, 27.5 / 25.9 and 38.1 / 33.8; 2M (7813) at 6, 11 and 21
+// 40.6 / 38.4, 49.5 / 43.5 and 69.1 / 59.8.
+constexpr uint32_t kBinLaunchTiles = 3072u;
 struct alignas(16) BinDesc {
     const InstDev *inst;
-    uint32_t tile0;    // first source tile of the instance
-    uint32_t ntile;    // tiles (<= kBinTiles)
+    uint32_t part, parts;   // takes part `part` of `parts` of the step's passes
 };
 
 struct StepCtl;

@@ -375,9 +375,10 @@ class Engine:
 
     def split(self, on=None, capacity=0):
         """Sets (when given) and returns split binning: the fired rows are
-        binned by a second launch per step, in groups of 32 tiles over the
-        whole GPU, instead of by the tiles whose neurons fired (capacity has
-        no effect).  Same results either way."""
+        binned by a second launch per step, in equal shares over the whole
+        GPU, instead of by the tiles whose neurons fired (off: only in engines
+        whose queues serve 786,432 neurons or more; capacity has no effect).
+        Same results either way."""
         if on is not None:
             _lib.check(self._lib.dtb_engine_split(self._h, c_int32(int(bool(on))), ctypes.c_uint32(int(capacity))))
         o, c = c_int32(0), ctypes.c_uint32(0)

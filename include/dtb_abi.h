@@ -262,9 +262,10 @@ int dtb_engine_queue_capacity(dtb_engine_t h, uint32_t floor, uint32_t shift);
 int dtb_engine_pull(dtb_engine_t h, int32_t on, uint32_t defer_min);
 /* Split binning (the binning stage of src/stage/presynaptic_voltage.cpp:
  * 122-225, scheduled differently): on = the fired rows are binned by a second
- * launch per step, in groups of 32 tiles over the whole GPU, instead of by the
- * tiles whose neurons fired.  capacity is kept and reported, and has no effect
- * (there is no list to bound).  Results never depend on either. */
+ * launch per step, in equal shares over the whole GPU, instead of by the tiles
+ * whose neurons fired; off = only where the engine's queues serve 786,432
+ * neurons or more.  capacity is kept and reported, and has no effect (the
+ * list holds every row).  Results never depend on either. */
 int dtb_engine_split(dtb_engine_t h, int32_t on, uint32_t capacity);
 int dtb_engine_get_split(dtb_engine_t h, int32_t *on, uint32_t *capacity);
 int dtb_engine_get_pull(dtb_engine_t h, int32_t *on, uint32_t *defer_min);
