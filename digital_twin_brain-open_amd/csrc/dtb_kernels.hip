@@ -507,6 +507,23 @@ __device__ __forceinline__ void direct_rows(unsigned long long *acc, const Inst 
     }
 }
 
+// The emitted rows of a thread's source tiles, all rounds in flight together:
+// per tile, after its 4 words of bits, a word of the count and the first ids.
+struct DirectIds {
+    unsigned long long b[kDirectRounds];
+
+    // bits: the instance's words of the set
+    __device__ __forceinline__ DirectIds(const unsigned long long *bits, uint32_t T, uint32_t tid)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < kDirectRounds; ++i)
+            if (i * kBlock < T) {
+                const uint32_t src = i * kBlock + tid;
+                b[i] = src < T ? gp(bits)[(size_t)src * kBitWords + 4u] : 0ull;
+            }
+    }
+};
+
 // Direct propagation: adds into acc (zeroed, as ls.n is; both visible) the
 // synapses onto tile t of every row emitted into set `set`.  Each thread
 // reads the emitted rows of up to kDirectRounds source tiles (the count and
@@ -515,22 +532,13 @@ __device__ __forceinline__ void direct_rows(unsigned long long *acc, const Inst 
 // (volleys), the tile pulls.  Called by the whole workgroup; ends without a
 // barrier.  Returns whether the tile pulled.
 template <uint32_t kFmt, typename Inst>
-__device__ __forceinline__ bool direct_tile(unsigned long long *acc, DirectList &ls, const Inst &I, uint32_t set,
-                                            uint32_t t, uint32_t tid)
+__device__ __forceinline__ bool direct_tile(unsigned long long *acc, DirectList &ls, const Inst &I,
+                                            const DirectIds &ids, uint32_t set, uint32_t t, uint32_t tid)
 {
     const uint32_t T = I.ntiles;
     typedef unsigned long long u64x4 __attribute__((ext_vector_type(4)));
-    // per tile: 4 words of bits, then a word of the count and the first ids
-    const auto ids = gp(I.bits + (size_t)set * T * kBitWords + 4u);
     const auto bits = (const __attribute__((address_space(1))) u64x4 *)gp(I.bits + (size_t)set * T * kBitWords);
-    // every round's rows in flight before the first is used
-    unsigned long long b4[kDirectRounds];
-#pragma unroll
-    for (uint32_t i = 0; i < kDirectRounds; ++i)
-        if (i * kBlock < T) {
-            const uint32_t src = i * kBlock + tid;
-            b4[i] = src < T ? ids[(size_t)src * kBitWords] : 0ull;
-        }
+    const unsigned long long(&b4)[kDirectRounds] = ids.b;
     // places in the list: one LDS add per wave
     uint32_t mine = 0;
 #pragma unroll
@@ -1031,16 +1039,27 @@ __device__ __forceinline__ float ou_step(float iou, float mu, float f1, float f2
     return iou + (f1 * (mu - iou) + f2s * xi);
 }
 
+// The step's normal draw of a tile with one population, one substep and the
+// OU current on.  Taken while the tile's loads are in flight: its 100
+// instructions wait for nothing but the step index (with the emitted rows'
+// words read as early: 200k x 250 9.8 -> 9.6 us a step, 10k 5.25 -> 5.10,
+// eight instances 12.7 -> 11.9).
+__device__ __forceinline__ float ou_draw(TilePtr d, uint32_t tid, int64_t step)
+{
+    constexpr uint32_t kOne = kTileOnePop | kTileOneSub | kTileOuOn;
+    return (d->flags & kOne) == kOne ? ou_normal(d->seed, d->begin + tid, (uint64_t)step) : 0.0f;
+}
+
 // Every substep of a tile whose neurons share one population, with one
 // substep per step (the usual case: straight-line code, the OU factors in
 // scalar registers).  Returns whether the lane's neuron emitted.
 __device__ __forceinline__ bool step_lane_one(TilePtr d, Lane &x, const ParamRec &q, float isyn, uint32_t li,
-                                              int64_t step)
+                                              int64_t step, float xi)
 {
     uint32_t f = x.fl & kFlagSpike;
     float Ieff = isyn;
     if (d->flags & kTileOuOn) {
-        x.iou = ou_step(x.iou, d->mu, d->f1, d->f2s, ou_normal(d->seed, li, (uint64_t)step));
+        x.iou = ou_step(x.iou, d->mu, d->f1, d->f2s, xi);
         Ieff = isyn + x.iou;
     }
     bool emit = lif(x, f, q, Ieff);
@@ -1084,10 +1103,12 @@ __device__ __forceinline__ bool step_lane_any(TilePtr d, InstPtr I, Lane &x, con
 
 // Fold of the delta, the recorded statistics, and every substep of OU + LIF
 // (or of the noise mode) of the tile's neurons; returns whether the lane's
-// neuron emitted a spike and writes the state back.
+// neuron emitted a spike and writes the state back.  xi: the step's normal
+// draw, where the tile has one (ou_draw).
 template <bool kStat>
 __device__ __forceinline__ bool step_lane(TilePtr d, Lane &x, const ParamRec &q, const float4 dl, bool active,
-                                          uint32_t tid, uint32_t lane, int64_t step, uint32_t &p, TileRec &rec)
+                                          uint32_t tid, uint32_t lane, int64_t step, float xi, uint32_t &p,
+                                          TileRec &rec)
 {
     const bool one_pop = (d->flags & kTileOnePop) != 0u;
     const uint32_t li = d->begin + tid;
@@ -1134,7 +1155,7 @@ __device__ __forceinline__ bool step_lane(TilePtr d, Lane &x, const ParamRec &q,
     bool emit = false;
     if (active) {
         if ((d->flags & (kTileOnePop | kTileOneSub)) == (kTileOnePop | kTileOneSub))
-            emit = step_lane_one(d, x, q, isyn, li, step);
+            emit = step_lane_one(d, x, q, isyn, li, step, xi);
         else
             emit = step_lane_any(d, I, x, q, isyn, li, step, p);
         *st_at<kStV, float>(d->state, tid) = x.V;
@@ -1348,7 +1369,11 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
         bool over = !gat && e.cnt > e.d->qcap;
         uint32_t cnt = gat ? 0u : min(e.cnt, e.d->qcap);
         pull = !gat && (e.d->flags & kTilePull) && (over || e.stamp == e.step + 1);
+        const uint32_t begin_word = kMode == kDirect ? (e.d->begin >> kTileBits) * kBitWords : 0u;
+        DirectIds ids(kMode == kDirect ? e.d->bits - begin_word + (size_t)par * e.d->ntiles * kBitWords : nullptr,
+                      kMode == kDirect ? e.d->ntiles : 0u, tid);
         clear_row(acc, tid);
+        const float xi = ou_draw(e.d, tid, e.step);
         if (tid == 0) {
             rec.count = 0u;
             if (kMode == kDirect)
@@ -1375,7 +1400,7 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
             cnt = 0u;
         }
         if (kMode == kDirect) {
-            if (direct_tile<kFmt>(acc, *ls, *cp(e.d->inst), par, e.d->begin >> kTileBits, tid) && tid == 0) {
+            if (direct_tile<kFmt>(acc, *ls, *cp(e.d->inst), ids, par, e.d->begin >> kTileBits, tid) && tid == 0) {
                 // the tile pulled; and its own rows, if any, went by the pull
                 CtlSlot &c = qp->ctl->slot[blockIdx.x & (kCtlSlots - 1u)];
                 gadd(&c.pulled, 1ull);
@@ -1402,7 +1427,7 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
                 gp(e.d->step)[par ^ 1u] = step + 1;   // no tile of this launch reads this slot
         }
         const float4 dl = kMode != kDirect && (e.d->flags & kTileGather) ? ahead : acc_to_delta(acc, tid);
-        emit = step_lane<kStat>(e.d, e.x, e.prm, dl, e.active, tid, lane, step, p, rec);
+        emit = step_lane<kStat>(e.d, e.x, e.prm, dl, e.active, tid, lane, step, xi, p, rec);
     }
 
     const TilePtr d = again(tp);
@@ -1992,7 +2017,8 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const TileDesc *__restri
         if (tid == 0)
             ls.n = 0u;
         __syncthreads();
-        direct_tile<kWeightAny>(acc, ls, I, set, d.begin >> kTileBits, tid);
+        const DirectIds ids(I.bits + (size_t)set * I.ntiles * kBitWords, I.ntiles, tid);
+        direct_tile<kWeightAny>(acc, ls, I, ids, set, d.begin >> kTileBits, tid);
         __syncthreads();
         if (tid < d.count)
             st4(I.dlt, d.begin + tid, acc_to_delta(acc, tid));
@@ -2052,7 +2078,8 @@ __global__ __launch_bounds__(kBlock) void k_settle(const TileDesc *__restrict__ 
         if (tid == 0)
             ls.n = 0u;
         __syncthreads();
-        direct_tile<kWeightAny>(acc, ls, I, set, d.begin >> kTileBits, tid);
+        const DirectIds ids(I.bits + (size_t)set * I.ntiles * kBitWords, I.ntiles, tid);
+        direct_tile<kWeightAny>(acc, ls, I, ids, set, d.begin >> kTileBits, tid);
     }
     const uint32_t cnt_raw = direct ? 0u : *cnt_p;
     const bool over = cnt_raw > d.qcap;
