@@ -200,9 +200,10 @@ constexpr uint32_t kDirectIds = 6;
 // size was slower), the emitted rows a tile lists in LDS at a time (with 1024
 // a 200k-neuron step of 1143 rows took 25.5 us, in two rounds, with 2048 18.2;
 // with 4096 five workgroups fit a CU and eight instances in one engine took
-// 14.7 us instead of 12.7), and the synapses a thread has in flight.
+// 14.7 us instead of 12.7), and the synapses a lane has in flight (4: 66k
+// neurons x 250 6.63 us, 2: 6.53).
 constexpr uint32_t kDirectMaxNeurons = 1u << 18;
-constexpr uint32_t kDirectRows = 2048, kDirectItems = 4;
+constexpr uint32_t kDirectRows = 2048, kDirectItems = 2;
 constexpr uint32_t kDirectRounds = (kDirectMaxNeurons / kBlock + kBlock - 1) / kBlock;   // tiles per thread
 
 // Weight pair formats kept on the device (include/weights.hpp:14-21 and the
