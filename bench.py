@@ -412,7 +412,9 @@ def main():
     else:
         layout_bytes = (LAYOUT_NEURON_BYTES * net.n + LAYOUT_ROW_BYTES * sp_step
                         + (LAYOUT_SYN_BYTES - 8 + wpair) * ev_step)
-    kname = "k_gather+k_step" if gather else ("k_step+k_bin" if args.split else "k_step")
+    # engines of 3072 queue tiles or more bin in a launch of their own
+    bin_launch = args.split or (net.n + 255) // 256 >= 3072
+    kname = "k_gather+k_step" if gather else ("k_step+k_bin" if bin_launch else "k_step")
     achieved = algo_bytes / (us * 1e-6) / 1e9
     traffic, traffic_src = (profiled_traffic(args.workload, args.neurons, layout_used, args.steps, args.warmup,
                                              bool(k_best)) if args.weights == "float32" else (None, None))

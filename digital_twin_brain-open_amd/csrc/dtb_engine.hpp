@@ -688,7 +688,7 @@ private:
     uint32_t split_cap_ = 0;               // as given to set_split
     DataAllocator<BinDesc> d_bins_;        // k_bin's workgroups
     uint32_t nbins_ = 0, bin_tiles_ = 0;   // their number (0: tiles bin their own rows), tiles of the largest queue instance
-    bool want_bin_launch(const std::vector<char> &direct);   // and builds the pass lists; false if they do not fit
+    bool want_bin_launch();   // and builds the pass lists; false if they do not fit
     uint32_t defer_min_ = kDeferMinDefault;
     void try_pull(Instance &p, hipStream_t s);   // builds p's in-edges if on and they fit
     DataAllocator<InstDev> d_insts_;
@@ -713,7 +713,12 @@ private:
                queue_shift_ == kQueueShiftDefault && defer_min_ == kDeferMinDefault && p.direct_allowed();
     }
     bool try_direct(Instance &p);          // builds p's tile offsets if they fit
-    uint32_t nqueue_tiles_ = 0;            // tiles of the queue and gather instances (first in the tables)
+    // Whether the engine takes direct propagation, for every instance (an
+    // engine with both kinds steps in two launches, one after the other), and
+    // builds what it needs: all want it, and they have at most kDirectTiles
+    // tiles together.
+    bool want_direct();
+    uint32_t nqueue_tiles_ = 0;            // tiles of queue and gather instances: all, or none
     bool tuned_direct_ = false;            // the autotuner's (dense, default pass) candidate ran direct
     HostStage tables_stage_, call_stage_;
     // Everything a captured step's launches take from the engine: graphs stay

@@ -121,15 +121,42 @@ bool Engine::try_direct(Instance &p)
     }
 }
 
-bool Engine::want_bin_launch(const std::vector<char> &direct)
+bool Engine::want_direct()
 {
     uint64_t tiles = 0;
+    for (auto &p : insts_) {
+        if (!p)
+            continue;
+        if (!wants_direct(*p))
+            return false;
+        tiles += (p->n() + kBlock - 1) / kBlock;
+    }
+    if (tiles > kDirectTiles)
+        return false;
+    for (auto &p : insts_) {
+        if (!p)
+            continue;
+        try_pull(*p, stream_);
+        if (!p->pull_built() || !try_direct(*p))
+            return false;
+    }
+    return true;
+}
+
+bool Engine::want_bin_launch()
+{
+    uint64_t tiles = 0;
+    double segments = 0.0, synapses = 0.0;   // tile segments of all rows, and their synapses
     bool want = false;
-    auto queued = [&](size_t i) { return insts_[i] && !direct[i] && !use_gather(*insts_[i]); };
+    auto queued = [&](size_t i) { return insts_[i] && !use_gather(*insts_[i]); };
     for (size_t i = 0; i < insts_.size(); ++i)
-        if (queued(i))
-            tiles += (insts_[i]->n() + kBlock - 1) / kBlock;
-    want = tiles > 0 && (split_ || tiles >= kBinLaunchTiles);
+        if (queued(i)) {
+            const double t = (insts_[i]->n() + kBlock - 1) / kBlock;
+            tiles += (uint64_t)t;
+            segments += insts_[i]->row_coverage() * t * insts_[i]->n();
+            synapses += (double)insts_[i]->nsyn();
+        }
+    want = tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;
@@ -359,25 +386,13 @@ void Engine::rebuild()
     std::vector<BinDesc> bins;
     bin_tiles_ = 0;
     uint32_t fmt = kWeightAny + 1;   // the instances' common weight format (kWeightAny: mixed)
-    // The tiles of the queue and gather instances come first (their index is
-    // their queue count's), then those of the direct ones.
-    std::vector<size_t> order;
-    std::vector<char> direct(insts_.size(), 0);
-    for (size_t slot = 0; slot < insts_.size(); ++slot)
-        if (insts_[slot] && wants_direct(*insts_[slot])) {
-            try_pull(*insts_[slot], stream_);
-            direct[slot] = insts_[slot]->pull_built() && try_direct(*insts_[slot]);
-        }
-    for (int d = 0; d < 2; ++d)
-        for (size_t slot = 0; slot < insts_.size(); ++slot)
-            if (insts_[slot] && direct[slot] == d)
-                order.push_back(slot);
-    nqueue_tiles_ = 0;
-    const bool bin_launch = want_bin_launch(direct);
+    const bool dir = want_direct();   // every instance, or none
+    const bool bin_launch = !dir && want_bin_launch();
     std::vector<CopyWords> put;   // the tables' copies, below
-    for (size_t slot : order) {
+    for (size_t slot = 0; slot < insts_.size(); ++slot) {
         Instance *p = insts_[slot].get();
-        const bool dir = direct[slot] != 0;
+        if (!p)
+            continue;
         const uint32_t idx = (uint32_t)table.size();
         tile_base_[slot] = (uint32_t)tiles.size();
         stat_ = stat_ || p->stat_mask() != 0;
@@ -406,7 +421,7 @@ void Engine::rebuild()
         if (!gat)
             try_pull(*p, stream_);
         const bool pl = !gat && pull_on_ && p->pull_built();
-        if (!dir && !wants_direct(*p) && !tuning_)
+        if (!dir && !tuning_)
             p->release_direct();   // (the old tables, settled above, were the last to use it)
         const bool passes = bin_launch && !gat && !dir;
         table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_, passes));
@@ -426,8 +441,6 @@ void Engine::rebuild()
             for (uint32_t k = 0; k < ids.size(); ++k)
                 samples.push_back(SampleDev{idx, ids[k], k, 0});
         }
-        if (!dir)
-            nqueue_tiles_ = (uint32_t)tiles.size();
         if (!gat && !dir) {
             total += p->n();
             coverage += p->row_coverage() * p->n();
@@ -442,17 +455,18 @@ void Engine::rebuild()
     }
     if (total > 0xffffffffull || tiles.size() > 0xffffffffull)
         throw Error(kInvalidParameter, "too many neurons in one engine");
+    nqueue_tiles_ = dir ? 0u : (uint32_t)tiles.size();
     // Workgroups are dealt to the 8 XCDs by index mod 8: each XCD gets a
     // contiguous range of the direct tiles, so tiles that share cache lines
     // of a row's offsets and synapses meet in one L2.
-    {
-        const size_t nd = tiles.size() - nqueue_tiles_;
+    if (dir) {
+        const size_t nd = tiles.size();
         std::vector<TileDesc> dealt(nd);
         for (size_t k = 0; k < nd; ++k) {
             const size_t x = k & 7u;
-            dealt[k] = tiles[nqueue_tiles_ + x * (nd >> 3) + std::min<size_t>(x, nd & 7u) + (k >> 3)];
+            dealt[k] = tiles[x * (nd >> 3) + std::min<size_t>(x, nd & 7u) + (k >> 3)];
         }
-        std::copy(dealt.begin(), dealt.end(), tiles.begin() + nqueue_tiles_);
+        tiles.swap(dealt);
     }
     ninst_ = (uint32_t)table.size();
     wfmt_ = fmt > kWeightAny ? kWeightF32 : fmt;

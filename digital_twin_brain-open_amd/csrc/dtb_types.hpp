@@ -203,6 +203,14 @@ constexpr uint32_t kDirectIds = 6;
 // 14.7 us instead of 12.7), and the synapses a lane has in flight (4: 66k
 // neurons x 250 6.63 us, 2: 6.53).
 constexpr uint32_t kDirectMaxNeurons = 1u << 18;
+// Tiles of an engine up to which it takes direct propagation: it shortens the
+// chain of one tile's waits, and past a few rounds of resident workgroups what
+// counts is their work.  Uniform networks of 20k-200k neurons, steps direct /
+// by queues: 1672 tiles 11.8 / 20.0 us, 4853 36.4 / 42.1, 10330 67.1 / 69.7,
+// 20345 128.9 / 119.6.  Served networks of 10k-1M neurons, the small ones
+// direct in a launch of their own: 1.24e10 synaptic events per second, all by
+// queues 1.35e10.
+constexpr uint32_t kDirectTiles = 8192;
 constexpr uint32_t kDirectRows = 2048, kDirectItems = 2;
 constexpr uint32_t kDirectRounds = (kDirectMaxNeurons / kBlock + kBlock - 1) / kBlock;   // tiles per thread
 
@@ -368,7 +376,10 @@ constexpr uint32_t kBinTiles = 16, kBinGroups = 512;
 // 33 spikes per second: 400k neurons (1563 tiles) 13.5 / 15.3, 15.7 / 16.0 and
 // 22.9 / 20.7 us; 600k (2344) 16.3 / 18.0, 19.5 / 19.6 and 28.8 / 25.9; 900k
 // (3516) 22.9 / 23.1, 27.5 / 25.9 and 38.1 / 33.8; 2M (7813) at 6, 11 and 21
-// 40.6 / 38.4, 49.5 / 43.5 and 69.1 / 59.8.
+// 40.6 / 38.4, 49.5 / 43.5 and 69.1 / 59.8.  And only where rows have two
+// synapses per tile they reach (voxel networks: three; neighbouring rows then
+// reach the same tiles): with uniformly drawn targets there is little to add
+// up first, 900k x 300 35.9 / 44.0, 2M x 300 53.8 / 63.2.
 constexpr uint32_t kBinLaunchTiles = 3072u;
 struct alignas(16) BinDesc {
     const InstDev *inst;

@@ -377,7 +377,8 @@ class Engine:
         """Sets (when given) and returns split binning: the fired rows are
         binned by a second launch per step, in equal shares over the whole
         GPU, instead of by the tiles whose neurons fired (off: only in engines
-        whose queues serve 786,432 neurons or more; capacity has no effect).
+        of 786,432 neurons or more whose rows have two synapses per tile they
+        reach; capacity has no effect).
         Same results either way."""
         if on is not None:
             _lib.check(self._lib.dtb_engine_split(self._h, c_int32(int(bool(on))), ctypes.c_uint32(int(capacity))))
