@@ -11,7 +11,7 @@
 //             (synaptic_current.cpp:7-105)
 //
 // One launch per step here (k_step; see the end of this comment for the
-// gather schedule's second launch).  Every workgroup of 256 threads owns a
+// second launches of the gather schedule and of large engines).  Every workgroup of 256 threads owns a
 // tile of 256 consecutive neurons of one instance, and per tile:
 //   1. reads the tile's queue (the synapses delivered to it: target index,
 //      channel pair, weight pair; contiguous, so the reads coalesce) and adds
@@ -29,10 +29,13 @@
 // fills set p ^ 1, so step k consumes exactly the synapses queued from the
 // spikes of step k - 1.  No global atomics touch the delta.
 //   With the gather schedule (instances with group offsets) a k_gather
-//   launch precedes each k_step: per group of 2048 target neurons it gathers
+//   launch precedes each k_step: per group of target neurons it gathers
 //   the last step's fired rows into the same exact LDS sums and writes the
 //   delta, which k_step folds instead of draining a queue; k_step lists its
 //   fired rows for the next k_gather instead of binning them.
+//   Small engines propagate directly: no queues, a tile reads the rows that
+//   every tile emitted in the step before (direct_tile).  Large ones bin in a
+//   launch of their own (k_bin) in place of 3.
 //   k_materialize writes the pending delta of every neuron (without consuming
 //   the queues) for sampling and state read-back; k_sample gathers samples.
 #include <hip/hip_ext.h>
@@ -1436,8 +1439,9 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
     const InstPtr I = cp(d->inst);
     const bool gat = (d->flags & kTileGather) != 0u;
     // Spike propagation (presynaptic_voltage.cpp:122-225): with gather the
-    // fired rows go to lists for the next k_gather; else the tile's emitted
-    // rows are left as bits for the k_bin launch that follows.
+    // fired rows go to lists for the next k_gather; else they are binned by
+    // the tile (below) or listed as passes for the k_bin launch that follows,
+    // or left as bits and ids (direct).
     const unsigned long long m = __ballot(emit);
     if (lane == 0)
         s_bits[w] = m;
@@ -1557,9 +1561,8 @@ __device__ __forceinline__ void step_tile(TilePtr tp, QueuePtr qp, uint32_t par,
     }
 }
 
-// The step of launch parity `par`: takes the input of set par, leaves the
-// emitted rows of set par ^ 1 as bits (fired lists with gather), reads the
-// step index from step[par] and advances it into step[par ^ 1].
+// The step of launch parity `par`: takes the input of set par, passes its
+// emitted rows on into set par ^ 1, reads the step index from step[par] and advances it into step[par ^ 1].
 // Seven waves per SIMD: at eight the compiler spills up to 14 registers, and
 // the 2M-neuron step takes 42.3 us instead of 40.5 (1200 rows per step), a
 // 10k-neuron step by direct propagation 5.7 instead of 5.3.

@@ -56,3 +56,13 @@ def test_more_tiles_than_one_window(dtb, orc, gpu):
 @pytest.mark.parametrize("n", [3071 * 256, 3071 * 256 + 1])
 def test_size_from_which_it_is_taken(dtb, orc, gpu, n):
     check(dtb, orc, [dtb.gen_uniform(n, 12, seed=5)], 40, 6.0)
+
+
+def test_taken_where_rows_share_tiles(dtb, orc, gpu):
+    """A voxel network of 3072 tiles whose rows have two synapses per tile
+    they reach (the uniform ones above have one)."""
+    net = dtb.gen_voxel(3072 * 256, 78, 220, seed=6)
+    rows = np.random.default_rng(1).integers(0, net.n, 500)
+    seg = [len(np.unique(net.col[net.rowptr[r]:net.rowptr[r + 1]] >> 8)) for r in rows]
+    assert 2.0 * np.mean(seg) < 0.98 * 220
+    check(dtb, orc, [net], 24, 9.0)
