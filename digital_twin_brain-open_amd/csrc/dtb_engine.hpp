@@ -103,8 +103,9 @@ void release(void *p);               // block from alloc; may still be in use by
 void reserve(size_t bytes);          // keeps at least this much for blocks of 1 MB and more
 void trim();                         // returns all unused memory to the runtime
 size_t cached_bytes(int device);     // bytes held in the cache
-// While one is alive on a thread, alloc on that thread throws instead of
-// taking memory (the entry points that promise not to allocate).
+// While one is alive on a thread, alloc on that thread (and HostStage::reserve)
+// throws instead of taking memory (the entry points that promise not to
+// allocate).
 struct NoAlloc {
     NoAlloc();
     ~NoAlloc();
@@ -218,10 +219,15 @@ public:
     HostStage(const HostStage &) = delete;
     HostStage &operator=(const HostStage &) = delete;
     // At least `bytes`; what it held before is lost when it grows, so no
-    // kernel may be using it.
+    // kernel may be using it.  Under NoAlloc it throws instead of growing (a
+    // caller inside a capture may make no allocating runtime call).
     unsigned char *reserve(size_t bytes)
     {
         if (bytes > cap_) {
+            if (devmem::NoAlloc::active())
+                throw Error(kInvalidParameter, "this call allocates no memory, but needs " + std::to_string(bytes) +
+                                                   " bytes of pinned host memory first (build the tables with one "
+                                                   "dtb_run or dtb_engine_run)");
             release();
             DTB_HIP(hipHostMalloc(&p_, bytes, hipHostMallocDefault));
             cap_ = bytes;

@@ -520,6 +520,9 @@ void Engine::rebuild()
         f(d_recs_, recs);
     };
     each_table([&](auto &, const auto &v) { bytes += v.size() * sizeof(v[0]); });
+    // sized for every sample that is set, like d_samples_: a recording that
+    // follows takes no pinned memory (dtb_run_noalloc)
+    bytes += (std::max(sample_set, samples.size()) - samples.size()) * sizeof(samples[0]);
     unsigned char *at = tables_stage_.reserve(std::max<size_t>(bytes, 1));
     each_table([&](auto &buf, const auto &v) {
         const size_t b = v.size() * sizeof(v[0]);
