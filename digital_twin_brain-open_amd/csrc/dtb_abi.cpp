@@ -612,6 +612,20 @@ int dtb_engine_get_schedule(dtb_engine_t h, int32_t *pass_k, int32_t *layout, in
     });
 }
 
+int dtb_engine_get_step_mode(dtb_engine_t h, int32_t *mode, uint64_t *tables_built)
+{
+    return guarded([&] {
+        const dtb::Engine &e = engine(h);
+        if (mode)
+            *mode = e.gathers()                                  ? DTB_STEP_GATHER
+                    : e.step_mode() == dtb::StepMode::direct     ? DTB_STEP_DIRECT
+                    : e.step_mode() == dtb::StepMode::bin_launch ? DTB_STEP_BIN_LAUNCH
+                                                                 : DTB_STEP_TILE_BIN;
+        if (tables_built)
+            *tables_built = e.tables_built();
+    });
+}
+
 int dtb_instance_propagation(dtb_engine_t h, int inst, int32_t *gather_allowed, int32_t *gather_in_use,
                              float *group_coverage)
 {

@@ -612,6 +612,15 @@ public:
     uint32_t defer_min() const { return defer_min_; }
     // (a direct instance pulls the steps whose emitted rows are many)
     bool uses_pull(const Instance &p) const { return pull_on_ && p.pull_built() && !use_gather(p); }
+    // How the tables of the last build step (gathers(): some of their
+    // instances gather), and how often an instance's tile offsets or pass
+    // lists were built.
+    StepMode step_mode() const
+    {
+        return nqueue_tiles_ < ntiles_ ? StepMode::direct : nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin;
+    }
+    bool gathers() const { return ngroups_ > 0; }
+    uint64_t tables_built() const { return tables_built_; }
     // Queue capacity per tile: min(synapses targeting it, floor +
     // (synapses >> shift)); shift 0 keeps the exact worst case.
     void set_queue_capacity(uint32_t floor, uint32_t shift);
@@ -695,6 +704,7 @@ private:
     DataAllocator<BinDesc> d_bins_;        // k_bin's workgroups
     uint32_t nbins_ = 0, bin_tiles_ = 0;   // their number (0: tiles bin their own rows), tiles of the largest queue instance
     bool want_bin_launch();   // and builds the pass lists; false if they do not fit
+    uint64_t tables_built_ = 0;            // tables_built()
     uint32_t defer_min_ = kDeferMinDefault;
     void try_pull(Instance &p, hipStream_t s);   // builds p's in-edges if on and they fit
     DataAllocator<InstDev> d_insts_;

@@ -111,6 +111,7 @@ bool Engine::try_direct(Instance &p)
         return false;
     try {
         p.ensure_direct(stream_);
+        ++tables_built_;
         return true;
     } catch (const Error &e) {
         // without device memory for the offsets the instance keeps queues
@@ -164,6 +165,7 @@ bool Engine::want_bin_launch()
             return false;
         try {
             insts_[i]->ensure_passes();
+            ++tables_built_;
         } catch (const Error &e) {
             // without device memory for the lists the tiles bin their own
             // rows (same results)

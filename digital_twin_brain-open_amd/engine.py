@@ -412,6 +412,19 @@ class Engine:
             _lib.check(self._lib.dtb_engine_get_schedule(self._h, byref(k), byref(l), byref(u)))
         return k.value, names[l.value], names.get(u.value, "dense")
 
+    STEP_MODES = ("tile_bin", "bin_launch", "direct", "gather")
+
+    def step_info(self):
+        """How the engine's last run (or table build) steps: {"mode":
+        "tile_bin" (emitted rows binned into queues by the tiles that fired),
+        "bin_launch" (by a second launch per step), "direct" (tiles read the
+        rows emitted in the step before, no queues) or "gather" (some
+        instance gathers), "tables_built": how often an instance's tile
+        offsets or pass lists were built}."""
+        m, b = c_int32(0), c_uint64(0)
+        _lib.check(self._lib.dtb_engine_get_step_mode(self._h, byref(m), byref(b)))
+        return {"mode": self.STEP_MODES[m.value], "tables_built": int(b.value)}
+
     def autotune(self, trial_steps=50):
         """Times every schedule on about trial_steps real steps, the schedules
         taking turns in 4-step windows (autotune_steps(trial_steps) steps in

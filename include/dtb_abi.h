@@ -303,6 +303,15 @@ int dtb_engine_get_schedule(dtb_engine_t h, int32_t *pass_k, int32_t *layout, in
  * simulation exactly as any other steps would; tune in the regime that will
  * be run (after the initial transient). */
 int dtb_engine_autotune(dtb_engine_t h, int64_t trial_steps, int32_t *pass_k, int32_t *layout, float *us_per_step);
+/* No counterpart in the reference.  How the tables of the last run or table
+ * build step: emitted rows binned into queues by the tiles whose neurons
+ * fired (TILE_BIN) or by a second launch per step (BIN_LAUNCH), tiles that
+ * take their input straight from the rows emitted in the step before
+ * (DIRECT), or, where some instance gathers, GATHER.  tables_built: how often
+ * the engine has built an instance's tile offsets (DIRECT) or pass lists
+ * (BIN_LAUNCH).  Any pointer may be NULL. */
+enum { DTB_STEP_TILE_BIN = 0, DTB_STEP_BIN_LAUNCH = 1, DTB_STEP_DIRECT = 2, DTB_STEP_GATHER = 3 };
+int dtb_engine_get_step_mode(dtb_engine_t h, int32_t *mode, uint64_t *tables_built);
 /* No counterpart in the reference.  Gather propagation of one instance:
  * whether it allows it (rows ordered by target group, rows of at most 65535
  * synapses, group offsets no larger than the synapse arrays), whether the

@@ -1,0 +1,136 @@
+"""Which step an engine takes (Engine.step_info) under every rule that chooses
+one, each checked bit for bit against the CPU oracle in the same run: direct
+propagation for all instances or none, its rounds of listed rows, the queue
+tiles and the sharing of tiles from which rows are binned in a launch of their
+own, and the settings that take either off."""
+import numpy as np
+import pytest
+
+from test_direct import LIMIT, reorder
+from test_gpu_parity import DT, assert_state_equal, run_oracle
+
+pytestmark = pytest.mark.gpu
+
+QUEUES = ("tile_bin", "bin_launch")
+
+
+def add(dtb, eng, net, seed, mu):
+    b = dtb.Block(net, delta_t=DT, seed=seed, engine=eng)
+    b.update_ou_background_stimuli(b.subblk_id, 4.0, mu, 0.1)
+    eng.configure(b.inst, 1, True)
+    return b
+
+
+def assert_oracle(orc, net, blk, steps, seed, mu):
+    ref, sim = run_oracle(orc, net, steps, seed, mu)
+    events = int((ref["raster"].astype(np.int64) * np.diff(net.rowptr)[None, :]).sum())
+    assert events > 0 and blk.counters() == (steps, events, int(ref["raster"].sum()))
+    assert_state_equal(blk.state(), sim)
+
+
+def reversed_rows(dtb, net):
+    """Rows by descending target: direct propagation is not allowed."""
+    return reorder(dtb, net, -net.col.astype(np.int64))
+
+
+@pytest.mark.parametrize("settings,mode", [
+    ({}, "direct"),
+    (dict(schedule=dict(layout="dense")), "tile_bin"),
+    (dict(schedule=dict(layout="spread")), "tile_bin"),
+    (dict(schedule=dict(pass_k=1, layout="auto")), "direct"),
+    (dict(schedule=dict(layout="gather")), "gather"),
+    (dict(split=dict(on=True)), "bin_launch"),
+    (dict(split=dict(on=True, capacity=3)), "bin_launch"),
+    (dict(pull=dict(on=False)), "tile_bin"),
+    (dict(pull=dict(defer_min=1)), "tile_bin"),
+    (dict(queue_capacity=dict(floor=64, shift=4)), "tile_bin"),
+])
+def test_mode_by_settings(dtb, orc, gpu, settings, mode):
+    net, steps = dtb.gen_uniform(5000, 60, seed=4), 150
+    eng = dtb.Engine(0)
+    try:
+        for name, kw in settings.items():
+            getattr(eng, name)(**kw)
+        b = add(dtb, eng, net, 3, 2.0)
+        eng.run(steps, graph_chunk=50)
+        assert eng.step_info()["mode"] == mode
+        assert_oracle(orc, net, b, steps, 3, 2.0)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("n,mode", [(2, "direct"), (255, "direct"), (257, "direct"), (LIMIT, "direct"),
+                                    (LIMIT + 1, "tile_bin")])
+def test_direct_by_size(dtb, orc, gpu, n, mode):
+    net, steps = dtb.gen_uniform(n, min(180, n - 1), seed=2), 40
+    eng = dtb.Engine(0)
+    try:
+        b = add(dtb, eng, net, 13, 5.0)
+        eng.run(steps)
+        assert eng.step_info()["mode"] == mode
+        assert_oracle(orc, net, b, steps, 13, 5.0)
+    finally:
+        eng.close()
+
+
+def test_direct_for_all_instances_or_none(dtb, orc, gpu):
+    """Unequal instances step directly; one that does not allow it takes all
+    of them to queues, and back when it leaves, with spikes pending."""
+    nets = [dtb.gen_uniform(3000, 60, seed=4), dtb.gen_voxel(30000, 12, 150, seed=3), dtb.gen_uniform(257, 20, seed=9)]
+    other = reversed_rows(dtb, dtb.gen_uniform(9000, 120, seed=2))
+    eng = dtb.Engine(0)
+    try:
+        blks = [add(dtb, eng, net, 70 + i, 2.0) for i, net in enumerate(nets)]
+        eng.run(120, graph_chunk=50)
+        assert eng.step_info()["mode"] == "direct"
+        guest = add(dtb, eng, other, 90, 2.0)
+        eng.run(101, graph_chunk=50)
+        assert eng.step_info()["mode"] == "tile_bin"
+        assert_oracle(orc, other, guest, 101, 90, 2.0)
+        eng.remove(guest.inst)
+        eng.run(60, graph_chunk=50)
+        assert eng.step_info()["mode"] == "direct"
+        for i, net in enumerate(nets):
+            assert_oracle(orc, net, blks[i], 281, 70 + i, 2.0)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("rate", [0.04, 0.085])
+def test_direct_rows_in_rounds(dtb, orc, gpu, rate):
+    """More rows than a tile lists at a time (2048), and fewer than from which
+    reading the in-edges is cheaper: two and three rounds in every step."""
+    g = tuple(np.asarray(dtb.DEFAULT_G_UI) * 0.002)
+    net, steps = dtb.gen_uniform(70_001, 400, seed=6, g_ui=g), 24
+    net.props[:, 0] = rate   # noise spikes per step
+    ref, sim = run_oracle(orc, net, steps, 19, 0.0, use_ou=False)
+    rows = ref["raster"].sum(axis=1)
+    edges = np.bincount(net.col >> 8, minlength=(net.n + 255) // 256).astype(np.float64)
+    pulls_from = 12 * edges * net.n / (64.0 * net.n + 24 * edges)
+    assert rows.min() > 2048 and rows.max() <= pulls_from.min()
+    eng = dtb.Engine(0)
+    try:
+        b = dtb.Block(net, delta_t=DT, seed=19, engine=eng)
+        out = b.run(steps, freqs=True, iou=False)
+        assert eng.step_info()["mode"] == "direct" and eng.propagation_stats()["pulled"] == 0
+        assert np.array_equal(out["freq"].sum(axis=1), rows)
+        assert_state_equal(b.state(), sim)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("kind,n,mode", [("voxel", 3071 * 256, "tile_bin"), ("voxel", 3071 * 256 + 1, "bin_launch"),
+                                         ("uniform", 3071 * 256 + 1, "tile_bin")])
+def test_binning_launch_by_tiles_and_sharing(dtb, orc, gpu, kind, n, mode):
+    """From 3072 tiles, and only where rows have two synapses per tile they
+    reach."""
+    net = dtb.gen_voxel(n, 78, 220, seed=6) if kind == "voxel" else dtb.gen_uniform(n, 12, seed=5)
+    steps, mu = (24, 9.0) if kind == "voxel" else (40, 6.0)
+    eng = dtb.Engine(0)
+    try:
+        b = add(dtb, eng, net, 40, mu)
+        eng.run(steps)
+        assert eng.step_info()["mode"] == mode
+        assert_oracle(orc, net, b, steps, 40, mu)
+    finally:
+        eng.close()
