@@ -148,7 +148,6 @@ bool Engine::want_bin_launch()
 {
     uint64_t tiles = 0;
     double segments = 0.0, synapses = 0.0;   // tile segments of all rows, and their synapses
-    bool want = false;
     auto queued = [&](size_t i) { return insts_[i] && !use_gather(*insts_[i]); };
     for (size_t i = 0; i < insts_.size(); ++i)
         if (queued(i)) {
@@ -157,7 +156,7 @@ bool Engine::want_bin_launch()
             segments += insts_[i]->row_coverage() * t * insts_[i]->n();
             synapses += (double)insts_[i]->nsyn();
         }
-    want = tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
+    const bool want = tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;
@@ -171,12 +170,12 @@ bool Engine::want_bin_launch()
             // rows (same results)
             if (e.code != kOutOfMemory)
                 throw;
-            want = false;
+            for (auto &p : insts_)
+                if (p)
+                    p->release_passes();
+            return false;
         }
     }
-    for (auto &p : insts_)
-        if (p && !want)
-            p->release_passes();
     return want;
 }
 
@@ -425,7 +424,9 @@ void Engine::rebuild()
         const bool pl = !gat && pull_on_ && p->pull_built();
         if (!dir && !tuning_)
             p->release_direct();   // (the old tables, settled above, were the last to use it)
-        const bool passes = bin_launch && !gat && !dir;
+        const bool passes = bin_launch && !gat;
+        if (!passes && !devmem::NoAlloc::active())
+            p->release_passes();
         table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_, passes));
         if (passes)
             put.push_back(p->pass_count_words());

@@ -134,3 +134,21 @@ def test_binning_launch_by_tiles_and_sharing(dtb, orc, gpu, kind, n, mode):
         assert_oracle(orc, net, b, steps, 40, mu)
     finally:
         eng.close()
+
+
+def test_pass_lists_returned_in_direct_propagation(dtb, gpu):
+    """The lists of the binning launch (131 kB here) go back when the engine
+    turns to direct propagation."""
+    eng = dtb.Engine(0)
+    try:
+        add(dtb, eng, dtb.gen_uniform(257, 20, seed=9), 3, 2.0)
+        eng.split(True)
+        eng.run(5)
+        assert eng.step_info()["mode"] == "bin_launch"
+        before = dtb.device_memory_cached(0)
+        eng.split(False)
+        eng.run(5)
+        assert eng.step_info()["mode"] == "direct"
+        assert dtb.device_memory_cached(0) - before > 64 * 1024
+    finally:
+        eng.close()
