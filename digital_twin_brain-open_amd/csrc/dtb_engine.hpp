@@ -603,7 +603,7 @@ public:
         if (on != split_ || cap != split_cap_) {
             split_ = on;
             split_cap_ = cap;
-            dirty_ = true;
+            routes_changed();
         }
     }
     bool split() const { return split_; }
@@ -734,6 +734,15 @@ private:
     // builds what it needs: all want it, and they have at most kDirectTiles
     // tiles together.
     bool want_direct();
+    // Offsets or pass lists did not fit: not tried again (each table build
+    // would build and return those that do fit) before the instances or the
+    // propagation settings change.
+    bool direct_short_ = false, passes_short_ = false;
+    void routes_changed()
+    {
+        dirty_ = true;
+        direct_short_ = passes_short_ = false;
+    }
     uint32_t nqueue_tiles_ = 0;            // tiles of queue and gather instances: all, or none
     bool tuned_direct_ = false;            // the autotuner's (dense, default pass) candidate ran direct
     HostStage tables_stage_, call_stage_;

@@ -48,12 +48,12 @@ int Engine::add(std::unique_ptr<Instance> inst)
     for (size_t i = 0; i < insts_.size(); ++i)
         if (!insts_[i]) {
             insts_[i] = std::move(inst);
-            dirty_ = true;
+            routes_changed();
             staged_.insert((int)i);
             return (int)i;
         }
     insts_.push_back(std::move(inst));
-    dirty_ = true;
+    routes_changed();
     staged_.insert((int)insts_.size() - 1);
     return (int)insts_.size() - 1;
 }
@@ -64,7 +64,7 @@ std::unique_ptr<Instance> Engine::remove(int id)
         throw Error(kInvalidParameter, "no such instance");
     settle();
     sync();
-    dirty_ = true;
+    routes_changed();
     staged_.erase(id);
     return std::move(insts_[id]);
 }
@@ -94,7 +94,7 @@ void Engine::set_schedule(uint32_t pass_k, int layout)
         pass_k_ = pass_k;
         count_layout_ = layout;
         tuned_direct_ = false;
-        dirty_ = true;   // graphs hold the old kernel; counts move to the new layout
+        routes_changed();   // graphs hold the old kernel; counts move to the new layout
     }
 }
 
@@ -124,6 +124,8 @@ bool Engine::try_direct(Instance &p)
 
 bool Engine::want_direct()
 {
+    if (direct_short_)
+        return false;
     uint64_t tiles = 0;
     for (auto &p : insts_) {
         if (!p)
@@ -138,8 +140,10 @@ bool Engine::want_direct()
         if (!p)
             continue;
         try_pull(*p, stream_);
-        if (!p->pull_built() || !try_direct(*p))
+        if (!p->pull_built() || !try_direct(*p)) {
+            direct_short_ = !devmem::NoAlloc::active();
             return false;
+        }
     }
     return true;
 }
@@ -156,7 +160,7 @@ bool Engine::want_bin_launch()
             segments += insts_[i]->row_coverage() * t * insts_[i]->n();
             synapses += (double)insts_[i]->nsyn();
         }
-    const bool want = tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
+    const bool want = !passes_short_ && tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;
@@ -173,6 +177,7 @@ bool Engine::want_bin_launch()
             for (auto &p : insts_)
                 if (p)
                     p->release_passes();
+            passes_short_ = true;
             return false;
         }
     }
@@ -275,7 +280,7 @@ void Engine::set_pull(bool on, uint32_t defer_min)
     if (on != pull_on_ || defer_min != defer_min_) {
         pull_on_ = on;
         defer_min_ = defer_min;
-        dirty_ = true;
+        routes_changed();
     }
 }
 
@@ -321,7 +326,7 @@ void Engine::set_queue_capacity(uint32_t floor, uint32_t shift)
         throw Error(kInvalidParameter, "queue capacity shift must be at most 31");
     queue_floor_ = floor;
     queue_shift_ = shift;
-    dirty_ = true;
+    routes_changed();
 }
 
 uint32_t Engine::queue_capacity(uint32_t synapses) const

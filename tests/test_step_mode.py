@@ -152,3 +152,42 @@ def test_pass_lists_returned_in_direct_propagation(dtb, gpu):
         assert dtb.device_memory_cached(0) - before > 64 * 1024
     finally:
         eng.close()
+
+
+def test_offsets_that_do_not_fit_are_tried_once(dtb, gpu):
+    """Where the offsets of one instance do not fit (313 MB, from a
+    reservation with 64 MB left), the engine keeps queues and does not build
+    and return those of the others at every run; it tries again when the
+    instances change."""
+    def fill(eng):
+        small = dtb.Block(dtb.gen_uniform(3000, 60, seed=4), delta_t=DT, seed=3, engine=eng)
+        return small, eng.add_fanout(200_000, 150, 5)
+
+    dtb.device_memory_trim()
+    dtb.device_memory_reserve(4 << 30)
+    eng = dtb.Engine(0)
+    try:
+        eng.schedule(layout="dense")
+        free = dtb.device_memory_cached(0)
+        fill(eng)
+        eng.run(2)
+        used = free - dtb.device_memory_cached(0)
+    finally:
+        eng.close()
+    dtb.device_memory_trim()
+    dtb.device_memory_reserve(used + (64 << 20))
+    eng = dtb.Engine(0)
+    try:
+        small, big = fill(eng)
+        small.run(3, freqs=True)
+        assert eng.step_info()["mode"] == "tile_bin"
+        built = eng.step_info()["tables_built"]
+        for _ in range(4):
+            small.run(3, freqs=True)
+        assert eng.step_info() == {"mode": "tile_bin", "tables_built": built}
+        eng.remove(big)
+        small.run(3, freqs=True)
+        assert eng.step_info() == {"mode": "direct", "tables_built": built + 1}
+    finally:
+        eng.close()
+        dtb.device_memory_trim()
