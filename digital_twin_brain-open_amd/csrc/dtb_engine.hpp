@@ -732,7 +732,7 @@ private:
     // Whether the engine takes direct propagation, for every instance (an
     // engine with both kinds steps in two launches, one after the other), and
     // builds what it needs: all want it, and they have at most kDirectTiles
-    // tiles together.
+    // tiles together (kDirectTilesStay while it steps so).
     bool want_direct();
     // Offsets or pass lists did not fit: not tried again (each table build
     // would build and return those that do fit) before the instances or the

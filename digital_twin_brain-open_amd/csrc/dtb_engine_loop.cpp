@@ -134,7 +134,7 @@ bool Engine::want_direct()
             return false;
         tiles += (p->n() + kBlock - 1) / kBlock;
     }
-    if (tiles > kDirectTiles)
+    if (tiles > (step_mode() == StepMode::direct ? kDirectTilesStay : kDirectTiles))
         return false;
     for (auto &p : insts_) {
         if (!p)

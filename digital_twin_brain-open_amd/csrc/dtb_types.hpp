@@ -211,6 +211,10 @@ constexpr uint32_t kDirectMaxNeurons = 1u << 18;
 // direct in a launch of their own: 1.24e10 synaptic events per second, all by
 // queues 1.35e10.
 constexpr uint32_t kDirectTiles = 8192;
+// An engine that steps directly goes on to here (10330 tiles, above, are still
+// no slower), so instances that come and go around the limit do not make it
+// build and return every instance's offsets at each change.
+constexpr uint32_t kDirectTilesStay = kDirectTiles + kDirectTiles / 4u;
 constexpr uint32_t kDirectRows = 2048, kDirectItems = 2;
 constexpr uint32_t kDirectRounds = (kDirectMaxNeurons / kBlock + kBlock - 1) / kBlock;   // tiles per thread
 

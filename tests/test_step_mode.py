@@ -191,3 +191,34 @@ def test_offsets_that_do_not_fit_are_tried_once(dtb, gpu):
     finally:
         eng.close()
         dtb.device_memory_trim()
+
+
+def test_direct_stays_past_the_tiles_it_starts_from(dtb, gpu):
+    """8192 tiles to start, 10240 to leave: an instance that comes and goes at
+    8,200 tiles does not make the others' offsets go and come back."""
+    n, k = 25_600, 30   # 100 tiles each
+    eng = dtb.Engine(0)
+    try:
+        ids = [eng.add_fanout(n, k, 7 + i) for i in range(81)]
+        eng.run(2)
+        assert eng.step_info() == {"mode": "direct", "tables_built": 81}
+        for turn in range(3):
+            extra = eng.add_fanout(n, k, 500 + turn)
+            eng.run(2)
+            assert eng.step_info() == {"mode": "direct", "tables_built": 82 + turn}
+            eng.remove(extra)
+            eng.run(2)
+            assert eng.step_info() == {"mode": "direct", "tables_built": 82 + turn}
+        ids += [eng.add_fanout(n, k, 600 + i) for i in range(22)]
+        eng.run(2)
+        assert eng.step_info()["mode"] == "tile_bin"   # 10300 tiles
+        for i in ids[90:]:
+            eng.remove(i)
+        eng.run(2)
+        assert eng.step_info()["mode"] == "tile_bin"   # 9000: not from here
+        for i in ids[81:90]:
+            eng.remove(i)
+        eng.run(2)
+        assert eng.step_info()["mode"] == "direct"
+    finally:
+        eng.close()
