@@ -367,8 +367,10 @@ void Instance::ensure_direct(hipStream_t s)
     const uint32_t ntile = (n_ + kBlock - 1) / kBlock;
     try {
         tidx_.resize((size_t)n_ * (ntile + 1u));
-        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ntile, kTileBits, tidx_.mutable_gpu_data(),
+        // (every word is written; up to 500 MB to clear otherwise)
+        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ntile, kTileBits, tidx_.gpu_uncleared(),
                                     s));
+        DTB_HIP(hipStreamSynchronize(s));
     } catch (...) {
         tidx_.resize(0);
         throw;
@@ -389,7 +391,7 @@ void Instance::ensure_passes()
         pass_count_.resize(2 * (size_t)kFiredLists * kFiredCountStride);
         pass_count_.mutable_gpu_data();
         passes_.resize((size_t)(kFiredLists * passcap_));
-        passes_.mutable_gpu_data();
+        passes_.gpu_uncleared();   // (entries past a list's count are not read)
     } catch (...) {
         release_passes();
         throw;

@@ -159,6 +159,14 @@ public:
         }
         return gpu_;
     }
+    // The device memory, not cleared when it is taken: for a buffer of which
+    // nothing is read that a kernel has not written.
+    T *gpu_uncleared()
+    {
+        if (gpu_ == nullptr && count_ > 0)
+            gpu_ = static_cast<T *>(devmem::alloc(size()));
+        return gpu_;
+    }
     const T *cpu_data() { return mutable_cpu_data(); }
     T *mutable_cpu_data()
     {
@@ -728,12 +736,13 @@ private:
         return (count_layout_ == kLayoutAuto || tuned_direct_) && !split_ && pull_on_ && queue_floor_ == kQueueFloorDefault &&
                queue_shift_ == kQueueShiftDefault && defer_min_ == kDeferMinDefault && p.direct_allowed();
     }
-    bool try_direct(Instance &p);          // builds p's tile offsets if they fit
-    // Whether the engine takes direct propagation, for every instance (an
-    // engine with both kinds steps in two launches, one after the other), and
-    // builds what it needs: all want it, and they have at most kDirectTiles
-    // tiles together (kDirectTilesStay while it steps so).
-    bool want_direct();
+    bool try_direct(Instance &p, hipStream_t s);   // builds p's tile offsets if they fit
+    // Whether the engine's instances, and `joining` with them, should step by
+    // direct propagation, all of them (an engine with both kinds steps in two
+    // launches, one after the other): all want it, and they have at most
+    // kDirectTiles tiles together (kDirectTilesStay while it steps so).
+    bool direct_by_rules(const Instance *joining = nullptr) const;
+    bool want_direct();                    // direct_by_rules(), and builds what it needs
     // Offsets or pass lists did not fit: not tried again (each table build
     // would build and return those that do fit) before the instances or the
     // propagation settings change.

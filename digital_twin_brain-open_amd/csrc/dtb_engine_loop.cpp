@@ -45,6 +45,10 @@ int Engine::add(std::unique_ptr<Instance> inst)
         inst->ensure_gather(admit_stream_);
     else
         try_pull(*inst, admit_stream_);
+    // Beside the steps of the others, like the in-edges (a table build would
+    // do it on their stream).
+    if (inst->pull_built() && direct_by_rules(inst.get()))
+        try_direct(*inst, admit_stream_);
     for (size_t i = 0; i < insts_.size(); ++i)
         if (!insts_[i]) {
             insts_[i] = std::move(inst);
@@ -103,14 +107,14 @@ bool Engine::use_gather(const Instance &p) const
     return p.gather_allowed() && count_layout_ == kLayoutGather;
 }
 
-bool Engine::try_direct(Instance &p)
+bool Engine::try_direct(Instance &p, hipStream_t s)
 {
     if (p.direct_built())
         return true;
     if (devmem::NoAlloc::active())
         return false;
     try {
-        p.ensure_direct(stream_);
+        p.ensure_direct(s);
         ++tables_built_;
         return true;
     } catch (const Error &e) {
@@ -122,25 +126,30 @@ bool Engine::try_direct(Instance &p)
     }
 }
 
+bool Engine::direct_by_rules(const Instance *joining) const
+{
+    uint64_t tiles = 0;
+    auto wanted = [&](const Instance &p) {
+        tiles += (p.n() + kBlock - 1) / kBlock;
+        return wants_direct(p);
+    };
+    if (joining && !wanted(*joining))
+        return false;
+    for (auto &p : insts_)
+        if (p && !wanted(*p))
+            return false;
+    return tiles <= (step_mode() == StepMode::direct ? kDirectTilesStay : kDirectTiles);
+}
+
 bool Engine::want_direct()
 {
-    if (direct_short_)
-        return false;
-    uint64_t tiles = 0;
-    for (auto &p : insts_) {
-        if (!p)
-            continue;
-        if (!wants_direct(*p))
-            return false;
-        tiles += (p->n() + kBlock - 1) / kBlock;
-    }
-    if (tiles > (step_mode() == StepMode::direct ? kDirectTilesStay : kDirectTiles))
+    if (direct_short_ || !direct_by_rules())
         return false;
     for (auto &p : insts_) {
         if (!p)
             continue;
         try_pull(*p, stream_);
-        if (!p->pull_built() || !try_direct(*p)) {
+        if (!p->pull_built() || !try_direct(*p, stream_)) {
             direct_short_ = !devmem::NoAlloc::active();
             return false;
         }

@@ -222,3 +222,26 @@ def test_direct_stays_past_the_tiles_it_starts_from(dtb, gpu):
         assert eng.step_info()["mode"] == "direct"
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("n,k", [(257, 20), (20_000, 100)])
+def test_offsets_built_when_an_instance_is_added(dtb, orc, gpu, n, k):
+    """Before its first step, beside the steps of the others; in memory that
+    other data filled before (rows of no synapses among them)."""
+    old = dtb.Engine(0)
+    add(dtb, old, dtb.gen_uniform(n, 2 * k, seed=8), 5, 9.0)
+    old.run(60)
+    old.close()
+    net = dtb.gen_uniform(n, k, seed=4)
+    keep = np.repeat(np.arange(n), np.diff(net.rowptr)) % 5 != 0
+    pre = np.repeat(np.arange(n), np.diff(net.rowptr))[keep]
+    net = dtb.NetworkArrays.from_edges(net.props, pre, net.col[keep], net.w[keep], net.kind_per_synapse()[keep])
+    eng = dtb.Engine(0)
+    try:
+        b = add(dtb, eng, net, 3, 3.0)
+        assert eng.step_info()["tables_built"] == 1
+        eng.run(100, graph_chunk=20)
+        assert eng.step_info() == {"mode": "direct", "tables_built": 1}
+        assert_oracle(orc, net, b, 100, 3, 3.0)
+    finally:
+        eng.close()
