@@ -324,20 +324,28 @@ void Instance::ensure_gather(hipStream_t s)
         fcount_.mutable_gpu_data();
         fired_.resize(2 * (size_t)kFiredLists * fired_capacity());
         fired_.mutable_gpu_data();
-        const uint32_t ng = ngroups(gather_bits_);
-        segidx_.resize((size_t)n_ * (ng + 1u));
-        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ng, gather_bits_,
-                                    segidx_.mutable_gpu_data(), s));
         grec_.resize((size_t)nsyn_ * grec_words(wfmt_));
         DTB_HIP(launch_build_grec(col_.gpu_data(), w_.gpu_data(), wfmt_, (uint64_t)nsyn_, grec_.mutable_gpu_data(),
                                   s));
+        for (;;) {
+            segidx_.resize((size_t)n_ * (ngroups(gather_bits_) + 1u));
+            try {
+                segidx_.mutable_gpu_data();
+                break;
+            } catch (const Error &e) {
+                // without device memory for the offsets of smaller groups:
+                // larger ones
+                if (e.code != kOutOfMemory || gather_bits_ == kGroupBits)
+                    throw;
+                ++gather_bits_;
+            }
+        }
+        DTB_HIP(launch_build_segidx(rowptr_.gpu_data(), col_.gpu_data(), n_, ngroups(gather_bits_), gather_bits_,
+                                    segidx_.mutable_gpu_data(), s));
         DTB_HIP(hipStreamSynchronize(s));
     } catch (...) {
         // out of device memory (or a failed build): nothing half-built stays
-        segidx_.resize(0);
-        grec_.resize(0);
-        fired_.resize(0);
-        fcount_.resize(0);
+        release_gather();
         throw;
     }
     gather_built_ = true;
