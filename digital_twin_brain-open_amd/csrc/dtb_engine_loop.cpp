@@ -145,6 +145,11 @@ bool Engine::want_direct()
 {
     if (direct_short_ || !direct_by_rules())
         return false;
+    // an engine holds offsets or pass lists, not both (the old tables,
+    // settled by the caller, were the last to use the lists)
+    for (auto &p : insts_)
+        if (p && !devmem::NoAlloc::active())
+            p->release_passes();
     for (auto &p : insts_) {
         if (!p)
             continue;

@@ -25,20 +25,26 @@ from .engine import DEFAULT_G_UI, Block, Engine, device_memory_cached, device_me
 
 # Device bytes per neuron of an instance: parameter class, V, i_ou,
 # refractory counter, flag, J, pending delta, spill accumulators (2 x 32),
-# blocked flag, row offset and per-wave counters; per synapse: column index
-# and weight pair; the two propagation queues hold 12-byte entries, per tile
-# min(S_t, QUEUE_FLOOR + S_t / 2^QUEUE_SHIFT) of its S_t synapses (the
-# engine's default capacity).
+# blocked flag, row offset, emitted and deferred rows' bits and per-wave
+# counters; per synapse: column index and weight pair; the two propagation
+# queues hold 12-byte entries, per tile min(S_t, QUEUE_FLOOR + S_t /
+# 2^QUEUE_SHIFT) of its S_t synapses (the engine's default capacity).
 BYTES_PER_NEURON = 2 + 4 + 4 + 4 + 1 + 16 + 16 + 64 + 1 + 8 + 1
 BYTES_PER_SYNAPSE = 4 + 8
 QUEUE_ENTRY_BYTES, QUEUE_FLOOR, QUEUE_SHIFT = 12, 4096, 3
-GATHER_GROUP, FIRED_LISTS = 2048, 64
-# Gather records: each synapse's column and weight pair side by side.
+# Gather propagation: groups of 2048 target neurons, halved (not below 256)
+# while there are fewer than 128 and the offsets stay within 12 bytes per
+# synapse; each synapse's column and weight pair side by side.
+GATHER_BITS, GATHER_BITS_MIN, GATHER_GROUPS, FIRED_LISTS = 11, 8, 128, 64
+OFFSET_BYTES_PER_SYNAPSE = 12
 GATHER_RECORD_BYTES = 12
 # Pull propagation: the in-edges (source | target | channel key and weight
-# pair per synapse), per tile its first in-edge, per wave of 64 neurons two
-# bitmap words per parity.
+# pair per synapse), per tile its first in-edge.
 PULL_BYTES_PER_SYNAPSE = 4 + 8
+# Direct propagation (instances of at most 2^18 neurons): 2-byte offsets per
+# row and tile; binning by a launch of its own: 64 lists of 8-byte entries,
+# one per 256 synapses of a row.
+DIRECT_NEURONS, PASS_SYNAPSES = 1 << 18, 256
 
 
 class Request:
@@ -55,21 +61,38 @@ class Request:
         self.v = None
         self.shed = False   # refused by admission control (waited past the server's limit)
 
-    def device_bytes(self, gather=False, pull=False):
+    def device_bytes(self, gather=False, pull=False, optional=True):
         """Device footprint; gather: also the gather buffers (2-byte offsets
-        per row and group of 2048 neurons, 64 fired lists per parity, a
-        12-byte record per synapse); pull
-        (without gather): also the in-edges of the pull propagation."""
+        per row and target group, 64 fired lists per parity, a 12-byte record
+        per synapse); pull (without gather): also the in-edges of the pull
+        propagation.  optional: with what the engine takes where memory
+        allows, and steps without otherwise: gather's smaller groups; the
+        offsets of direct propagation (with pull) or the pass lists of a
+        binning launch, whichever is larger (an engine has one or the
+        other)."""
         syn = self.n * self.k
         tiles = (self.n + 255) // 256
         queue = min(syn, tiles * QUEUE_FLOOR + (syn >> QUEUE_SHIFT))   # bound on the sum over tiles
         b = self.n * BYTES_PER_NEURON + syn * BYTES_PER_SYNAPSE + 2 * QUEUE_ENTRY_BYTES * queue
         if gather:
-            groups = (self.n + GATHER_GROUP - 1) // GATHER_GROUP
+            bits = GATHER_BITS
+            groups = (self.n + (1 << bits) - 1) >> bits
+            while optional and bits > GATHER_BITS_MIN and groups < GATHER_GROUPS:
+                finer = (self.n + (1 << (bits - 1)) - 1) >> (bits - 1)
+                if self.n * (finer + 1) * 2 > OFFSET_BYTES_PER_SYNAPSE * syn:
+                    break
+                bits, groups = bits - 1, finer
             fcap = (tiles + FIRED_LISTS - 1) // FIRED_LISTS * 256
-            b += self.n * (groups + 1) * 2 + 2 * FIRED_LISTS * (fcap + 32) * 4 + syn * GATHER_RECORD_BYTES
-        elif pull:
-            b += syn * PULL_BYTES_PER_SYNAPSE + (tiles + 1) * 8 + 4 * ((self.n + 63) // 64) * 8 + 16
+            return b + self.n * (groups + 1) * 2 + 2 * FIRED_LISTS * (fcap + 32) * 4 + syn * GATHER_RECORD_BYTES
+        if pull:
+            b += syn * PULL_BYTES_PER_SYNAPSE + (tiles + 1) * 8
+        if optional:
+            passes = (self.k + PASS_SYNAPSES - 1) // PASS_SYNAPSES
+            lists = 8 * FIRED_LISTS * ((tiles + FIRED_LISTS - 1) // FIRED_LISTS) * 256 * passes
+            offsets = 2 * self.n * (tiles + 1)
+            direct = (pull and self.n <= DIRECT_NEURONS and syn < 1 << 32 and offsets <= OFFSET_BYTES_PER_SYNAPSE * syn
+                      and (self.n * tiles <= 4 * syn or 1.0 - (1.0 - 1.0 / tiles) ** self.k >= 0.125))
+            b += max(lists + 2 * FIRED_LISTS * 32 * 4, offsets if direct else 0)
         return b
 
     def latency(self):
@@ -138,6 +161,9 @@ class Server:
     def close(self):
         self.engine.close()
 
+    def _bytes(self, r, optional=True):
+        return r.device_bytes(self.gather, self.pull, optional)
+
     def _admit(self, r):
         eng = self.engine
         inst = eng.add_fanout(r.n, r.k, r.net_seed, g_ui=r.g_ui, dt=self.dt, seed=r.seed)
@@ -169,9 +195,9 @@ class Server:
         which bounds the latency of the served ones (None: every request is
         served)."""
         for r in requests:
-            if r.device_bytes(self.gather, self.pull) > self.budget:
+            if self._bytes(r, optional=False) > self.budget:
                 raise ValueError("request %d needs %d bytes, more than the HBM budget"
-                                 % (r.rid, r.device_bytes(self.gather, self.pull)))
+                                 % (r.rid, self._bytes(r, optional=False)))
         pending = collections.deque(sorted(requests, key=lambda r: r.arrival))
         active = {}    # inst -> (request, block, remaining steps)
         used = 0
@@ -193,7 +219,7 @@ class Server:
                 while pending and clock - pending[0].arrival > shed_after:
                     pending.popleft().shed = True
             while (pending and not wait_retire and pending[0].arrival - offset <= now
-                   and used + pending[0].device_bytes(self.gather, self.pull) <= self.budget
+                   and (used + self._bytes(pending[0]) <= self.budget or not used)
                    and (max_resident is None or len(active) + len(joining) < max_resident)):
                 r = pending.popleft()
                 ta = time.monotonic()
@@ -212,7 +238,7 @@ class Server:
                 t_admit += time.monotonic() - ta
                 r.admitted = time.monotonic() - t0 + offset
                 joining[b.inst] = [r, b, r.steps]
-                used += r.device_bytes(self.gather, self.pull)
+                used += self._bytes(r)
 
         joining = {}   # admitted while a chunk runs: they step from the next chunk on
         while pending or active or joining:
@@ -256,7 +282,7 @@ class Server:
                 self._retire(r, b)
                 t_retire += time.monotonic() - ta
                 r.finished = time.monotonic() - t0 + offset
-                used -= r.device_bytes(self.gather, self.pull)
+                used -= self._bytes(r)
                 done_count += 1
                 wait_retire = False
         wall = time.monotonic() - t0
