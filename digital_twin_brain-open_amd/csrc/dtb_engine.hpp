@@ -733,7 +733,7 @@ private:
     // takes 7.0 ms, by queues and spill 2.2.)
     bool wants_direct(const Instance &p) const
     {
-        return (count_layout_ == kLayoutAuto || tuned_direct_) && !split_ && pull_on_ && queue_floor_ == kQueueFloorDefault &&
+        return (count_layout_ == kLayoutAuto || tuned_ == Tuned::automatic) && !split_ && pull_on_ && queue_floor_ == kQueueFloorDefault &&
                queue_shift_ == kQueueShiftDefault && defer_min_ == kDeferMinDefault && p.direct_allowed();
     }
     bool try_direct(Instance &p, hipStream_t s);   // builds p's tile offsets if they fit
@@ -753,7 +753,13 @@ private:
         direct_short_ = passes_short_ = false;
     }
     uint32_t nqueue_tiles_ = 0;            // tiles of queue and gather instances: all, or none
-    bool tuned_direct_ = false;            // the autotuner's (dense, default pass) candidate ran direct
+    // A schedule of the autotuner's: its (dense, default pass) candidate
+    // stands for the automatic choice among direct propagation, the binning
+    // launch and binning in the tiles; the other queue candidates are what
+    // they name, with the rows binned in the tiles (a binning launch knows no
+    // pass size, so they would all time the same kernels).
+    enum class Tuned { no, automatic, named };
+    Tuned tuned_ = Tuned::no;
     HostStage tables_stage_, call_stage_;
     // Everything a captured step's launches take from the engine: graphs stay
     // as long as it does (what changes from run to run is in the tables).

@@ -94,10 +94,10 @@ void Engine::set_schedule(uint32_t pass_k, int layout)
         throw Error(kInvalidParameter, "pass size must be 1, 2 or 4 synapses per lane");
     if (layout != kLayoutAuto && layout != kLayoutDense && layout != kLayoutSpread && layout != kLayoutGather)
         throw Error(kInvalidParameter, "unknown propagation layout");
-    if (pass_k != pass_k_ || layout != count_layout_ || tuned_direct_) {
+    if (pass_k != pass_k_ || layout != count_layout_ || tuned_ != Tuned::no) {
         pass_k_ = pass_k;
         count_layout_ = layout;
-        tuned_direct_ = false;
+        tuned_ = Tuned::no;
         routes_changed();   // graphs hold the old kernel; counts move to the new layout
     }
 }
@@ -148,7 +148,7 @@ bool Engine::want_direct()
     // an engine holds offsets or pass lists, not both (the old tables,
     // settled by the caller, were the last to use the lists)
     for (auto &p : insts_)
-        if (p && !devmem::NoAlloc::active())
+        if (p && !tuning_ && !devmem::NoAlloc::active())
             p->release_passes();
     for (auto &p : insts_) {
         if (!p)
@@ -174,7 +174,7 @@ bool Engine::want_bin_launch()
             segments += insts_[i]->row_coverage() * t * insts_[i]->n();
             synapses += (double)insts_[i]->nsyn();
         }
-    const bool want = !passes_short_ && tiles > 0 && (split_ || (tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
+    const bool want = !passes_short_ && tiles > 0 && (split_ || (tuned_ != Tuned::named && tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;
@@ -227,11 +227,13 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
     // buffers) the seventh turn runs the default schedule and is not a
     // candidate, so the number of steps does not depend on the networks.
     int nc = gather_possible() ? 7 : 6;
-    // The default pass with dense counts stands for the automatic layout:
-    // direct propagation for the instances that allow it.
     auto set_candidate = [&](int s) {
         set_schedule(ks[s], layouts[s]);
-        tuned_direct_ = layouts[s] == kLayoutDense && ks[s] == kPassKDefault;
+        const Tuned t = layouts[s] == kLayoutDense && ks[s] == kPassKDefault ? Tuned::automatic : Tuned::named;
+        if (t != tuned_) {
+            tuned_ = t;
+            routes_changed();
+        }
     };
     // The cost of a step follows the network's activity, which drifts and
     // bursts; so the schedules take turns in short windows (kAutotuneWindow
@@ -240,9 +242,10 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
     // loads every kernel variant (and builds the gather offsets).
     const int64_t rounds = (trial_steps + kAutotuneWindow - 1) / kAutotuneWindow;
     double t_sum[7] = {0, 0, 0, 0, 0, 0, 0};
-    // The gather buffers stay built between the gather turns (a table build
-    // would otherwise return them at every other turn and build them again);
-    // the first table build after the tuning returns them unless gather won.
+    // The gather buffers, tile offsets and pass lists stay built between their
+    // turns (a table build would otherwise return them at every other turn
+    // and build them again); the first table build after the tuning returns
+    // what the winner does not use.
     struct Tuning {
         bool &flag;
         explicit Tuning(bool &f) : flag(f) { flag = true; }
@@ -282,7 +285,7 @@ void Engine::autotune(int64_t trial_steps, uint32_t *best_k, int *best_layout, f
     const uint32_t bk = ks[bi];
     const int bl = layouts[bi];
     set_candidate(bi);
-    dirty_ = true;   // the next table build returns gather buffers no longer used
+    dirty_ = true;   // the next table build returns what is no longer used
     if (best_k)
         *best_k = bk;
     if (best_layout)
@@ -444,7 +447,7 @@ void Engine::rebuild()
         if (!dir && !tuning_)
             p->release_direct();   // (the old tables, settled above, were the last to use it)
         const bool passes = bin_launch && !gat;
-        if (!passes && !devmem::NoAlloc::active())
+        if (!passes && !tuning_ && !devmem::NoAlloc::active())
             p->release_passes();
         table.push_back(p->dev(tile_base_[slot], gat, dir, pl, defer_min_, passes));
         if (passes)

@@ -431,7 +431,9 @@ class Engine:
         all; they advance the simulation), and keeps the fastest; returns
         (pass_k, layout, mean us per step as {(layout, pass_k): us}); the
         gather schedule is a candidate (and in the table) only when some
-        instance allows it."""
+        instance allows it.  ("dense", 2) stands for the automatic choice of
+        the step (step_info); the other queue schedules bin rows in the tiles
+        that fired."""
         k, l = c_int32(0), c_int32(0)
         us = np.zeros(7, dtype=np.float32)
         _lib.check(self._lib.dtb_engine_autotune(self._h, int(trial_steps), byref(k), byref(l), _ptr(us)))

@@ -297,9 +297,10 @@ int dtb_engine_get_schedule(dtb_engine_t h, int32_t *pass_k, int32_t *layout, in
  * allows it; otherwise its turns run the default schedule, untimed for the
  * choice.  Steps run in all: 7 (2 + r (2 + 4)), r = ceil(trial_steps / 4).
  * us_per_step[7] (optional) = mean per schedule, [dense K=1, 2, 4, spread
- * K=1, 2, 4, gather] (gather 0 when not a candidate; dense K=2 runs, and if
- * chosen keeps, the automatic layout's direct propagation where an instance
- * allows it).  The steps advance the
+ * K=1, 2, 4, gather] (gather 0 when not a candidate).  dense K=2 runs, and if
+ * chosen keeps, the automatic choice: direct propagation or a binning launch
+ * where their rules take them; the other queue schedules bin rows in the
+ * tiles, unless split binning is on.  The steps advance the
  * simulation exactly as any other steps would; tune in the regime that will
  * be run (after the initial transient). */
 int dtb_engine_autotune(dtb_engine_t h, int64_t trial_steps, int32_t *pass_k, int32_t *layout, float *us_per_step);

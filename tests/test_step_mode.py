@@ -245,3 +245,29 @@ def test_offsets_built_when_an_instance_is_added(dtb, orc, gpu, n, k):
         assert_oracle(orc, net, b, 100, 3, 3.0)
     finally:
         eng.close()
+
+
+def test_autotuner_compares_the_binning_launch_with_binning_in_tiles(dtb, orc, gpu):
+    """3072 tiles of a voxel network, nearly silent: ("dense", 2) is the
+    binning launch, every other queue schedule bins in the tiles, and what is
+    kept is what was timed."""
+    net = dtb.gen_voxel(3072 * 256, 78, 220, seed=6)
+    steps = 30
+    eng = dtb.Engine(0)
+    try:
+        b = add(dtb, eng, net, 40, 9.0)
+        eng.run(steps)
+        assert eng.step_info()["mode"] == "bin_launch"
+        for _ in range(4):
+            k, layout, us = eng.autotune(16)
+            print(k, layout, us, flush=True)
+            eng.run(2)
+            steps += eng.autotune_steps(16) + 2
+            assert eng.step_info()["mode"] == ("gather" if layout == "gather" else
+                                               "bin_launch" if (layout, k) == ("dense", 2) else "tile_bin")
+        eng.schedule(layout="auto")
+        eng.run(2)
+        assert eng.step_info()["mode"] == "bin_launch"
+        assert b.counters()[0] == steps + 2
+    finally:
+        eng.close()
