@@ -1067,20 +1067,21 @@ struct Instance::StateStage {
     StateStage(HostStage &host, uint32_t count)
     {
         unsigned char *p = nullptr;
-        if (count * kPerNeuron <= kCallStageBytes) {
-            cap = count;
-            p = host.reserve(kCallStageBytes);
-        } else {
-            // at most 1M neurons (34 MB) at a time; fewer when memory is short
-            for (cap = std::min<uint32_t>(count, 1u << 20);; cap /= 2) {
-                try {
-                    p = base = static_cast<unsigned char *>(devmem::alloc((size_t)cap * kPerNeuron));
-                    break;
-                } catch (const Error &e) {
-                    if (e.code != kOutOfMemory || cap <= 256)
-                        throw;
-                }
+        constexpr uint32_t kHostNeurons = kCallStageBytes / kPerNeuron;
+        // at most 1M neurons (34 MB) at a time; fewer when memory is short,
+        // and in the end the pinned memory's
+        for (cap = std::min<uint32_t>(count, 1u << 20); cap > kHostNeurons && p == nullptr;) {
+            try {
+                p = base = static_cast<unsigned char *>(devmem::alloc((size_t)cap * kPerNeuron));
+            } catch (const Error &e) {
+                if (e.code != kOutOfMemory && !devmem::NoAlloc::active())
+                    throw;
+                cap /= 2;
             }
+        }
+        if (p == nullptr) {
+            cap = std::min(count, kHostNeurons);
+            p = host.reserve(kCallStageBytes);
         }
         a.J = reinterpret_cast<float4 *>(p);
         a.V = reinterpret_cast<float *>(p + (size_t)cap * 16);
@@ -1114,7 +1115,7 @@ void Instance::read_state(HostStage &stage, float *V, int32_t *t, uint8_t *f, ui
             DTB_HIP(hipStreamSynchronize(s));
         auto copy = [&](auto *dst, const auto *src, size_t per) {
             if (dst != nullptr && st.base == nullptr)
-                std::memcpy(dst, src, m * per * sizeof(*dst));
+                std::memcpy(dst + (size_t)b * per, src, m * per * sizeof(*dst));
             else if (dst != nullptr)
                 DTB_HIP(hipMemcpyAsync(dst + (size_t)b * per, src, m * per * sizeof(*dst), hipMemcpyDeviceToHost, s));
         };
@@ -1145,7 +1146,7 @@ void Instance::write_state(HostStage &stage, const float *V, const int32_t *t, c
         const size_t m = std::min(st.cap, n_ - b);
         auto copy = [&](auto *dst, const auto *src, size_t per) {
             if (src != nullptr && st.base == nullptr)
-                std::memcpy(dst, src, m * per * sizeof(*src));
+                std::memcpy(dst, src + (size_t)b * per, m * per * sizeof(*src));
             else if (src != nullptr)
                 DTB_HIP(hipMemcpyAsync(dst, src + (size_t)b * per, m * per * sizeof(*src), hipMemcpyHostToDevice, s));
         };
@@ -1155,6 +1156,8 @@ void Instance::write_state(HostStage &stage, const float *V, const int32_t *t, c
         copy(a.iou, iou, 1);
         copy(reinterpret_cast<float *>(a.J), J, 4);
         DTB_HIP(launch_write_state(state_view(), b, (uint32_t)m, a, s));
+        if (st.base == nullptr)
+            DTB_HIP(hipStreamSynchronize(s));   // the next neurons go into the same memory
     }
     DTB_HIP(hipStreamSynchronize(s));
 }
