@@ -894,6 +894,18 @@ void Instance::begin_record(int64_t step0, int64_t steps, bool freq, bool sample
     rec_freq_ = freq;
     rec_samples_ = samples;
     rec_stat_mask_ = stat_mask;
+    // The samples first: the sums' slots can do with less.
+    auto take_samples = [&] {
+        const size_t m = (size_t)steps * samples_.size();
+        rec_spike_.resize(m);
+        rec_v_.resize(m);
+        rec_isyn_.resize(m);
+        rec_iou_.resize(m);
+        rec_spike_.mutable_gpu_data();
+        rec_v_.mutable_gpu_data();
+        rec_isyn_.mutable_gpu_data();
+        rec_iou_.mutable_gpu_data();
+    };
     auto allocate = [&](bool slots) {
         layout_record(steps, freq, stat_mask != 0, slots);
         if (stat_mask != 0) {
@@ -906,27 +918,34 @@ void Instance::begin_record(int64_t step0, int64_t steps, bool freq, bool sample
         }
     };
     try {
-        allocate(true);
-    } catch (const Error &e) {
-        // no device memory for the slots: one per row, as without them
-        if (e.code != kOutOfMemory || rec_slots_ == 1)
-            throw;
-        allocate(false);
+        if (samples) {
+            try {
+                take_samples();
+            } catch (const Error &e) {
+                if (e.code != kOutOfMemory)
+                    throw;
+                rec_stat_.resize(0);   // an earlier record's slots
+                rec_counts_.resize(0);
+                take_samples();
+            }
+        }
+        try {
+            allocate(true);
+        } catch (const Error &e) {
+            // no device memory for the slots: one per row, as without them
+            if (e.code != kOutOfMemory || rec_slots_ == 1)
+                throw;
+            allocate(false);
+        }
+    } catch (...) {
+        end_record();   // no step may write a record whose buffers are not there
+        throw;
     }
-    const CopyWords clear[2] = {{rec_stat_.mutable_gpu_data(), nullptr, stat_mask != 0 ? rec_stat_.size() / 4 : 0},
-                                {rec_counts_.mutable_gpu_data(), nullptr, freq ? rec_counts_.size() / 4 : 0}};
+    const CopyWords clear[2] = {{stat_mask != 0 ? rec_stat_.mutable_gpu_data() : nullptr, nullptr,
+                                 stat_mask != 0 ? rec_stat_.size() / 4 : 0},
+                                {freq ? rec_counts_.mutable_gpu_data() : nullptr, nullptr,
+                                 freq ? rec_counts_.size() / 4 : 0}};
     DTB_HIP(launch_copy_words(clear, 2, s));
-    if (samples) {
-        const size_t m = (size_t)steps * samples_.size();
-        rec_spike_.resize(m);
-        rec_v_.resize(m);
-        rec_isyn_.resize(m);
-        rec_iou_.resize(m);
-        rec_spike_.mutable_gpu_data();
-        rec_v_.mutable_gpu_data();
-        rec_isyn_.mutable_gpu_data();
-        rec_iou_.mutable_gpu_data();
-    }
 }
 
 void Instance::begin_record_at(int64_t steps, bool freq, bool samples, uint32_t stat_mask, const RecordBuffers &b,

@@ -57,3 +57,76 @@ def test_gather_takes_larger_groups(dtb, gpu, limit):
     assert got[0][0] == got[1][0] and got[0][0][2] > 1000
     for key in ("V", "J", "i_ou"):
         assert np.array_equal(bits(got[0][1][key]), bits(got[1][1][key])), key
+
+
+@pytest.mark.parametrize("earlier", [False, True])
+def test_samples_come_before_the_slots_of_the_sums(dtb, gpu, limit, earlier):
+    """2000 rows of 10,000 samples (260 MB) fit with 16 MB to spare; the
+    population sums' slots (33 MB), or those an earlier record left, must not
+    take them first."""
+    n, steps = 1 << 18, 2000
+    ids = np.arange(0, n, 26, dtype=np.uint32)[:10_000]
+    kw = dict(freqs=True, vmean=True, output_sample_spike=True, output_sample_vmemb=True, output_sample_isynaptic=True,
+              output_sample_iou=True)
+
+    def block(eng):
+        b = dtb.Block(None, delta_t=0.1, engine=eng, inst=eng.add_fanout(n, 20, 5, seed=3))
+        b.update_ou_background_stimuli(b.subblk_id, 4.0, 5.0, 0.1)
+        b.set_samples(ids)
+        b.run(1, freqs=True)
+        return b
+
+    limit(block, 13 * steps * ids.size + (16 << 20))
+    eng = dtb.Engine(0)
+    try:
+        b = block(eng)
+        if earlier:
+            b.run(1000, freqs=True, vmean=True)
+        got = b.run(steps, **kw)
+    finally:
+        eng.close()
+    dtb.device_memory_trim()
+    eng = dtb.Engine(0)
+    try:
+        b = block(eng)
+        if earlier:
+            b.run(1000, freqs=True, vmean=True)
+        parts = [b.run(steps // 4, **kw) for _ in range(4)]
+    finally:
+        eng.close()
+    assert got["freq"].sum() > 1000
+    for key in ("freq", "vmean", "spike", "vmemb", "isynaptic", "iou"):
+        want = np.concatenate([p[key] for p in parts])
+        assert np.array_equal(bits(got[key]) if want.dtype == np.float32 else got[key],
+                              bits(want) if want.dtype == np.float32 else want), key
+
+
+def test_a_run_refused_for_its_record_leaves_none(dtb, gpu, limit):
+    """A recorded run whose samples do not fit is refused; the steps after it
+    record nothing, and a smaller record works."""
+    n = 1 << 18
+    ids = np.arange(0, n, 26, dtype=np.uint32)[:10_000]
+
+    def block(eng):
+        b = dtb.Block(None, delta_t=0.1, engine=eng, inst=eng.add_fanout(n, 20, 5, seed=3))
+        b.update_ou_background_stimuli(b.subblk_id, 4.0, 5.0, 0.1)
+        b.set_samples(ids)
+        b.run(10, freqs=True)
+        return b
+
+    limit(block, 64 << 20)
+    got = []
+    for refused in (True, False):
+        eng = dtb.Engine(0)
+        try:
+            b = block(eng)
+            if refused:
+                with pytest.raises(dtb.DtbError) as e:
+                    b.run(4000, freqs=True, output_sample_vmemb=True)
+                assert e.value.status == 101   # OUT_OF_MEMORY
+            eng.run(100)
+            got.append((b.run(60, freqs=True)["freq"], b.counters(), b.state()["V"]))
+        finally:
+            eng.close()
+    assert got[0][0].sum() > 100 and np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+    assert np.array_equal(bits(got[0][2]), bits(got[1][2]))
