@@ -9,8 +9,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <exception>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <unordered_set>
@@ -18,6 +16,7 @@
 #include "dtb_devgen.hpp"
 #include "dtb_gen.hpp"
 #include "dtb_kernels.hpp"
+#include "dtb_parts.hpp"
 
 namespace dtb {
 
@@ -514,47 +513,6 @@ struct ParamRecEq {
     bool operator()(const ParamRec &x, const ParamRec &y) const { return same_bits(x, y); }
 };
 
-}  // namespace
-
-namespace {
-// Threads for a pass over n neurons' property rows (88 bytes each, so one
-// thread waits for memory): 200k neurons' parameters re-derived took 1.1 ms
-// on one thread.
-uint32_t host_parts(uint32_t n)
-{
-    const uint32_t hw = std::thread::hardware_concurrency();
-    return std::max(1u, std::min({hw ? hw : 4u, 8u, n / 16384u}));
-}
-
-// f(0) .. f(parts - 1), each on a thread of its own; rethrows the first error.
-template <typename F>
-void for_parts(uint32_t parts, F &&f)
-{
-    std::vector<std::exception_ptr> err(parts);
-    std::vector<std::thread> th;
-    auto run = [&](uint32_t k) {
-        try {
-            f(k);
-        } catch (...) {
-            err[k] = std::current_exception();
-        }
-    };
-    uint32_t k = 1;
-    try {
-        for (; k < parts; ++k)
-            th.emplace_back(run, k);
-    } catch (const std::system_error &) {
-        // no more threads: this one does the rest
-    }
-    for (; k < parts; ++k)
-        run(k);
-    run(0);
-    for (auto &t : th)
-        t.join();
-    for (auto &e : err)
-        if (e)
-            std::rethrow_exception(e);
-}
 }  // namespace
 
 void Instance::derive_params(hipStream_t s)
