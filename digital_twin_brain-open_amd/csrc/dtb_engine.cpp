@@ -1165,8 +1165,8 @@ InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, u
         d.passcap = passcap_;
     }
     if (direct) {
-        if (!direct_built() || gather)
-            throw Error(kInternal, "direct propagation needs the tile offsets and no gather");
+        if (!direct_built() || gather || !pull)
+            throw Error(kInternal, "direct propagation needs the tile offsets, the in-edges and no gather");
         d.tidx = tidx_.gpu_data();
     }
     if (pull) {
@@ -1244,7 +1244,6 @@ TileDesc Instance::tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, 
     r.pop0 = pop0;
     r.ntiles = d.ntiles;
     r.flags = (d.use_ou ? kTileOu : 0u) | (d.crec ? kTilePull : 0u) | (d.segidx ? kTileGather : 0u) |
-              (d.tidx ? kTileDirect : 0u) |
               (d.t_steps == 1 ? kTileOneSub : 0u) | (d.rec_stat ? kTileStat : 0u);
     if (tile_cls_[t] != 0u) {
         r.flags |= kTileUniform;

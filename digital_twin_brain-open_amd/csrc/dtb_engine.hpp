@@ -623,10 +623,7 @@ public:
     // How the tables of the last build step (gathers(): some of their
     // instances gather), and how often an instance's tile offsets or pass
     // lists were built.
-    StepMode step_mode() const
-    {
-        return nqueue_tiles_ < ntiles_ ? StepMode::direct : nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin;
-    }
+    StepMode step_mode() const { return mode_; }
     bool gathers() const { return ngroups_ > 0; }
     uint64_t tables_built() const { return tables_built_; }
     // Queue capacity per tile: min(synapses targeting it, floor +
@@ -683,7 +680,7 @@ public:
 private:
     void rebuild();
     void launch_step();        // one step at parity par_, then par_ ^= 1
-    void launch_step_k(hipEvent_t *ev = nullptr);   // ev: 8 events (start and stop of up to four kernels)
+    void launch_step_k(hipEvent_t *ev = nullptr);   // ev: 6 events (start and stop of up to three kernels)
     void launch_aux();         // materialize + sample after a step, if samples are set
     void drop_graphs();
     QueueSet queues();
@@ -752,7 +749,7 @@ private:
         dirty_ = true;
         direct_short_ = passes_short_ = false;
     }
-    uint32_t nqueue_tiles_ = 0;            // tiles of queue and gather instances: all, or none
+    StepMode mode_ = StepMode::tile_bin;   // of every tile in the tables
     // A schedule of the autotuner's: its (dense, default pass) candidate
     // stands for the automatic choice among direct propagation, the binning
     // launch and binning in the tiles; the other queue candidates are what
@@ -765,7 +762,7 @@ private:
     // as long as it does (what changes from run to run is in the tables).
     struct GraphKey {
         const void *tiles, *insts, *queues, *qtiles, *qcnt, *bins, *groups, *samples, *recs;
-        uint32_t ntiles, nqueue_tiles, nbins, bin_tiles, ngroups, nsamples, cshift, pass_k, wfmt, stat;
+        uint32_t ntiles, mode, nbins, bin_tiles, ngroups, nsamples, cshift, pass_k, wfmt, stat;
     };
     GraphKey graph_key_{};
     hipGraphExec_t graph_[2] = {nullptr, nullptr};   // by starting parity

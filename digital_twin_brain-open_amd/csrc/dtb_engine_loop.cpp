@@ -480,7 +480,6 @@ void Engine::rebuild()
     }
     if (total > 0xffffffffull || tiles.size() > 0xffffffffull)
         throw Error(kInvalidParameter, "too many neurons in one engine");
-    nqueue_tiles_ = dir ? 0u : (uint32_t)tiles.size();
     // Workgroups are dealt to the 8 XCDs by index mod 8: each XCD gets a
     // contiguous range of the direct tiles, so tiles that share cache lines
     // of a row's offsets and synapses meet in one L2.
@@ -522,6 +521,7 @@ void Engine::rebuild()
         cshift_ = (total > 0 && coverage / (double)total > kSpreadCoverage) ? kCountShiftSpread : kCountShiftDense;
     grow(d_qcnt_, count_words(2 * std::max<size_t>(tiles.size(), 1), cshift_));
     nbins_ = (uint32_t)bins.size();
+    mode_ = dir && ntiles_ > 0 ? StepMode::direct : nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin;
     grow(d_bins_, bins.size());
     d_bins_.mutable_gpu_data();
     // Allocate (zero-filled) everything the step kernels touch before any
@@ -571,7 +571,7 @@ void Engine::rebuild()
     key.samples = d_samples_.gpu_data();
     key.recs = d_recs_.gpu_data();
     key.ntiles = ntiles_;
-    key.nqueue_tiles = nqueue_tiles_;
+    key.mode = (uint32_t)mode_;
     key.nbins = nbins_;
     key.bin_tiles = bin_tiles_;
     key.ngroups = ngroups_;
@@ -598,12 +598,10 @@ void Engine::launch_step_k(hipEvent_t *ev)
     // start and stop events of the i-th kernel, or none
     auto e = [&](int i) { return ev ? ev[i] : nullptr; };
     DTB_HIP(launch_gather(d_groups_.gpu_data(), ngroups_, d_insts_.gpu_data(), par_, wfmt_, e(0), e(1), stream_));
-    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), nqueue_tiles_, nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin,
-                               pass_k_, d_queues_.gpu_data(), par_, wfmt_, stat_, e(2), e(3), stream_));
+    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data(), ntiles_, mode_, pass_k_, d_queues_.gpu_data(), par_, wfmt_, stat_,
+                               e(2), e(3), stream_));
     DTB_HIP(launch_bin_kernel(d_bins_.gpu_data(), nbins_, bin_tiles_, d_queues_.gpu_data(), par_, wfmt_, e(4), e(5),
                               stream_));
-    DTB_HIP(launch_step_kernel(d_tiles_.gpu_data() + nqueue_tiles_, ntiles_ - nqueue_tiles_, StepMode::direct, pass_k_,
-                               d_queues_.gpu_data(), par_, wfmt_, stat_, e(6), e(7), stream_));
 }
 
 void Engine::launch_aux()
@@ -746,35 +744,31 @@ void Engine::run_timed(int64_t steps, float *ms_step)
     if (ninst_ == 0 || steps <= 0)
         return;
     pending_ = true;
-    // Every kernel of a step (k_gather, k_step over the queue and gather
-    // tiles, k_bin, k_step over the direct tiles: those with a grid) records
-    // its own start and stop events at the dispatch boundaries, on the engine
-    // stream; they are read back once per chunk so the launch pipeline is not
-    // drained every step.
-    const uint32_t grid[4] = {ngroups_, nqueue_tiles_, nbins_, ntiles_ - nqueue_tiles_};
-    int last = 0;
-    for (int i = 0; i < 4; ++i)
-        if (grid[i] > 0)
-            last = i;
+    // Every kernel of a step (k_gather, k_step, k_bin: those with a grid)
+    // records its own start and stop events at the dispatch boundaries, on
+    // the engine stream; they are read back once per chunk so the launch
+    // pipeline is not drained every step.
+    const uint32_t grid[3] = {ngroups_, ntiles_, nbins_};
+    const int last = nbins_ > 0 ? 2 : 1;
     const int64_t chunk = 256;
-    std::vector<hipEvent_t> ev((size_t)(8 * chunk));
+    std::vector<hipEvent_t> ev((size_t)(6 * chunk));
     for (auto &e : ev)
         DTB_HIP(hipEventCreate(&e));
     double ts = 0.0;
     for (int64_t base = 0; base < steps; base += chunk) {
         const int64_t m = std::min<int64_t>(chunk, steps - base);
         for (int64_t k = 0; k < m; ++k) {
-            launch_step_k(&ev[(size_t)(8 * k)]);
+            launch_step_k(&ev[(size_t)(6 * k)]);
             par_ ^= 1u;
             launch_aux();
         }
-        DTB_HIP(hipEventSynchronize(ev[(size_t)(8 * (m - 1) + 2 * last + 1)]));
+        DTB_HIP(hipEventSynchronize(ev[(size_t)(6 * (m - 1) + 2 * last + 1)]));
         for (int64_t k = 0; k < m; ++k)
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < 3; ++i) {
                 if (grid[i] == 0)
                     continue;
                 float a = 0.0f;
-                DTB_HIP(hipEventElapsedTime(&a, ev[(size_t)(8 * k + 2 * i)], ev[(size_t)(8 * k + 2 * i + 1)]));
+                DTB_HIP(hipEventElapsedTime(&a, ev[(size_t)(6 * k + 2 * i)], ev[(size_t)(6 * k + 2 * i + 1)]));
                 ts += a;
             }
     }

@@ -588,12 +588,10 @@ __device__ __forceinline__ bool direct_tile(unsigned long long *acc, DirectList 
     // segment a line of columns and one of weights per few synapses; the
     // in-edges are one stream (a volley step of 200k x 150 pulls in 110-146
     // us, with every row in rounds 7 ms).
-    if (I.crec != nullptr) {
-        const uint64_t in_edges = (uint64_t)(gp(I.cptr)[t + 1] - gp(I.cptr)[t]);
-        if ((uint64_t)n * (64u * (uint64_t)I.n + 24u * in_edges) > 12u * in_edges * (uint64_t)I.n) {
-            pull_tile<kFmt>(acc, I, set, t, true, tid);
-            return true;
-        }
+    const uint64_t in_edges = (uint64_t)(gp(I.cptr)[t + 1] - gp(I.cptr)[t]);
+    if ((uint64_t)n * (64u * (uint64_t)I.n + 24u * in_edges) > 12u * in_edges * (uint64_t)I.n) {
+        pull_tile<kFmt>(acc, I, set, t, true, tid);
+        return true;
     }
     // ranks: rows of the threads before, then a thread's own in tile order
     const uint32_t lane = tid & (kWave - 1u), w = tid / kWave;

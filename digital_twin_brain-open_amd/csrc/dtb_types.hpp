@@ -263,7 +263,6 @@ constexpr uint32_t kTilePull = 16u;      // pull propagation
 constexpr uint32_t kTileGather = 32u;    // gather propagation
 constexpr uint32_t kTileOneSub = 64u;    // one substep per step
 constexpr uint32_t kTileStat = 128u;     // population statistics are recorded
-constexpr uint32_t kTileDirect = 256u;   // direct propagation
 struct alignas(128) TileDesc {
     unsigned char *state;    // the tile's state block
     const QSyn *queue;       // its queue of set 0
