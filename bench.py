@@ -8,9 +8,10 @@ the voxel, 30% from a sparse lognormal voxel-to-voxel matrix at 5% density),
 (mean 5.0, sigma 0.1, tau 4 ms, about 10 Hz), one parameter record per
 population (400).  Synthetic, seeded.
 
-A step is one launch of the step kernel (delta accumulation, neuron update
-and spike binning) over the whole block with the network resident in HBM;
-the timed steps are replayed from HIP graphs of 100 steps, as a run does.
+A step is one or two launches (delta accumulation and neuron update; spike
+binning in the same launch or in one of its own, as the engine's rules take
+it) over the whole block with the network resident in HBM; the timed steps are
+replayed from HIP graphs of 100 steps, as a run does.
 Prints one JSON line.
 
 The line also carries "ensemble": the data-assimilation ensemble (64
@@ -26,9 +27,11 @@ same 100 requests are also served as a backlog (all waiting at the start)
 for the server's capacity.
 """
 import argparse
+import hashlib
 import importlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -51,8 +54,9 @@ AUTOTUNE_STEPS = 7 * (2 + (AUTOTUNE_TRIAL + 3) // 4 * 6)   # Engine.autotune_ste
 # rocprofv3 FETCH_SIZE + WRITE_SIZE per launch, scaled by a device-copy
 # calibration, of profiled runs: each summary names its window (workload,
 # neurons, propagation layout, timed steps, warm-up steps, whether the
-# autotuner ran) and is used only for a run of exactly that window.
-PROFILES = ("k_step_voxel2M_in500.md", "k_step_voxel2M_in500_steps20_warmup5.md",
+# autotuner ran), its kernels and the device code that ran, and is used only
+# for a run of exactly that window with those kernels from the same code.
+PROFILES = ("k_step_voxel2M_in500.md", "k_step_voxel2M_in500_steps20_warmup5.md", "k_step_direct_voxel200k_in500.md",
             "k_gather_k_step_uniform500k_in5000.md")
 
 # Algorithmic HBM bytes of one step, as the step is defined on per-neuron
@@ -75,26 +79,57 @@ LAYOUT_SYN_BYTES = 12 + 2 * 12
 # With gather propagation (k_gather, then k_step): per neuron the delta
 # (16 B) is written by k_gather and read by k_step; per fired row 16 B (row
 # offset, fired-list entry written and read) and its two 2-byte offsets for
-# each group of 2048 neurons; per delivered synapse 12 B (column index +
-# weight pair, no queue).
+# each target group; per delivered synapse 12 B (column index + weight pair,
+# no queue).
 GATHER_NEURON_BYTES = LAYOUT_NEURON_BYTES + 2 * 16
 GATHER_ROW_BYTES, GATHER_ROW_GROUP_BYTES = 16, 4
 GATHER_SYN_BYTES = 12
+# With direct propagation: per fired row 16 B and its two 2-byte offsets for
+# each tile of 256 neurons; per delivered synapse 12 B.
+DIRECT_ROW_TILE_BYTES, DIRECT_SYN_BYTES = 4, 12
+
+# The kernels of a step by Engine.step_info()["mode"].
+STEP_KERNELS = {"tile_bin": "k_step", "bin_launch": "k_step+k_bin", "direct": "k_step (direct)",
+                "gather": "k_gather+k_step"}
 
 
-def profiled_traffic(workload, neurons, layout, steps, warmup, autotuned):
-    """(HBM bytes per launch measured with rocprofv3 counters over exactly
-    this window (workload, size, layout, timed and warm-up steps, whether the
-    autotuner ran), the summary that holds it), or (None, None)."""
-    want = "window: workload=%s neurons=%d layout=%s steps=%d warmup=%d autotuned=%d" % (
-        workload, neurons, layout, steps, warmup, int(autotuned))
+def gather_groups(n):
+    """Target groups of k_gather: of 2048 neurons, or fewer (not below 256)
+    while there are less than 128."""
+    bits = 11
+    while bits > 8 and -(-n >> bits) < 128:
+        bits -= 1
+    return -(-n >> bits)
+
+
+def device_source():
+    """Hash of the device code (comments and white space left out)."""
+    h = hashlib.sha256()
+    for name in ("dtb_kernels.hip", "dtb_types.hpp", "dtb_rng.hpp"):
+        with open(os.path.join(ROOT, "digital_twin_brain-open_amd", "csrc", name)) as f:
+            text = re.sub(r"//[^\n]*|/\*.*?\*/", "", f.read(), flags=re.S)
+        h.update("".join(text.split()).encode())
+    return h.hexdigest()[:16]
+
+
+def profiled_traffic(workload, neurons, layout, steps, warmup, autotuned, kernel=None, source=None):
+    """(HBM bytes per step measured with rocprofv3 counters over exactly this
+    window (workload, size, layout, timed and warm-up steps, whether the
+    autotuner ran), the summary that holds it), or (None, None).  kernel,
+    source: only of these kernels (STEP_KERNELS) and this device code."""
+    want = ["window: workload=%s neurons=%d layout=%s steps=%d warmup=%d autotuned=%d" % (
+        workload, neurons, layout, steps, warmup, int(autotuned))]
+    if kernel is not None:
+        want.append("kernels: " + kernel)
+    if source is not None:
+        want.append("device_source: " + source)
     for name in PROFILES:
         path = os.path.join(ROOT, "profiles", name)
         if not os.path.exists(path):
             continue
         with open(path) as f:
             lines = [x.strip() for x in f]
-        if want not in lines:
+        if any(w not in lines for w in want):
             continue
         for line in lines:
             if line.startswith("traffic_bytes_per_launch:"):
@@ -371,7 +406,8 @@ def main():
         eng.run(args.warmup, graph_chunk=GRAPH_CHUNK)
     eng.sync()
     pk, _, layout_used = eng.schedule()
-    schedule = {"pass_synapses": 64 * pk, "count_layout": layout_used, "autotuned": bool(k_best),
+    mode = eng.step_info()["mode"]
+    schedule = {"pass_synapses": 64 * pk, "count_layout": layout_used, "step": mode, "autotuned": bool(k_best),
                 "trial_us_per_step": {"%s/%d" % (lay, 64 * kk): round(us, 2) for (lay, kk), us in table.items()}}
     step0, ev0, sp0 = eng.counters(blk.inst)
     prop0 = eng.propagation_stats()
@@ -404,20 +440,22 @@ def main():
     wpair = net.w.dtype.itemsize * 2
     syn_bytes = ALGO_SYN_BYTES - 8 + wpair
     algo_bytes = ALGO_NEURON_BYTES * net.n + ALGO_ROW_BYTES * sp_step + syn_bytes * ev_step
-    gather = layout_used == "gather"
-    if gather:
-        ngroups = (net.n + 2047) // 2048
-        layout_bytes = (GATHER_NEURON_BYTES * net.n + (GATHER_ROW_BYTES + GATHER_ROW_GROUP_BYTES * ngroups) * sp_step
+    if mode == "gather":
+        layout_bytes = (GATHER_NEURON_BYTES * net.n
+                        + (GATHER_ROW_BYTES + GATHER_ROW_GROUP_BYTES * gather_groups(net.n)) * sp_step
                         + (GATHER_SYN_BYTES - 8 + wpair) * ev_step)
+    elif mode == "direct":
+        layout_bytes = (LAYOUT_NEURON_BYTES * net.n
+                        + (LAYOUT_ROW_BYTES + DIRECT_ROW_TILE_BYTES * -(-net.n // 256)) * sp_step
+                        + (DIRECT_SYN_BYTES - 8 + wpair) * ev_step)
     else:
         layout_bytes = (LAYOUT_NEURON_BYTES * net.n + LAYOUT_ROW_BYTES * sp_step
                         + (LAYOUT_SYN_BYTES - 8 + wpair) * ev_step)
-    # engines of 3072 queue tiles or more bin in a launch of their own
-    bin_launch = args.split or (net.n + 255) // 256 >= 3072
-    kname = "k_gather+k_step" if gather else ("k_step+k_bin" if bin_launch else "k_step")
+    kname = STEP_KERNELS[mode]
     achieved = algo_bytes / (us * 1e-6) / 1e9
     traffic, traffic_src = (profiled_traffic(args.workload, args.neurons, layout_used, args.steps, args.warmup,
-                                             bool(k_best)) if args.weights == "float32" else (None, None))
+                                             bool(k_best), kname, device_source())
+                            if args.weights == "float32" else (None, None))
     eager = args.steps < GRAPH_CHUNK
 
     res = {
