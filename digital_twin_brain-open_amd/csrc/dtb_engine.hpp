@@ -386,8 +386,6 @@ public:
     // Synapses whose target lies in tile `tile` (2^kTileBits neurons): the
     // exact queue bound of the binning.
     uint32_t tile_synapses(uint32_t tile) const;
-    // 1 + the parameter class of every neuron of tile `tile` if they share
-    // one, else 0.
     // Zeroes both spill accumulators (the queues of this instance were
     // cleared).
     void clear_spill(hipStream_t s);
@@ -395,7 +393,6 @@ public:
     // contents need no initialisation: only the first `count` entries of a
     // tile's queue are ever read).
     void ensure_queue(uint64_t slots);
-    uint32_t tile_class(uint32_t tile) const { return tile_cls_.at(tile); }
     // Mean over rows of the fraction of this instance's tiles that the row's
     // synapses reach (tile segments of the row / tiles).
     double row_coverage() const { return row_coverage_; }
@@ -438,7 +435,7 @@ public:
     CopyWords deferred_words();   // the same as a launch_copy_words segment
     const int64_t *step_words() { return step_.gpu_data(); }   // [2], the larger one is the step index
 
-    // Direct propagation: possible when every row is ordered by target and at
+    // Direct propagation: possible when every row is ordered by tile and at
     // most kGatherMaxRow long, the instance has at most kDirectMaxNeurons
     // neurons, the tile offsets ([n][ntiles + 1] x 2 bytes) are no larger
     // than the synapse arrays and a row has enough synapses for its lookups.
@@ -499,8 +496,9 @@ private:
     DataAllocator<int64_t> step_;
     static constexpr size_t kStepPad = 16;
     DataAllocator<unsigned long long> counters_;   // per wave: events, spikes
-    // [steps][rec_slots_][stride], with more than one slot followed by the
-    // rows of the slots' sums ([npop], [npop][kStatFields])
+    // Records of the run, [steps][rec_slots_][stride]: counts per population,
+    // and its sums ([npop][kStatFields]); the slots of a row are added up
+    // when it is fetched.
     DataAllocator<uint32_t> rec_counts_;
     DataAllocator<long long> rec_stat_;
     size_t count_slots() const { return (size_t)rec_len_ * rec_slots_ * rec_cstride_; }

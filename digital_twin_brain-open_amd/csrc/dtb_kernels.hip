@@ -641,7 +641,7 @@ __device__ __forceinline__ float4 receptor_currents(const float4 g, const float4
 // Atomics on one 128-byte line are served one after the other (about 8 ns
 // each: a block of two populations and 469 tiles took 97 us per step with
 // one line per step, 9 us without statistics), so a record has rec_slots
-// slots of whole lines, a tile adding into slot (tile % slots); k_fold_slots
+// slots of whole lines, a tile adding into slot (tile % slots); k_fetch_rows
 // adds the slots up when the record is fetched.
 template <typename Inst>
 __device__ __forceinline__ uint32_t *rec_count_row(const Inst &I, int64_t row, uint32_t begin)

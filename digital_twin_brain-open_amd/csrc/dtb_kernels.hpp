@@ -32,12 +32,12 @@ hipError_t launch_bin_kernel(const BinDesc *groups, uint32_t ngroups, uint32_t m
 hipError_t launch_gather(const GroupDesc *groups, uint32_t ngroups, const InstDev *insts, uint32_t par, uint32_t wfmt,
                          hipEvent_t start, hipEvent_t stop, hipStream_t stream);
 
-// Offsets per target group of 2^shift neurons ([n][ngroups + 1], rows ordered
-// by target group).
 // Gather records ([nsyn][grec_words(wfmt)]: column, weight pair bits).
 hipError_t launch_build_grec(const uint32_t *col, const void *w, uint32_t wfmt, uint64_t nsyn, uint32_t *rec,
                              hipStream_t stream);
 
+// Offsets per target group of 2^shift neurons ([n][ngroups + 1], rows ordered
+// by target group; tiles: shift kTileBits).
 hipError_t launch_build_segidx(const int64_t *rowptr, const uint32_t *col, uint32_t n, uint32_t ngroups,
                                uint32_t shift, uint16_t *segidx, hipStream_t stream);
 
