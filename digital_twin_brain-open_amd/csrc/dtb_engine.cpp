@@ -1224,7 +1224,7 @@ InstDev Instance::dev(uint32_t tile_base, bool gather, bool direct, bool pull, u
 }
 
 TileDesc Instance::tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, uint32_t idx, uint32_t pop0,
-                             uint64_t qoff, uint32_t qcap) const
+                             uint64_t qoff, uint32_t qcap)
 {
     TileDesc r{};
     r.begin = t * kBlock;
@@ -1255,8 +1255,10 @@ TileDesc Instance::tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, 
         r.flags |= kTileOnePop;
         if (d.use_ou && ou_on_[pop0]) {
             r.flags |= kTileOuOn;
-            ou_factors(dt_ / (float)t_steps_, ou_tau_[pop0], ou_sigma_[pop0], &r.f1, &r.f2s);
-            r.mu = ou_mean_[pop0];
+            const PopDev &pop = pops_.cpu_data()[pop0];
+            r.f1 = pop.f1;
+            r.f2s = pop.f2s;
+            r.mu = pop.mu;
         }
     }
     return r;

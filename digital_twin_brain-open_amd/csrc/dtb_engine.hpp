@@ -379,7 +379,7 @@ public:
     // the instance's descriptor `d`, idx its index; pop0: population of the
     // tile's first neuron; qoff, qcap: its queue.
     TileDesc tile_desc(uint32_t t, const InstDev &d, const InstDev *inst, uint32_t idx, uint32_t pop0, uint64_t qoff,
-                       uint32_t qcap) const;
+                       uint32_t qcap);
     // Distinct parameter records (classes); n() when stored per neuron.
     uint32_t param_classes() const { return (uint32_t)prm_.count(); }
     SampleRecDev sample_rec();

@@ -376,19 +376,40 @@ QueueSet Engine::queues()
     return q;
 }
 
+namespace {
+// Workgroups of k_bin for an instance of nt tiles.
+uint32_t bin_parts(uint32_t nt)
+{
+    return std::min(kBinGroups, (nt + kBinTiles - 1) / kBinTiles);
+}
+
+// Place in the launch of direct tile j of n.  Workgroups are dealt to the 8
+// XCDs by index mod 8: each XCD gets a contiguous range of the tiles, so tiles
+// that share cache lines of a row's offsets and synapses meet in one L2.
+size_t dealt(size_t j, size_t n)
+{
+    const size_t q = n >> 3, r = n & 7u;   // the first r ranges have q + 1 tiles
+    const size_t x = j < r * (q + 1) ? j / (q + 1) : r + (j - r * (q + 1)) / q;
+    return (j - (x * q + std::min(x, r))) * 8 + x;
+}
+}  // namespace
+
 void Engine::rebuild()
 {
     settle();   // the queues are reallocated below; nothing pending may be lost
     DTB_HIP(hipStreamSynchronize(stream_));   // the last tables have left their staging memory
     staged_.clear();
     std::vector<InstDev> table;
-    std::vector<TileDesc> tiles;
-    std::vector<QueueTile> qtiles;
-    size_t ninst = 0, ntile_all = 0;
+    size_t ninst = 0, ntile = 0, sample_set = 0, group_max = 0, bin_max = 0;
     for (auto &p : insts_)
         if (p) {
+            const uint32_t nt = (p->n() + kBlock - 1) / kBlock;
             ++ninst;
-            ntile_all += (p->n() + kBlock - 1) / kBlock;
+            ntile += nt;
+            sample_set += p->samples().size();
+            bin_max += bin_parts(nt);
+            if (use_gather(*p))
+                group_max += p->ngroups(p->gather_bits());
         }
     // The tables only grow (the kernels get their lengths as arguments), so
     // a rebuild after the largest set so far allocates nothing.
@@ -397,8 +418,16 @@ void Engine::rebuild()
             buf.resize(std::max<size_t>(n, 1));
     };
     grow(d_insts_, ninst);
-    tiles.reserve(ntile_all);
-    qtiles.reserve(ntile_all);
+    // The tables go to the device from pinned memory.  The tiles' are written
+    // there at once (by way of vectors, 2M neurons' 1.1 MB made a rebuild
+    // 60-100 us longer); it holds every sample that is set, recorded or not,
+    // so a recording that follows takes no pinned memory (dtb_run_noalloc).
+    TileDesc *tiles = reinterpret_cast<TileDesc *>(
+        tables_stage_.reserve(ntile * (sizeof(TileDesc) + sizeof(QueueTile)) + ninst * (sizeof(InstDev) + sizeof(SampleRecDev)) +
+                              sizeof(QueueSet) + group_max * sizeof(GroupDesc) + bin_max * sizeof(BinDesc) +
+                              sample_set * sizeof(SampleDev)));
+    QueueTile *qtiles = reinterpret_cast<QueueTile *>(tiles + ntile);
+    size_t tile = 0;   // written so far
     std::vector<GroupDesc> groups;
     std::vector<SampleDev> samples;
     std::vector<SampleRecDev> recs;
@@ -417,13 +446,13 @@ void Engine::rebuild()
         if (!p)
             continue;
         const uint32_t idx = (uint32_t)table.size();
-        tile_base_[slot] = (uint32_t)tiles.size();
+        tile_base_[slot] = (uint32_t)tile;
         stat_ = stat_ || p->stat_mask() != 0;
         fmt = fmt == kWeightAny + 1 || fmt == p->weight_format() ? p->weight_format() : kWeightAny;
         uint64_t qtotal = 0;   // this instance's queue slots per parity
         for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
             const uint32_t cap = queue_capacity(p->tile_synapses(t));
-            qtiles.push_back(QueueTile{qtotal, cap, 0u});
+            qtiles[tile + t] = QueueTile{qtotal, cap, 0u};
             qtotal += cap;
         }
         // Each instance owns its queues (both parities and the read-ahead
@@ -457,8 +486,10 @@ void Engine::rebuild()
         for (uint32_t b = 0, t = 0; b < p->n(); b += kBlock, ++t) {
             while (pb[q + 1] <= b)
                 ++q;
-            const QueueTile &qt = qtiles[tile_base_[slot] + t];
-            tiles.push_back(p->tile_desc(t, table.back(), d_insts_.gpu_data() + idx, idx, q, qt.off, qt.cap));
+            const QueueTile &qt = qtiles[tile];
+            tiles[dir ? dealt(tile, ntile) : tile] =
+                p->tile_desc(t, table.back(), d_insts_.gpu_data() + idx, idx, q, qt.off, qt.cap);
+            ++tile;
         }
         recs.push_back(p->sample_rec());
         if (recs.back().nsample > 0) {
@@ -472,41 +503,25 @@ void Engine::rebuild()
             if (passes) {
                 const uint32_t nt = (p->n() + kBlock - 1) / kBlock;
                 bin_tiles_ = std::max(bin_tiles_, nt);
-                const uint32_t parts = std::min(kBinGroups, (nt + kBinTiles - 1) / kBinTiles);
+                const uint32_t parts = bin_parts(nt);
                 for (uint32_t k = 0; k < parts; ++k)
                     bins.push_back(BinDesc{d_insts_.gpu_data() + idx, k, parts});
             }
         }
     }
-    if (total > 0xffffffffull || tiles.size() > 0xffffffffull)
+    if (total > 0xffffffffull || ntile > 0xffffffffull)
         throw Error(kInvalidParameter, "too many neurons in one engine");
-    // Workgroups are dealt to the 8 XCDs by index mod 8: each XCD gets a
-    // contiguous range of the direct tiles, so tiles that share cache lines
-    // of a row's offsets and synapses meet in one L2.
-    if (dir) {
-        const size_t nd = tiles.size();
-        std::vector<TileDesc> dealt(nd);
-        for (size_t k = 0; k < nd; ++k) {
-            const size_t x = k & 7u;
-            dealt[k] = tiles[x * (nd >> 3) + std::min<size_t>(x, nd & 7u) + (k >> 3)];
-        }
-        tiles.swap(dealt);
-    }
     ninst_ = (uint32_t)table.size();
     wfmt_ = fmt > kWeightAny ? kWeightF32 : fmt;
-    ntiles_ = (uint32_t)tiles.size();
+    ntiles_ = (uint32_t)ntile;
     ngroups_ = (uint32_t)groups.size();
     nsamples_ = (uint32_t)samples.size();
     grow(d_groups_, groups.size());
-    grow(d_tiles_, tiles.size());
-    grow(d_qtiles_, qtiles.size());
+    grow(d_tiles_, ntile);
+    grow(d_qtiles_, ntile);
     // sized by the samples set, recorded or not: a recording run then finds
     // the table built
-    size_t sample_set = 0;
-    for (auto &p : insts_)
-        if (p)
-            sample_set += p->samples().size();
-    grow(d_samples_, std::max(samples.size(), sample_set));
+    grow(d_samples_, sample_set);
     grow(d_recs_, recs.size());
     // Auto: dense, unless rows reach most of their instance's tiles (the
     // reservations of many waves then meet on the same lines).  Measured with
@@ -519,7 +534,7 @@ void Engine::rebuild()
         cshift_ = kCountShiftSpread;
     else
         cshift_ = (total > 0 && coverage / (double)total > kSpreadCoverage) ? kCountShiftSpread : kCountShiftDense;
-    grow(d_qcnt_, count_words(2 * std::max<size_t>(tiles.size(), 1), cshift_));
+    grow(d_qcnt_, count_words(2 * std::max<size_t>(ntile, 1), cshift_));
     nbins_ = (uint32_t)bins.size();
     mode_ = dir && ntiles_ > 0 ? StepMode::direct : nbins_ > 0 ? StepMode::bin_launch : StepMode::tile_bin;
     grow(d_bins_, bins.size());
@@ -530,34 +545,28 @@ void Engine::rebuild()
     d_samples_.mutable_gpu_data();
     d_recs_.mutable_gpu_data();
     d_groups_.mutable_gpu_data();
-    // All tables in one launch, from pinned memory: a copy call each and the
-    // wait for the last were 60 of a short call's 240 us.
+    // All tables in one launch: a copy call each and the wait for the last
+    // were 60 of a short call's 240 us.
     const std::vector<QueueSet> qset(1, queues());
-    size_t bytes = 0;
-    auto each_table = [&](auto &&f) {
-        f(d_insts_, table);
-        f(d_tiles_, tiles);
-        f(d_qtiles_, qtiles);
-        f(d_bins_, bins);
-        f(d_queues_, qset);
-        f(d_groups_, groups);
-        f(d_samples_, samples);
-        f(d_recs_, recs);
+    unsigned char *at = reinterpret_cast<unsigned char *>(qtiles + ntile);
+    auto put_table = [&](auto &buf, const auto *src, size_t n) {
+        static_assert(sizeof(src[0]) % 4 == 0, "tables are whole words");
+        if (n > 0)
+            put.push_back(CopyWords{buf.mutable_gpu_data(), src, n * sizeof(src[0]) / 4});
     };
-    each_table([&](auto &, const auto &v) { bytes += v.size() * sizeof(v[0]); });
-    // sized for every sample that is set, like d_samples_: a recording that
-    // follows takes no pinned memory (dtb_run_noalloc)
-    bytes += (std::max(sample_set, samples.size()) - samples.size()) * sizeof(samples[0]);
-    unsigned char *at = tables_stage_.reserve(std::max<size_t>(bytes, 1));
-    each_table([&](auto &buf, const auto &v) {
-        const size_t b = v.size() * sizeof(v[0]);
-        static_assert(sizeof(v[0]) % 4 == 0, "tables are whole words");
-        if (b == 0)
-            return;
-        std::memcpy(at, v.data(), b);
-        put.push_back(CopyWords{buf.mutable_gpu_data(), at, b / 4});
-        at += b;
-    });
+    auto stage_table = [&](auto &buf, const auto &v) {
+        std::memcpy(at, v.data(), v.size() * sizeof(v[0]));
+        put_table(buf, reinterpret_cast<decltype(v.data())>(at), v.size());
+        at += v.size() * sizeof(v[0]);
+    };
+    put_table(d_tiles_, tiles, ntile);
+    put_table(d_qtiles_, qtiles, ntile);
+    stage_table(d_insts_, table);
+    stage_table(d_bins_, bins);
+    stage_table(d_queues_, qset);
+    stage_table(d_groups_, groups);
+    stage_table(d_samples_, samples);
+    stage_table(d_recs_, recs);
     put.push_back(CopyWords{d_qcnt_.mutable_gpu_data(), nullptr, d_qcnt_.size() / 4});
     DTB_HIP(launch_copy_words(put.data(), (int)put.size(), stream_));
     GraphKey key{};
