@@ -51,6 +51,15 @@ dtb::Engine &engine(dtb_engine_t h)
     return *h->eng;
 }
 
+// The engine with its device current: for calls that allocate or launch (a
+// caller's thread may have another device current).
+dtb::Engine &engine_here(dtb_engine_t h)
+{
+    dtb::Engine &e = engine(h);
+    DTB_HIP(hipSetDevice(e.device()));
+    return e;
+}
+
 void need(bool ok, const char *what)
 {
     if (!ok)
@@ -199,7 +208,7 @@ int dtb_set_ou(dtb_engine_t h, int inst, const uint32_t *brain_ids, const float 
     return guarded([&] {
         need(n >= 0, "negative count");
         need(n == 0 || (brain_ids && mean && deviation && correlation_time), "OU arrays are required");
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle_for(inst);
         e.get(inst)->set_ou(brain_ids, mean, deviation, correlation_time, (size_t)n, e.stream_for(inst));
@@ -222,7 +231,7 @@ int dtb_update_props(dtb_engine_t h, int inst, const uint32_t *neuron_ids, const
 {
     return guarded([&] {
         need(n >= 0 && (n == 0 || (neuron_ids && prop_ids && vals)), "property arrays are required");
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle_for(inst);
         e.get(inst)->update_props(neuron_ids, prop_ids, vals, (size_t)n, e.stream_for(inst));
@@ -235,7 +244,7 @@ int dtb_update_prop_cols(dtb_engine_t h, int inst, const uint32_t *prop_ids, con
 {
     return guarded([&] {
         need(n >= 0 && (n == 0 || (prop_ids && brain_ids && vals)), "property arrays are required");
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle_for(inst);
         e.get(inst)->update_prop_cols(prop_ids, brain_ids, vals, (size_t)n, assign != 0, e.stream_for(inst));
@@ -491,7 +500,7 @@ int dtb_engine_run(dtb_engine_t h, int64_t steps, int32_t graph_chunk)
 int dtb_configure(dtb_engine_t h, int inst, int32_t t_steps, int32_t use_ou)
 {
     return guarded([&] {
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle_for(inst);
         if (e.get(inst)->configure_run(t_steps, use_ou != 0, e.stream_for(inst)))
@@ -689,7 +698,7 @@ int dtb_read_state(dtb_engine_t h, int inst, float *v, int32_t *t_ref_count, uin
                    float *i_ou, float *j, float *i_syn)
 {
     return guarded([&] {
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle();   // the pending delta of the last step is folded into J
         e.get(inst)->read_state(e.call_stage(), v, t_ref_count, f, emitted, i_ou, j, i_syn, e.stream());
@@ -700,7 +709,7 @@ int dtb_write_state(dtb_engine_t h, int inst, const float *v, const int32_t *t_r
                     const float *i_ou, const float *j)
 {
     return guarded([&] {
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle();
         e.get(inst)->write_state(e.call_stage(), v, t_ref_count, f, i_ou, j, e.stream());
@@ -772,7 +781,7 @@ int dtb_gamma_prop_cols(dtb_engine_t h, int inst, const uint32_t *prop_ids, cons
 {
     return guarded([&] {
         need(n >= 0 && (n == 0 || (prop_ids && brain_ids && concentration && rate)), "gamma arrays are required");
-        dtb::Engine &e = engine(h);
+        dtb::Engine &e = engine_here(h);
         e.get(inst);
         e.settle_for(inst);
         e.get(inst)->gamma_prop_cols(prop_ids, brain_ids, concentration, rate, (size_t)n, e.stream_for(inst));
