@@ -225,6 +225,7 @@ Instance::Instance(const FanoutSpec &f, float dt, uint64_t seed, hipStream_t s)
     // expected distinct tiles (groups) among K uniform targets, as a fraction
     row_coverage_ = 1.0 - std::pow(1.0 - 1.0 / ntile, (double)f.K);
     group_coverage_ = 1.0 - std::pow(1.0 - 1.0 / ngroups(), (double)f.K);
+    shared_segments_ = row_coverage_ * row_coverage_ * (double)ntile * (double)n_;
     // rows are ordered by target, K <= 8192
     gather_ok_ = (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
     src_pass_.assign(ntile, 0u);
@@ -295,7 +296,32 @@ void Instance::count_tile_synapses(const NetworkHost &net)
     group_coverage_ = (double)gs / ((double)n_ * (double)ngroups());
     gather_ok_ = ordered && nsyn_ > 0 && (double)n_ * (ngroups() + 1.0) * 2.0 <= 12.0 * (double)nsyn_;
     choose_groups(by_tile);
+    sample_sharing(net);
     direct_ok_ = by_tile && direct_fits();
+}
+
+void Instance::sample_sharing(const NetworkHost &net)
+{
+    const uint32_t ntile = (n_ + kBlock - 1) / kBlock;
+    const uint32_t rows = std::min(n_, kSharingRows);
+    std::vector<uint32_t> mark(ntile, 0u);   // 2 k + 1: reached by the k-th sampled row, 2 k + 2: and counted
+    uint64_t shared = 0, seen = 0;
+    uint32_t k = 0;
+    for (; k < rows && seen < ((uint64_t)1 << 20); ++k) {   // (rows of tens of thousands: fewer of them)
+        const uint32_t r = (uint32_t)((uint64_t)n_ * k / rows);
+        const uint32_t s = (uint32_t)(((uint64_t)r + kSharingDistance) % n_);
+        for (int64_t j = net.rowptr[r]; j < net.rowptr[r + 1]; ++j)
+            mark[(net.col[j] & kColMask) >> kTileBits] = 2u * k + 1u;
+        for (int64_t j = net.rowptr[s]; j < net.rowptr[s + 1]; ++j) {
+            uint32_t &m = mark[(net.col[j] & kColMask) >> kTileBits];
+            if (m == 2u * k + 1u) {
+                ++m;
+                ++shared;
+            }
+        }
+        seen += (uint64_t)(net.rowptr[r + 1] - net.rowptr[r]) + (uint64_t)(net.rowptr[s + 1] - net.rowptr[s]);
+    }
+    shared_segments_ = k > 0 ? (double)shared / k * n_ : 0.0;
 }
 
 void Instance::choose_groups(bool by_tile)

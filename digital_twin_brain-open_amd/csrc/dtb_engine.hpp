@@ -396,6 +396,9 @@ public:
     // Mean over rows of the fraction of this instance's tiles that the row's
     // synapses reach (tile segments of the row / tiles).
     double row_coverage() const { return row_coverage_; }
+    // (Row, tile) pairs of all rows that the row kSharingDistance neurons on
+    // reaches too, estimated from kSharingRows rows.
+    double shared_segments() const { return shared_segments_; }
 
     // Gather propagation (k_gather): possible when every row is ordered by
     // target group, no row is longer than kGatherMaxRow and the group offsets
@@ -515,6 +518,8 @@ private:
     RecordBuffers rec_ext_{};
     std::vector<uint32_t> tile_syn_;      // synapses per target tile
     double row_coverage_ = 0.0;           // mean fraction of the tiles one row reaches
+    double shared_segments_ = 0.0;        // shared_segments()
+    void sample_sharing(const NetworkHost &net);
     double group_coverage_ = 0.0;         // mean fraction of the gather groups one row reaches
     bool gather_ok_ = false;              // gather_allowed()
     uint32_t gather_bits_ = kGroupBits;   // gather_bits()

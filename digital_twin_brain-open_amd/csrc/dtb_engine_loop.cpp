@@ -165,7 +165,7 @@ bool Engine::want_direct()
 bool Engine::want_bin_launch()
 {
     uint64_t tiles = 0;
-    double segments = 0.0, synapses = 0.0;   // tile segments of all rows, and their synapses
+    double segments = 0.0, synapses = 0.0, shared = 0.0;   // tile segments of all rows, their synapses, shared ones
     auto queued = [&](size_t i) { return insts_[i] && !use_gather(*insts_[i]); };
     for (size_t i = 0; i < insts_.size(); ++i)
         if (queued(i)) {
@@ -173,8 +173,10 @@ bool Engine::want_bin_launch()
             tiles += (uint64_t)t;
             segments += insts_[i]->row_coverage() * t * insts_[i]->n();
             synapses += (double)insts_[i]->nsyn();
+            shared += insts_[i]->shared_segments();
         }
-    const bool want = !passes_short_ && tiles > 0 && (split_ || (tuned_ != Tuned::named && tiles >= kBinLaunchTiles && 2.0 * segments <= synapses));
+    const bool rules = tiles >= kBinLaunchTiles && 2.0 * segments <= synapses && shared >= kBinLaunchShared;
+    const bool want = !passes_short_ && tiles > 0 && (split_ || (rules && tuned_ != Tuned::named));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;

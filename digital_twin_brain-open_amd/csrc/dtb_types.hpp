@@ -384,6 +384,16 @@ constexpr uint32_t kBinTiles = 16, kBinGroups = 512;
 // reach the same tiles): with uniformly drawn targets there is little to add
 // up first, 900k x 300 35.9 / 44.0, 2M x 300 53.8 / 63.2.
 constexpr uint32_t kBinLaunchTiles = 3072u;
+// And only where the rows that fire in one step share tiles: the (row, tile)
+// pairs of all rows that a row 512 neurons on reaches too (about the distance
+// of two rows at 20 spikes per second).  Voxels of 10k neurons have 4.5e7 and
+// more from 800k neurons and 150 synapses on; of 200 neurons they have none,
+// and steps in the tiles / by k_bin are 1M x 60 21.6 / 27.0 us, 1M x 200 24.3 /
+// 29.6, 800k x 100 19.1 / 25.4, 2M x 200 41.9 / 44.9; of 1000 neurons 1M x 200
+// (1.2e7) 23.6 / 27.5, of 2500 (2.5e7) 23.3 / 26.1, of 1500 2M x 300 (4.2e7)
+// 40.9 / 40.9, at 16 spikes per second 47.8 / 45.9.
+constexpr double kBinLaunchShared = 3.5e7;
+constexpr uint32_t kSharingDistance = 512, kSharingRows = 256;
 struct alignas(16) BinDesc {
     const InstDev *inst;
     uint32_t part, parts;   // takes part `part` of `parts` of the step's passes

@@ -378,8 +378,8 @@ class Engine:
         binned by a second launch per step, in equal shares over the whole
         GPU, instead of by the tiles whose neurons fired (off: only in engines
         of 786,432 neurons or more whose rows have two synapses per tile they
-        reach; capacity has no effect).
-        Same results either way."""
+        reach and share these tiles with rows some hundred neurons away;
+        capacity has no effect).  Same results either way."""
         if on is not None:
             _lib.check(self._lib.dtb_engine_split(self._h, c_int32(int(bool(on))), ctypes.c_uint32(int(capacity))))
         o, c = c_int32(0), ctypes.c_uint32(0)

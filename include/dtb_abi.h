@@ -264,8 +264,10 @@ int dtb_engine_pull(dtb_engine_t h, int32_t on, uint32_t defer_min);
  * 122-225, scheduled differently): on = the fired rows are binned by a second
  * launch per step, in equal shares over the whole GPU, instead of by the tiles
  * whose neurons fired; off = only in engines of 786,432 neurons or more whose
- * rows have two synapses per tile they reach.  capacity is kept and reported, and has no effect (the
- * list holds every row).  Results never depend on either. */
+ * rows have two synapses per tile they reach and share these tiles with rows
+ * some hundred neurons away (voxels of thousands of neurons).  capacity is
+ * kept and reported, and has no effect (the list holds every row).  Results
+ * never depend on either. */
 int dtb_engine_split(dtb_engine_t h, int32_t on, uint32_t capacity);
 int dtb_engine_get_split(dtb_engine_t h, int32_t *on, uint32_t *capacity);
 int dtb_engine_get_pull(dtb_engine_t h, int32_t *on, uint32_t *defer_min);

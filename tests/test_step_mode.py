@@ -120,12 +120,18 @@ def test_direct_rows_in_rounds(dtb, orc, gpu, rate):
 
 
 @pytest.mark.parametrize("kind,n,mode", [("voxel", 3071 * 256, "tile_bin"), ("voxel", 3071 * 256 + 1, "bin_launch"),
-                                         ("uniform", 3071 * 256 + 1, "tile_bin")])
+                                         ("uniform", 3071 * 256 + 1, "tile_bin"),
+                                         ("small voxels", 3072 * 256, "tile_bin")])
 def test_binning_launch_by_tiles_and_sharing(dtb, orc, gpu, kind, n, mode):
     """From 3072 tiles, and only where rows have two synapses per tile they
-    reach."""
-    net = dtb.gen_voxel(n, 78, 220, seed=6) if kind == "voxel" else dtb.gen_uniform(n, 12, seed=5)
-    steps, mu = (24, 9.0) if kind == "voxel" else (40, 6.0)
+    reach (uniform ones have one) and share these with the rows that fire
+    beside them (voxels of 196 neurons share none)."""
+    net = dtb.gen_uniform(n, 12, seed=5) if kind == "uniform" else \
+        dtb.gen_voxel(n, 78 if kind == "voxel" else 4000, 220 if kind == "voxel" else 100, seed=6)
+    rows = np.random.default_rng(1).integers(0, n, 300)
+    seg = np.mean([len(np.unique(net.col[net.rowptr[r]:net.rowptr[r + 1]] >> 8)) for r in rows])
+    assert (2.0 * seg <= net.nsyn / n) == (kind != "uniform")
+    steps, mu = (40, 6.0) if kind == "uniform" else (24, 9.0)
     eng = dtb.Engine(0)
     try:
         b = add(dtb, eng, net, 40, mu)
