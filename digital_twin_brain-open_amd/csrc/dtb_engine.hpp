@@ -429,6 +429,8 @@ public:
     bool pull_allowed() const { return n_ <= kPullMaxNeurons && nsyn_ > 0; }
     // Device bytes ensure_pull allocates.
     uint64_t pull_bytes() const;
+    uint64_t direct_bytes() const { return (uint64_t)n_ * ((n_ + kBlock - 1) / kBlock + 1u) * sizeof(uint16_t); }
+    uint64_t pass_bytes() const { return (uint64_t)kFiredLists * passcap_ * sizeof(unsigned long long); }
     void ensure_pull(hipStream_t s);
     void release_pull();
     bool pull_built() const { return pull_built_; }
@@ -745,12 +747,30 @@ private:
     bool want_direct();                    // direct_by_rules(), and builds what it needs
     // Offsets or pass lists did not fit: not tried again (each table build
     // would build and return those that do fit) before the instances or the
-    // propagation settings change.
-    bool direct_short_ = false, passes_short_ = false;
+    // propagation settings change, or as much memory as was missing is given
+    // back to the library.
+    struct Short {
+        bool on = false, base_set = false;
+        size_t need = 0, base = 0;
+
+        void failed(size_t bytes) { *this = Short{true, false, bytes, 0}; }
+        // Whether it still holds, at a table build with `cached` bytes free in
+        // the library (the first one after the failure sets the base).
+        bool holds(size_t cached)
+        {
+            if (on && !base_set) {
+                base_set = true;
+                base = cached;
+            }
+            on = on && cached < base + need;
+            return on;
+        }
+    };
+    Short direct_short_, passes_short_;
     void routes_changed()
     {
         dirty_ = true;
-        direct_short_ = passes_short_ = false;
+        direct_short_.on = passes_short_.on = false;
     }
     StepMode mode_ = StepMode::tile_bin;   // of every tile in the tables
     // A schedule of the autotuner's: its (dense, default pass) candidate

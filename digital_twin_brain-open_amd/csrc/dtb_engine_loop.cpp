@@ -143,7 +143,7 @@ bool Engine::direct_by_rules(const Instance *joining) const
 
 bool Engine::want_direct()
 {
-    if (direct_short_ || !direct_by_rules())
+    if (!direct_by_rules() || direct_short_.holds(devmem::cached_bytes(device_)))
         return false;
     // an engine holds offsets or pass lists, not both (the old tables,
     // settled by the caller, were the last to use the lists)
@@ -155,7 +155,8 @@ bool Engine::want_direct()
             continue;
         try_pull(*p, stream_);
         if (!p->pull_built() || !try_direct(*p, stream_)) {
-            direct_short_ = !devmem::NoAlloc::active();
+            if (!devmem::NoAlloc::active())
+                direct_short_.failed(p->pull_built() ? p->direct_bytes() : p->pull_bytes());
             return false;
         }
     }
@@ -176,7 +177,8 @@ bool Engine::want_bin_launch()
             shared += insts_[i]->shared_segments();
         }
     const bool rules = tiles >= kBinLaunchTiles && 2.0 * segments <= synapses && shared >= kBinLaunchShared;
-    const bool want = !passes_short_ && tiles > 0 && (split_ || (rules && tuned_ != Tuned::named));
+    const bool want = tiles > 0 && (split_ || (rules && tuned_ != Tuned::named)) &&
+                      !passes_short_.holds(devmem::cached_bytes(device_));
     for (size_t i = 0; i < insts_.size() && want; ++i) {
         if (!queued(i) || insts_[i]->passes_built())
             continue;
@@ -193,7 +195,7 @@ bool Engine::want_bin_launch()
             for (auto &p : insts_)
                 if (p)
                     p->release_passes();
-            passes_short_ = true;
+            passes_short_.failed(insts_[i]->pass_bytes());
             return false;
         }
     }

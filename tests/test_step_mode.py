@@ -277,3 +277,50 @@ def test_autotuner_compares_the_binning_launch_with_binning_in_tiles(dtb, orc, g
         assert b.counters()[0] == steps + 2
     finally:
         eng.close()
+
+
+def test_offsets_are_tried_again_when_memory_is_free(dtb, gpu):
+    """The offsets of 313 MB do not fit beside another engine's instance; once
+    that is gone, the next run steps directly."""
+    def big(eng):
+        b = dtb.Block(None, delta_t=DT, engine=eng, inst=eng.add_fanout(200_000, 150, 5))
+        b.run(3, freqs=True)
+        return b
+
+    def guest(eng):
+        eng.schedule(layout="dense")
+        eng.add_fanout(100_000, 150, 6)
+        eng.run(1)
+
+    used = []
+    for what in (guest, lambda e: (e.schedule(layout="dense"), big(e))):
+        dtb.device_memory_trim()
+        dtb.device_memory_reserve(4 << 30)
+        eng = dtb.Engine(0)
+        try:
+            free = dtb.device_memory_cached(0)
+            what(eng)
+            used.append(free - dtb.device_memory_cached(0))
+        finally:
+            eng.close()
+    dtb.device_memory_trim()
+    dtb.device_memory_reserve(sum(used) + (64 << 20))
+    other, eng = dtb.Engine(0), dtb.Engine(0)
+    try:
+        # the guest last, so that its range and the free one beside it are one
+        eng.schedule(layout="dense")
+        b = big(eng)
+        guest(other)
+        eng.schedule(layout="auto")
+        for _ in range(3):
+            b.run(3, freqs=True)
+            assert eng.step_info()["mode"] == "tile_bin"
+        other.close()
+        other = None
+        b.run(3, freqs=True)
+        assert eng.step_info()["mode"] == "direct"
+    finally:
+        if other:
+            other.close()
+        eng.close()
+        dtb.device_memory_trim()
