@@ -393,7 +393,7 @@ constexpr uint32_t kBinLaunchTiles = 3072u;
 // (1.2e7) 23.6 / 27.5, of 2500 (2.5e7) 23.3 / 26.1, of 1500 2M x 300 (4.2e7)
 // 40.9 / 40.9, at 16 spikes per second 47.8 / 45.9.
 constexpr double kBinLaunchShared = 3.5e7;
-constexpr uint32_t kSharingDistance = 512, kSharingRows = 256;
+constexpr uint32_t kSharingDistance = 512, kSharingRows = 64;
 struct alignas(16) BinDesc {
     const InstDev *inst;
     uint32_t part, parts;   // takes part `part` of `parts` of the step's passes
